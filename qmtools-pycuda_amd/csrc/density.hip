@@ -163,7 +163,7 @@ __device__ __forceinline__ void phi_f64_body(int blk, const MolView& m, const Ge
         if (e < kExpCut) radial += pc.y * exp(-e);   // beyond: below 2e-22 of the coefficient
       }
     }
-    double* __restrict__ col = phi + (int64_t)sh.bf * ld + t;
+    double* __restrict__ col = phi + (int64_t)(pts ? sh.bf_user : sh.bf) * ld + t;   // point lists: caller's order
     shell_emit<double>(sh.L, dx, dy, dz, radial, [&](int c, double val) { col[(int64_t)c * ld] = val; });
   }
   for (int f = m.nbf; f < nbf_pad; ++f) phi[(int64_t)f * ld + t] = 0.0;
@@ -627,7 +627,10 @@ __device__ __forceinline__ bool tile_coords(int b, int nrt, int ncb, int& rt, in
   const int xcd = b & 7, slot = b >> 3;
   const int rl = slot / ncb;
   cb = ncb - 1 - (slot - rl * ncb);
-  rt = rl * 8 + xcd;
+  // row tile 8 rl + xcd, turned by a hash of rl within its group of 8: with tiles per grid row a multiple of
+  // 8, a fixed xcd would own fixed x ranges of the grid, and the one through the molecule's middle would
+  // finish last (the CUs were busy 64-81% of the launch)
+  rt = rl * 8 + ((xcd + (int)((unsigned)rl * 2654435761u >> 29)) & 7);
   return rt < nrt;
 }
 
@@ -645,15 +648,41 @@ __device__ __forceinline__ void lds_dma16(const void* gsrc, const void* lds_wave
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(l), "v"(gsrc) : "memory");
 }
 
+// A wave-uniform value or address that the compiler holds in vector registers (a field of a table in
+// memory), moved to scalar ones.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+template <typename T>
+__device__ __forceinline__ const T* uniform(const T* p) {
+  const uint64_t a = (uint64_t)(uintptr_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  return (const T*)(uintptr_t)((uint64_t)hi << 32 | lo);
+}
+
+// Element i of a table that no kernel of this launch writes, i and p wave uniform: read through the constant
+// address space, so that it becomes a scalar load.  (The stores of the kernel might alias a plain pointer for
+// all that the compiler knows, which makes every table read a vector load.)
+template <typename V, typename T>
+__device__ __forceinline__ V table(const T* p, int64_t i) {
+  typedef const V __attribute__((address_space(4))) CV;
+  return *(CV*)(uintptr_t)(p + i);
+}
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ DevShell table_shell(const DevShell* p, int i) {
+  static_assert(sizeof(DevShell) == 32, "two 16-byte words");
+  const v4i a = table<v4i>((const v4i*)(p + i), 0), b = table<v4i>((const v4i*)(p + i), 1);
+  const int cut = b.y;   // a value: bit_cast of the vector element itself takes element 0
+  return DevShell{a.x, a.y, a.z, a.w, b.x, __builtin_bit_cast(float, cut), b.z, b.w};
+}
+
 // saddr form of lds_dma16: wave-uniform 64-bit base (SGPRs) plus a 32-bit byte offset per lane;
 // lds_addr is the wave's LDS byte address (M0).
 __device__ __forceinline__ void lds_dma16_s(const void* sbase, unsigned voff, unsigned lds_addr) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
 }
-
-// k per stage of the DMA-fed FP64 tiles (ring of 32 / kF64Ks stages).  Stages of 8 k in a ring
-// of 4 (one more stage of lookahead, twice the barriers) measured 4% slower than 16 k in a ring of 2.
-constexpr int kF64Ks = 16;
 
 // Row-dot of the transposed FP64 tiles (M was the first MFMA operand): lane
 // (li, lk) register q of tile (r, c) is X[t = li][n = lk + 4 q]; 16 lanes read 16
@@ -747,162 +776,345 @@ __device__ __forceinline__ void tiled_f64_body(int rt, int cb, const double* __r
   if (t < kTT) part[(int64_t)cb * ldp + row0 + t] = red[0][t] + red[1][t];
 }
 
-// Tiled FP64 contraction fed by LDS DMA (variant 4): the 128 x 128 workgroup
-// tiles and per-tile MFMA order of tiled_f64_body, with waves of 16 rows x all
-// 128 columns (so that every wave skips the same tiles of the triangle and the
-// diagonal stages have compile-time tiles, with no runtime tile selection and no
-// cross-wave row-dot reduction); both operands go global -> LDS by
-// global_load_lds_dwordx4 (lane i of a wave brings points / columns 2i, 2i+1 of
-// one k row, so a wave fills one padded LDS row) into a two-stage ring, issued
-// right after the barrier that opens the previous stage.  The loads come from
-// inline assembly (lds_dma16), the wait before each barrier is explicit.
-// KS k per stage in a ring of NB stages (NB KS = 32: the same 72 KB of LDS); stage st + NB - 1 is
-// requested right after the barrier that opens stage st.  The row-dot is summed in the K loop from
-// the LDS copy of the basis values of each diagonal stage (below), not re-read from global memory.
-template <int KS, int NB>
-__device__ __forceinline__ void tiled_f64_dma_body(int rt, int cb, const double* __restrict__ phi, int ld,
-                                                   const double* __restrict__ M, int np, int nbf, int ncb,
-                                                   double* __restrict__ part, int ldp,
-                                                   const uint32_t* __restrict__ amask = nullptr, int nw = 0) {
-  static_assert(KS % 4 == 0 && (2 * KS) % 8 == 0, "stages of whole MFMA k-steps, rows split over 8 waves");
-  static_assert(KS == 16, "the diagonal stages below are the block's 8 tiles of 16 columns");
-  constexpr int RPW = 2 * KS / 8;   // rows of one operand fetched per wave and stage
-  __shared__ __align__(16) double ring[NB][2][KS][kTT + kTPad];
+// ---------------------------------------------------------------------------
+// Block tiles (the default contractions).  A row tile is a compact block of 8 x 4 x 4 voxels
+// (128 points) instead of 128 consecutive points of an x line: seen from a nucleus it spans a third of
+// the distance, so fewer basis functions reach into it.  k_tile_list lists the tile's active groups of
+// consecutive functions (16 in FP64, 32 in the split path), i.e. those with a shell whose cutoff reaches the tile's bounding box;
+// everything after it works on that list alone: the basis-value kernel evaluates and stores only the
+// listed groups, packed, and the contraction runs the triangle of the listed groups as if they were the
+// whole basis.  What is left out are exact zeros (the basis-value kernels write 0 beyond a shell's
+// cutoff), so the sums are the same bit for bit with every group listed (QM_TUNE_TILE_SKIP = 0).
+// On 60 atoms in a 28 bohr box 45% of the FP64 groups (52% of the split ones) are active and 26% (33%) of the
+// triangle is left.  60 atoms at 256^3, density call: FP64 110 -> 43 ms, split 25.3 -> 16.7 ms.
+constexpr int kBTX = 8, kBTY = 4, kBTZ = 4;
+static_assert(kBTX * kBTY * kBTZ == kTT, "a block tile is one row tile");
+constexpr int kMaxGroups = 2048;   // groups per tile that a workgroup can list in LDS
+
+struct BlockTiles {
+  int T0, nT;             // tiles T0 .. T0 + nT - 1 of the grid (x fastest)
+  int nsub;               // row tile rt = s nT + (T - T0) holds sub-point s of tile T's voxels
+  int ng;                 // groups of the whole basis: stride of a tile's list, values and partial sums
+  const uint16_t* list;   // [row tile][ng]: active groups in increasing order
+  const int* cnt;         // [row tile]: how many
+};
+
+__host__ __device__ inline int64_t block_tiles(const GeomView& g) {
+  return (int64_t)((g.nx + kBTX - 1) / kBTX) * ((g.ny + kBTY - 1) / kBTY) * ((g.nz + kBTZ - 1) / kBTZ);
+}
+
+__device__ __forceinline__ void block_origin(const GeomView& g, int T, int& i0, int& j0, int& k0) {
+  const int ntx = (g.nx + kBTX - 1) / kBTX, nty = (g.ny + kBTY - 1) / kBTY;
+  const int q = T / ntx;
+  i0 = (T - q * ntx) * kBTX;
+  k0 = q / nty * kBTZ;
+  j0 = (q - q / nty * nty) * kBTY;
+}
+
+// Position of point p of row tile rt (same arithmetic as chunk_point); points of an edge tile beyond the
+// grid repeat its last plane, row or column and are not stored.
+__device__ __forceinline__ void block_point(const GeomView& g, const BlockTiles& b, int rt, int p, double& x, double& y,
+                                            double& z) {
+  const int s = rt / b.nT;
+  int i0, j0, k0;
+  block_origin(g, b.T0 + (rt - s * b.nT), i0, j0, k0);
+  const int i = min(i0 + (p & 7), g.nx - 1), j = min(j0 + ((p >> 3) & 3), g.ny - 1), k = min(k0 + (p >> 5), g.nz - 1);
+  const int sx = s % b.nsub, sy = (s / b.nsub) % b.nsub, sz = s / (b.nsub * b.nsub);
+  const double inv = 1.0 / b.nsub;
+  x = g.ox + ((double)i + (sx + 0.5) * inv) * g.h;
+  y = g.oy + ((double)j + (sy + 0.5) * inv) * g.h;
+  z = g.oz + ((double)k + (sz + 0.5) * inv) * g.h;
+}
+
+// The list of row tile rt (one workgroup of 128 threads).  Conservative: a shell is tested against the
+// tile's bounding box with a relative margin of 1e-6 on the squared cutoff.
+template <int GS>   // log2 of the functions per group
+__device__ __forceinline__ void tile_list_body(const MolView& m, const GeomView& g, const BlockTiles& b, int rt,
+                                               int all, uint16_t* __restrict__ list, int* __restrict__ cnt) {
+  __shared__ uint32_t words[kMaxGroups / 32];
+  double lo[3], hi[3];
+  block_point(g, b, rt, 0, lo[0], lo[1], lo[2]);
+  block_point(g, b, rt, kTT - 1, hi[0], hi[1], hi[2]);
+  for (int w = threadIdx.x; w < kMaxGroups / 32; w += kTT)
+    words[w] = !all || 32 * w >= b.ng ? 0u : b.ng - 32 * w >= 32 ? 0xffffffffu : (1u << (b.ng - 32 * w)) - 1u;
+  __syncthreads();
+  if (!all)
+    for (int sidx = threadIdx.x; sidx < m.nshell; sidx += kTT) {
+      const DevShell sh = m.shells[sidx];
+      const double4 a = m.atoms[sh.atom];
+      const double c[3] = {a.x, a.y, a.z};
+      double d2 = 0.0;
+      for (int d = 0; d < 3; ++d) {
+        const double e = fmax(0.0, fmax(lo[d] - c[d], c[d] - hi[d]));
+        d2 += e * e;
+      }
+      if (d2 <= (double)sh.rcut2 * (1.0 + 1e-6))
+        for (int q = sh.bf >> GS; q <= (sh.bf + 2 * sh.L) >> GS; ++q) atomicOr(&words[q >> 5], 1u << (q & 31));
+    }
+  __syncthreads();
+  if (threadIdx.x < 64) {   // wave 0: lane l lists the groups of word l
+    uint32_t w = words[threadIdx.x];
+    const int n = __popc(w);
+    int incl = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(incl, d, 64);
+      if ((int)threadIdx.x >= d) incl += v;
+    }
+    uint16_t* __restrict__ out = list + (int64_t)rt * b.ng + (incl - n);
+    for (; w; w &= w - 1) *out++ = (uint16_t)(32 * threadIdx.x + __builtin_ctz(w));
+    if (threadIdx.x == 63) cnt[rt] = incl;
+  }
+}
+
+template <int GS>
+__global__ __launch_bounds__(kTT) void k_tile_list(MolView m, GeomView g, BlockTiles b, int all,
+                                                   uint16_t* __restrict__ list, int* __restrict__ cnt) {
+  tile_list_body<GS>(m, g, b, blockIdx.x, all, list, cnt);
+}
+
+// Walks the listed groups of a row tile as runs of consecutive functions (wave uniform): run(j, fj, f0, f1)
+// for each run f0 .. f1 - 1, whose first function lies in the tile's j-th group, which starts at function fj.
+// Part y of ny takes an equal share of the list, in units of 8 functions.
+template <int GS, typename F>
+__device__ __forceinline__ void for_runs(const uint16_t* __restrict__ list, int cnt, int y, int ny, F&& run) {
+  constexpr int US = GS - 3;   // log2 of the units per group
+  auto entry = [&](int i) __attribute__((always_inline)) -> int {   // 16-bit entries by 4-byte scalar loads
+    const uintptr_t a = (uintptr_t)(list + i);
+    return table<uint32_t>((const uint32_t*)(a & ~(uintptr_t)3), 0) >> (8 * (a & 2)) & 0xffff;
+  };
+  const unsigned units = (unsigned)cnt << US;
+  const int last = (int)(units * (y + 1) / ny);
+  for (int u = (int)(units * y / ny); u < last;) {
+    const int j = u >> US, g0 = entry(j);
+    int e = j + 1;
+    while (e << US < last && entry(e) == g0 + (e - j)) ++e;
+    const int stop = min(e << US, last);
+    run(j, g0 << GS, (g0 << GS) + 8 * (u - (j << US)), (g0 << GS) + 8 * (stop - (j << US)));
+    u = stop;
+  }
+}
+
+// FP64 basis values of the listed groups: group j of row tile rt at phi + (rt ng + j) 2048, function-major
+// ([16][128]).  One thread per point; a shell that straddles two groups is evaluated once per run.
+__device__ __forceinline__ void phi_f64_blocks_body(const MolView& m, const int2* __restrict__ kg, const GeomView& g,
+                                                    const BlockTiles& b, int rt, int p, int part, int nparts,
+                                                    double* __restrict__ phi) {
+  const DevShell* shells = uniform(m.shells);
+  const double4* atoms = uniform(m.atoms);
+  const double2* prims = uniform(m.prims);
+  const int nshell = uniform(m.nshell), nbf = uniform(m.nbf);
+  kg = uniform(kg);
+  double x, y, z;
+  block_point(g, b, rt, p, x, y, z);
+  double* __restrict__ mine = phi + (int64_t)rt * b.ng * (16 * kTT) + p;
+  for_runs<4>(uniform(b.list) + (int64_t)rt * uniform(b.ng), table<int>(uniform(b.cnt), rt), part, nparts,
+              [&](int j, int fj, int f0, int f1) __attribute__((always_inline)) {
+    double* __restrict__ col = mine + ((int64_t)j * 16 - fj) * kTT;   // function f of the run at col[f kTT]
+    int atom = -1;
+    double dx = 0, dy = 0, dz = 0, r2 = 0;
+    for (int s = table<int>((const int*)(kg + (f0 >> 3)), 0); s < nshell; ++s) {
+      const DevShell sh = table_shell(shells, s);
+      if (sh.bf >= f1) break;
+      if (sh.atom != atom) {
+        atom = sh.atom;
+        const v4d a = table<v4d>((const v4d*)atoms, atom);
+        dx = x - a.x;
+        dy = y - a.y;
+        dz = z - a.z;
+        r2 = dx * dx + dy * dy + dz * dz;
+      }
+      double radial = 0.0;
+      if (r2 <= (double)sh.rcut2) {
+        for (int q = 0; q < sh.nprim; ++q) {
+          const v2d pc = table<v2d>((const v2d*)prims, sh.poff + q);
+          const double e = pc.x * r2;
+          if (e < kExpCut) radial += pc.y * exp(-e);   // beyond: below 2e-22 of the coefficient
+        }
+      }
+      double* __restrict__ at = col + (int64_t)sh.bf * kTT;
+      if (sh.bf >= f0 && sh.bf + 2 * sh.L < f1) {
+        shell_emit<double>(sh.L, dx, dy, dz, radial, [&](int c, double val) { at[c * kTT] = val; });
+      } else {
+        shell_emit<double>(sh.L, dx, dy, dz, radial, [&](int c, double val) {
+          if (sh.bf + c >= f0 && sh.bf + c < f1) at[c * kTT] = val;
+        });
+      }
+    }
+    for (int f = max(nbf, f0); f < f1; ++f) col[(int64_t)f * kTT] = 0.0;   // padding of the last group
+  });
+}
+
+constexpr int kPhiTiles = kPhiThreads / 64;   // row tiles per workgroup of the split basis-value launch
+
+__global__ __launch_bounds__(kPhiThreads) void k_phi_f64_blocks(MolView m, const int2* __restrict__ kg, GeomView g,
+                                                                BlockTiles b, int nrt, double* __restrict__ phi) {
+  const int rt = __builtin_amdgcn_readfirstlane(blockIdx.x * (kPhiThreads / kTT) + threadIdx.x / kTT);
+  if (rt < nrt) phi_f64_blocks_body(m, kg, g, b, rt, threadIdx.x % kTT, blockIdx.y, gridDim.y, phi);
+}
+
+// FP64 contraction of block tiles (variant 4), fed by LDS DMA: a workgroup of 8 waves owns one row tile
+// and takes its column blocks of 8 listed groups (128 columns) one after the other, the longest first; wave w
+// owns rows 16 w .. 16 w + 15 and all 8 column tiles, so every wave skips the same tiles of the triangle and the
+// diagonal stages have compile-time tiles.  Stages are the listed groups in order (16 k each).  Both operands
+// go global -> LDS by global_load_lds_dwordx4 (lane i of a wave brings points / columns 2i, 2i + 1 of one k row,
+// so a wave fills one padded LDS row) into a two-stage ring, issued right after the barrier that opens the
+// previous stage, across the end of a column block too; the packed basis values of a stage are 16 KB in one
+// piece, M's rows and columns are picked by the list.  Column blocks are right-aligned on the list: only the
+// last one (the cheapest) holds padding, as columns below group 0.  The loads come from inline assembly
+// (lds_dma16_s); the wait before each barrier is explicit.  The row-dot of a column tile is summed in the
+// stage that completes it, from the LDS copy of the basis values, and goes to part[tile][group][point]: one
+// partial sum per group, so that the sum over groups does not depend on which groups share a block.
+__device__ __forceinline__ void f64_block_tile(int rt, int y, int ny, const double* __restrict__ phi,
+                                               const double* __restrict__ M, int np, const BlockTiles& b,
+                                               double* __restrict__ part) {
+  constexpr int KS = 16, RPW = 2 * KS / 8;   // k per stage; rows of one operand fetched per wave and stage
+  __shared__ __align__(16) double ring[2][2][KS][kTT + kTPad];
+  __shared__ uint16_t seq[kMaxGroups];
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int li = lane & 15, lk = lane >> 4;
-  // Column blocks are right-aligned on ne = nbf rounded up to 16: block cb covers columns
-  // c0 .. c0 + 127 with c0 = 128 cb - shift, so only block 0 (the cheapest, k < c0 + 128) holds
-  // padding, as columns below 0; rows and columns of M from nbf on are zero and are not visited.
-  const int ne = (nbf + 15) / 16 * 16;
-  const int row0 = rt * kTT, c0 = cb * kTT - (ncb * kTT - ne);
-  const int jd = c0 / KS;   // c0 is a multiple of 16: stage jd + j is the block's diagonal stage j
+  rt = uniform(rt);
+  np = uniform(np);
+  const int ng = uniform(b.ng);
+  const int nact = uniform(b.cnt[rt]);
+  if (8 * y >= nact) return;
+  phi = uniform(phi);
+  M = uniform(M);
+  part = (double*)uniform(part) + (int64_t)rt * ng * kTT + 16 * wave + li;
+  for (int i = t; i < nact; i += kTWG) seq[i] = b.list[(int64_t)rt * ng + i];
+  __syncthreads();
   // wave w brings k rows RPW (w % 4) .. RPW (w % 4) + RPW - 1 of operand w / 4 (0: basis values, 1: M)
   const int op = wave >> 2, k0 = RPW * (wave & 3);
-  const double* src = op == 0 ? phi + row0 + 2 * lane : M + min(max(c0 + 2 * lane, 0), np - 2);   // clamped: unused
-  const int64_t lds_ld = op == 0 ? ld : np;
-
-  // Wave w owns rows 16 w .. 16 w + 15 and all 8 tiles of 16 columns of the block, so every wave
-  // drops the same tiles out of the triangle and completes the same tile in each diagonal stage.
-  // Groups of 16 functions whose basis values are all zero on this row tile (activity bit clear,
-  // k_tile_mask) add only zero products.  A block with no active group among its own columns writes
-  // zeros before its first load; otherwise the stages below the block's diagonal run only for the
-  // active groups (their list is compacted into LDS), loads included, and the eight diagonal stages
-  // always run.  Every decision is uniform per workgroup.
-  const uint32_t* __restrict__ mk = amask ? amask + (int64_t)rt * nw : nullptr;
-  auto act = [&](int st) __attribute__((always_inline)) -> bool {
-    return !mk || ((mk[st >> 5] >> (st & 31)) & 1u);
+  const unsigned lring =
+      uniform((int)(unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)&ring[0][op][k0][0]);
+  // operand rows: the tile's packed basis values (row 16 q + k), M (row 16 seq[q] + k).  Selected without a
+  // branch: with one the compiler keeps a second copy of the accumulators (161 VGPRs, one workgroup per CU)
+  const char* src = op == 0 ? (const char*)(phi + (int64_t)rt * ng * (16 * kTT)) : (const char*)M;
+  const int64_t ld = 8 * (int64_t)(op == 0 ? kTT : np);
+  // this lane's 16 bytes of a row: points 2 lane, 2 lane + 1, or columns of the block that starts at group c
+  auto lane_offset = [&](int c) __attribute__((always_inline)) -> unsigned {
+    const unsigned m = 128u * seq[max(c + (lane >> 3), 0)] + 16u * (lane & 7);
+    return op == 0 ? 16u * lane : m;
   };
-  if (mk) {
-    bool any = false;
-    for (int j = 0; j < 8; ++j) any = any || (jd + j >= 0 && act(jd + j));
-    if (!any) {
-      if (lk == 0) part[(int64_t)cb * ldp + row0 + 16 * wave + li] = 0.0;
-      return;
-    }
-  }
-  constexpr int kSeqMax = 256;   // below-diagonal stages listed in LDS (16 kSeqMax functions)
-  __shared__ int seq[kSeqMax + 1];
-  const bool compact = mk && jd <= kSeqMax;
-  int nloop = jd > 0 ? jd : 0;
-  if (compact) {
-    if (wave == 0) {   // wave 0 lists the active stages below the diagonal in order
-      int cnt = 0;
-      for (int b = 0; b < jd; b += 64) {
-        const int st = b + lane;
-        const bool a = st < jd && act(st);
-        const uint64_t bal = __ballot(a);
-        if (a) seq[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = st;
-        cnt += __popcll(bal);
+  auto issue = [&](int q, int slot, unsigned voff) __attribute__((always_inline)) {
+    const int listed = uniform((int)seq[q]);
+    const char* base = src + (16 * (op == 0 ? q : listed) + k0) * ld;
+#pragma unroll
+    for (int j = 0; j < RPW; ++j)
+      lds_dma16_s(base + j * ld, voff, lring + (unsigned)slot * (unsigned)sizeof(ring[0]) + j * (unsigned)sizeof(ring[0][0][0]));
+  };
+  int c0 = nact - 8 * (y + 1);   // the block's first column group, negative: padding
+  int slot = 0;                  // ring slot of the stage being computed
+  unsigned voff = lane_offset(c0);
+  issue(0, 0, voff);
+  for (;; c0 -= 8 * ny) {
+    const int npos = c0 + 8;     // stages 0 .. npos - 1; stage c0 + j is the block's diagonal stage j
+    const int cn = c0 - 8 * ny;  // the next block's first group
+    d4 acc[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) acc[c] = d4{0, 0, 0, 0};
+    // opens stage q: this thread's loads have landed, everyone's after the barrier, and everyone is done
+    // with the stage before, whose slot receives the next stage (of this block, or the next block's first)
+    auto open = [&](int q) __attribute__((always_inline)) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      const bool last = q + 1 == npos;
+      if (last) voff = lane_offset(cn);
+      if (!last || cn > -8) issue(last ? 0 : q + 1, slot ^ 1, voff);
+    };
+    // MFMAs of one stage for the tiles first .. 7 (transposed tiles: M first)
+    auto body = [&](auto first) __attribute__((always_inline)) {
+      constexpr int cs = decltype(first)::value;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks += 4) {
+        double bm[8];
+        const double a = ring[slot][0][ks + lk][16 * wave + li];
+#pragma unroll
+        for (int c = cs; c < 8; ++c) bm[c] = ring[slot][1][ks + lk][c * 16 + li];
+#pragma unroll
+        for (int c = cs; c < 8; ++c) acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(bm[c], a, acc[c], 0, 0, 0);
       }
-      if (lane == 0) seq[kSeqMax] = cnt;
+    };
+    // stages below the block's diagonal (none in the last block): every tile, no row-dot
+    for (int q = 0; q < c0; ++q) {
+      open(q);
+      body(std::integral_constant<int, 0>());
+      slot ^= 1;
     }
-    __syncthreads();
-    nloop = __builtin_amdgcn_readfirstlane(seq[kSeqMax]);
+    // The eight diagonal stages.  M is zero below its diagonal: in diagonal stage j tile c still needs
+    // products while c >= j, and tile j gets its last ones; its A operand in the ring slot holds the basis
+    // values of exactly its columns (k = n = lk + 4 q for lane (li, lk), register q).
+    auto diag = [&](auto jc) __attribute__((always_inline)) {
+      constexpr int J = decltype(jc)::value;
+      const int q = c0 + J;
+      if (q < 0) return;
+      open(q);
+      body(jc);
+      double pr = 0.0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pr = fma(acc[J][r], ring[slot][0][lk + 4 * r][16 * wave + li], pr);
+      pr += __shfl_xor(pr, 16);
+      pr += __shfl_xor(pr, 32);
+      part[(int64_t)q * kTT] = pr;   // the four lane groups store the same value (no branch)
+      slot ^= 1;
+    };
+    diag(std::integral_constant<int, 0>());
+    diag(std::integral_constant<int, 1>());
+    diag(std::integral_constant<int, 2>());
+    diag(std::integral_constant<int, 3>());
+    diag(std::integral_constant<int, 4>());
+    diag(std::integral_constant<int, 5>());
+    diag(std::integral_constant<int, 6>());
+    diag(std::integral_constant<int, 7>());
+    if (cn <= -8) break;
   }
-  // the ring's stage sequence: position p < nloop is a listed stage below the diagonal, then the
-  // diagonal stages jd + j0 .. jd + 7 (j0 > 0 only for block 0, whose first columns are padding)
-  const int j0 = jd < 0 ? -jd : 0;
-  const int npos = nloop + 8 - j0;
-  auto stage_of = [&](int q) __attribute__((always_inline)) -> int {
-    return q < nloop ? (compact ? __builtin_amdgcn_readfirstlane(seq[q]) : q) : jd + j0 + (q - nloop);
-  };
-  auto issue = [&](int q) __attribute__((always_inline)) {
-    const int st = stage_of(q);
-#pragma unroll
-    for (int j = 0; j < RPW; ++j) {
-      const int k = k0 + j;
-      lds_dma16(src + (int64_t)(st * KS + k) * lds_ld, &ring[q % NB][op][k][0]);
-    }
-  };
-  d4 acc[8];
-  double pr = 0.0;   // this lane's row-dot partial sum (row 16 w + li)
-#pragma unroll
-  for (int c = 0; c < 8; ++c) acc[c] = d4{0, 0, 0, 0};
-#pragma unroll
-  for (int q = 0; q < NB - 1; ++q)
-    if (q < npos) issue(q);
-  // opens position q: this thread's loads of q are done once at most RPW (NB - 2) newer ones are
-  // pending, everyone's after the barrier, and everyone is done with q - 1, whose slot is refilled
-  auto open = [&](int q) __attribute__((always_inline)) {
-    const int newer = min(NB - 2, npos - 1 - q);
-    if (RPW == 2 && newer >= 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    else if (RPW == 2 && newer == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (q + NB - 1 < npos) issue(q + NB - 1);
-  };
-  // MFMAs of one stage for the tiles first .. 7 (transposed tiles: M first)
-  auto body = [&](int buf, auto first) __attribute__((always_inline)) {
-    constexpr int cs = decltype(first)::value;
-#pragma unroll
-    for (int ks = 0; ks < KS; ks += 4) {
-      double b[8];
-      const double a = ring[buf][0][ks + lk][16 * wave + li];
-#pragma unroll
-      for (int c = cs; c < 8; ++c) b[c] = ring[buf][1][ks + lk][c * 16 + li];
-#pragma unroll
-      for (int c = cs; c < 8; ++c) acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[c], a, acc[c], 0, 0, 0);
-    }
-  };
-  // Row-dot of the tile a diagonal stage completes: tile c (columns n0 = c0 + 16 c ..) gets its last
-  // products in the stage with KS st = n0, whose A operand in the ring slot holds the basis values of
-  // exactly its columns (k = n - n0 = lk + 4 q for lane (li, lk), register q).  Tiles are summed in
-  // column order.
-  auto rowdot = [&](int buf, auto tile) __attribute__((always_inline)) {
-    constexpr int c = decltype(tile)::value;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) pr = fma(acc[c][q], ring[buf][0][lk + 4 * q][16 * wave + li], pr);
-  };
-  // stages below the block's diagonal (none in block 0): every tile, no row-dot
-  for (int q = 0; q < nloop; ++q) {
-    open(q);
-    if (compact || act(q)) body(q % NB, std::integral_constant<int, 0>());
-  }
-  // The eight diagonal stages.  M is zero below its diagonal: in diagonal stage j tile c still needs
-  // products while KS j <= 16 c + 15, i.e. c >= j, and tile j gets its last ones.  Block 0 starts at
-  // stage 0 = diagonal stage -jd; its tiles below column 0 are those below -jd, skipped too.
-  auto diag = [&](auto jc) __attribute__((always_inline)) {
-    constexpr int J = decltype(jc)::value;
-    if (J < j0) return;
-    const int q = nloop + J - j0;
-    open(q);
-    body(q % NB, jc);
-    rowdot(q % NB, jc);
-  };
-  diag(std::integral_constant<int, 0>());
-  diag(std::integral_constant<int, 1>());
-  diag(std::integral_constant<int, 2>());
-  diag(std::integral_constant<int, 3>());
-  diag(std::integral_constant<int, 4>());
-  diag(std::integral_constant<int, 5>());
-  diag(std::integral_constant<int, 6>());
-  diag(std::integral_constant<int, 7>());
-  pr += __shfl_xor(pr, 16);
-  pr += __shfl_xor(pr, 32);
-  if (lk == 0) part[(int64_t)cb * ldp + row0 + 16 * wave + li] = pr;
 }
 
+__global__ __launch_bounds__(kTWG, 4) void k_contract_f64_blocks(const double* __restrict__ phi,
+                                                                 const double* __restrict__ M, int np, BlockTiles b,
+                                                                 int nrt, int ny, double* __restrict__ part) {
+  int rt, y;
+  if (tile_coords(blockIdx.x, nrt, ny, rt, y)) f64_block_tile(rt, ny - 1 - y, ny, phi, M, np, b, part);
+}
+
+// Density of a voxel: partial sums of its row tiles in list order (FP64: one per group; split: two per block
+// of 4 groups), times scale, summed over its sub-points.  One thread per tile point.
+template <bool SPLIT>
+__device__ __forceinline__ int block_parts(int cnt) { return SPLIT ? (cnt + 3) / 4 * 2 : cnt; }
+
+template <bool SPLIT, typename TO>
+__device__ __forceinline__ void blocks_finish_body(int64_t idx, const GeomView& g, const BlockTiles& b,
+                                                   const double* __restrict__ part, double scale,
+                                                   TO* __restrict__ out) {
+  const int tl = (int)(idx / kTT), p = (int)(idx % kTT);
+  if (tl >= b.nT) return;
+  int i, j, k;
+  block_origin(g, b.T0 + tl, i, j, k);
+  i += p & 7;
+  j += (p >> 3) & 3;
+  k += p >> 5;
+  if (i >= g.nx || j >= g.ny || k >= g.nz) return;
+  const int stride = block_parts<SPLIT>(b.ng);
+  double v = 0.0;
+  for (int s = 0; s < b.nsub * b.nsub * b.nsub; ++s) {
+    const int rt = s * b.nT + tl;
+    const int n = block_parts<SPLIT>(b.cnt[rt]);
+    const double* __restrict__ mine = part + (int64_t)rt * stride * kTT + p;
+    double r = 0.0;
+    for (int q = 0; q < n; ++q) r += mine[(int64_t)q * kTT];
+    v += r * scale;
+  }
+  store_rho<TO>(out, i + (int64_t)g.nx * (j + (int64_t)g.ny * k), v);
+}
+
+template <bool SPLIT, typename TO>
+__global__ __launch_bounds__(256) void k_blocks_finish(GeomView g, BlockTiles b, const double* __restrict__ part,
+                                                       double scale, TO* __restrict__ out) {
+  blocks_finish_body<SPLIT, TO>((int64_t)blockIdx.x * 256 + threadIdx.x, g, b, part, scale, out);
+}
+
+// ---------------------------------------------------------------------------
 // Tiled 16-bit split contraction: the tiling, triangle, workgroup order and
 // partial sums of the FP64 tiled kernel, with stages of 32 k.  The M planes are
 // copied as stored (K8-interleaved); X = Ah Bh + Ah Bl + Al Bh in FP32.
@@ -1103,180 +1315,306 @@ __global__ __launch_bounds__(64 * WR * WC) void k_contract_split_tiles(const voi
   tiled_split_body<T16, WR, WC, PRE>(rt, cb, phi, ld, pscale, p_hi, p_lo, np, part, ld);
 }
 
-// Tiled split contraction on pre-split basis values with both operands
-// fetched by LDS DMA (global_load_lds_dwordx4: each lane's 16 bytes land at
-// M0 + 16 lane, so a wave fills 1 KB of LDS without touching registers) into a
-// two-stage ring of 32 k: stage st + 1 is requested right after the barrier
-// that opens stage st, so its loads run behind stage st's MFMAs while the
-// workgroup's registers stay free (two workgroups share a CU).  The ring slot
-// written at stage st was last read at stage st - 1, which every wave has
-// finished once it passes stage st's barrier.  The loads are issued from inline
-// assembly (M0 holds the LDS address) so that the compiler does not wait for
-// them before each LDS read; the explicit s_waitcnt vmcnt before the barrier
-// waits for them instead.  No other code in this kernel uses M0.  The transposed
-// MFMA order per tile is that of tiled_split_body<PRE>; the row-dot sums are
-// formed here in the K loop, from the LDS copy of the basis values (below).
-//
-// The stage loop is split so that its code has no runtime tile selection: the
-// stages below the block's diagonal run every tile with no row-dot, and the four
-// diagonal stages are unrolled with compile-time first tile and row-dot tile.
-// The two waves of a SIMD take interleaved 16-column tiles, so both drop out of
-// the triangle alike and no diagonal stage branches on the wave.  (A version that
-// selected tiles at run time spent 43 VALU instructions per 24 MFMAs in a full
-// stage, 16 of them register moves; this one spends 4, with 80 VGPRs.)  Measured
-// and dropped: persistent workgroups that prefetch the next tile's first stage
-// (slower: the row tiles' column blocks drift apart); a three- or four-slot ring
-// at one workgroup per CU (two waves per SIMD: 35% slower); warming L2 with a
-// dummy DMA of stage st + 2 (10% slower).
+// ---------------------------------------------------------------------------
+// Block tiles of the 16-bit split path (variant 3): groups of 32 functions (one MFMA k step), basis values of
+// the listed groups scaled and split by the basis-value kernel, group j of row tile rt at
+// phi + (rt ng + j) 8192: hi plane [4 k groups][128 points][8], then lo.  Values, (hi, lo) packing and
+// the LDS transpose are those of phi_split_body.
+// A wave takes a whole tile, two points per lane (64 apart), so that the scalar work of a shell (its record,
+// nucleus and primitives, the loop, the store addresses) is paid once per tile; the next shell's record is
+// loaded ahead, and shells with common exponents share their exponentials (`pair`).  1.77 M points of 606
+// functions: 0.91 -> 0.61 ms against one point per lane.  (The same in phi_f64_blocks_body measured 0.44 -> 0.46
+// to 0.51 ms per 0.88 M points: that kernel is bound by its writes, 4.6 to 4.9 TB/s.)
+template <int NT, typename T16>   // NT: threads per workgroup
+__device__ __forceinline__ void phi_split_blocks_body(const MolView& m, const float2* __restrict__ prim_l2e,
+                                                      const int2* __restrict__ kg, const GeomView& g,
+                                                      const BlockTiles& b, int rt, int lane, int part, int nparts,
+                                                      float S, T16* __restrict__ phi) {
+#pragma clang fp contract(off)
+  __shared__ uint32_t stage[8][2 * NT];   // word [f % 8][point] of a wave's two points per lane
+  const DevShell* shells = uniform(m.shells);
+  const double4* atoms = uniform(m.atoms);
+  const float2* prims = uniform(prim_l2e);
+  const int nshell = uniform(m.nshell), nbf = uniform(m.nbf);
+  kg = uniform(kg);
+  double x[2], y[2], z[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) block_point(g, b, rt, lane + 64 * i, x[i], y[i], z[i]);
+  uint32_t* __restrict__ mine = &stage[0][2 * (threadIdx.x & ~63) + lane];
+  T16* __restrict__ tile = phi + (int64_t)rt * b.ng * (64 * kTT) + 8 * lane;
+  for_runs<5>(uniform(b.list) + (int64_t)rt * uniform(b.ng), table<int>(uniform(b.cnt), rt), part, nparts, [&](int j, int fj, int f0, int f1)
+                                                                        __attribute__((always_inline)) {
+    T16* __restrict__ out = tile + (int64_t)j * (64 * kTT);
+    auto store = [&](int i, int f, float xs) __attribute__((always_inline)) {   // xs: the value already times S
+      const T16 hq = (T16)xs;
+      const T16 lq = (T16)(xs - (float)hq);
+      mine[(f & 7) * (2 * NT) + 64 * i] = bits16(hq) | (bits16(lq) << 16);
+    };
+    auto flush = [&](int f) __attribute__((always_inline)) {   // f: last of its 8 functions
+      T16* __restrict__ o = out + (int64_t)((f - fj) >> 5) * (64 * kTT) + ((f >> 3) & 3) * (8 * kTT);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        uint32_t w[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) w[q] = mine[q * (2 * NT) + 64 * i];
+        uint4 H, L;
+        H.x = __builtin_amdgcn_perm(w[1], w[0], 0x05040100u);
+        H.y = __builtin_amdgcn_perm(w[3], w[2], 0x05040100u);
+        H.z = __builtin_amdgcn_perm(w[5], w[4], 0x05040100u);
+        H.w = __builtin_amdgcn_perm(w[7], w[6], 0x05040100u);
+        L.x = __builtin_amdgcn_perm(w[1], w[0], 0x07060302u);
+        L.y = __builtin_amdgcn_perm(w[3], w[2], 0x07060302u);
+        L.z = __builtin_amdgcn_perm(w[5], w[4], 0x07060302u);
+        L.w = __builtin_amdgcn_perm(w[7], w[6], 0x07060302u);
+        *(uint4*)(o + 8 * 64 * i) = H;
+        *(uint4*)(o + 8 * 64 * i + 32 * kTT) = L;
+      }
+    };
+    int atom = -1, s = table<int>((const int*)(kg + (f0 >> 3)), 0);
+    float dx[2], dy[2], dz[2], r2[2], next[2];
+    bool have = false;
+    if (s < nshell) {
+      DevShell sh = table_shell(shells, s);
+      for (; sh.bf < f1;) {
+        const DevShell ahead = table_shell(shells, min(s + 1, nshell - 1));
+        if (sh.atom != atom) {   // r^2 in FP64, rounded once: exp(-a r^2) amplifies its error by a r^2
+          atom = sh.atom;
+          const v4d a = table<v4d>((const v4d*)atoms, atom);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const double ex = x[i] - a.x, ey = y[i] - a.y, ez = z[i] - a.z;
+            dx[i] = (float)ex;
+            dy[i] = (float)ey;
+            dz[i] = (float)ez;
+            r2[i] = (float)dist2(ex, ey, ez);
+          }
+        }
+        float radial[2] = {0.f, 0.f};
+        if (have) {
+          radial[0] = next[0];
+          radial[1] = next[1];
+          have = false;
+        } else {
+          have = sh.pair != 0;
+          next[0] = next[1] = 0.f;
+          if (fminf(r2[0], r2[1]) <= sh.rcut2) {
+            for (int q = 0; q < sh.nprim; ++q) {
+              const v2f pc = table<v2f>((const v2f*)prims, sh.poff + q);
+              const float c2 = have ? table<v2f>((const v2f*)prims, sh.pair - 1 + q).y : 0.f;
+#pragma unroll
+              for (int i = 0; i < 2; ++i) {
+                const float v = __builtin_amdgcn_exp2f(-pc.x * r2[i]);
+                radial[i] = __builtin_fmaf(pc.y, v, radial[i]);
+                next[i] = __builtin_fmaf(c2, v, next[i]);
+              }
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+              if (!(r2[i] <= sh.rcut2)) radial[i] = next[i] = 0.f;
+          }
+        }
+        // functions of a straddling shell outside the run are dropped (uniform)
+        auto emit = [&](auto lc) __attribute__((always_inline)) {
+          constexpr int L = decltype(lc)::value;
+          float v[2][5];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) shell_values<float>(L, dx[i], dy[i], dz[i], radial[i] * S, v[i]);
+#pragma unroll
+          for (int c = 0; c < 2 * L + 1; ++c) {
+            const int f = sh.bf + c;
+            if (f >= f0 && f < f1) {
+              store(0, f, v[0][c]);
+              store(1, f, v[1][c]);
+              if ((f & 7) == 7) flush(f);
+            }
+          }
+        };
+        if (sh.L == 0) emit(std::integral_constant<int, 0>());
+        else if (sh.L == 1) emit(std::integral_constant<int, 1>());
+        else emit(std::integral_constant<int, 2>());
+        if (++s >= nshell) break;
+        sh = ahead;
+      }
+    }
+    for (int f = max(nbf, f0); f < f1; ++f) {   // padding of the last group
+      store(0, f, 0.f);
+      store(1, f, 0.f);
+      if ((f & 7) == 7) flush(f);
+    }
+  });
+}
 
 template <typename T16>
-__device__ __forceinline__ void tiled_dma_body(int rt, int cb, const T16* __restrict__ a_hi, int ld,
-                                               const T16* __restrict__ p_hi, const T16* __restrict__ p_lo, int np,
-                                               int nbf, int ncb, double* __restrict__ part, int ldp) {
+__global__ __launch_bounds__(kPhiThreads) void k_phi_split_blocks(MolView m, const float2* __restrict__ prim_l2e,
+                                                                  const int2* __restrict__ kg, GeomView g,
+                                                                  BlockTiles b, int nrt, float S,
+                                                                  T16* __restrict__ phi) {
+  const int rt = __builtin_amdgcn_readfirstlane(blockIdx.x * kPhiTiles + threadIdx.x / 64);
+  if (rt < nrt)
+    phi_split_blocks_body<kPhiThreads, T16>(m, prim_l2e, kg, g, b, rt, threadIdx.x % 64, blockIdx.y, gridDim.y, S, phi);
+}
+
+// Split contraction of block tiles, fed by LDS DMA (variant 3): a workgroup owns one row tile and takes
+// its column blocks of 4 listed groups (128 columns) one after the other, the longest first.  Stages are the
+// listed groups in order (32 k).  Both operands go global -> LDS by global_load_lds_dwordx4 into a two-stage
+// ring, issued right after the barrier that opens the previous stage, so the loads run behind that stage's
+// MFMAs while the registers stay free (two workgroups share a CU); the slot written was last read in the
+// stage before, which every wave has finished once it passes the barrier.  The loads come from inline
+// assembly (M0 holds the LDS address) so that the compiler does not wait for them before each LDS read; the
+// explicit s_waitcnt vmcnt before the barrier does.  M goes first into the MFMAs, so a 16 x 16 tile of X
+// comes out transposed (lane (li, lk), register q = X[t = li][n = 4 lk + q]) and the row-dot reads the 4
+// consecutive functions of one point as one 8-byte word per plane, in the stage that completes the tile.
+// Waves are 4 x 2: wave (wr, wc) owns rows 32 wr .. 32 wr + 31 and the interleaved 16-column tiles 2 c + wc, so
+// the two waves of a SIMD drop out of the triangle alike and the diagonal stages have compile-time tiles.
+// Column blocks are right-aligned on the list: only the last one holds padding, as columns below group 0.
+// The finishing pass divides by S^2 (folded into its scale) and adds the two wc halves of every block.
+template <typename T16>
+__device__ __forceinline__ void split_block_tile(int rt, int y, int ny, const T16* __restrict__ phi,
+                                                 const T16* __restrict__ p_hi, const T16* __restrict__ p_lo, int np,
+                                                 const BlockTiles& b, int np_part, double* __restrict__ part) {
   typedef typename Vec8<T16>::type V8;
   constexpr int WR = 4, WC = 2, TRW = kTT / WR, TCW = kTT / WC, RT = TRW / 16, CT = TCW / 16;
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   // ring slot: 4 operand planes (A hi, A lo, B hi, B lo) of [4 k groups][128] 16-byte words
   __shared__ u32x4 ring[2][4][4][kTT];
-  __shared__ double red[WC][kTT];
-  const char* __restrict__ a_hi_b = (const char*)a_hi;
-  const char* __restrict__ a_lo_b = (const char*)(a_hi + (int64_t)np * ld);
+  __shared__ uint16_t seq[kMaxGroups];
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int wr = wave & 3, wc = wave >> 2;   // waves w, w + 4 share a SIMD
   const int li = lane & 15, lk = lane >> 4;
-  // column blocks right-aligned on ne = nbf rounded up to 32 (as in tiled_f64_dma_body): only
-  // block 0 holds padding, as columns below 0, skipped like tiles below the diagonal
-  const int ne = (nbf + 31) / 32 * 32;
-  const int row0 = rt * kTT, c0 = cb * kTT - (ncb * kTT - ne);
-  const int nst = (c0 + kTT) / 32;
-  const int jd = c0 / 32;   // c0 is a multiple of 32: stage jd + j is the block's diagonal stage j
-  // thread t fetches word t of each plane: k group g = t / 128, row / column ii = t % 128.  The
-  // stage's base address is wave-uniform (SGPRs, saddr form); the lane's byte offset within the
-  // stage is at most 64 ld < 2^32 (a plane of basis values is at most 2 GiB).
-  const int g = t / kTT, ii = t % kTT;
-  const int bcol = min(max(c0 + ii, 0), np - 1);   // clamped columns are never used
-  const unsigned oa = (unsigned)(g * ld + ii) * 16u;
-  const unsigned ob = (unsigned)(g * np + bcol) * 16u;
-  const unsigned lring = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)&ring[0][0][0][0] + 1024u * wave;
-  auto issue = [&](int st) __attribute__((always_inline)) {
-    const unsigned l = lring + (unsigned)(st & 1) * (unsigned)sizeof(ring[0]);
-    // 4 k groups of 16 bytes per stage; the tile's first row goes into the uniform base
-    const int64_t sa = (int64_t)st * 64 * ld + (int64_t)row0 * 16, sb = (int64_t)st * 64 * np;
-    lds_dma16_s(a_hi_b + sa, oa, l);
-    lds_dma16_s(a_lo_b + sa, oa, l + (unsigned)sizeof(ring[0][0]));
-    lds_dma16_s((const char*)p_hi + sb, ob, l + 2u * (unsigned)sizeof(ring[0][0]));
-    lds_dma16_s((const char*)p_lo + sb, ob, l + 3u * (unsigned)sizeof(ring[0][0]));
-  };
-  f4 acc[RT][CT];
-  double pr[RT];   // this lane's row-dot partial sums (rows wr TRW + 16 r + li)
-  // Wave (wr, wc) owns rows wr TRW .. + TRW - 1 and the interleaved 16-column tiles 2 c + wc, c =
-  // 0 .. CT - 1, of the block (columns c0 + 32 c + 16 wc ..), so that both waves of a SIMD drop
-  // tiles out of the triangle alike.  MFMAs of one stage for the tiles first .. CT - 1:
-  auto body = [&](int slot, auto first) __attribute__((always_inline)) {
-    constexpr int cs = decltype(first)::value;
-    V8 ah[RT], al[RT], bh[CT], bl[CT];
-#pragma unroll
-    for (int r = 0; r < RT; ++r) {
-      ah[r] = __builtin_bit_cast(V8, ring[slot][0][lk][wr * TRW + r * 16 + li]);
-      al[r] = __builtin_bit_cast(V8, ring[slot][1][lk][wr * TRW + r * 16 + li]);
-    }
-#pragma unroll
-    for (int c = cs; c < CT; ++c) {
-      bh[c] = __builtin_bit_cast(V8, ring[slot][2][lk][32 * c + 16 * wc + li]);
-      bl[c] = __builtin_bit_cast(V8, ring[slot][3][lk][32 * c + 16 * wc + li]);
-    }
-    // transposed tiles (M first); each product runs over all tiles before the next, so consecutive
-    // MFMAs are independent (a tile's three products keep their order)
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-      for (int c = cs; c < CT; ++c) acc[r][c] = Vec8<T16>::mma(bh[c], al[r], acc[r][c]);
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-      for (int c = cs; c < CT; ++c) acc[r][c] = Vec8<T16>::mma(bl[c], ah[r], acc[r][c]);
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-      for (int c = cs; c < CT; ++c) acc[r][c] = Vec8<T16>::mma(bh[c], ah[r], acc[r][c]);
-  };
-  // Row-dot of the tile a stage completes: the wave's tile c (columns n0 = c0 + 32 c + 16 wc ..)
-  // gets its last products in stage (n0 + 15) / 32 = diagonal stage c, whose A operand in the ring
-  // slot holds the basis values of exactly its columns (k = n).  Lane (li, lk), register q of a
-  // tile is X[t = li][n = 4 lk + q]: the 4 values of one point sit in one 8-byte word of each
-  // plane.  Each wave sums its tiles in column order.
-  auto rowdot = [&](int slot, auto tile) __attribute__((always_inline)) {
-    constexpr int c = decltype(tile)::value;
-    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-    typedef __bf16 b4 __attribute__((ext_vector_type(4)));
-    typedef typename std::conditional<std::is_same<T16, _Float16>::value, h4, b4>::type V4;
-    const int kg = 2 * wc + (lk >> 1);   // k group of n - 32 st = 16 wc + 4 lk + q
-#pragma unroll
-    for (int r = 0; r < RT; ++r) {
-      const int row = wr * TRW + r * 16 + li;
-      const V4 h = __builtin_bit_cast(V4, ((const uint2*)&ring[slot][0][kg][row])[lk & 1]);
-      const V4 l = __builtin_bit_cast(V4, ((const uint2*)&ring[slot][1][kg][row])[lk & 1]);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) pr[r] += (double)(acc[r][c][q] * ((float)h[q] + (float)l[q]));
-    }
-  };
-#pragma unroll
-  for (int r = 0; r < RT; ++r) {
-    pr[r] = 0.0;
-#pragma unroll
-    for (int c = 0; c < CT; ++c) acc[r][c] = f4{0, 0, 0, 0};
-  }
-  // opens stage st: this thread's loads of st have landed, every thread's have after the barrier,
-  // and every wave is done with st - 1, whose slot receives st + 1
-  auto open = [&](int st) __attribute__((always_inline)) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (st + 1 < nst) issue(st + 1);
-  };
-  issue(0);
-  // stages below the block's diagonal (none in block 0): every tile, no row-dot
-  for (int st = 0; st < jd; ++st) {
-    open(st);
-    body(st & 1, std::integral_constant<int, 0>());
-  }
-  // The four diagonal stages, with compile-time tiles.  M is zero below its diagonal: in diagonal
-  // stage j, the wave's tile c (columns c0 + 32 c + 16 wc ..) still needs products while 32 j <
-  // 32 c + 16 wc + 16, i.e. c >= j, and tile j gets its last ones.  Block 0 starts at stage 0 =
-  // diagonal stage -jd; its tiles below column 0 are those below -jd, skipped too.
-  auto diag = [&](auto jc) __attribute__((always_inline)) {
-    constexpr int J = decltype(jc)::value;
-    const int st = jd + J;
-    if (st < 0) return;
-    open(st);
-    body(st & 1, jc);
-    __builtin_amdgcn_sched_barrier(0);
-    rowdot(st & 1, jc);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  diag(std::integral_constant<int, 0>());
-  diag(std::integral_constant<int, 1>());
-  diag(std::integral_constant<int, 2>());
-  diag(std::integral_constant<int, 3>());
-#pragma unroll
-  for (int r = 0; r < RT; ++r) {
-    double p = pr[r];
-    p += __shfl_xor(p, 16);
-    p += __shfl_xor(p, 32);
-    if (lk == 0) red[wc][wr * TRW + r * 16 + li] = p;
-  }
+  rt = uniform(rt);
+  np = uniform(np);
+  const int ng = uniform(b.ng);
+  const int nact = uniform(b.cnt[rt]);
+  if (4 * y >= nact) return;
+  const char* a_b = (const char*)(uniform(phi) + (int64_t)rt * ng * (64 * kTT));
+  const char* h_b = (const char*)uniform(p_hi);
+  const char* l_b = (const char*)uniform(p_lo);
+  part = (double*)uniform(part) + (int64_t)rt * uniform(np_part) * kTT + wr * TRW + li;
+  for (int i = t; i < nact; i += kTWG) seq[i] = b.list[(int64_t)rt * ng + i];
   __syncthreads();
-  if (t < kTT) part[(int64_t)cb * ldp + row0 + t] = red[0][t] + red[1][t];
+  // thread t fetches word t of each plane: k group t / 128, row / column t % 128.  Bases are wave uniform
+  // (SGPRs), lane offsets below 64 np < 2^32 bytes.
+  const unsigned oa = 16u * t;
+  const int g = t / kTT, ii = t % kTT;
+  auto column_offset = [&](int c) __attribute__((always_inline)) -> unsigned {
+    return (unsigned)(g * np + 32 * (int)seq[max(c + (ii >> 5), 0)] + (ii & 31)) * 16u;
+  };
+  const unsigned lring = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)&ring[0][0][0][0] + 1024u * wave;
+  auto issue = [&](int q, int slot, unsigned ob) __attribute__((always_inline)) {
+    const unsigned l = lring + (unsigned)slot * (unsigned)sizeof(ring[0]);
+    const int64_t sa = (int64_t)q * (128 * kTT), sb = (int64_t)uniform((int)seq[q]) * 64 * np;
+    lds_dma16_s(a_b + sa, oa, l);
+    lds_dma16_s(a_b + sa + 64 * kTT, oa, l + (unsigned)sizeof(ring[0][0]));
+    lds_dma16_s(h_b + sb, ob, l + 2u * (unsigned)sizeof(ring[0][0]));
+    lds_dma16_s(l_b + sb, ob, l + 3u * (unsigned)sizeof(ring[0][0]));
+  };
+  int c0 = nact - 4 * (y + 1);   // the block's first column group, negative: padding
+  int slot = 0;
+  unsigned ob = column_offset(c0);
+  issue(0, 0, ob);
+  for (int cbi = y;; cbi += ny, c0 -= 4 * ny) {
+    const int npos = c0 + 4;     // stages 0 .. npos - 1; stage c0 + j is the block's diagonal stage j
+    const int cn = c0 - 4 * ny;  // the next block's first group
+    f4 acc[RT][CT];
+    double pr[RT];   // this lane's row-dot partial sums (rows wr TRW + 16 r + li)
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      pr[r] = 0.0;
+#pragma unroll
+      for (int c = 0; c < CT; ++c) acc[r][c] = f4{0, 0, 0, 0};
+    }
+    // opens stage q: this thread's loads have landed, everyone's after the barrier, and everyone is done
+    // with the stage before, whose slot receives the next stage (of this block, or the next block's first)
+    auto open = [&](int q) __attribute__((always_inline)) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      const bool last = q + 1 == npos;
+      if (last) ob = column_offset(cn);
+      if (!last || cn > -4) issue(last ? 0 : q + 1, slot ^ 1, ob);
+    };
+    // MFMAs of one stage for the wave's tiles first .. CT - 1; each product runs over all tiles before the
+    // next, so consecutive MFMAs are independent (a tile's three products keep their order)
+    auto body = [&](auto first) __attribute__((always_inline)) {
+      constexpr int cs = decltype(first)::value;
+      V8 ah[RT], al[RT], bh[CT], bl[CT];
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        ah[r] = __builtin_bit_cast(V8, ring[slot][0][lk][wr * TRW + r * 16 + li]);
+        al[r] = __builtin_bit_cast(V8, ring[slot][1][lk][wr * TRW + r * 16 + li]);
+      }
+#pragma unroll
+      for (int c = cs; c < CT; ++c) {
+        bh[c] = __builtin_bit_cast(V8, ring[slot][2][lk][32 * c + 16 * wc + li]);
+        bl[c] = __builtin_bit_cast(V8, ring[slot][3][lk][32 * c + 16 * wc + li]);
+      }
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int c = cs; c < CT; ++c) acc[r][c] = Vec8<T16>::mma(bh[c], al[r], acc[r][c]);
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int c = cs; c < CT; ++c) acc[r][c] = Vec8<T16>::mma(bl[c], ah[r], acc[r][c]);
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int c = cs; c < CT; ++c) acc[r][c] = Vec8<T16>::mma(bh[c], ah[r], acc[r][c]);
+    };
+    // stages below the block's diagonal (none in the last block): every tile, no row-dot
+    for (int q = 0; q < c0; ++q) {
+      open(q);
+      body(std::integral_constant<int, 0>());
+      slot ^= 1;
+    }
+    // The four diagonal stages: in stage j the wave's tile c still needs products while c >= j, and tile j
+    // gets its last ones; the stage's A operand holds the basis values of exactly its columns (k = n).
+    auto diag = [&](auto jc) __attribute__((always_inline)) {
+      constexpr int J = decltype(jc)::value;
+      const int q = c0 + J;
+      if (q < 0) return;
+      open(q);
+      body(jc);
+      __builtin_amdgcn_sched_barrier(0);
+      typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+      typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+      typedef typename std::conditional<std::is_same<T16, _Float16>::value, h4, b4>::type V4;
+      const int kg = 2 * wc + (lk >> 1);   // k group of n - 32 q = 16 wc + 4 lk + i
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        const int row = wr * TRW + r * 16 + li;
+        const V4 h = __builtin_bit_cast(V4, ((const uint2*)&ring[slot][0][kg][row])[lk & 1]);
+        const V4 l = __builtin_bit_cast(V4, ((const uint2*)&ring[slot][1][kg][row])[lk & 1]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pr[r] += (double)(acc[r][J][i] * ((float)h[i] + (float)l[i]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      slot ^= 1;
+    };
+    diag(std::integral_constant<int, 0>());
+    diag(std::integral_constant<int, 1>());
+    diag(std::integral_constant<int, 2>());
+    diag(std::integral_constant<int, 3>());
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      double v = pr[r];
+      v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      part[(int64_t)(2 * cbi + wc) * kTT + 16 * r] = v;   // the four lane groups store the same value (no branch)
+    }
+    if (cn <= -4) break;
+  }
 }
 
 template <typename T16>
-__global__ __launch_bounds__(512, 4) void k_contract_split_dma(const void* __restrict__ phi, int ld,
-                                                            const T16* __restrict__ p_hi, const T16* __restrict__ p_lo,
-                                                            int np, int nbf, int nrt, int ncb,
-                                                            double* __restrict__ part) {
-  int rt, cb;
-  if (!tile_coords(blockIdx.x, nrt, ncb, rt, cb)) return;
-  tiled_dma_body<T16>(rt, cb, (const T16*)phi, ld, p_hi, p_lo, np, nbf, ncb, part, ld);
+__global__ __launch_bounds__(512, 4) void k_contract_split_blocks(const T16* __restrict__ phi,
+                                                                  const T16* __restrict__ p_hi,
+                                                                  const T16* __restrict__ p_lo, int np, BlockTiles b,
+                                                                  int np_part, int nrt, int ny,
+                                                                  double* __restrict__ part) {
+  int rt, y;
+  if (tile_coords(blockIdx.x, nrt, ny, rt, y))
+    split_block_tile<T16>(rt, ny - 1 - y, ny, phi, p_hi, p_lo, np, b, np_part, part);
 }
 
 // ---------------------------------------------------------------------------
@@ -1919,77 +2257,12 @@ __global__ __launch_bounds__(kTWG) void k_contract_f64_rows(const double* __rest
   tiled_f64_rows_body(rt, cb, phi, ld, M, np, part, ld);
 }
 
-template <bool DMA>
 __global__ __launch_bounds__(kTWG) void k_contract_f64_tiles(const double* __restrict__ phi, int ld,
-                                                             const double* __restrict__ M, int np, int nbf, int nrt,
-                                                             int ncb, double* __restrict__ part,
-                                                             const uint32_t* __restrict__ amask, int nw) {
+                                                             const double* __restrict__ M, int np, int nrt, int ncb,
+                                                             double* __restrict__ part) {
   int rt, cb;
   if (!tile_coords(blockIdx.x, nrt, ncb, rt, cb)) return;
-  if (DMA) tiled_f64_dma_body<kF64Ks, 32 / kF64Ks>(rt, cb, phi, ld, M, np, nbf, ncb, part, ld, amask, nw);
-  else tiled_f64_body(rt, cb, phi, ld, M, np, part, ld);
-}
-
-// Activity of each row tile's groups of 16 basis functions: bit q of mask[rt nw + q / 32] is set
-// when some point of the tile is within the cutoff (r^2 <= rcut2) of a shell with a function in
-// group q.  A clear bit means the tile's basis values in the group are all exactly zero (the
-// basis-value kernels write 0 beyond a shell's cutoff).  Conservative: the distance is taken to the
-// bounding box of the tile's points, against the cutoff with a relative margin of 1e-6.
-__device__ __forceinline__ void tile_mask_body(const MolView& m, const GeomView& g, int64_t v0, int nvox, int nsub,
-                                               int npts, int rt, int nw, uint32_t* __restrict__ mask) {
-  __shared__ double box[kTT / 64][6];
-  __shared__ uint32_t words[64];
-  const int t = rt * kTT + threadIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  double b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};   // lo xyz, hi xyz
-  if (t < npts) {
-    double x, y, z;
-    chunk_point(g, v0, nvox, nsub, t, x, y, z);
-    b[0] = b[3] = x;
-    b[1] = b[4] = y;
-    b[2] = b[5] = z;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      b[d] = fmin(b[d], __shfl_xor(b[d], off, 64));
-      b[3 + d] = fmax(b[3 + d], __shfl_xor(b[3 + d], off, 64));
-    }
-  if (lane == 0)
-    for (int d = 0; d < 6; ++d) box[wave][d] = b[d];
-  for (int w = threadIdx.x; w < nw; w += kTT) words[w] = 0u;
-  __syncthreads();
-  double lo[3], hi[3];
-  for (int d = 0; d < 3; ++d) {
-    lo[d] = box[0][d];
-    hi[d] = box[0][3 + d];
-    for (int w = 1; w < kTT / 64; ++w) {
-      lo[d] = fmin(lo[d], box[w][d]);
-      hi[d] = fmax(hi[d], box[w][3 + d]);
-    }
-  }
-  if (lo[0] <= hi[0]) {   // the tile holds at least one point
-    for (int sidx = threadIdx.x; sidx < m.nshell; sidx += kTT) {
-      const DevShell sh = m.shells[sidx];
-      const double4 a = m.atoms[sh.atom];
-      const double c[3] = {a.x, a.y, a.z};
-      double d2 = 0.0;
-      for (int d = 0; d < 3; ++d) {
-        const double e = fmax(0.0, fmax(lo[d] - c[d], c[d] - hi[d]));
-        d2 += e * e;
-      }
-      if (d2 <= (double)sh.rcut2 * (1.0 + 1e-6))
-        for (int q = sh.bf >> 4; q <= (sh.bf + 2 * sh.L) >> 4; ++q) atomicOr(&words[q >> 5], 1u << (q & 31));
-    }
-  }
-  __syncthreads();
-  for (int w = threadIdx.x; w < nw; w += kTT) mask[(int64_t)rt * nw + w] = words[w];
-}
-
-__global__ __launch_bounds__(kTT) void k_tile_mask(MolView m, GeomView g, int64_t v0, int nvox, int nsub, int npts,
-                                                   int nw, uint32_t* __restrict__ mask) {
-  tile_mask_body(m, g, v0, nvox, nsub, npts, blockIdx.x, nw, mask);
+  tiled_f64_body(rt, cb, phi, ld, M, np, part, ld);
 }
 
 // rho_t = scale * sum_cb part[cb][t] (fixed order), optionally / pscale_t
@@ -2272,8 +2545,92 @@ void launch_contract_split(hipStream_t s, int ld, const float* phi, const float*
 #undef QM_SPLIT_CASE
 }
 
+float split_phi_scale(const qm_mol* m);
+
+// Workgroups per row tile (ncb column blocks at most).  Bases of up to two blocks: one, because a workgroup's
+// start (count, list, first loads: about 7 us) costs more than a second block holds (246 functions, FP64,
+// 6.6 M points: 3.0 ms with one, 4.2 ms with two), unless the tiles alone do not fill the 512 workgroup slots.
+// Larger ones: several, side by side on one XCD, so that the blocks of a tile share its basis values in L2
+// (606 functions, 0.88 M points: FP64 2.05 / 1.90 / 1.71 / 1.66 ms with 1 / 2 / 3 / 5; split, 1.77 M points,
+// 0.94 / 0.88 / 0.82 / 0.81 ms, but a batch of 5-80 atoms 11.1 / 12.5 / 11.5 / 13.0 ms).
+inline int block_split(int nrt, int ncb, bool f64) {
+  if (ncb <= 2) return nrt >= 512 ? 1 : ncb;
+  return f64 ? ncb : 3;
+}
+// Workgroups per four tiles in the basis-value launch (blk of them): 2048 workgroups of four waves fill the
+// chip; with fewer the list (n8 units of 8 functions at most) is shared out.
+inline int phi_split(int blk, int n8) { return std::max(1, std::min({n8, 64, 2048 / std::max(blk, 1)})); }
+
+// Block tiles (the default contractions): chunks of tiles whose basis values fit kPhiBudget with every
+// group listed (a tile leaves the part of its space that it does not need untouched).
+// FP64 (T = double, groups of 16) or split (T = _Float16 / __bf16, groups of 32; M in hi and lo planes).
+template <typename T, typename TO>
+int density_blocks(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, int nsub, TO* out) {
+  constexpr bool f64 = std::is_same<T, double>::value;
+  constexpr int GS = f64 ? 4 : 5;
+  const int np = mol->nbf_pad, ng = (mol->nbf + (1 << GS) - 1) >> GS;
+  const int ncb = f64 ? (ng + 7) / 8 : (ng + 3) / 4, nparts = f64 ? ng : 2 * ncb;
+  const int nsub3 = nsub * nsub * nsub;
+  const GeomView gv = geom_view(g);
+  const MolView mv = mol->view();
+  const int64_t ntiles = block_tiles(gv);
+  const size_t tile_bytes = (f64 ? sizeof(double) : 4) * (size_t)kTT * (ng << GS);
+  int64_t nT = std::max<int64_t>((int64_t)(kPhiBudget / tile_bytes) / nsub3, 1);
+  nT = std::min(nT, std::min(ntiles, std::max<int64_t>((1 << 22) / nsub3, 1)));
+  const int64_t rows = nT * nsub3;
+  T* phi = nullptr;
+  double* part = nullptr;
+  char* lists = nullptr;
+  int rc = QM_OK;
+  if ((rc = qm_ws(ctx, s, WS_PHI, tile_bytes * rows, (void**)&phi))) return rc;
+  if ((rc = qm_ws(ctx, s, WS_PART, sizeof(double) * kTT * (size_t)nparts * rows, (void**)&part))) return rc;
+  if ((rc = qm_ws(ctx, s, WS_MASK, (sizeof(int) + sizeof(uint16_t) * (size_t)ng) * rows, (void**)&lists))) return rc;
+  int* cnt = (int*)lists;
+  uint16_t* list = (uint16_t*)(lists + sizeof(int) * rows);
+  const float S = f64 ? 1.f : split_phi_scale(mol);
+  const double h3 = g->step * g->step * g->step;
+  const double scale = (f64 ? h3 : h3 / mol->pfac / ((double)S * S)) / nsub3;
+  const T* M = (const T*)(f64 ? (const void*)mol->M64 : std::is_same<T, _Float16>::value ? mol->P16 : mol->Pb16);
+  for (int64_t T0 = 0; T0 < ntiles; T0 += nT) {
+    const BlockTiles b{(int)T0, (int)std::min(nT, ntiles - T0), nsub, ng, list, cnt};
+    const int nrt = b.nT * nsub3, pblk = f64 ? (nrt + 1) / 2 : (nrt + kPhiTiles - 1) / kPhiTiles;
+    const dim3 pgrid(pblk, phi_split(pblk, ng << (GS - 3)));
+    const int ny = block_split(nrt, ncb, f64);
+    const dim3 cgrid(tile_grid(nrt, ny));
+    {
+      ProfScope ps(ctx, s, f64 ? QM_K_PHI : QM_K_PHI_SPLIT);
+      hipLaunchKernelGGL(k_tile_list<GS>, dim3(nrt), dim3(kTT), 0, s, mv, gv, b, f64 && !ctx->tile_skip, list, cnt);
+      if constexpr (f64)
+        hipLaunchKernelGGL(k_phi_f64_blocks, pgrid, dim3(kPhiThreads), 0, s, mv, (const int2*)mol->kgroups, gv, b, nrt,
+                           phi);
+      else
+        hipLaunchKernelGGL(k_phi_split_blocks<T>, pgrid, dim3(kPhiThreads), 0, s, mv, (const float2*)mol->prims_l2e,
+                           (const int2*)mol->kgroups, gv, b, nrt, S, phi);
+    }
+    QM_CHECK_LAUNCH(ctx);
+    ProfScope pc(ctx, s, f64 ? QM_K_DENSITY_CONTRACT : QM_K_DENSITY_SPLIT);
+    if constexpr (f64)
+      hipLaunchKernelGGL(k_contract_f64_blocks, cgrid, dim3(kTWG), 0, s, (const double*)phi, M, np, b, nrt, ny, part);
+    else
+      hipLaunchKernelGGL(k_contract_split_blocks<T>, cgrid, dim3(512), 0, s, (const T*)phi, M, M + (int64_t)np * np, np,
+                         b, nparts, nrt, ny, part);
+    QM_CHECK_LAUNCH(ctx);
+    hipLaunchKernelGGL((k_blocks_finish<!f64, TO>), dim3((unsigned)(((int64_t)b.nT * kTT + 255) / 256)), dim3(256), 0, s,
+                       gv, b, (const double*)part, scale, out);
+    QM_CHECK_LAUNCH(ctx);
+  }
+  return QM_OK;
+}
+
+// a tile's groups fit a workgroup's list: 32768 basis functions in FP64, where larger bases take variant 2
+// (a split basis beyond 65536 functions would need 34 GB for M and is refused by its allocation)
+inline bool f64_blocks(const qm_ctx* ctx, const qm_mol* mol) {
+  return ctx->f64_variant == 4 && (mol->nbf + 15) / 16 <= kMaxGroups;
+}
+
 template <typename TO>
 int density_fp64(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, int nsub, TO* out) {
+  if (f64_blocks(ctx, mol)) return density_blocks<double, TO>(ctx, mol, s, g, nsub, out);
   const int np = mol->nbf_pad;
   const int nsub3 = nsub * nsub * nsub;
   const int64_t nvox_tot = npoints(g);
@@ -2291,16 +2648,10 @@ int density_fp64(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, int 
     rc = qm_ws(ctx, s, WS_RHO, sizeof(double) * ldmax, (void**)&rho);
     if (rc) return rc;
   }
-  const bool tiled = ctx->f64_variant >= 2;   // 2 tiles, 3 rows, 4 tiles fed by LDS DMA
+  const bool tiled = ctx->f64_variant >= 2;   // 2 tiles, 3 rows
   const int ncb = ctx->f64_variant == 3 ? np / kRN : (np + kTT - 1) / kTT;
   double* part = nullptr;
   if (tiled && (rc = qm_ws(ctx, s, WS_PART, sizeof(double) * (size_t)ncb * ldmax, (void**)&part))) return rc;
-  // activity bits of the row tiles' 16-function groups (the LDS-DMA tile kernel skips zero groups)
-  const int nw = (np / 16 + 31) / 32;
-  uint32_t* mask = nullptr;
-  if (ctx->f64_variant == 4 && ctx->tile_skip && nw <= 64 &&
-      (rc = qm_ws(ctx, s, WS_MASK, sizeof(uint32_t) * (size_t)nw * (ldmax / kTT), (void**)&mask)))
-    return rc;
   const GeomView gv = geom_view(g);
   const MolView mv = mol->view();
   const double h3 = g->step * g->step * g->step;
@@ -2320,17 +2671,9 @@ int density_fp64(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, int 
       if (ctx->f64_variant == 3)
         hipLaunchKernelGGL(k_contract_f64_rows, dim3(tile_grid(nrt, ncb)), dim3(kTWG), 0, s, (const double*)phi, ld,
                            (const double*)mol->M64, np, nrt, ncb, part);
-      else if (ctx->f64_variant == 4) {
-        if (mask)
-          hipLaunchKernelGGL(k_tile_mask, dim3(nrt), dim3(kTT), 0, s, mv, gv, v0, nv, nsub, npts, nw, mask);
-        hipLaunchKernelGGL(k_contract_f64_tiles<true>, dim3(tile_grid(nrt, ncb)), dim3(kTWG), 0, s,
-                           (const double*)phi, ld, (const double*)mol->M64, np, mol->nbf, nrt, ncb, part,
-                           (const uint32_t*)mask, nw);
-      } else {
-        hipLaunchKernelGGL(k_contract_f64_tiles<false>, dim3(tile_grid(nrt, ncb)), dim3(kTWG), 0, s,
-                           (const double*)phi, ld, (const double*)mol->M64, np, mol->nbf, nrt, ncb, part,
-                           (const uint32_t*)nullptr, 0);
-      }
+      else
+        hipLaunchKernelGGL(k_contract_f64_tiles, dim3(tile_grid(nrt, ncb)), dim3(kTWG), 0, s, (const double*)phi, ld,
+                           (const double*)mol->M64, np, nrt, ncb, part);
       QM_CHECK_LAUNCH(ctx);
       if (nsub3 == 1) {
         hipLaunchKernelGGL(k_tiles_finish<TO>, dim3((npts + 255) / 256), dim3(256), 0, s, (const double*)part, ld, ncb,
@@ -2386,7 +2729,7 @@ inline bool split_pre(int v) { return v == 1 || v == 3; }
 
 template <typename T16>
 void launch_split_tiles(hipStream_t s, int v, int blocks, const void* phi, int ld, const float* pscale,
-                        const T16* Ph, const T16* Pl, int np, int nbf, int nrt, int ncb, double* part) {
+                        const T16* Ph, const T16* Pl, int np, int nrt, int ncb, double* part) {
   switch (v) {
     case 1:
       hipLaunchKernelGGL((k_contract_split_tiles<T16, 4, 2, true>), dim3(blocks), dim3(512), 0, s, phi, ld, pscale,
@@ -2395,10 +2738,6 @@ void launch_split_tiles(hipStream_t s, int v, int blocks, const void* phi, int l
     case 2:
       hipLaunchKernelGGL((k_contract_split_tiles<T16, 2, 2>), dim3(blocks), dim3(256), 0, s, phi, ld, pscale, Ph, Pl,
                          np, nrt, ncb, part);
-      break;
-    case 3:
-      hipLaunchKernelGGL(k_contract_split_dma<T16>, dim3(blocks), dim3(512), 0, s, phi, ld, Ph, Pl, np, nbf, nrt, ncb,
-                         part);
       break;
     default:
       hipLaunchKernelGGL((k_contract_split_tiles<T16, 4, 2>), dim3(blocks), dim3(512), 0, s, phi, ld, pscale, Ph, Pl,
@@ -2523,6 +2862,7 @@ int density_split(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, int
   // tables too large for the fused kernel's LDS: basis values written pre-split, LDS DMA tiles
   const int variant = ctx->split_tm == 4 ? 3 : ctx->split_tm;
   if (variant == 5) return density_wide<T16, TO>(ctx, mol, s, g, nsub, out);
+  if (variant == 3) return density_blocks<T16, TO>(ctx, mol, s, g, nsub, out);
   const int np = mol->nbf_pad;
   const int nsub3 = nsub * nsub * nsub;
   const int64_t nvox_tot = npoints(g);
@@ -2573,8 +2913,7 @@ int density_split(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, int
     ProfScope pc(ctx, s, QM_K_DENSITY_SPLIT);
     if (tiled) {
       const int nrt = ld / kTT;
-      launch_split_tiles<T16>(s, variant, tile_grid(nrt, ncb), phi, ld, pscale, Phi, Plo, np, mol->nbf, nrt, ncb,
-                              part);
+      launch_split_tiles<T16>(s, variant, tile_grid(nrt, ncb), phi, ld, pscale, Phi, Plo, np, nrt, ncb, part);
       QM_CHECK_LAUNCH(ctx);
       // pre-split: both factors of the row-dot carry S, divided out here with the volume element
       const float* ps = pre ? nullptr : (const float*)pscale;
@@ -2818,9 +3157,9 @@ struct BChunk {
   int ncb;
   int blk0_phi;         // first block in the round's basis-value (and tiled finish) launch
   int blk0;             // first block in its contraction launch
-  const int2* kg;       // fused kernel: the molecule's function-group table
-  uint32_t* mask;       // FP64 LDS-DMA tiles: activity bits of the row tiles' 16-function groups (or null)
-  int nw;               // mask words per row tile
+  const int2* kg;       // the molecule's function-group table
+  BlockTiles b;         // block tiles: ld / 128 row tiles, their lists and counts
+  int ny;               // block tiles: workgroups per row tile
 };
 
 __device__ __forceinline__ int find_chunk(const BChunk* __restrict__ c, int n, int b, bool phi_launch) {
@@ -2926,25 +3265,76 @@ __global__ __launch_bounds__(kTWG) void kb_contract_f64_rows(const BChunk* __res
   tiled_f64_rows_body(rt, cb, (const double*)q.phi, q.ld, (const double*)q.ph, q.nbf_pad, q.part, q.ld);
 }
 
-// activity bits of every chunk of a round, numbered as the basis-value launch (two 128-point tiles
-// per block of that launch); chunks without a mask are left alone
-__global__ __launch_bounds__(kTT) void kb_tile_mask(const BChunk* __restrict__ c, int n) {
+// block tiles: chunks numbered as the basis-value launch (two row tiles per block of that launch)
+template <int GS>
+__global__ __launch_bounds__(kTT) void kb_tile_list(const BChunk* __restrict__ c, int n, int all) {
   const int pb = blockIdx.x >> 1;
   const BChunk& q = c[find_chunk(c, n, pb, true)];
   const int rt = (pb - q.blk0_phi) * 2 + (blockIdx.x & 1);
-  if (!q.mask || rt >= q.ld / kTT) return;   // uniform per workgroup
-  tile_mask_body(q.mol, q.g, q.v0, q.nvox, 1, q.nvox, rt, q.nw, q.mask);
+  if (rt >= q.b.nT) return;   // uniform per workgroup
+  tile_list_body<GS>(q.mol, q.g, q.b, rt, all, (uint16_t*)q.b.list, (int*)q.b.cnt);
 }
 
-template <bool DMA>
+__global__ __launch_bounds__(kPhiThreads) void kb_phi_f64_blocks(const BChunk* __restrict__ c, int n) {
+  const BChunk& q = c[find_chunk(c, n, blockIdx.x, true)];
+  const int rt = __builtin_amdgcn_readfirstlane((blockIdx.x - q.blk0_phi) * 2 + threadIdx.x / kTT);
+  if (rt < q.b.nT) phi_f64_blocks_body(q.mol, q.kg, q.g, q.b, rt, threadIdx.x % kTT, blockIdx.y, gridDim.y, (double*)q.phi);
+}
+
+__global__ __launch_bounds__(kTWG, 4) void kb_contract_f64_blocks(const BChunk* __restrict__ c, int n) {
+  const BChunk& q = c[find_chunk(c, n, blockIdx.x, false)];
+  int rt, y;
+  if (tile_coords(blockIdx.x - q.blk0, q.b.nT, q.ny, rt, y))
+    f64_block_tile(rt, q.ny - 1 - y, q.ny, (const double*)q.phi, (const double*)q.ph, q.nbf_pad, q.b, q.part);
+}
+
+template <typename T16>
+__global__ __launch_bounds__(kTT) void kb_phi_split_blocks(const BChunk* __restrict__ c, int n) {
+  const BChunk& q = c[find_chunk(c, n, blockIdx.x, true)];
+  const int rt = __builtin_amdgcn_readfirstlane((blockIdx.x - q.blk0_phi) * 2 + threadIdx.x / 64);
+  if (rt < q.b.nT)
+    phi_split_blocks_body<kTT, T16>(q.mol, q.l2e, q.kg, q.g, q.b, rt, threadIdx.x % 64, blockIdx.y, gridDim.y, q.phis,
+                               (T16*)q.phi);
+}
+
+template <typename T16>
+__global__ __launch_bounds__(512, 4) void kb_contract_split_blocks(const BChunk* __restrict__ c, int n) {
+  const BChunk& q = c[find_chunk(c, n, blockIdx.x, false)];
+  int rt, y;
+  if (tile_coords(blockIdx.x - q.blk0, q.b.nT, q.ny, rt, y))
+    split_block_tile<T16>(rt, q.ny - 1 - y, q.ny, (const T16*)q.phi, (const T16*)q.ph, (const T16*)q.pl, q.nbf_pad, q.b,
+                          2 * q.ncb, q.part);
+}
+
+template <bool SPLIT, typename TO>
+__global__ __launch_bounds__(kPhiThreads) void kb_blocks_finish(const BChunk* __restrict__ c, int n) {
+  const BChunk& q = c[find_chunk(c, n, blockIdx.x, true)];
+  blocks_finish_body<SPLIT, TO>((int64_t)(blockIdx.x - q.blk0_phi) * kPhiThreads + threadIdx.x, q.g, q.b, q.part,
+                                q.scale, (TO*)q.out);
+}
+
+// the basis-value launches of a round of block tiles
+template <typename T>
+void launch_batch_blocks_phi(hipStream_t s, const BChunk* c, int n, int pairs, int ng, int all) {
+  constexpr bool f64 = std::is_same<T, double>::value;
+  const dim3 grid(pairs, phi_split(pairs, f64 ? 2 * ng : 4 * ng));
+  hipLaunchKernelGGL(kb_tile_list<f64 ? 4 : 5>, dim3(2 * pairs), dim3(kTT), 0, s, c, n, all);
+  if constexpr (f64) hipLaunchKernelGGL(kb_phi_f64_blocks, grid, dim3(kPhiThreads), 0, s, c, n);
+  else hipLaunchKernelGGL(kb_phi_split_blocks<T>, grid, dim3(kTT), 0, s, c, n);
+}
+
+template <bool SPLIT>
+void launch_batch_blocks_finish(hipStream_t s, const BChunk* c, int n, int blocks, int out_dtype) {
+  if (out_dtype == QM_F64)
+    hipLaunchKernelGGL((kb_blocks_finish<SPLIT, double>), dim3(blocks), dim3(kPhiThreads), 0, s, c, n);
+  else hipLaunchKernelGGL((kb_blocks_finish<SPLIT, float>), dim3(blocks), dim3(kPhiThreads), 0, s, c, n);
+}
+
 __global__ __launch_bounds__(kTWG) void kb_contract_f64_tiles(const BChunk* __restrict__ c, int n) {
   const BChunk& q = c[find_chunk(c, n, blockIdx.x, false)];
   int rt, cb;
   if (!tile_coords(blockIdx.x - q.blk0, q.ld / kTT, q.ncb, rt, cb)) return;
-  if (DMA)
-    tiled_f64_dma_body<kF64Ks, 32 / kF64Ks>(rt, cb, (const double*)q.phi, q.ld, (const double*)q.ph, q.nbf_pad,
-                                            q.mol.nbf, q.ncb, q.part, q.ld, q.mask, q.nw);
-  else tiled_f64_body(rt, cb, (const double*)q.phi, q.ld, (const double*)q.ph, q.nbf_pad, q.part, q.ld);
+  tiled_f64_body(rt, cb, (const double*)q.phi, q.ld, (const double*)q.ph, q.nbf_pad, q.part, q.ld);
 }
 
 template <typename T16, int WR, int WC, bool PRE = false>
@@ -2957,20 +3347,10 @@ __global__ __launch_bounds__(64 * WR * WC) void kb_contract_split_tiles(const BC
 }
 
 template <typename T16>
-__global__ __launch_bounds__(512, 4) void kb_contract_split_dma(const BChunk* __restrict__ c, int n) {
-  const BChunk& q = c[find_chunk(c, n, blockIdx.x, false)];
-  int rt, cb;
-  if (!tile_coords(blockIdx.x - q.blk0, q.ld / kTT, q.ncb, rt, cb)) return;
-  tiled_dma_body<T16>(rt, cb, (const T16*)q.phi, q.ld, (const T16*)q.ph, (const T16*)q.pl, q.nbf_pad, q.mol.nbf, q.ncb,
-                      q.part, q.ld);
-}
-
-template <typename T16>
 void launch_batch_split_tiles(hipStream_t s, int v, int blocks, const BChunk* c, int n) {
   switch (v) {
     case 1: hipLaunchKernelGGL((kb_contract_split_tiles<T16, 4, 2, true>), dim3(blocks), dim3(512), 0, s, c, n); break;
     case 2: hipLaunchKernelGGL((kb_contract_split_tiles<T16, 2, 2>), dim3(blocks), dim3(256), 0, s, c, n); break;
-    case 3: hipLaunchKernelGGL(kb_contract_split_dma<T16>, dim3(blocks), dim3(512), 0, s, c, n); break;
     default: hipLaunchKernelGGL((kb_contract_split_tiles<T16, 4, 2>), dim3(blocks), dim3(512), 0, s, c, n); break;
   }
 }
@@ -3004,6 +3384,7 @@ struct Round {
   std::vector<std::pair<int, std::pair<size_t, size_t>>> groups;   // (nt, [first, count))
   std::vector<int> group_blocks;
   int phi_blocks;
+  int max_ncb = 1;                          // column blocks of the round's largest chunk
 };
 
 // Charge normalisation of every molecule of a batch: Q <- Q sum Z / sum Q (device-side factors).
@@ -3136,15 +3517,22 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
   const bool tiled = f64 ? ctx->f64_variant >= 2 : split_tiled(sv);
   // basis values written scaled and split (same bytes as FP32)
   const bool pre = !f64 && split_pre(sv);
+  // partial sums of a chunk: one per group (block tiles) or column block and point
+  auto part_bytes = [f64](const BChunk& c) {
+    return sizeof(double) * (size_t)(!c.b.nT ? c.ncb : f64 ? c.b.ng : 2 * c.ncb) * c.ld;
+  };
+  bool blocks = f64 || sv == 3;   // block tiles
+  for (int i = 0; f64 && i < nmol; ++i) blocks = blocks && f64_blocks(ctx, mols[i]);
+  const int gs = f64 ? 4 : 5;     // log2 of the functions per group
   // chunks per molecule, packed into rounds of at most kPhiBudget bytes of basis values
   std::vector<BChunk> table;
   std::vector<Round> rounds;
   std::vector<BChunk> cur;
   size_t cur_bytes = 0, cur_ps = 0, cur_part = 0;
-  size_t mask_bytes = 0;   // activity bits of every chunk (FP64 LDS-DMA tiles), kept for the whole call
+  size_t cnt_bytes = 0, list_bytes = 0;   // group lists of every chunk's block tiles, kept for the whole call
   auto flush = [&]() {
     if (cur.empty()) return;
-    Round r;
+    Round r{};
     r.first = table.size();
     r.count = cur.size();
     std::stable_sort(cur.begin(), cur.end(), [](const BChunk& a, const BChunk& b) { return a.nt < b.nt; });
@@ -3157,14 +3545,16 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
     size_t k = 0;
     while (k < cur.size()) {
       size_t e = k;
-      int blocks = 0;
+      int nblk = 0;
       while (e < cur.size() && cur[e].nt == cur[k].nt) {
-        cur[e].blk0 = blocks;
-        blocks += tiled ? tile_grid(cur[e].ld / kTT, cur[e].ncb) : cur[e].ld / tm;   // tiled: multiples of 8
+        cur[e].blk0 = nblk;
+        const int per = blocks ? cur[e].ny : cur[e].ncb;
+        nblk += tiled ? tile_grid(cur[e].ld / kTT, per) : cur[e].ld / tm;   // tiled: multiples of 8
+        r.max_ncb = std::max(r.max_ncb, cur[e].ncb);
         ++e;
       }
       r.groups.push_back({cur[k].nt, {r.first + k, e - k}});
-      r.group_blocks.push_back(blocks);
+      r.group_blocks.push_back(nblk);
       k = e;
     }
     table.insert(table.end(), cur.begin(), cur.end());
@@ -3177,9 +3567,12 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
   for (int i = 0; i < nmol; ++i) {
     qm_mol* m = mols[i];
     const int np = m->nbf_pad;
-    const int64_t N = npoints(&geoms[i]);
+    // block tiles: points of whole tiles, in tile order
+    const int ng = (m->nbf + (1 << gs) - 1) >> gs;
+    const int nphi = blocks ? ng << gs : np;   // functions stored per point
+    const int64_t N = blocks ? block_tiles(geom_view(&geoms[i])) * kTT : npoints(&geoms[i]);
     const int64_t cap = std::max<int64_t>(kTileM, std::min<int64_t>(kBatchChunk,
-                                          (int64_t)(kPhiBudget / ((size_t)np * elt)) / kTileM * kTileM));
+                                          (int64_t)(kPhiBudget / ((size_t)nphi * elt)) / kTileM * kTileM));
     for (int64_t v0 = 0; v0 < N; v0 += cap) {
       BChunk c{};
       c.mol = m->view();
@@ -3191,19 +3584,23 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
       c.nbf_pad = np;
       c.nt = tiled ? 0 : pick_nt(np);     // tiled chunks form one launch per round
       c.ncb = (f64 && ctx->f64_variant == 3) ? np / kRN : (np + kTT - 1) / kTT;
-      if (f64 && ctx->f64_variant == 4 && ctx->tile_skip && (np / 16 + 31) / 32 <= 64) {
-        c.nw = (np / 16 + 31) / 32;
-        c.mask = (uint32_t*)(uintptr_t)mask_bytes;   // offset for now, rebased below
-        mask_bytes += sizeof(uint32_t) * (size_t)c.nw * (c.ld / kTT);
+      if (blocks) {
+        c.kg = m->kgroups;
+        c.ncb = f64 ? (ng + 7) / 8 : (ng + 3) / 4;
+        c.ny = block_split(c.ld / kTT, c.ncb, f64);
+        c.b = BlockTiles{(int)(v0 / kTT), c.ld / kTT, 1, ng, (const uint16_t*)(uintptr_t)list_bytes,
+                         (const int*)(uintptr_t)cnt_bytes};   // offsets for now, rebased below
+        list_bytes += sizeof(uint16_t) * (size_t)ng * c.b.nT;
+        cnt_bytes += sizeof(int) * (size_t)c.b.nT;
       }
-      const size_t bytes = (size_t)np * c.ld * elt;
+      const size_t bytes = (size_t)nphi * c.ld * elt;
       if (cur_bytes + bytes > kPhiBudget) flush();
       c.phi = (void*)(uintptr_t)cur_bytes;            // offsets for now, rebased below
       c.pscale = (float*)(uintptr_t)cur_ps;
       c.part = (double*)(uintptr_t)cur_part;
       cur_bytes += bytes;
       cur_ps += (size_t)c.ld * sizeof(float);
-      if (tiled) cur_part += sizeof(double) * (size_t)c.ncb * c.ld;
+      if (tiled) cur_part += part_bytes(c);
       const double h3 = geoms[i].step * geoms[i].step * geoms[i].step;
       if (f64) {
         c.ph = ctx->f64_variant == 1 ? m->P64 : m->M64;   // the LDS-staged kernel takes the triangular form
@@ -3228,9 +3625,9 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
     size_t b = 0, p = 0, q = 0;
     for (size_t k = 0; k < r.count; ++k) {
       const BChunk& c = table[r.first + k];
-      b = std::max(b, (size_t)(uintptr_t)c.phi + (size_t)c.nbf_pad * c.ld * elt);
+      b = std::max(b, (size_t)(uintptr_t)c.phi + (size_t)(c.b.nT ? c.b.ng << gs : c.nbf_pad) * c.ld * elt);
       p = std::max(p, (size_t)(uintptr_t)c.pscale + (size_t)c.ld * sizeof(float));
-      if (tiled) q = std::max(q, (size_t)(uintptr_t)c.part + sizeof(double) * (size_t)c.ncb * c.ld);
+      if (tiled) q = std::max(q, (size_t)(uintptr_t)c.part + part_bytes(c));
     }
     max_bytes = std::max(max_bytes, b);
     max_ps = std::max(max_ps, p);
@@ -3242,9 +3639,12 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
   if (tiled && (rc = qm_ws(ctx, s, WS_PART, max_part, &pt))) return rc;
   if ((rc = qm_ws(ctx, s, WS_BATCH, sizeof(BChunk) * table.size(), &dtab))) return rc;
   void* mk = nullptr;
-  if (mask_bytes && (rc = qm_ws(ctx, s, WS_MASK, mask_bytes, &mk))) return rc;
+  if (blocks && (rc = qm_ws(ctx, s, WS_MASK, cnt_bytes + list_bytes, &mk))) return rc;
   for (BChunk& c : table) {
-    c.mask = c.nw ? (uint32_t*)((char*)mk + (size_t)(uintptr_t)c.mask) : nullptr;
+    if (blocks) {
+      c.b.cnt = (const int*)((char*)mk + (size_t)(uintptr_t)c.b.cnt);
+      c.b.list = (const uint16_t*)((char*)mk + cnt_bytes + (size_t)(uintptr_t)c.b.list);
+    }
     c.phi = (char*)phi + (size_t)(uintptr_t)c.phi;
     c.pscale = (float*)((char*)ps + (size_t)(uintptr_t)c.pscale);
     c.part = tiled ? (double*)((char*)pt + (size_t)(uintptr_t)c.part) : nullptr;
@@ -3255,11 +3655,14 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
   for (const Round& r : rounds) {
     {
       ProfScope pp(ctx, s, f64 ? QM_K_PHI : QM_K_PHI_SPLIT);
-      if (f64) {
+      const BChunk* c = dt + r.first;
+      const int n = (int)r.count, ng = (f64 ? 8 : 4) * r.max_ncb;
+      if (blocks && f64) launch_batch_blocks_phi<double>(s, c, n, r.phi_blocks, ng, !ctx->tile_skip);
+      else if (blocks && precision == QM_PREC_F16X3) launch_batch_blocks_phi<_Float16>(s, c, n, r.phi_blocks, ng, 0);
+      else if (blocks) launch_batch_blocks_phi<__bf16>(s, c, n, r.phi_blocks, ng, 0);
+      else if (f64)
         hipLaunchKernelGGL(kb_phi_f64, dim3(r.phi_blocks), dim3(kPhiThreads), 0, s, dt + r.first, (int)r.count);
-        if (mask_bytes)
-          hipLaunchKernelGGL(kb_tile_mask, dim3(2 * r.phi_blocks), dim3(kTT), 0, s, dt + r.first, (int)r.count);
-      } else if (pre && precision == QM_PREC_F16X3)
+      else if (pre && precision == QM_PREC_F16X3)
         hipLaunchKernelGGL(kb_phi_split<_Float16>, dim3(r.phi_blocks), dim3(kPhiThreads), 0, s, dt + r.first,
                            (int)r.count);
       else if (pre)
@@ -3273,37 +3676,44 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
       const int nt = r.groups[gi].first;
       const BChunk* gc = dt + r.groups[gi].second.first;
       const int gn = (int)r.groups[gi].second.second;
-      const int blocks = r.group_blocks[gi];
+      const int nblk = r.group_blocks[gi];
       ProfScope pc(ctx, s, f64 ? QM_K_DENSITY_CONTRACT : QM_K_DENSITY_SPLIT);
       if (tiled) {
         if (f64 && ctx->f64_variant == 3)
-          hipLaunchKernelGGL(kb_contract_f64_rows, dim3(blocks), dim3(kTWG), 0, s, gc, gn);
-        else if (f64 && ctx->f64_variant == 4)
-          hipLaunchKernelGGL(kb_contract_f64_tiles<true>, dim3(blocks), dim3(kTWG), 0, s, gc, gn);
+          hipLaunchKernelGGL(kb_contract_f64_rows, dim3(nblk), dim3(kTWG), 0, s, gc, gn);
+        else if (blocks) {
+          const dim3 grid(nblk);
+          if (f64) hipLaunchKernelGGL(kb_contract_f64_blocks, grid, dim3(kTWG), 0, s, gc, gn);
+          else if (precision == QM_PREC_F16X3)
+            hipLaunchKernelGGL(kb_contract_split_blocks<_Float16>, grid, dim3(512), 0, s, gc, gn);
+          else hipLaunchKernelGGL(kb_contract_split_blocks<__bf16>, grid, dim3(512), 0, s, gc, gn);
+        }
         else if (f64)
-          hipLaunchKernelGGL(kb_contract_f64_tiles<false>, dim3(blocks), dim3(kTWG), 0, s, gc, gn);
+          hipLaunchKernelGGL(kb_contract_f64_tiles, dim3(nblk), dim3(kTWG), 0, s, gc, gn);
         else if (precision == QM_PREC_F16X3)
-          launch_batch_split_tiles<_Float16>(s, sv, blocks, gc, gn);
+          launch_batch_split_tiles<_Float16>(s, sv, nblk, gc, gn);
         else
-          launch_batch_split_tiles<__bf16>(s, sv, blocks, gc, gn);
+          launch_batch_split_tiles<__bf16>(s, sv, nblk, gc, gn);
         QM_CHECK_LAUNCH(ctx);
         // finish over the whole round: chunk blocks numbered as in the basis-value launch
         const int per_point = !f64 && !pre;   // per-point scales to divide out
-        if (out_dtype == QM_F64)
+        if (blocks && f64) launch_batch_blocks_finish<false>(s, dt + r.first, (int)r.count, r.phi_blocks, out_dtype);
+        else if (blocks) launch_batch_blocks_finish<true>(s, dt + r.first, (int)r.count, r.phi_blocks, out_dtype);
+        else if (out_dtype == QM_F64)
           hipLaunchKernelGGL(kb_tiles_finish<double>, dim3(r.phi_blocks), dim3(kPhiThreads), 0, s, dt + r.first,
                              (int)r.count, per_point);
         else
           hipLaunchKernelGGL(kb_tiles_finish<float>, dim3(r.phi_blocks), dim3(kPhiThreads), 0, s, dt + r.first,
                              (int)r.count, per_point);
       } else if (f64) {
-        if (out_dtype == QM_F64) launch_batch_f64<double>(s, nt, gc, gn, blocks, ctx->f64_variant == 1);
-        else launch_batch_f64<float>(s, nt, gc, gn, blocks, ctx->f64_variant == 1);
+        if (out_dtype == QM_F64) launch_batch_f64<double>(s, nt, gc, gn, nblk, ctx->f64_variant == 1);
+        else launch_batch_f64<float>(s, nt, gc, gn, nblk, ctx->f64_variant == 1);
       } else if (precision == QM_PREC_F16X3) {
-        if (out_dtype == QM_F64) launch_batch_split<_Float16, double>(s, nt, tm, gc, gn, blocks);
-        else launch_batch_split<_Float16, float>(s, nt, tm, gc, gn, blocks);
+        if (out_dtype == QM_F64) launch_batch_split<_Float16, double>(s, nt, tm, gc, gn, nblk);
+        else launch_batch_split<_Float16, float>(s, nt, tm, gc, gn, nblk);
       } else {
-        if (out_dtype == QM_F64) launch_batch_split<__bf16, double>(s, nt, tm, gc, gn, blocks);
-        else launch_batch_split<__bf16, float>(s, nt, tm, gc, gn, blocks);
+        if (out_dtype == QM_F64) launch_batch_split<__bf16, double>(s, nt, tm, gc, gn, nblk);
+        else launch_batch_split<__bf16, float>(s, nt, tm, gc, gn, nblk);
       }
       QM_CHECK_LAUNCH(ctx);
     }

@@ -23,9 +23,10 @@ struct DevShell {
   int L;        // 0..2
   int nprim;    // primitives
   int poff;     // first primitive
-  int bf;       // first basis function
+  int bf;       // first basis function, internal order (qm_mol_create: shells by cutoff, then along a chain of atoms)
   float rcut2;  // squared distance (bohr^2) beyond which every primitive is cut
-  int pad_[2];
+  int bf_user;  // first basis function in the caller's order (rows of the density matrix, qm_basis_points)
+  int pair;     // 1 + first primitive of the next shell if that one has the same nucleus and exponents, else 0
 };
 
 struct MolView {
@@ -72,7 +73,7 @@ enum WsSlot {
   WS_BATCH2,
   WS_VNE,          // diffusion V_ne partials and loop state
   WS_PART,         // per-column-block partial densities of the tiled contraction
-  WS_MASK,         // per-row-tile activity bits of the basis-function groups
+  WS_MASK,         // per-tile lists of the active basis-function groups
   WS_COUNT
 };
 
@@ -113,7 +114,7 @@ struct qm_ctx {
   void* gto_staged = nullptr;           // pinned staging of GTO distribution tables (grown as needed;
   size_t gto_staged_bytes = 0;          // every upload from it completes before the build returns)
   int split_tm = 3;                     // split contraction variant (0..3 tiled, 4 fused, 64 / 128 all-columns)
-  int f64_variant = 4;                  // FP64 contraction: 0 wave-cyclic, 1 dense per-wave, 2 tiled, 3 rows, 4 tiled + DMA
+  int f64_variant = 4;                  // FP64 contraction: 0 wave-cyclic, 1 dense per-wave, 2 tiled, 3 rows, 4 block tiles + DMA
   int jacobi_zs = 0;                    // z planes per Jacobi sweep workgroup (0 = chosen per grid)
   int jacobi_pairs = 1;                 // FP32 two-sweep passes with two columns per lane (even nx)
   int tile_skip = 1;                    // contractions skip basis-function groups that are zero on a row tile
@@ -128,13 +129,13 @@ struct qm_mol {
   double2* prims = nullptr;
   float2* prims_l2e = nullptr;      // (alpha log2 e, coeff) in FP32 for the FP32 basis kernel
   int2* kgroups = nullptr;          // per 8 functions (nbf_pad / 8): shell of the first function, its m index
-  // host copies (used to build per-request tables)
+  // host copies (used to build per-request tables), shells in the internal order
   std::vector<double> xyz, Z;
   std::vector<DevShell> h_shells;
   std::vector<double> h_alpha, h_coeff;
   // density matrix: total P_eff = 2 * (tril(dm) + tril(dm,-1)^T), nbf_pad^2, zero padded
   bool has_dm = false;
-  std::vector<double> h_P;          // nbf x nbf total P_eff (host)
+  std::vector<double> h_P;          // nbf x nbf total P_eff (host, internal order)
   double* P64 = nullptr;            // [nbf_pad][nbf_pad]
   double* M64 = nullptr;            // upper triangle of P, off-diagonal doubled (same shape)
   void* P16 = nullptr;              // fp16 hi/lo, K8-interleaved, 2 planes

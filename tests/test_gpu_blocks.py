@@ -1,0 +1,75 @@
+"""Block tiles of the density contractions (8 x 4 x 4 voxels, lists of active function groups) at their edges:
+grids smaller than a tile, part-filled edge tiles, sub-points, tiles with no active group, the shell order."""
+import ctypes
+
+import numpy
+import pytest
+from conftest import BASIS
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(mol):
+    from oracle.basisfile import read_basis
+    from oracle.system import make_system
+    return make_system(mol.types, mol.coords, mol.dm, read_basis(BASIS))
+
+
+def _raw(mol, geom, subgrid, prec):
+    import torch
+    from qmtools import _native as nat
+    from qmtools.qmtools import device_molecule
+    out = torch.full((geom[0] * geom[1] * geom[2],), float("nan"), dtype=torch.float64, device="cuda")
+    nat.call("qm_density", device_molecule(mol).handle, nat.stream(), ctypes.byref(nat.geom(geom)), subgrid, prec,
+             nat.QM_F64, nat.dptr(out), 0, None)
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (7, 3, 5), (8, 4, 4), (9, 4, 5), (33, 2, 17), (17, 21, 6)])
+@pytest.mark.parametrize("natoms,subgrid", [(1, 1), (1, 3), (12, 1), (30, 2)])
+def test_block_tiles_ragged(shape, natoms, subgrid):
+    """The same gates as on full grids: 1e-10 (FP64), 1e-6 (split) of the largest value."""
+    import qmtools
+    from oracle import density as od
+    from qmtools import _native as nat, synth
+    mol = synth.synthetic_molecule(natoms, 6, qmtools.BasisSet(BASIS))
+    h = 0.7
+    o = mol.coords.mean(0) - 0.5 * h * numpy.array(shape) + 0.1
+    print("[case] block tiles", shape, natoms, subgrid, flush=True)
+    want = od.density_grid_raw(_system(mol), *shape, h, o, subgrid)
+    for prec, tol in ((nat.QM_PREC_FP64, 1e-10), (nat.QM_PREC_F16X3, 1e-6)):
+        got = _raw(mol, (*shape, h, tuple(o)), subgrid, prec)
+        assert numpy.abs(got - want).max() <= tol * numpy.abs(want).max()
+
+
+def test_block_tiles_without_active_groups():
+    """A grid whose far tiles are beyond every cutoff: exactly zero there, the oracle's values elsewhere."""
+    import qmtools
+    from oracle import density as od
+    from qmtools import _native as nat, synth
+    mol = synth.synthetic_molecule(4, 9, qmtools.BasisSet(BASIS))
+    shape, h = (80, 5, 4), 1.0
+    o = mol.coords.mean(0) - 2.0
+    print("[case] block tiles, inactive", flush=True)
+    want = od.density_grid_raw(_system(mol), *shape, h, o, 1)
+    for prec, tol in ((nat.QM_PREC_FP64, 1e-10), (nat.QM_PREC_F16X3, 1e-6)):
+        got = _raw(mol, (*shape, h, tuple(o)), 1, prec)
+        assert numpy.abs(got - want).max() <= tol * numpy.abs(want).max()
+        assert (got.reshape(4, 5, 80)[:, :, 40:] == 0.0).all()
+
+
+def test_basis_points_in_the_callers_order():
+    """qm_basis_points writes rows in the caller's function order, whatever the internal shell order."""
+    import torch
+    import qmtools
+    from oracle import density as od
+    from qmtools import _native as nat, synth
+    from qmtools.qmtools import device_molecule
+    mol = synth.synthetic_molecule(9, 4, qmtools.BasisSet(BASIS))
+    pts = numpy.random.default_rng(3).normal(size=(70, 3)) * 3.0
+    want = od.basis_on_points(_system(mol), pts).T
+    d = torch.tensor(pts.ravel(), device="cuda")
+    phi = torch.empty(mol.nbf * 70, dtype=torch.float64, device="cuda")
+    nat.call("qm_basis_points", device_molecule(mol).handle, nat.stream(), nat.dptr(d), 70, nat.dptr(phi))
+    got = phi.cpu().numpy().reshape(mol.nbf, 70)
+    assert numpy.abs(got - want).max() <= 1e-13 * numpy.abs(want).max()
