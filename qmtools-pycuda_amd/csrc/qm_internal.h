@@ -74,6 +74,7 @@ enum WsSlot {
   WS_VNE,          // diffusion V_ne partials and loop state
   WS_PART,         // per-column-block partial densities of the tiled contraction
   WS_MASK,         // per-tile lists of the active basis-function groups
+  WS_SINE,         // sine-transform matrices and partial sums
   WS_COUNT
 };
 

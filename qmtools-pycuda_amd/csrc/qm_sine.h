@@ -1,0 +1,42 @@
+// Sine transforms of a grid's interior (sine.hip), used by the relaxations' closed forms.
+#pragma once
+
+#include "qm_internal.h"
+
+struct SinePlan {
+  int nx, ny;               // grid row and plane sizes
+  int m[3], ld[3];          // interior points per axis, row length of S
+  const double* S[3];       // S_kn = sqrt(2 / (m + 1)) sin(pi k n / (m + 1)), zero padded
+  const double* s2[3];      // sin^2(pi k / (2 (m + 1))), k = 1 .. m
+  double* part;             // partial sums of an x pass
+  double* sum;              // their sum
+  int* flag;                // set when a residual is not finite
+};
+
+enum { SINE_JACOBI = 0, SINE_VNE = 1 };     // which sweep's eigenvalue a
+enum { SINE_SUM = 0, SINE_POWER = 1 };      // (1 - a^n) / (1 - a), a^n
+
+struct SineFactor {
+  int sweep, kind;
+  double n;                 // whole number below 2^53
+  int odd;                  // n is odd
+  double w0, w1, w2, w3;    // SINE_VNE: 1 - a = w0 - (w1 sum c + w2 sum c c' + w3 c c' c''), c = cos theta per axis
+};
+
+bool qm_sine_fits(const qm_geom* g);   // every axis has 1 .. 1024 interior points
+// tables in the context's workspace, valid on s until the next plan; clears the flag
+int qm_sine_plan(qm_ctx* ctx, hipStream_t s, const qm_geom* g, SinePlan* p);
+// The passes read and write interior points only and work in place where one buffer is given.
+// x and y transforms of (one Jacobi sweep of v) - v; sets the plan's flag if that is not finite somewhere
+int qm_sine_residual_xy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* rho, const double* v, double h,
+                        double* out);
+int qm_sine_xy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* a);
+int qm_sine_z(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* a);
+// z transform, factor, z and y transforms
+int qm_sine_z_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const SineFactor& f, double* a);
+// factor times a spectrum, z and y transforms (the same bits as qm_sine_z and then this, or the call above)
+int qm_sine_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const SineFactor& f, const double* spectrum,
+                     double* out);
+int qm_sine_x_add(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, double* v);   // v += x transform of a
+// sum over the interior of |x transform of a| (v null) or |v + x transform of a|; waits for s
+int qm_sine_x_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, const double* v, double* host_sum);

@@ -1,0 +1,343 @@
+// Sine transforms (DST-I) of the interior of a grid, as FP64 matrix products.
+//
+// Both relaxations of the library are linear and act on the interior points only, with the outer layer
+// held: the Jacobi sweep (reference kernel_hartree.cu:85-171) and the diffusion V_ne sweep (kernel_vne.cu:13-128).
+// Their neighbour sums are diagonal in the products of sin(pi k n / (m + 1)) along each axis (m interior
+// points), so a given number of sweeps has a closed form: with increments d_j = A^j d_0 the field after n
+// sweeps is V_0 + sum_{j<n} d_j, a multiplication by (1 - a^n) / (1 - a) between two transforms, a being the
+// eigenvalue of the sweep.  A fixed sweep count is then 6 one-axis transforms whatever the count, and the
+// change of the n-th sweep (the convergence test) is 3 transforms of a^(n-1) times the stored spectrum.
+//
+// One axis is a product with the symmetric m x m matrix S_kn = sqrt(2 / (m + 1)) sin(pi k n / (m + 1)), which
+// is its own inverse.  A matrix product takes 2 m flops per point where an FFT would take about
+// 2.5 log2 m per real point, but it runs on the FP64 matrix cores for any m (an FFT of the odd extension has
+// length 2 (m + 1) = 510 for 256 points, with factors 17 and 51), and one pass reads and writes each
+// value once like an FFT pass: 256^3, 6 transforms: 50 GFLOP, 1.6 GB.
+//
+// Kernel: a workgroup of 8 waves owns 16 LT lines and keeps their values in LDS ([line tile][n][16 lines]:
+// an MFMA operand row is 128 contiguous bytes, and 4 consecutive rows cover all 64 banks); wave w owns the row tiles w,
+// w + 8, .. of the result and reads S from L2 (64 points: 32 KB, 254: 516 KB) straight into operands.  Lines are
+// read whole before anything is stored, so a pass works in place.
+#include <algorithm>
+#include <cmath>
+
+#include <type_traits>
+
+#include "qm_sine.h"
+
+namespace {
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+constexpr int kThreads = 512;
+constexpr int kMaxM = 1024;       // interior points per axis (139 KB of LDS)
+
+enum Load { LOAD_PLAIN, LOAD_RESIDUAL, LOAD_SCALED };
+enum Store { STORE_PLAIN, STORE_ADD, STORE_SUM, STORE_SUMV };
+
+struct Args {
+  SinePlan p;
+  const double* in;
+  double* out;              // STORE_ADD: the field that receives the sum; STORE_SUMV: the field
+  const double* rho;        // LOAD_RESIDUAL: in is V, the result is one Jacobi sweep minus V
+  double hinv;
+  SineFactor f;
+  double* part;             // STORE_SUM: sum |x|, STORE_SUMV: sum |out + x|, one per workgroup
+};
+
+// q = 1 - a and c = 1 + a of the sweep's eigenvalue a at mode (kx, ky, kz) (0-based), both without
+// cancellation at their small ends for the Jacobi sweep: a = (cos x + cos y + cos z) / 3.
+// Returns a^n (SINE_POWER) or (1 - a^n) / (1 - a) (SINE_SUM).
+__device__ __forceinline__ double factor(const SinePlan& p, const SineFactor& f, int kx, int ky, int kz) {
+  double q, c;
+  const double sx = p.s2[0][kx], sy = p.s2[1][ky], sz = p.s2[2][kz];   // sin^2(theta / 2)
+  if (f.sweep == SINE_JACOBI) {
+    q = (sx + sy + sz) * (2.0 / 3.0);
+    c = (p.s2[0][p.m[0] - 1 - kx] + p.s2[1][p.m[1] - 1 - ky] + p.s2[2][p.m[2] - 1 - kz]) * (2.0 / 3.0);
+  } else {
+    const double cx = 1.0 - 2.0 * sx, cy = 1.0 - 2.0 * sy, cz = 1.0 - 2.0 * sz;
+    q = f.w0 - (f.w1 * (cx + cy + cz) + f.w2 * (cx * cy + cx * cz + cy * cz) + f.w3 * cx * cy * cz);
+    c = 2.0 - q;
+  }
+  // log |a| from the smaller of 1 - a and 1 + a (with a near 0 both may round to just above 1)
+  const bool pos = q < 1.0;
+  const double la = log1p(-fmin(pos ? q : c, 1.0));
+  if (f.kind == SINE_POWER) {
+    const double v = exp(f.n * la);
+    return !pos && f.odd ? -v : v;
+  }
+  if (fabs(q) < 1e-290) return f.n;
+  if (pos) return -expm1(f.n * la) / q;
+  const double v = exp(f.n * la);
+  return (1.0 - (f.odd ? -v : v)) / q;
+}
+
+template <int LT, int RT, int AX, int LOAD, bool MID, int STORE>
+__global__ __launch_bounds__(kThreads) void k_sine(Args a) {
+  __shared__ __align__(16) double x[LT][128 * RT][16];
+  __shared__ int64_t base[16 * LT];   // first interior point of each line
+  __shared__ int2 mode[16 * LT];      // its indices along the two other axes
+  const SinePlan& p = a.p;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  const int m = p.m[AX], ld = p.ld[AX];
+  const int m0 = AX == 0 ? p.m[1] : p.m[0];   // fast one of the other axes
+  const int m1 = AX == 2 ? p.m[1] : p.m[2];
+  const int64_t nx = p.nx, nxy = (int64_t)p.nx * p.ny;
+  const int64_t stride = AX == 0 ? 1 : AX == 1 ? nx : nxy;
+  const int64_t nl = (int64_t)m0 * m1, l0 = (int64_t)blockIdx.x * (16 * LT);
+  if (t < 16 * LT) {
+    const int64_t l = min(l0 + t, nl - 1);
+    const int u = (int)(l % m0), w = (int)(l / m0);
+    base[t] = AX == 0 ? 1 + nx * (1 + u) + nxy * (1 + w)
+                      : AX == 1 ? (1 + u) + nx + nxy * (1 + w) : (1 + u) + nx * (1 + w) + nxy;
+    mode[t] = make_int2(u, w);
+  }
+  __syncthreads();
+  // mode (kx, ky, kz) of element n of line t
+  auto fac = [&](int line, int n) __attribute__((always_inline)) -> double {
+    const int2 u = mode[line];
+    return AX == 0 ? factor(p, a.f, n, u.x, u.y) : AX == 1 ? factor(p, a.f, u.x, n, u.y) : factor(p, a.f, u.x, u.y, n);
+  };
+  const int rows = (m + 15) / 16 * 16;
+  bool bad = false;
+  // lines along x: 16 threads per 128 bytes of a line; else consecutive threads take neighbouring lines
+  for (int e = t; e < rows * 16 * LT; e += kThreads) {
+    const int line = AX == 0 ? (e >> 4) % (16 * LT) : e % (16 * LT);
+    const int n = AX == 0 ? (e & 15) + 16 * ((e >> 4) / (16 * LT)) : e / (16 * LT);
+    double v = 0.0;
+    if (n < m) {
+      const int64_t idx = base[line] + n * stride;
+      if (LOAD == LOAD_RESIDUAL) {
+        const double* __restrict__ V = a.in;
+        double s = V[idx - 1] + V[idx + 1];
+        s += V[idx + nx];
+        s += V[idx - nx];
+        s += V[idx + nxy];
+        s += V[idx - nxy];
+        v = fma(-a.rho[idx], a.hinv, s) * (1.0 / 6.0) - V[idx];
+        bad = bad || !(fabs(v) < INFINITY);
+      } else {
+        v = a.in[idx];
+        if (LOAD == LOAD_SCALED) v *= fac(line, n);
+      }
+    }
+    x[line >> 4][n][line & 15] = v;
+  }
+  if (LOAD == LOAD_RESIDUAL && bad) atomicOr(p.flag, 1);
+  __syncthreads();
+
+  const double* __restrict__ S = p.S[AX];
+  d4 acc[RT][LT];
+  auto product = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int l = 0; l < LT; ++l) acc[r][l] = d4{0, 0, 0, 0};
+    const double* __restrict__ Sw = S + (int64_t)lk * ld + 16 * wave + li;
+    auto run = [&](auto nrc) __attribute__((always_inline)) {
+      constexpr int NR = decltype(nrc)::value;
+#pragma unroll 4
+      for (int n0 = 0; n0 < m; n0 += 4) {   // rows m .. of S and of x are zero
+        double b[LT], s[NR > 0 ? NR : 1];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) s[r] = Sw[(int64_t)n0 * ld + 128 * r];
+#pragma unroll
+        for (int l = 0; l < LT; ++l) b[l] = x[l][n0 + lk][li];
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+          for (int l = 0; l < LT; ++l)   // along x the lines go first, so that 16 lanes store 16 points of a line
+            acc[r][l] = AX == 0 ? __builtin_amdgcn_mfma_f64_16x16x4f64(b[l], s[r], acc[r][l], 0, 0, 0)
+                                : __builtin_amdgcn_mfma_f64_16x16x4f64(s[r], b[l], acc[r][l], 0, 0, 0);
+      }
+    };
+    // row tiles of this wave: wave + 8 r < rows / 16 (uniform)
+    const int nr = max(0, (rows / 16 - wave + 7) / 8);
+    if (nr == RT) run(std::integral_constant<int, RT>());
+    else if (RT > 1 && nr == RT - 1) run(std::integral_constant<int, RT - 1>());
+    else if (RT > 2 && nr == RT - 2) run(std::integral_constant<int, (RT > 2 ? RT - 2 : 0)>());
+    else if (RT > 3 && nr == RT - 3) run(std::integral_constant<int, (RT > 3 ? RT - 3 : 0)>());
+    else if (RT > 4 && nr == RT - 4) run(std::integral_constant<int, (RT > 4 ? RT - 4 : 0)>());
+  };
+  // element of acc[r][l][q]: along x (line 16 l + 4 q + lk, n = 16 (wave + 8 r) + li), else the reverse
+  auto each = [&](auto&& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int l = 0; l < LT; ++l)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int line = 16 * l + (AX == 0 ? 4 * q + lk : li);
+          const int n = 16 * (wave + 8 * r) + (AX == 0 ? li : 4 * q + lk);
+          if (n < m) f(line, n, acc[r][l][q]);
+        }
+  };
+  product();
+  if (MID) {
+    __syncthreads();
+    each([&](int line, int n, double v) { x[line >> 4][n][line & 15] = v * fac(line, n); });
+    __syncthreads();
+    product();
+  }
+  double sum = 0.0;
+  each([&](int line, int n, double v) {
+    if (l0 + line >= nl) return;
+    const int64_t idx = base[line] + n * stride;
+    if (STORE == STORE_PLAIN) a.out[idx] = v;
+    else if (STORE == STORE_ADD) a.out[idx] += v;
+    else if (STORE == STORE_SUM) sum += fabs(v);
+    else sum += fabs(a.out[idx] + v);
+  });
+  if (STORE == STORE_SUM || STORE == STORE_SUMV) {
+    __shared__ double red[8];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
+    if (lane == 0) red[wave] = sum;
+    __syncthreads();
+    if (t == 0) {
+      double s = 0.0;
+      for (int w = 0; w < 8; ++w) s += red[w];
+      a.part[blockIdx.x] = s;
+    }
+  }
+}
+
+// S_kn with zero columns up to ld and zero rows up to a multiple of 4, and sin^2(pi k / (2 (m + 1)))
+__global__ __launch_bounds__(256) void k_sine_tables(SinePlan p) {
+  const int ax = blockIdx.y, m = p.m[ax], ld = p.ld[ax];
+  const int rows = (m + 3) / 4 * 4;
+  double* __restrict__ S = const_cast<double*>(p.S[ax]);
+  double* __restrict__ s2 = const_cast<double*>(p.s2[ax]);
+  if (ax == 0 && blockIdx.x == 0 && threadIdx.x == 0) *p.flag = 0;
+  const double scale = sqrt(2.0 / (m + 1));
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < rows * ld; i += gridDim.x * 256) {
+    const int n = i / ld, k = i - n * ld;
+    const int64_t r = (int64_t)(n + 1) * (k + 1) % (2 * (m + 1));
+    S[i] = n < m && k < m ? scale * sinpi((double)r / (m + 1)) : 0.0;
+    if (i < m) {
+      const double h = sinpi((double)(i + 1) / (2 * (m + 1)));
+      s2[i] = h * h;
+    }
+  }
+}
+
+template <int LT, int RT, int AX, int LOAD, bool MID, int STORE>
+void launch(hipStream_t s, const Args& a) {
+  const int64_t nl = (int64_t)(AX == 0 ? a.p.m[1] : a.p.m[0]) * (AX == 2 ? a.p.m[1] : a.p.m[2]);
+  hipLaunchKernelGGL((k_sine<LT, RT, AX, LOAD, MID, STORE>), dim3((unsigned)((nl + 16 * LT - 1) / (16 * LT))),
+                     dim3(kThreads), 0, s, a);
+}
+
+// 32 lines per workgroup (34 or 68 KB of LDS, two workgroups per CU) up to 256 points, 16 beyond
+template <int AX, int LOAD, bool MID, int STORE>
+int pass(qm_ctx* ctx, hipStream_t s, const Args& a) {
+  const int m = a.p.m[AX];
+  if (m <= 128) launch<2, 1, AX, LOAD, MID, STORE>(s, a);
+  else if (m <= 256) launch<2, 2, AX, LOAD, MID, STORE>(s, a);
+  else if (m <= 512) launch<1, 4, AX, LOAD, MID, STORE>(s, a);
+  else launch<1, 8, AX, LOAD, MID, STORE>(s, a);
+  QM_CHECK_LAUNCH(ctx);
+  return QM_OK;
+}
+
+Args plain_args(const SinePlan& p, const double* in, double* out) {
+  Args a{};
+  a.p = p;
+  a.in = in;
+  a.out = out;
+  return a;
+}
+
+}  // namespace
+
+bool qm_sine_fits(const qm_geom* g) {
+  const int n[3] = {g->nx, g->ny, g->nz};
+  for (int d = 0; d < 3; ++d)
+    if (n[d] < 3 || n[d] - 2 > kMaxM) return false;
+  return true;
+}
+
+int qm_sine_plan(qm_ctx* ctx, hipStream_t s, const qm_geom* g, SinePlan* p) {
+  const int n[3] = {g->nx, g->ny, g->nz};
+  p->nx = g->nx;
+  p->ny = g->ny;
+  size_t doubles = 0, off[3], most = 0;
+  for (int d = 0; d < 3; ++d) {
+    p->m[d] = n[d] - 2;
+    p->ld[d] = (p->m[d] + 15) / 16 * 16;
+    off[d] = doubles;
+    most = std::max(most, (size_t)((p->m[d] + 3) / 4 * 4) * p->ld[d]);
+    doubles += (size_t)((p->m[d] + 3) / 4 * 4) * p->ld[d] + p->ld[d];
+  }
+  // partial sums of an x pass, then the flag
+  const size_t nparts = ((size_t)p->m[1] * p->m[2] + 15) / 16;
+  double* w = nullptr;
+  int rc = qm_ws(ctx, s, WS_SINE, sizeof(double) * (doubles + nparts + 4), (void**)&w);
+  if (rc) return rc;
+  for (int d = 0; d < 3; ++d) {
+    p->S[d] = w + off[d];
+    p->s2[d] = p->S[d] + (size_t)((p->m[d] + 3) / 4 * 4) * p->ld[d];
+  }
+  p->part = w + doubles;
+  p->sum = p->part + nparts;
+  p->flag = (int*)(p->sum + 1);
+  hipLaunchKernelGGL(k_sine_tables, dim3((unsigned)std::min<size_t>(512, (most + 255) / 256), 3), dim3(256), 0, s, *p);
+  QM_CHECK_LAUNCH(ctx);
+  return QM_OK;
+}
+
+int qm_sine_residual_xy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* rho, const double* v, double h,
+                        double* out) {
+  Args a = plain_args(p, v, out);
+  a.rho = rho;
+  a.hinv = 1.0 / h;
+  int rc = pass<0, LOAD_RESIDUAL, false, STORE_PLAIN>(ctx, s, a);
+  if (rc) return rc;
+  return pass<1, LOAD_PLAIN, false, STORE_PLAIN>(ctx, s, plain_args(p, out, out));
+}
+
+int qm_sine_xy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* a) {
+  int rc = pass<0, LOAD_PLAIN, false, STORE_PLAIN>(ctx, s, plain_args(p, a, a));
+  if (rc) return rc;
+  return pass<1, LOAD_PLAIN, false, STORE_PLAIN>(ctx, s, plain_args(p, a, a));
+}
+
+int qm_sine_z(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* a) {
+  return pass<2, LOAD_PLAIN, false, STORE_PLAIN>(ctx, s, plain_args(p, a, a));
+}
+
+int qm_sine_z_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const SineFactor& f, double* a) {
+  Args r = plain_args(p, a, a);
+  r.f = f;
+  int rc = pass<2, LOAD_PLAIN, true, STORE_PLAIN>(ctx, s, r);
+  if (rc) return rc;
+  return pass<1, LOAD_PLAIN, false, STORE_PLAIN>(ctx, s, plain_args(p, a, a));
+}
+
+int qm_sine_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const SineFactor& f, const double* spectrum,
+                     double* out) {
+  Args r = plain_args(p, spectrum, out);
+  r.f = f;
+  int rc = pass<2, LOAD_SCALED, false, STORE_PLAIN>(ctx, s, r);
+  if (rc) return rc;
+  return pass<1, LOAD_PLAIN, false, STORE_PLAIN>(ctx, s, plain_args(p, out, out));
+}
+
+int qm_sine_x_add(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, double* v) {
+  return pass<0, LOAD_PLAIN, false, STORE_ADD>(ctx, s, plain_args(p, a, v));
+}
+
+int qm_sine_x_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, const double* v, double* host_sum) {
+  Args r = plain_args(p, a, const_cast<double*>(v));
+  r.part = p.part;
+  int rc = v ? pass<0, LOAD_PLAIN, false, STORE_SUMV>(ctx, s, r) : pass<0, LOAD_PLAIN, false, STORE_SUM>(ctx, s, r);
+  if (rc) return rc;
+  const int64_t nl = (int64_t)p.m[1] * p.m[2], lines = p.m[0] <= 256 ? 32 : 16;
+  if ((rc = qm_reduce_dev(ctx, s, QM_RED_SUM, QM_F64, p.part, nullptr, (nl + lines - 1) / lines, p.sum))) return rc;
+  QM_CHECK_HIP(ctx, hipMemcpyAsync(ctx->host_scalars + 2, p.sum, sizeof(double), hipMemcpyDeviceToHost, s));
+  QM_CHECK_HIP(ctx, hipStreamSynchronize(s));
+  *host_sum = ctx->host_scalars[2];
+  return QM_OK;
+}

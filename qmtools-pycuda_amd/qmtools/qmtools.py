@@ -207,7 +207,7 @@ class QMTools:
         done = ctypes.c_int64(0)
         delta = ctypes.c_double(-1.0)
         if p == "fp64":
-            tmp = v.clone()
+            tmp = _device.torch().empty_like(v)   # scratch: its first sweep writes every point
             prec, every = nat.QM_PREC_FP64, int(check_every)
             tptr = nat.dptr(tmp)
         else:

@@ -1,0 +1,77 @@
+"""Relaxations in closed form by sine transforms: sizes at the edges of the matrix tiles, the convergence
+check, and the inputs that are left to the sweeps."""
+import ctypes
+
+import numpy
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _jacobi(shape, rho, v0, sweeps, tol=-1.0, every=0, h=0.3):
+    import torch
+    from qmtools import _native as nat
+    g = nat.geom((*shape, h, (0.0, 0.0, 0.0)))
+    dr, dv = torch.tensor(rho, device="cuda"), torch.tensor(v0, device="cuda")
+    dt = torch.full_like(dv, 7.0)
+    done, delta = ctypes.c_int64(0), ctypes.c_double(0)
+    rc = nat.library().qm_jacobi(nat.context(), nat.stream(), ctypes.byref(g), nat.QM_PREC_FP64, nat.dptr(dr),
+                                 nat.dptr(dv), nat.dptr(dt), sweeps, tol, every, ctypes.byref(done),
+                                 ctypes.byref(delta))
+    return rc, dv.cpu().numpy(), done.value, delta.value
+
+
+def _inputs(shape, seed=5):
+    from oracle import jacobi as oj
+    rng = numpy.random.default_rng(seed)
+    n = shape[0] * shape[1] * shape[2]
+    return rng.standard_normal(n), numpy.where(oj.boundary_mask(*shape), rng.standard_normal(n), 0.0)
+
+
+@pytest.mark.parametrize("n", [3, 4, 17, 18, 19, 34, 130, 131, 257, 258, 259, 514, 515, 1026, 1027])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_fixed_sweeps_along_each_axis(n, axis):
+    """1 .. 1025 interior points along one axis (1025: left to the sweeps); the gate of the FP64 sweeps, 1e-12."""
+    from oracle import jacobi as oj
+    shape = [9, 7, 8]
+    shape[axis] = n
+    rho, v0 = _inputs(shape)
+    print("[case] closed form", shape, flush=True)
+    rc, got, done, _ = _jacobi(shape, rho, v0, 131)
+    want = oj.jacobi(rho, *shape, 0.3, 131, bvals=v0, v0=v0)
+    assert rc == 0 and done == 131
+    assert numpy.abs(got - want).max() <= 1e-12 * numpy.abs(want).max()
+
+
+@pytest.mark.parametrize("shape", [(24, 17, 20), (40, 12, 31)])
+def test_check_stops_at_the_first_one_below_tolerance(shape):
+    """The bisected check is the first whose delta, from plain sweeps, is at most the tolerance."""
+    from oracle import jacobi as oj
+    rho, v0 = _inputs(shape, 8)
+    print("[case] closed form check", shape, flush=True)
+    v, deltas = v0, []
+    for _ in range(30):
+        v = oj.jacobi(rho, *shape, 0.3, 39, bvals=v0, v0=v)
+        t = oj.sweep(v, rho, *shape, 0.3, v0)
+        deltas.append(float(numpy.abs(t - v).sum()))
+        v = t
+    for c in (0, 3, 17, 29):
+        tol = deltas[c] * 1.0001
+        rc, got, done, delta = _jacobi(shape, rho, v0, 40 * 30, tol, 40)
+        assert rc == 0 and done == 40 * (c + 1)
+        assert delta == pytest.approx(deltas[c], rel=1e-9)
+        want = oj.jacobi_closed_form(rho, *shape, 0.3, done, bvals=v0)
+        assert numpy.abs(got - want).max() <= 1e-12 * numpy.abs(want).max()
+
+
+def test_values_that_are_not_finite_stay_local():
+    """A NaN charge spreads one point per sweep, as with plain sweeps."""
+    shape = (120, 8, 8)
+    rho, v0 = _inputs(shape)
+    rho[60 + 120 * (4 + 8 * 4)] = numpy.nan
+    print("[case] closed form, NaN", flush=True)
+    rc, got, done, _ = _jacobi(shape, rho, v0, 45)
+    row = got.reshape(8, 8, 120)[4, 4]
+    assert rc == 0 and done == 45
+    assert numpy.isnan(row[60 - 44:60 + 45:2]).all()
+    assert numpy.isfinite(row[:60 - 46]).all() and numpy.isfinite(row[60 + 46:]).all()
