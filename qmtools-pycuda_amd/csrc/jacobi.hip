@@ -768,28 +768,8 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   bool converged = dhi <= tol;
   double delta = dhi;
   if (converged) {
-    int64_t lo = 0, hi = checks;   // delta(lo) > tol >= delta(hi); check 0 stands for "no check yet"
-    double dlo = 0.0;
-    for (int step = 0; hi - lo > 1; ++step) {
-      int64_t c = lo + (hi - lo) / 2;
-      if (lo > 0 && step % 3 != 2 && dhi > 0.0 && tol > 0.0) {
-        // where the line through (lo, log dlo) and (hi, log dhi) meets log tol
-        const double f = (std::log(dlo) - std::log(tol)) / (std::log(dlo) - std::log(dhi));
-        c = lo + (int64_t)std::llround(f * (double)(hi - lo));
-        c = std::max(lo + 1, std::min(hi - 1, c));
-      }
-      double d = 0.0;
-      if ((rc = delta_at(c, &d))) return rc;
-      if (d <= tol) {
-        hi = c;
-        dhi = d;
-      } else {
-        lo = c;
-        dlo = d;
-      }
-    }
-    at = hi * check_every;
-    delta = dhi;
+    if ((rc = qm_sine_first_below(checks, dhi, tol, delta_at, &at, &delta))) return rc;
+    at *= check_every;
   }
   if ((rc = qm_sine_scale_zy(ctx, s, p, sweeps_factor(SINE_SUM, at), tmp, w))) return rc;
   double total = 0.0;
@@ -804,15 +784,11 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   return QM_OK;
 }
 
-// Sweep counts from which the closed form is taken: it costs what 21 sweeps do at 256^3 (1.32 ms against 64 us a
-// sweep; its 12 n flops a point grow with the axis, a sweep's 24 bytes do not) and about 20 on small grids
-// (eight launches against one replayed node a sweep).  256^3, 2000 sweeps: 128.5 -> 1.47 ms with the charge and
-// the boundary; 72 x 64 x 56 to a delta of 1e-4: 45 -> 0.62 ms.
-inline int64_t closed_form_sweeps(const qm_geom* g) { return 32 + std::max({g->nx, g->ny, g->nz}) / 16; }
-
+// 256^3, 2000 sweeps: 128.5 -> 1.47 ms with the charge and the boundary; 72 x 64 x 56 to a delta of 1e-4:
+// 45 -> 0.62 ms.
 int jacobi_fp64(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const double* rho, double* v, double* tmp,
                 int64_t max_sweeps, double tol, int check_every, int64_t* done_out, double* delta_out) {
-  if (max_sweeps >= closed_form_sweeps(g) && qm_sine_fits(g)) {
+  if (max_sweeps >= qm_sine_sweeps(g) && qm_sine_fits(g)) {
     bool finished = false, conv = false;
     int64_t sweeps = 0;
     double d = -1.0;

@@ -1,6 +1,8 @@
 // Sine transforms of a grid's interior (sine.hip), used by the relaxations' closed forms.
 #pragma once
 
+#include <functional>
+
 #include "qm_internal.h"
 
 struct SinePlan {
@@ -20,7 +22,7 @@ struct SineFactor {
   int sweep, kind;
   double n;                 // whole number below 2^53
   int odd;                  // n is odd
-  double w0, w1, w2, w3;    // SINE_VNE: 1 - a = w0 - (w1 sum c + w2 sum c c' + w3 c c' c''), c = cos theta per axis
+  double w0, w1, w2, w3;    // SINE_VNE: 1 - a = w0 + w1 sum (1 - c) + w2 sum (1 - c c') + w3 (1 - c c' c''), c = cos theta
 };
 
 bool qm_sine_fits(const qm_geom* g);   // every axis has 1 .. 1024 interior points
@@ -37,6 +39,18 @@ int qm_sine_z_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const Sine
 // factor times a spectrum, z and y transforms (the same bits as qm_sine_z and then this, or the call above)
 int qm_sine_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const SineFactor& f, const double* spectrum,
                      double* out);
+int qm_sine_x(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* a);
 int qm_sine_x_add(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, double* v);   // v += x transform of a
 // sum over the interior of |x transform of a| (v null) or |v + x transform of a|; waits for s
 int qm_sine_x_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, const double* v, double* host_sum);
+// First check 1 .. n whose delta is at most tol, given that delta does not grow and delta(n) = dn <= tol, by
+// bisection in the logarithm of delta.
+int qm_sine_first_below(int64_t n, double dn, double tol, const std::function<int(int64_t, double*)>& delta_at,
+                        int64_t* at, double* delta);
+// Sweep counts from which a closed form is taken: it costs what 21 sweeps do at 256^3 (1.32 ms against 64 us a
+// sweep; its 12 n flops a point grow with the axis, a sweep's 24 bytes do not) and about 20 on small grids
+// (eight launches against one replayed node a sweep).
+inline int64_t qm_sine_sweeps(const qm_geom* g) {
+  const int n = g->nx > g->ny ? g->nx : g->ny;
+  return 32 + (n > g->nz ? n : g->nz) / 16;
+}

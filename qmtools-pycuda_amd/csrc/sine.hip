@@ -45,8 +45,9 @@ struct Args {
   double* part;             // STORE_SUM: sum |x|, STORE_SUMV: sum |out + x|, one per workgroup
 };
 
-// q = 1 - a and c = 1 + a of the sweep's eigenvalue a at mode (kx, ky, kz) (0-based), both without
-// cancellation at their small ends for the Jacobi sweep: a = (cos x + cos y + cos z) / 3.
+// q = 1 - a and c = 1 + a of the sweep's eigenvalue a at mode (kx, ky, kz) (0-based), from sin^2 of the half
+// angles, without cancellation where they are small: a = (cos x + cos y + cos z) / 3 (Jacobi), or one minus the
+// row sum's distance from 1 and the weights times 1 - cos, 1 - cos cos', 1 - cos cos' cos'' (V_ne, where c stays near 2).
 // Returns a^n (SINE_POWER) or (1 - a^n) / (1 - a) (SINE_SUM).
 __device__ __forceinline__ double factor(const SinePlan& p, const SineFactor& f, int kx, int ky, int kz) {
   double q, c;
@@ -55,8 +56,9 @@ __device__ __forceinline__ double factor(const SinePlan& p, const SineFactor& f,
     q = (sx + sy + sz) * (2.0 / 3.0);
     c = (p.s2[0][p.m[0] - 1 - kx] + p.s2[1][p.m[1] - 1 - ky] + p.s2[2][p.m[2] - 1 - kz]) * (2.0 / 3.0);
   } else {
-    const double cx = 1.0 - 2.0 * sx, cy = 1.0 - 2.0 * sy, cz = 1.0 - 2.0 * sz;
-    q = f.w0 - (f.w1 * (cx + cy + cz) + f.w2 * (cx * cy + cx * cz + cy * cz) + f.w3 * cx * cy * cz);
+    const double yz = 2.0 * (sy + sz - 2.0 * sy * sz);   // 1 - cos y cos z
+    q = f.w0 + f.w1 * (2.0 * (sx + sy + sz)) + f.w2 * (2.0 * (sx + sy - 2.0 * sx * sy) + 2.0 * (sx + sz - 2.0 * sx * sz) + yz) +
+        f.w3 * (2.0 * sx + (1.0 - 2.0 * sx) * yz);
     c = 2.0 - q;
   }
   // log |a| from the smaller of 1 - a and 1 + a (with a near 0 both may round to just above 1)
@@ -252,6 +254,34 @@ Args plain_args(const SinePlan& p, const double* in, double* out) {
 
 }  // namespace
 
+int qm_sine_first_below(int64_t n, double dn, double tol, const std::function<int(int64_t, double*)>& delta_at,
+                        int64_t* at, double* delta) {
+  int64_t lo = 0, hi = n;   // delta(lo) > tol >= delta(hi); 0 stands for "no check yet"
+  double dlo = 0.0, dhi = dn;
+  for (int step = 0; hi - lo > 1; ++step) {
+    int64_t c = lo + (hi - lo) / 2;
+    if (lo > 0 && step % 3 != 2 && dhi > 0.0 && tol > 0.0) {
+      // where the line through (lo, log dlo) and (hi, log dhi) meets log tol
+      const double f = (std::log(dlo) - std::log(tol)) / (std::log(dlo) - std::log(dhi));
+      c = lo + (int64_t)std::llround(f * (double)(hi - lo));
+      c = std::max(lo + 1, std::min(hi - 1, c));
+    }
+    double d = 0.0;
+    const int rc = delta_at(c, &d);
+    if (rc) return rc;
+    if (d <= tol) {
+      hi = c;
+      dhi = d;
+    } else {
+      lo = c;
+      dlo = d;
+    }
+  }
+  *at = hi;
+  *delta = dhi;
+  return QM_OK;
+}
+
 bool qm_sine_fits(const qm_geom* g) {
   const int n[3] = {g->nx, g->ny, g->nz};
   for (int d = 0; d < 3; ++d)
@@ -298,8 +328,12 @@ int qm_sine_residual_xy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const dou
   return pass<1, LOAD_PLAIN, false, STORE_PLAIN>(ctx, s, plain_args(p, out, out));
 }
 
+int qm_sine_x(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* a) {
+  return pass<0, LOAD_PLAIN, false, STORE_PLAIN>(ctx, s, plain_args(p, a, a));
+}
+
 int qm_sine_xy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* a) {
-  int rc = pass<0, LOAD_PLAIN, false, STORE_PLAIN>(ctx, s, plain_args(p, a, a));
+  int rc = qm_sine_x(ctx, s, p, a);
   if (rc) return rc;
   return pass<1, LOAD_PLAIN, false, STORE_PLAIN>(ctx, s, plain_args(p, a, a));
 }

@@ -8,6 +8,7 @@
 #include <cmath>
 
 #include "qm_internal.h"
+#include "qm_sine.h"
 
 namespace {
 
@@ -306,6 +307,71 @@ __global__ __launch_bounds__(256) void k_vne_finish(const double* __restrict__ p
   }
 }
 
+// The FP64 loop in closed form by sine transforms (sine.hip): from 0 with source s, n sweeps give
+// sum_{j<n} A^j s, and the n-th changes the field by A^(n-1) s.  Taken where A has no negative weight and no
+// row sum above 1 (the usual parameters: a voxel keeps 1 - 16.79 DIF - ADS >= 0, and ADS >= 2.31 DIF), because then
+// sum |A^(n-1) s| never grows and the first pair at the tolerance is found by bisection.  *finished stays
+// false where that does not hold, or where the sweeps' rounding (about 1e-16 of the field) decides the test.
+// v is the work buffer (its outer layer stays 0), tmp holds the spectrum.
+// 120 x 120 x 64, 974 pairs: 27.1 -> 0.5 ms.
+int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, double ads, double dif, double tol,
+                    int64_t cap, dim3 grid, dim3 block, int zs, const VneState* st, double* v, double* tmp,
+                    bool* finished, int64_t* pairs, double* delta, int* conv) {
+  *finished = false;
+  const long double D = dif, r2 = std::sqrt(2.0L), r3 = std::sqrt(3.0L);
+  const double gap = (double)((long double)ads - D * (6.0L + 12.0L / r2 + 8.0L / r3 - (long double)kVneSelf));   // 1 - row sum
+  if (!(dif >= 0.0) || !(1.0 - dif * kVneSelf - ads >= 0.0) || !(gap >= 0.0)) return QM_OK;
+  const double n = (double)npoints(g);
+  SinePlan p;
+  int rc;
+  if ((rc = qm_sine_plan(ctx, s, g, &p))) return rc;
+  ProfScope ps(ctx, s, QM_K_VNE, (int)std::min<int64_t>(cap, 1 << 30));
+  // the first sweep of a zero field is the source
+  hipLaunchKernelGGL(k_vne_sweep<double>, grid, block, 0, s, (const double*)v, tmp, (const double4*)mol->atoms,
+                     mol->natoms, geom_view(g), zs, ads, dif, (double*)nullptr, st);
+  QM_CHECK_LAUNCH(ctx);
+  if ((rc = qm_sine_xy(ctx, s, p, tmp)) || (rc = qm_sine_z(ctx, s, p, tmp))) return rc;
+  auto factor = [&](int kind, int64_t sweeps) {
+    SineFactor f{};
+    f.sweep = SINE_VNE;
+    f.kind = kind;
+    f.n = (double)sweeps;
+    f.odd = (int)(sweeps & 1);
+    f.w0 = gap;
+    f.w1 = 2.0 * dif;
+    f.w2 = (double)(4.0L * D / r2);
+    f.w3 = (double)(8.0L * D / r3);
+    return f;
+  };
+  auto delta_at = [&](int64_t pr, double* d) -> int {
+    int r = qm_sine_scale_zy(ctx, s, p, factor(SINE_POWER, 2 * pr - 1), tmp, v);
+    if (!r) r = qm_sine_x_sum(ctx, s, p, v, nullptr, d);
+    *d /= n;
+    return r;
+  };
+  // the pair that exceeds maxiters is not tested
+  int64_t at = cap;
+  double d = 0.0;
+  bool ok = false;
+  if (cap > 1) {
+    if ((rc = delta_at(cap - 1, &d))) return rc;
+    ok = d <= tol;
+    if (ok && (rc = qm_sine_first_below(cap - 1, d, tol, delta_at, &at, &d))) return rc;
+  }
+  if (!ok && (rc = delta_at(cap, &d))) return rc;
+  double total = 0.0;
+  if ((rc = qm_sine_scale_zy(ctx, s, p, factor(SINE_SUM, 2 * at), tmp, v))) return rc;
+  if ((rc = qm_sine_x_sum(ctx, s, p, v, nullptr, &total))) return rc;
+  const double floor = 1e-12 * total / n;
+  if (!(floor < INFINITY) || !(d < INFINITY) || (tol < floor && d < floor)) return QM_OK;
+  if ((rc = qm_sine_x(ctx, s, p, v))) return rc;
+  *pairs = at;
+  *delta = d;
+  *conv = ok ? 1 : 0;
+  *finished = true;
+  return QM_OK;
+}
+
 template <typename T>
 int vne_diffusion(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, double ads, double dif, double tol,
                   double maxiters, T* v, T* tmp, int64_t* pairs_out, double* delta_out, int* conv_out) {
@@ -332,6 +398,24 @@ int vne_diffusion(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, dou
   // the loop runs at least one pair and stops once the count exceeds maxiters:
   // at most max(1, floor(maxiters) + 1) pairs, and nothing is queued beyond that
   const int64_t cap = std::max<int64_t>(1, (int64_t)std::floor(std::max(maxiters, -1.0)) + 1);
+  if constexpr (std::is_same<T, double>::value) {
+    if (1.0 > tol && 2 * cap >= qm_sine_sweeps(g) && qm_sine_fits(g)) {
+      bool finished = false;
+      int64_t np = 0;
+      double d = 0.0;
+      int ok = 0;
+      if ((rc = vne_closed_form(ctx, mol, s, g, ads, dif, tol, cap, grid, block, zs, st, v, tmp, &finished, &np, &d, &ok)))
+        return rc;
+      if (finished) {
+        if (pairs_out) *pairs_out = np;
+        if (delta_out) *delta_out = d;
+        if (conv_out) *conv_out = ok;
+        return QM_OK;
+      }
+      QM_CHECK_HIP(ctx, hipMemsetAsync(v, 0, sizeof(T) * n, s));
+      QM_CHECK_HIP(ctx, hipMemsetAsync(tmp, 0, sizeof(T) * n, s));
+    }
+  }
   int64_t queued = 0;
   int64_t chunk = 8;
   VneState hs{};

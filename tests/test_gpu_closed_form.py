@@ -75,3 +75,35 @@ def test_values_that_are_not_finite_stay_local():
     assert rc == 0 and done == 45
     assert numpy.isnan(row[60 - 44:60 + 45:2]).all()
     assert numpy.isfinite(row[:60 - 46]).all() and numpy.isfinite(row[60 + 46:]).all()
+
+
+@pytest.mark.parametrize("adsorb,diff,tol,maxiters", [(0.1, 0.01, 1e-9, None), (0.05, 0.02, 1e-9, None),
+                                                      (0.05, 0.02, 1e-6, 400.5), (0.02, 0.02, 1e-6, 40),
+                                                      (0.4, 0.05, 1e-9, None), (0.05, 0.02, -1.0, 24)])
+@pytest.mark.parametrize("shape", [(24, 16, 40), (19, 33, 18)])
+def test_vne_pairs_and_field(shape, adsorb, diff, tol, maxiters):
+    """The pair count, convergence and field of the plain loop, in and out of the closed form's parameter range
+    (ADS = DIF grows; DIF = 0.05 with ADS = 0.4 leaves a negative self weight); 1e-12, the sweeps' gate."""
+    import torch
+    import qmtools
+    from conftest import BASIS
+    from oracle import vne as ov
+    from qmtools import _native as nat, synth
+    from qmtools.qmtools import device_molecule
+    mol = synth.synthetic_molecule(6, 3, qmtools.BasisSet(BASIS))
+    h = 0.5
+    o = mol.coords.mean(0) - 0.5 * h * numpy.array(shape)
+    n = shape[0] * shape[1] * shape[2]
+    cap = 10 * n ** (1.0 / 3) if maxiters is None else maxiters
+    print("[case] vne closed form", shape, adsorb, diff, tol, cap, flush=True)
+    v = torch.empty(n, dtype=torch.float64, device="cuda")
+    t = torch.empty_like(v)
+    pairs, delta, conv = ctypes.c_int64(0), ctypes.c_double(0), ctypes.c_int(0)
+    nat.call("qm_vne_diffusion", device_molecule(mol).handle, nat.stream(),
+             ctypes.byref(nat.geom((*shape, h, tuple(o)))), nat.QM_F64, adsorb, diff, tol, float(cap), nat.dptr(v),
+             nat.dptr(t), ctypes.byref(pairs), ctypes.byref(delta), ctypes.byref(conv))
+    want, wp, wd, wc = ov.vne_diffusion(mol.types, mol.coords, *shape, h, o, adsorb, diff, tol, cap)
+    assert pairs.value == wp and bool(conv.value) == wc
+    assert delta.value == pytest.approx(wd, rel=1e-6)
+    got = v.cpu().numpy().reshape(want.shape)
+    assert numpy.abs(got - want).max() <= 1e-12 * numpy.abs(want).max()
