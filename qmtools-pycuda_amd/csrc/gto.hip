@@ -13,14 +13,17 @@
 // The density-matrix contraction is done once per molecule on the host: every
 // primitive pair becomes a Hermite charge distribution (p, P, D_tuv) with
 //   D_tuv = -f (2 pi/p) K c_a c_b sum_{ma,mb} P_(a ma),(b mb) sum_cart E_t E_u E_v
-// (f = 2 for distinct shells), so that V_el(C) = sum_dist sum_tuv D_tuv R_tuv.
+// (f = 2 for distinct shells), so that V_el(C) = sum_dist sum_tuv D_tuv R_tuv.  Shells of one nucleus and L
+// with the same exponents (a general contraction) share their primitive pairs: their D_tuv are added
+// before anything is evaluated, and on one nucleus the pairs (i, j) and (j, i) are one distribution too.
+// cc-pVDZ: 196 instead of 484 pairs for two carbon atoms.
 // The device kernel then only evaluates Boys functions and R_tuv per point.
 // This has no singularity at T = 0 (the reference's closed forms divide by
 // powers of T = gamma |PC|^2 and lose precision there).
 //
 // Boys function F_n(T): for T < 40, Taylor expansion (8 terms) around the
-// nearest point of a 0.1-spaced table of F_0..F_11 and e^-T (computed on the host
-// from the all-positive series e^-T sum (2T)^k / ((2n+1)...(2n+2k+1))), then
+// nearest point of a 0.1-spaced table of F_L+k / k! (one table per L, so that a term is one multiply-add) and
+// e^-T (computed on the host from the all-positive series e^-T sum (2T)^k / ((2n+1)...(2n+2k+1))), then
 // downward recursion F_{n-1} = (2T F_n + e^-T)/(2n-1); for T >= 40,
 // F_0 = sqrt(pi/T)/2 and upward recursion (e^-40 is below FP64 resolution of F).
 #include <algorithm>
@@ -36,11 +39,11 @@ namespace {
 
 constexpr int kLmax = 4;                 // La + Lb <= 4
 constexpr int kNTUV = 35;                // (t,u,v) with t+u+v <= 4
-constexpr int kBoysN = 13;               // F_0 .. F_11 (up to L + 7 for L <= 4), then e^-T
+constexpr int kTaylor = 8;               // terms F_L+k / k! of a table row, then e^-T
+constexpr int kBoysN = kTaylor + 1;
 constexpr int kBoysPts = 401;            // T = 0, 0.1, ..., 40
 constexpr double kBoysStep = 0.1;
 constexpr double kBoysTmax = 40.0;
-constexpr int kThreads = 256;
 constexpr double kGtoScreen = 1e-17;      // largest dropped contribution of one distribution (hartree)
 
 __host__ __device__ constexpr int ntuv(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
@@ -48,15 +51,15 @@ __host__ __device__ constexpr int tuv_index(int t, int u, int v) {
   return (t + u + v) * (t + u + v + 1) * (t + u + v + 2) / 6 + (u + v) * (u + v + 1) / 2 + v;
 }
 
-struct HDist {
-  double p, Px, Py, Pz;
-  double D[kNTUV];
-};
+// A distribution of L = La + Lb in the table: p, Px, Py, Pz, then D_tuv for t + u + v <= L (tuv_index order).
+__host__ __device__ constexpr int dist_doubles(int L) { return 4 + ntuv(L); }
 
 // ------------------------------------------------------------------ device
-// 1 / k for the Taylor factors and 1 / (2n - 1) for the recursion: multiplications by
-// rounded reciprocals instead of FP64 divisions (each a ~10-instruction sequence)
-__device__ constexpr double kInvInt[10] = {0.0, 1.0, 1.0 / 2, 1.0 / 3, 1.0 / 4, 1.0 / 5, 1.0 / 6, 1.0 / 7, 1.0 / 8, 1.0 / 9};
+// 1 / (2n - 1) for the recursion and 1 / k! for e^d: multiplications by rounded reciprocals instead of FP64
+// divisions (each a ~10-instruction sequence)
+__device__ constexpr double kInvInt[8] = {0.0, 1.0, 1.0 / 2, 1.0 / 3, 1.0 / 4, 1.0 / 5, 1.0 / 6, 1.0 / 7};
+__device__ constexpr double kInvFact[10] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040,
+                                            1.0 / 40320, 1.0 / 362880};
 
 template <int L>
 __device__ __forceinline__ void boys(double T, const double* __restrict__ tab, double* F) {
@@ -65,16 +68,16 @@ __device__ __forceinline__ void boys(double T, const double* __restrict__ tab, d
     const double d = i * kBoysStep - T;       // T = Ti - d, |d| <= 0.05
     const double* row = tab + i * kBoysN;
     // F_L(T) = sum_k F_{L+k}(Ti) d^k / k!
-    double f = row[L + 7];
+    double f = row[kTaylor - 1];
 #pragma unroll
-    for (int k = 6; k >= 0; --k) f = row[L + k] + f * d * kInvInt[k + 1];
+    for (int k = kTaylor - 2; k >= 0; --k) f = fma(f, d, row[k]);
     F[L] = f;
     // e^-T = e^-Ti e^d: the table's last column holds e^-Ti, e^d is its Taylor series to d^9
     // (remainder below 3e-20)
-    double ed = 1.0;
+    double ed = kInvFact[9];
 #pragma unroll
-    for (int k = 9; k >= 1; --k) ed = 1.0 + d * ed * kInvInt[k];
-    const double ex = row[kBoysN - 1] * ed;
+    for (int k = 8; k >= 0; --k) ed = fma(ed, d, kInvFact[k]);
+    const double ex = row[kTaylor] * ed;
 #pragma unroll
     for (int n = L; n >= 1; --n) F[n - 1] = (2.0 * T * F[n] + ex) * kInvInt[2 * n - 1];
   } else {
@@ -87,10 +90,13 @@ __device__ __forceinline__ void boys(double T, const double* __restrict__ tab, d
   }
 }
 
+// The table is constant during a launch and its address wave uniform: read through scalar loads.
+typedef const double __attribute__((address_space(4))) TableDouble;
+
 // sum_tuv D_tuv R^0_tuv for t+u+v <= L, R from the Hermite recursion (Helgaker eq. 9.9.18-20)
 template <int L>
 __device__ __forceinline__ double hermite_contract(double X, double Y, double Z, const double* rn,
-                                                   const double* __restrict__ D) {
+                                                   TableDouble* D) {
   constexpr int N = ntuv(L);
   double cur[N], nxt[N];
   cur[0] = rn[L];
@@ -131,13 +137,13 @@ __device__ __forceinline__ double hermite_contract(double X, double Y, double Z,
 }
 
 template <int L>
-__device__ __forceinline__ double dist_sum(const HDist* __restrict__ ds, int lo, int hi, double cx, double cy,
+__device__ __forceinline__ double dist_sum(const double* __restrict__ ds, int lo, int hi, double cx, double cy,
                                            double cz, const double* __restrict__ tab) {
   double acc = 0.0;
   for (int d = lo; d < hi; ++d) {
-    const HDist& h = ds[d];
-    const double p = h.p;
-    const double X = h.Px - cx, Y = h.Py - cy, Z = h.Pz - cz;
+    TableDouble* h = (TableDouble*)(uintptr_t)(ds + (int64_t)d * dist_doubles(L));
+    const double p = h[0];
+    const double X = h[1] - cx, Y = h[2] - cy, Z = h[3] - cz;
     const double T = p * (X * X + Y * Y + Z * Z);
     double F[L + 1];
     boys<L>(T, tab, F);
@@ -148,46 +154,63 @@ __device__ __forceinline__ double dist_sum(const HDist* __restrict__ ds, int lo,
       rn[n] = m * F[n];
       m *= -2.0 * p;
     }
-    acc += hermite_contract<L>(X, Y, Z, rn, h.D);
+    acc += hermite_contract<L>(X, Y, Z, rn, h + 4);
   }
   return acc;
 }
 
 struct DistLists {
-  const HDist* d[kLmax + 1];
+  const double* d[kLmax + 1];
   int n[kLmax + 1];
 };
 
+// Point of thread t of workgroup b: a list in order; a grid in blocks of 8^3 per workgroup and 4^3 per wave, so
+// that the points of a wave mostly take the same branch of the Boys function.  idx < 0: none.
+__device__ __forceinline__ int64_t gto_point(const double* __restrict__ pts, const GeomView& g, int64_t npts, int64_t b,
+                                             int t, double& cx, double& cy, double& cz) {
+  if (pts) {
+    const int64_t idx = b * 512 + t, u = idx < npts ? idx : npts - 1;
+    cx = pts[3 * u];
+    cy = pts[3 * u + 1];
+    cz = pts[3 * u + 2];
+    return idx < npts ? idx : -1;
+  }
+  const int nbx = (g.nx + 7) / 8, nby = (g.ny + 7) / 8;
+  const int64_t q = b / nbx;
+  const int i = (int)(b - q * nbx) * 8 + (t & 3) + 4 * ((t >> 6) & 1);
+  const int j = (int)(q % nby) * 8 + ((t >> 2) & 3) + 4 * ((t >> 7) & 1);
+  const int k = (int)(q / nby) * 8 + ((t >> 4) & 3) + 4 * (t >> 8);
+  const int ic = min(i, g.nx - 1), jc = min(j, g.ny - 1), kc = min(k, g.nz - 1);
+  cx = g.ox + ic * g.h;
+  cy = g.oy + jc * g.h;
+  cz = g.oz + kc * g.h;
+  return i < g.nx && j < g.ny && k < g.nz ? i + (int64_t)g.nx * (j + (int64_t)g.ny * k) : -1;
+}
+
 // partial[chunk][pt] = sum over this chunk's slice of every L list
-// 512 threads share one 42 KB LDS copy of the table (two workgroups per CU; 4 waves per SIMD)
+// 512 threads share one 29 KB LDS copy of the table of one L at a time.  FP64 VALU bound.  60 atoms, 10^4
+// points: 3.1 -> 1.7 ms with shared primitive pairs and one multiply-add per Taylor term; 16 atoms,
+// 48 x 40 x 56 nodes: 2.9 -> 1.3 ms, with the nodes taken in 4^3 blocks.
 constexpr int kGtoThreads = 512;
 __global__ __launch_bounds__(kGtoThreads) void k_gto(DistLists lists, const double* __restrict__ boys_tab,
                                                      const double* __restrict__ pts, GeomView g, int64_t npts,
                                                      int nchunk, double* __restrict__ partial) {
   __shared__ double tab[kBoysPts * kBoysN];
-  for (int i = threadIdx.x; i < kBoysPts * kBoysN; i += kGtoThreads) tab[i] = boys_tab[i];
-  __syncthreads();
-  const int64_t t = (int64_t)blockIdx.x * kGtoThreads + threadIdx.x;
   const int chunk = blockIdx.y;
   double cx, cy, cz;
-  const int64_t tt = t < npts ? t : npts - 1;
-  if (pts) {
-    cx = pts[3 * tt];
-    cy = pts[3 * tt + 1];
-    cz = pts[3 * tt + 2];
-  } else {
-    const int64_t i = tt % g.nx, j = (tt / g.nx) % g.ny, k = tt / ((int64_t)g.nx * g.ny);
-    cx = g.ox + i * g.h;
-    cy = g.oy + j * g.h;
-    cz = g.oz + k * g.h;
-  }
+  const int64_t idx = gto_point(pts, g, npts, blockIdx.x, threadIdx.x, cx, cy, cz);
   double acc = 0.0;
-#define QM_GTO_L(LL)                                                             \
-  {                                                                              \
-    const int n = lists.n[LL];                                                   \
-    const int per = (n + nchunk - 1) / nchunk;                                   \
-    const int lo = min(n, chunk * per), hi = min(n, lo + per);                   \
-    if (hi > lo) acc += dist_sum<LL>(lists.d[LL], lo, hi, cx, cy, cz, tab);     \
+#define QM_GTO_L(LL)                                                                                                 \
+  {                                                                                                                  \
+    const int n = lists.n[LL];                                                                                       \
+    const int per = (n + nchunk - 1) / nchunk;                                                                       \
+    const int lo = min(n, chunk * per), hi = min(n, lo + per);                                                       \
+    if (hi > lo) { /* the same for the whole workgroup */                                                            \
+      __syncthreads();                                                                                               \
+      for (int i = threadIdx.x; i < kBoysPts * kBoysN; i += kGtoThreads) tab[i] = boys_tab[LL * kBoysPts * kBoysN + i]; \
+      __syncthreads();                                                                                               \
+      acc += dist_sum<LL>(lists.d[LL], lo, hi, cx, cy, cz, tab);                                                     \
+    }                                                                                                                \
   }
   QM_GTO_L(0)
   QM_GTO_L(1)
@@ -195,7 +218,7 @@ __global__ __launch_bounds__(kGtoThreads) void k_gto(DistLists lists, const doub
   QM_GTO_L(3)
   QM_GTO_L(4)
 #undef QM_GTO_L
-  if (t < npts) partial[(int64_t)chunk * npts + t] = acc;
+  if (idx >= 0) partial[(int64_t)chunk * npts + idx] = acc;
 }
 
 // out[t] = sum_chunks partial + sum_A Z_A / |C - R_A| (|C - R_A| > 1e-8, kernel_hartree.cu:851-865)
@@ -229,10 +252,13 @@ __global__ void k_gto_finish(const double* __restrict__ partial, int nchunk, con
 
 // ------------------------------------------------------------------ host: tables
 std::vector<double> make_boys_table() {
-  std::vector<double> tab(kBoysPts * kBoysN);
+  constexpr int nf = kLmax + kTaylor;   // F_0 .. F_11
+  std::vector<double> tab((size_t)(kLmax + 1) * kBoysPts * kBoysN);
   for (int i = 0; i < kBoysPts; ++i) {
     const double T = i * kBoysStep;
-    for (int n = 0; n < kBoysN - 1; ++n) {
+    long double F[nf];
+    const long double e = std::exp(-(long double)T);
+    for (int n = 0; n < nf; ++n) {
       // e^-T sum_k (2T)^k / ((2n+1)(2n+3)...(2n+2k+1)): positive terms, no cancellation
       long double term = 1.0L / (2 * n + 1), s = term;
       for (int k = 1; k < 2000; ++k) {
@@ -240,9 +266,17 @@ std::vector<double> make_boys_table() {
         s += term;
         if (term < s * 1e-21L) break;
       }
-      tab[i * kBoysN + n] = (double)(std::exp(-(long double)T) * s);
+      F[n] = e * s;
     }
-    tab[i * kBoysN + kBoysN - 1] = (double)std::exp(-(long double)T);
+    for (int L = 0; L <= kLmax; ++L) {
+      double* row = &tab[((size_t)L * kBoysPts + i) * kBoysN];
+      long double fact = 1.0L;
+      for (int k = 0; k < kTaylor; ++k) {
+        row[k] = (double)(F[L + k] / fact);
+        fact *= k + 1;
+      }
+      row[kTaylor] = (double)e;
+    }
   }
   return tab;
 }
@@ -315,123 +349,163 @@ void host_parallel(int n, F&& f) {
 }
 
 struct GtoCache {
-  HDist* dev = nullptr;
-  int off[kLmax + 1] = {0, 0, 0, 0, 0};
+  double* dev = nullptr;
+  size_t off[kLmax + 1] = {0, 0, 0, 0, 0};   // first double of each L's distributions
   int n[kLmax + 1] = {0, 0, 0, 0, 0};
   double* boys = nullptr;
 };
 
+// Shells of one nucleus and L with the same exponents, evaluated as one: their primitive pairs coincide.
+struct ShellSet {
+  int atom, L, nprim, poff;
+  std::vector<int> shells;
+};
+
 int build_distributions(qm_ctx* ctx, qm_mol* mol, hipStream_t s, GtoCache& c) {
-  const int nsh = mol->nshell, nbf = mol->nbf;
+  const int nbf = mol->nbf;
   // Cartesian term lists per (L, m index)
   std::vector<CartTerm> terms[3][5];
   for (int L = 0; L <= 2; ++L)
     for (int mi = 0; mi < 2 * L + 1; ++mi) terms[L][mi] = cart_terms(L, mi);
-  // distributions of shell A with the shells B <= A, per L, in the order (B, primitive of A,
-  // primitive of B); the table is the concatenation over A in increasing order, the same whether
-  // the shells are built by one thread or several
-  struct ShellOut {
-    std::vector<HDist> l[kLmax + 1];
+  std::vector<ShellSet> sets;
+  {
+    std::vector<std::vector<int>> of_atom(mol->natoms);   // sets of each nucleus
+    for (int k = 0; k < mol->nshell; ++k) {
+      const DevShell& sh = mol->h_shells[k];
+      int found = -1;
+      for (int i : of_atom[sh.atom]) {
+        bool same = sets[i].L == sh.L && sets[i].nprim == sh.nprim;
+        for (int q = 0; same && q < sh.nprim; ++q)
+          same = mol->h_alpha[sets[i].poff + q] == mol->h_alpha[sh.poff + q];
+        if (same) found = i;
+      }
+      if (found < 0) {
+        of_atom[sh.atom].push_back((int)sets.size());
+        sets.push_back({sh.atom, sh.L, sh.nprim, sh.poff, {k}});
+      } else {
+        sets[found].shells.push_back(k);
+      }
+    }
+  }
+  const int nset = (int)sets.size();
+  // distributions of set A with the sets B <= A, per L, in the order (B, primitive of A, primitive of B);
+  // the table is the concatenation over A in increasing order, the same whether the sets are built by one
+  // thread or several
+  struct SetOut {
+    std::vector<double> l[kLmax + 1];
   };
-  std::vector<ShellOut> per(nsh);
-  auto build_shell = [&](int sa) {
-    const DevShell& A = mol->h_shells[sa];
+  std::vector<SetOut> per(nset);
+  auto build_set = [&](int sa) {
+    const ShellSet& A = sets[sa];
     const double* RA = &mol->xyz[3 * A.atom];
+    // Cartesian pair (exponents ea, eb) with its weight sum_{ma,mb} P_ab fa fb for every pair of shells of the sets
+    struct CW {
+      int ea[3], eb[3];
+      std::vector<double> w;   // [shell of A][shell of B]
+    };
     for (int sb = 0; sb <= sa; ++sb) {
-      const DevShell& B = mol->h_shells[sb];
+      const ShellSet& B = sets[sb];
       const double* RB = &mol->xyz[3 * B.atom];
-      const double f = (sa == sb) ? 1.0 : 2.0;
-      // Cartesian pair weights W[(ex_a),(ex_b)] = sum_{ma,mb} P_ab fa fb over matching exponents
-      struct CW {
-        int ea[3], eb[3];
-        double w;
-      };
+      const size_t na = A.shells.size(), nb = B.shells.size();
       std::vector<CW> cw;
       double wmax = 0.0;
-      for (int ma = 0; ma < 2 * A.L + 1; ++ma)
-        for (int mb = 0; mb < 2 * B.L + 1; ++mb) {
-          const double P = mol->h_P[(size_t)(A.bf + ma) * nbf + (B.bf + mb)];
-          if (P == 0.0) continue;
-          for (const CartTerm& ta : terms[A.L][ma])
-            for (const CartTerm& tb : terms[B.L][mb]) {
-              const double w = P * ta.c * tb.c;
-              bool merged = false;
-              for (CW& x : cw)
-                if (x.ea[0] == ta.e[0] && x.ea[1] == ta.e[1] && x.ea[2] == ta.e[2] && x.eb[0] == tb.e[0] &&
-                    x.eb[1] == tb.e[1] && x.eb[2] == tb.e[2]) {
-                  x.w += w;
-                  merged = true;
-                  break;
+      for (size_t ka = 0; ka < na; ++ka)
+        for (size_t kb = 0; kb < nb; ++kb) {
+          const DevShell &SA = mol->h_shells[A.shells[ka]], &SB = mol->h_shells[B.shells[kb]];
+          for (int ma = 0; ma < 2 * A.L + 1; ++ma)
+            for (int mb = 0; mb < 2 * B.L + 1; ++mb) {
+              const double P = mol->h_P[(size_t)(SA.bf + ma) * nbf + (SB.bf + mb)];
+              if (P == 0.0) continue;
+              for (const CartTerm& ta : terms[A.L][ma])
+                for (const CartTerm& tb : terms[B.L][mb]) {
+                  CW* x = nullptr;
+                  for (CW& y : cw)
+                    if (y.ea[0] == ta.e[0] && y.ea[1] == ta.e[1] && y.ea[2] == ta.e[2] && y.eb[0] == tb.e[0] &&
+                        y.eb[1] == tb.e[1] && y.eb[2] == tb.e[2])
+                      x = &y;
+                  if (!x) {
+                    cw.push_back({{ta.e[0], ta.e[1], ta.e[2]}, {tb.e[0], tb.e[1], tb.e[2]},
+                                  std::vector<double>(na * nb, 0.0)});
+                    x = &cw.back();
+                  }
+                  x->w[ka * nb + kb] += P * ta.c * tb.c;
                 }
-              if (!merged) cw.push_back({{ta.e[0], ta.e[1], ta.e[2]}, {tb.e[0], tb.e[1], tb.e[2]}, w});
             }
         }
-      for (const CW& x : cw) wmax = std::max(wmax, std::fabs(x.w));
+      for (const CW& x : cw)
+        for (double w : x.w) wmax = std::max(wmax, std::fabs(w));
       if (cw.empty() || wmax == 0.0) continue;
       const int L = A.L + B.L;
       const double AB[3] = {RA[0] - RB[0], RA[1] - RB[1], RA[2] - RB[2]};
       const double AB2 = AB[0] * AB[0] + AB[1] * AB[1] + AB[2] * AB[2];
-      for (int ia = 0; ia < A.nprim; ++ia) {
-        const double a = mol->h_alpha[A.poff + ia], ca = mol->h_coeff[A.poff + ia];
-        for (int ib = 0; ib < B.nprim; ++ib) {
-          const double b = mol->h_alpha[B.poff + ib], cb = mol->h_coeff[B.poff + ib];
-          const double p = a + b;
-          const double K = std::exp(-a * b / p * AB2);
-          const double pref = -f * 2.0 * M_PI / p * K * ca * cb;
-          // exact zero contributions only (exp underflow or zero coefficient)
-          if (pref == 0.0) continue;
-          double E[3][3][3][6];
-          for (int d = 0; d < 3; ++d) hermite_E(a, b, AB[d], E[d]);
-          HDist h{};
-          h.p = p;
-          h.Px = (a * RA[0] + b * RB[0]) / p;
-          h.Py = (a * RA[1] + b * RB[1]) / p;
-          h.Pz = (a * RA[2] + b * RB[2]) / p;
-          for (const CW& x : cw) {
-            const double w = pref * x.w;
-            for (int t = 0; t <= x.ea[0] + x.eb[0]; ++t) {
-              const double et = E[0][x.ea[0]][x.eb[0]][t];
-              if (et == 0.0) continue;
-              for (int u = 0; u <= x.ea[1] + x.eb[1]; ++u) {
-                const double eu = E[1][x.ea[1]][x.eb[1]][u];
-                if (eu == 0.0) continue;
-                for (int v = 0; v <= x.ea[2] + x.eb[2]; ++v) {
-                  const double ev = E[2][x.ea[2]][x.eb[2]][v];
-                  h.D[tuv_index(t, u, v)] += w * et * eu * ev;
-                }
-              }
+      double D[kNTUV];
+      // adds the pair (ia, ib) to D; false if it contributes nothing (exp underflow or zero coefficients)
+      auto add_pair = [&](int ia, int ib, double f) -> bool {
+        const double a = mol->h_alpha[A.poff + ia], b = mol->h_alpha[B.poff + ib], p = a + b;
+        const double pref = -f * 2.0 * M_PI / p * std::exp(-a * b / p * AB2);
+        bool any = false;
+        double E[3][3][3][6];
+        for (const CW& x : cw) {
+          double w = 0.0;
+          for (size_t ka = 0; ka < na; ++ka)
+            for (size_t kb = 0; kb < nb; ++kb)
+              w += mol->h_coeff[mol->h_shells[A.shells[ka]].poff + ia] * mol->h_coeff[mol->h_shells[B.shells[kb]].poff + ib] *
+                   x.w[ka * nb + kb];
+          w *= pref;
+          if (w == 0.0) continue;
+          if (!any)
+            for (int d = 0; d < 3; ++d) hermite_E(a, b, AB[d], E[d]);
+          any = true;
+          for (int t = 0; t <= x.ea[0] + x.eb[0]; ++t) {
+            const double et = E[0][x.ea[0]][x.eb[0]][t];
+            if (et == 0.0) continue;
+            for (int u = 0; u <= x.ea[1] + x.eb[1]; ++u) {
+              const double eu = E[1][x.ea[1]][x.eb[1]][u];
+              if (eu == 0.0) continue;
+              for (int v = 0; v <= x.ea[2] + x.eb[2]; ++v)
+                D[tuv_index(t, u, v)] += w * et * eu * E[2][x.ea[2]][x.eb[2]][v];
             }
           }
+        }
+        return any;
+      };
+      for (int ia = 0; ia < A.nprim; ++ia) {
+        // one set with itself: (ia, ib) and (ib, ia) have the same centre and exponent
+        for (int ib = 0; ib < (sa == sb ? ia + 1 : B.nprim); ++ib) {
+          std::fill(D, D + kNTUV, 0.0);
+          bool any = add_pair(ia, ib, sa == sb ? 1.0 : 2.0);
+          if (sa == sb && ia != ib) any = add_pair(ib, ia, 1.0) || any;
+          if (!any) continue;
+          const double a = mol->h_alpha[A.poff + ia], b = mol->h_alpha[B.poff + ib], p = a + b;
           // Screening: |sum_tuv D_tuv R_tuv(C)| <= sum_tuv |D_tuv| (2p)^{n/2} 2^n n! for every point C
           // (n = t+u+v; Hermite-function bound on the derivatives of F_0), so a distribution whose
           // bound is below kGtoScreen changes no potential by more than that.
-          double bound = 0.0;
-          for (int t = 0; t <= L; ++t)
-            for (int u = 0; t + u <= L; ++u)
-              for (int v = 0; t + u + v <= L; ++v) {
-                const int n = t + u + v;
-                double g = std::pow(2.0 * p, 0.5 * n);
-                for (int k = 1; k <= n; ++k) g *= 2.0 * k;
-                bound += std::fabs(h.D[tuv_index(t, u, v)]) * g;
-              }
+          double bound = 0.0, g = 1.0;
+          for (int n = 0, k = 0; n <= L; ++n) {
+            for (; k < ntuv(n); ++k) bound += std::fabs(D[k]) * g;
+            g *= std::sqrt(2.0 * p) * 2.0 * (n + 1);
+          }
           if (bound < kGtoScreen) continue;
-          per[sa].l[L].push_back(h);
+          std::vector<double>& out = per[sa].l[L];
+          const double head[4] = {p, (a * RA[0] + b * RB[0]) / p, (a * RA[1] + b * RB[1]) / p, (a * RA[2] + b * RB[2]) / p};
+          out.insert(out.end(), head, head + 4);
+          out.insert(out.end(), D, D + ntuv(L));
         }
       }
     }
   };
-  // shells taken largest first (shell A pairs with A + 1 shells)
-  host_parallel(nsh, [&](int k) { build_shell(nsh - 1 - k); });
-  // table offsets: L-major, shells in increasing order within each L
-  std::vector<size_t> at((size_t)(kLmax + 1) * nsh);
+  // sets taken largest first (set A pairs with A + 1 sets)
+  host_parallel(nset, [&](int k) { build_set(nset - 1 - k); });
+  // table offsets: L-major, sets in increasing order within each L
+  std::vector<size_t> at((size_t)(kLmax + 1) * nset);
   size_t tot = 0;
   for (int L = 0; L <= kLmax; ++L) {
-    c.off[L] = (int)tot;
-    for (int sa = 0; sa < nsh; ++sa) {
-      at[(size_t)L * nsh + sa] = tot;
+    c.off[L] = tot;
+    for (int sa = 0; sa < nset; ++sa) {
+      at[(size_t)L * nset + sa] = tot;
       tot += per[sa].l[L].size();
     }
-    c.n[L] = (int)(tot - c.off[L]);
+    c.n[L] = (int)((tot - c.off[L]) / dist_doubles(L));
   }
   // stream-ordered: kernels queued earlier on s still read the previous table
   if (c.dev) {
@@ -440,7 +514,7 @@ int build_distributions(qm_ctx* ctx, qm_mol* mol, hipStream_t s, GtoCache& c) {
   }
   if (tot) {
     // the context's pinned staging buffer (the last upload from it finished: synchronised below)
-    const size_t bytes = sizeof(HDist) * tot;
+    const size_t bytes = sizeof(double) * tot;
     if (bytes > ctx->gto_staged_bytes) {
       if (ctx->gto_staged) QM_CHECK_HIP(ctx, hipHostFree(ctx->gto_staged));
       ctx->gto_staged = nullptr;
@@ -448,14 +522,14 @@ int build_distributions(qm_ctx* ctx, qm_mol* mol, hipStream_t s, GtoCache& c) {
       QM_CHECK_HIP(ctx, hipHostMalloc(&ctx->gto_staged, bytes, hipHostMallocDefault));
       ctx->gto_staged_bytes = bytes;
     }
-    HDist* staged = (HDist*)ctx->gto_staged;
-    // the shells' lists go to their places in the staging buffer
-    host_parallel(nsh, [&](int sa) {
+    double* staged = (double*)ctx->gto_staged;
+    // the sets' lists go to their places in the staging buffer
+    host_parallel(nset, [&](int sa) {
       for (int L = 0; L <= kLmax; ++L)
         if (!per[sa].l[L].empty())
-          std::copy(per[sa].l[L].begin(), per[sa].l[L].end(), staged + at[(size_t)L * nsh + sa]);
+          std::copy(per[sa].l[L].begin(), per[sa].l[L].end(), staged + at[(size_t)L * nset + sa]);
     });
-    QM_CHECK_HIP(ctx, hipMallocAsync((void**)&c.dev, sizeof(HDist) * tot, s));
+    QM_CHECK_HIP(ctx, hipMallocAsync((void**)&c.dev, bytes, s));
     QM_CHECK_HIP(ctx, hipMemcpyAsync(c.dev, staged, bytes, hipMemcpyHostToDevice, s));
     QM_CHECK_HIP(ctx, hipStreamSynchronize(s));   // the staging buffer is rewritten by the next build
   }
@@ -493,7 +567,8 @@ int gto_eval(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const double* pts, const G
     dl.n[L] = c->n[L];
     total += c->n[L];
   }
-  const int64_t pblocks = (npts + kGtoThreads - 1) / kGtoThreads;
+  const int64_t pblocks = pts ? (npts + kGtoThreads - 1) / kGtoThreads
+                              : (int64_t)((gv.nx + 7) / 8) * ((gv.ny + 7) / 8) * ((gv.nz + 7) / 8);
   // enough workgroups for 256 CUs: split the distributions over chunks when points are few
   int nchunk = (int)std::max<int64_t>(1, std::min<int64_t>(256, 2048 / std::max<int64_t>(pblocks, 1)));
   nchunk = std::max(1, std::min(nchunk, std::max(1, total / 64)));
