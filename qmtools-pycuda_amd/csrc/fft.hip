@@ -9,13 +9,24 @@
 //     G(d) = -h^3/(4 pi |d|), G(0) = -h^3 C0/(4 pi h), C0 = 2 (3 asinh(1/sqrt2) - pi/4)
 //     (the average of 1/|u| over the voxel), G^ cached per geometry.
 //
-// Layout: complex buffer in C order [n0][n1][n2] (axis 2 contiguous).  One
-// kernel per axis; a workgroup loads B lines into LDS (coalesced: for axis 2
-// the lines are contiguous, otherwise the B lines are adjacent along axis 2),
-// runs the Stockham stages out of place between two LDS planes, and writes
-// back.  Twiddles exp(-2 pi i m/n) come from a per-length table in LDS; a
-// radix-R stage uses the same table for its R-point DFT.  Zero padding is
-// exploited by transforming only the lines that can be non-zero.
+// The charge is real, so its transform is Hermitian and half of it is kept: complex work buffer
+// [n0][m1][hs] in C order, the k <= m2 / 2 of axis 2 (hs: that count rounded up to 128 bytes, so the
+// groups of adjacent lines of the other two axes start on cache lines).  One kernel per pass:
+//   z    two real lines packed as one complex line, separated by symmetry on the way out
+//   y    complex lines of i < n0, k <= m2 / 2
+//   x    forward, factor in k space, inverse, on the lines held on chip
+//   y    inverse, keeping j < n1
+//   z    the two half lines of a pair joined as one complex line, its real and imaginary parts stored
+//        as the two lines of the potential
+// Zero padding is never stored or cleared: positions beyond the grid are read as zero and only
+// positions that are read later are written.
+//
+// A workgroup takes B lines.  The first stage of a transform reads its inputs from memory straight
+// into registers and the last stage writes its outputs from registers (both touch positions i + j n / R
+// for one i, adjacent lanes adjacent addresses), so only the exchanges between stages go through LDS;
+// in the x pass the last forward and first inverse stage have the same radix and so the same points,
+// and the product with the factor happens in registers between the two.  Twiddles
+// exp(-2 pi i m/n) come from a per-length table in LDS.
 #include <algorithm>
 #include <cmath>
 #include <map>
@@ -38,7 +49,7 @@ template <typename R, bool POW2>
 struct FftPts {
   static constexpr int kMax = sizeof(R) == 4 && POW2 ? 8192 : 4096;
 };
-constexpr int kMaxStages = 24;
+constexpr int kMaxStages = 12;   // 4096 = 2^12
 
 template <typename R>
 struct Cx {
@@ -50,25 +61,20 @@ __device__ __forceinline__ Cx<R> cmul(Cx<R> a, Cx<R> b) {
   return Cx<R>{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
 }
 
-// LDS index skew: one empty slot after every W complex values, W = 256 bytes / value size
-// (16 for complex128, 32 for complex64), so that a W-value run spans the 64 banks once and
-// the strided accesses of the Stockham stages (stride RR in the first stage's writes) and of
-// the twiddle table land on distinct banks.  Lines are LS slots apart, LS = W/8 mod W, so the
-// 8 lines that one LDS cycle serves in the load and store phases of a strided axis (8 lines
-// x W/8 consecutive points) do not share banks either.
-template <typename R>
-struct Skew {
-  static constexpr int S = sizeof(R) == 8 ? 4 : 5;   // log2 W
-};
-template <typename R>
-__host__ __device__ __forceinline__ int sk(int i) { return i + (i >> Skew<R>::S); }
-template <typename R>
-__host__ __device__ __forceinline__ int line_slots(int n) {
-  constexpr int W = 1 << Skew<R>::S;
-  return (n + (n >> Skew<R>::S) + W - 1) / W * W + W / 8;
+// a times the table value b = exp(-i t) (DIR -1, forward) or its conjugate (DIR 1, inverse)
+template <int DIR, typename R>
+__device__ __forceinline__ Cx<R> twiddle(Cx<R> a, Cx<R> b) {
+  return cmul(a, Cx<R>{b.x, DIR < 0 ? b.y : -b.y});
 }
-template <typename R>
-__host__ __device__ __forceinline__ int table_slots(int n) { return n + (n >> Skew<R>::S) + 1; }
+
+// LDS index skew: one empty slot after every 32 complex values, so that the strided accesses of the
+// stages (stride RR in the first stage's writes) and of the twiddle table spread over the banks, and an
+// odd number of slots per line, so that adjacent lines at one position do too.  FP64, 240 x 256 x 200
+// in free space, whole solve: 1011 us; lines 2 (4, 8) slots past a multiple of 16: 1032 (1097, 1337);
+// a slot after every 8 (16) values: 1143 (1025), none: 1056.  Complex64 differs by less than 1 %.
+__host__ __device__ __forceinline__ int sk(int i) { return i + (i >> 5); }
+__host__ __device__ __forceinline__ int line_slots(int n) { return (n + (n >> 5) + 15) / 16 * 16 + 1; }
+__host__ __device__ __forceinline__ int table_slots(int n) { return n + (n >> 5) + 1; }
 
 // Division by a run-time divisor 1 <= d < 2^16 of dividends x < 2^16: q = umulhi(x, ceil(2^32 / d))
 // is exact (the product overshoots x / d by less than x / 2^32 < 2^-16 <= 1 / d, which cannot reach
@@ -95,152 +101,233 @@ struct AxisPlan {
   FastDiv pdiv[kMaxStages];     // by the span
 };
 
+// What one axis pass does with its lines.  TURN_*: forward, k-space factor, inverse (axis 0).
+enum Kind { FORWARD, INVERSE, TURN_FREE, TURN_PERIODIC, FROM_REAL, TO_REAL };
+// How: power-of-two lengths; other lengths of radices <= 10; any length (two LDS planes).
+enum Path { POW2, RADIX, GENERIC };
+
 struct AxisLines {
   int64_t stride;     // distance between consecutive elements of a line
-  int nl0, nl1;       // lines: l0 in [0, nl0), l1 in [0, nl1)
+  int nl0, nl1;       // lines: l0 in [0, nl0), l1 in [0, nl1); real passes: l1 counts pairs of lines
   int64_t s0, s1;     // line base = l0 * s0 + l1 * s1
   int B;              // lines per workgroup (consecutive l1)
   FastDiv bdiv;       // by B
+  FastDiv hdiv;       // by n / 2 + 1
   int nin;            // positions >= nin of a line are zero on input (not loaded)
   int nout;           // positions >= nout are not needed after the pass (not stored)
+  int nr1, nr2;       // real passes: lines per l0 and points per line of the real array
 };
 
 // Transform of the free-space Green's function for one padded shape, computed at unit grid step:
 // the transform is real and even in every axis, so one octant is kept, o1 = m1 / 2 + 1 and
 // o2 = m2 / 2 + 1 wide; the value at grid step h is g[min(i, m0 - i)][min(j, m1 - j)][min(k, m2 - k)]
 // times scale = h^2 (Angstrom), since g(d) = 1 / |d| scales as 1 / h and the voxel volume as h^3.
+// TURN_PERIODIC reads the shape, the grid step and the normalisation of the inverse transform.
 template <typename R>
-struct GreenView {
+struct FactorView {
   const R* g;
   int m0, m1, m2;
   int o1, o2;
   R scale;
+  double step, norm;
 };
 
-// R-point DFT of x (forward sign through the table; the inverse uses a conjugated table).
-// w1 = table index step of exp(-2 pi i / R).
-template <typename R, int RR>
-__device__ __forceinline__ void dft(Cx<R>* x, const Cx<R>* __restrict__ tw, int w1) {
+// R-point DFT of x with W = exp(i DIR 2 pi / R), DIR = -1 (forward) or 1.  The odd radices pair x_q with
+// x_R-q: real parts of W^k multiply the sums, imaginary parts the differences (radix 5: 16 multiplications
+// and no table read, against 16 complex products with table values for the plain sum).  Radices 6 and 10 are radix 3 and 5 of the sums and differences of opposite points, in the
+// prime-factor order, which needs no inner twiddles.
+template <typename R, int RR, int DIR>
+__device__ __forceinline__ void dft(Cx<R>* x) {
+  constexpr R dir = (R)DIR;
   if (RR == 2) {
     const Cx<R> a = x[0], b = x[1];
     x[0] = Cx<R>{a.x + b.x, a.y + b.y};
     x[1] = Cx<R>{a.x - b.x, a.y - b.y};
-  } else if (RR == 4) {
-    const Cx<R> a0{x[0].x + x[2].x, x[0].y + x[2].y}, a1{x[0].x - x[2].x, x[0].y - x[2].y};
-    const Cx<R> b0{x[1].x + x[3].x, x[1].y + x[3].y}, b1{x[1].x - x[3].x, x[1].y - x[3].y};
-    const Cx<R> b1w = cmul(b1, tw[sk<R>(w1)]);   // exp(-+ i pi/2)
-    x[0] = Cx<R>{a0.x + b0.x, a0.y + b0.y};
-    x[1] = Cx<R>{a1.x + b1w.x, a1.y + b1w.y};
-    x[2] = Cx<R>{a0.x - b0.x, a0.y - b0.y};
-    x[3] = Cx<R>{a1.x - b1w.x, a1.y - b1w.y};
-  } else if (RR == 8) {
-    // X_2r = DFT4(x_m + x_m+4)_r, X_2r+1 = DFT4((x_m - x_m+4) W8^m)_r; W8^m = tw[m w1], W4 = W8^2
-    Cx<R> a[4], b[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      a[q] = Cx<R>{x[q].x + x[q + 4].x, x[q].y + x[q + 4].y};
-      b[q] = Cx<R>{x[q].x - x[q + 4].x, x[q].y - x[q + 4].y};
-    }
-    b[1] = cmul(b[1], tw[sk<R>(w1)]);
-    b[2] = cmul(b[2], tw[sk<R>(2 * w1)]);
-    b[3] = cmul(b[3], tw[sk<R>(3 * w1)]);
-    const Cx<R> w4 = tw[sk<R>(2 * w1)];
-    auto dft4 = [&](const Cx<R>* c, Cx<R>& o0, Cx<R>& o1, Cx<R>& o2, Cx<R>& o3) {
-      const Cx<R> d0{c[0].x + c[2].x, c[0].y + c[2].y}, d1{c[0].x - c[2].x, c[0].y - c[2].y};
-      const Cx<R> d2{c[1].x + c[3].x, c[1].y + c[3].y};
-      const Cx<R> d3 = cmul(Cx<R>{c[1].x - c[3].x, c[1].y - c[3].y}, w4);
+  } else if (RR == 4 || RR == 8) {
+    // out_r = sum_m c_m W4^(m r), W4 = i dir
+    auto dft4 = [&](const Cx<R>& c0, const Cx<R>& c1, const Cx<R>& c2, const Cx<R>& c3, Cx<R>& o0, Cx<R>& o1, Cx<R>& o2,
+                    Cx<R>& o3) __attribute__((always_inline)) {
+      const Cx<R> d0{c0.x + c2.x, c0.y + c2.y}, d1{c0.x - c2.x, c0.y - c2.y};
+      const Cx<R> d2{c1.x + c3.x, c1.y + c3.y};
+      const Cx<R> d3{-dir * (c1.y - c3.y), dir * (c1.x - c3.x)};
       o0 = Cx<R>{d0.x + d2.x, d0.y + d2.y};
       o1 = Cx<R>{d1.x + d3.x, d1.y + d3.y};
       o2 = Cx<R>{d0.x - d2.x, d0.y - d2.y};
       o3 = Cx<R>{d1.x - d3.x, d1.y - d3.y};
     };
-    dft4(a, x[0], x[2], x[4], x[6]);
-    dft4(b, x[1], x[3], x[5], x[7]);
-  } else {
-    Cx<R> y[RR];
+    if (RR == 4) {
+      const Cx<R> c0 = x[0], c1 = x[1], c2 = x[2], c3 = x[3];
+      dft4(c0, c1, c2, c3, x[0], x[1], x[2], x[3]);
+    } else {
+      // X_2r = DFT4(x_m + x_m+4)_r, X_2r+1 = DFT4((x_m - x_m+4) W8^m)_r, W8 = (1 + i dir) / sqrt 2
+      Cx<R> a[4], b[4];
 #pragma unroll
-    for (int j = 0; j < RR; ++j) {
-      Cx<R> acc = x[0];
-#pragma unroll
-      for (int q = 1; q < RR; ++q) {
-        const Cx<R> t = cmul(x[q], tw[sk<R>(((j * q) % RR) * w1)]);
-        acc.x += t.x;
-        acc.y += t.y;
+      for (int q = 0; q < 4; ++q) {
+        a[q] = Cx<R>{x[q].x + x[q + 4].x, x[q].y + x[q + 4].y};
+        b[q] = Cx<R>{x[q].x - x[q + 4].x, x[q].y - x[q + 4].y};
       }
-      y[j] = acc;
+      const R h = (R)0.70710678118654752440, hd = h * dir;
+      b[1] = Cx<R>{h * b[1].x - hd * b[1].y, h * b[1].y + hd * b[1].x};
+      b[2] = Cx<R>{-dir * b[2].y, dir * b[2].x};
+      b[3] = Cx<R>{-h * b[3].x - hd * b[3].y, -h * b[3].y + hd * b[3].x};
+      dft4(a[0], a[1], a[2], a[3], x[0], x[2], x[4], x[6]);
+      dft4(b[0], b[1], b[2], b[3], x[1], x[3], x[5], x[7]);
     }
+  } else if (RR == 6 || RR == 10) {
+    // m = H a + 2 b, r = H c + (H + 1) d (mod 2H, H odd): W_2H^(m r) = (-1)^(a c) W_H^(b d)
+    constexpr int H = RR / 2;
+    Cx<R> u[H], v[H];
 #pragma unroll
-    for (int j = 0; j < RR; ++j) x[j] = y[j];
+    for (int b = 0; b < H; ++b) {
+      const Cx<R> p = x[2 * b], q = x[(2 * b + H) % RR];
+      u[b] = Cx<R>{p.x + q.x, p.y + q.y};
+      v[b] = Cx<R>{p.x - q.x, p.y - q.y};
+    }
+    dft<R, RR == 6 ? 3 : 5, DIR>(u);
+    dft<R, RR == 6 ? 3 : 5, DIR>(v);
+#pragma unroll
+    for (int d = 0; d < H; ++d) {
+      x[(H + 1) * d % RR] = u[d];
+      x[(H + (H + 1) * d) % RR] = v[d];
+    }
+  } else {
+    constexpr int H = RR / 2;
+    // cos and sin of 2 pi k / RR, k = 0 .. H
+    constexpr double C3[2] = {1.0, -0.5}, S3[2] = {0.0, 0.86602540378443864676};
+    constexpr double C5[3] = {1.0, 0.30901699437494742410, -0.80901699437494742410};
+    constexpr double S5[3] = {0.0, 0.95105651629515357212, 0.58778525229247312917};
+    constexpr double C7[4] = {1.0, 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624};
+    constexpr double S7[4] = {0.0, 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048};
+    Cx<R> sum[H + 1], dif[H + 1];
+    Cx<R> y0 = x[0];
+#pragma unroll
+    for (int q = 1; q <= H; ++q) {
+      sum[q] = Cx<R>{x[q].x + x[RR - q].x, x[q].y + x[RR - q].y};
+      dif[q] = Cx<R>{x[q].x - x[RR - q].x, x[q].y - x[RR - q].y};
+      y0.x += sum[q].x;
+      y0.y += sum[q].y;
+    }
+    Cx<R> lo[H + 1], hi[H + 1];
+#pragma unroll
+    for (int j = 1; j <= H; ++j) {
+      Cx<R> a = x[0], b{0, 0};
+#pragma unroll
+      for (int q = 1; q <= H; ++q) {
+        const int k = j * q % RR, kk = k <= H ? k : RR - k;
+        const double cd = RR == 3 ? C3[kk] : RR == 5 ? C5[kk] : C7[kk];
+        const double sd = RR == 3 ? S3[kk] : RR == 5 ? S5[kk] : S7[kk];
+        const R c = (R)cd, sn = (R)(k <= H ? sd : -sd);
+        a.x += c * sum[q].x;
+        a.y += c * sum[q].y;
+        b.x += sn * dif[q].x;
+        b.y += sn * dif[q].y;
+      }
+      // a + i dir b and its mirror
+      lo[j] = Cx<R>{a.x - dir * b.y, a.y + dir * b.x};
+      hi[j] = Cx<R>{a.x + dir * b.y, a.y - dir * b.x};
+    }
+    x[0] = y0;
+#pragma unroll
+    for (int j = 1; j <= H; ++j) {
+      x[j] = lo[j];
+      x[RR - j] = hi[j];
+    }
   }
 }
 
-// One radix-RR Stockham stage in place: all inputs of the thread's butterflies
-// are read into registers, then (after a barrier) the outputs are written.
-// POW2: n, p and RR are powers of two, so the line / butterfly / twiddle indices come from
-// shifts and masks instead of integer divisions by run-time values.
-template <typename R, int RR, bool POW2 = false>
-__device__ __forceinline__ void stage_inplace(Cx<R>* buf, const Cx<R>* __restrict__ tw, int n, int B, int p,
-                                              FastDiv mdiv = FastDiv{0}, FastDiv pdiv = FastDiv{0}) {
-  const int LS = line_slots<R>(n);
-  constexpr int MAXB = (FftPts<R, POW2>::kMax / kFftThreads + RR - 1) / RR;   // butterflies per thread (B n <= kMax)
+// One radix-RR Stockham stage on a workgroup's B lines.  EDGE 0: LDS to LDS in place (all inputs of the
+// thread's butterflies are read into registers, then, after a barrier, the outputs are written).
+// EDGE 1: the first stage, inputs through io.load, no twiddles.  EDGE 2: the last stage, outputs through
+// io.store.  EDGE 3: the last forward stage, io.factor and the first inverse stage (span 1) in one.
+// Butterflies of the first and last stage follow the order of the lines in memory (ROWS: line-major,
+// else line-minor).  P2: n, p, B and RR are powers of two, so the line / butterfly / twiddle indices
+// come from shifts and masks instead of divisions by run-time values.
+template <typename R, int RR, int DIR, int EDGE, bool P2, typename IO>
+__device__ __forceinline__ void stage(const IO& io, Cx<R>* buf, const Cx<R>* __restrict__ tw, int n, int B, int LS,
+                                      int p, FastDiv mdiv, FastDiv pdiv) {
+  constexpr int MAXB = (FftPts<R, P2>::kMax / kFftThreads + RR - 1) / RR;   // butterflies per thread (B n <= kMax)
   const int m = n / RR;
   const int tstep = n / (p * RR);
   const int total = B * m;
-  const int lm = POW2 ? __builtin_ctz(m) : 0;
-  auto split = [&](int bf, int& l, int& i, int& k) __attribute__((always_inline)) {
-    if (POW2) {
-      l = bf >> lm;
-      i = bf & (m - 1);
-      k = i & (p - 1);
-    } else {   // bf < B n <= 4096
-      l = fdiv(bf, mdiv);
-      i = bf - l * m;
-      k = i - fdiv(i, pdiv) * p;
+  const int lm = P2 ? __builtin_ctz(m) : 0, lb = P2 ? __builtin_ctz(B) : 0;
+  const bool rows = EDGE == 0 || io.rows();
+  auto split = [&](int bf, int& l, int& i) __attribute__((always_inline)) {   // bf < B n <= kMax
+    if (rows) {
+      l = P2 ? bf >> lm : fdiv(bf, mdiv);
+      i = P2 ? bf & (m - 1) : bf - l * m;
+    } else {
+      i = P2 ? bf >> lb : fdiv(bf, io.bdiv());
+      l = P2 ? bf & (B - 1) : bf - i * B;
     }
+  };
+  // the span of the last stage is m, of the first stage 1
+  auto rem = [&](int i) __attribute__((always_inline)) {
+    return EDGE == 1 ? 0 : EDGE >= 2 ? i : P2 ? i & (p - 1) : i - fdiv(i, pdiv) * p;
   };
   Cx<R> x[MAXB][RR];
 #pragma unroll
   for (int b = 0; b < MAXB; ++b) {
     const int bf = threadIdx.x + b * kFftThreads;
     if (bf < total) {
-      int l, i, k;
-      split(bf, l, i, k);
-      const Cx<R>* src = buf + l * LS;
+      int l, i;
+      split(bf, l, i);
+      if (EDGE == 1) {
+        io.template load<RR>(l, i, m, x[b]);
+      } else {
+        const int k = rem(i);
+        const Cx<R>* src = buf + l * LS;
 #pragma unroll
-      for (int j = 0; j < RR; ++j) {
-        Cx<R> v = src[sk<R>(i + j * m)];
-        // j k tstep <= (RR - 1)(p - 1) n / (p RR) < n: the twiddle index needs no reduction
-        if (k) v = cmul(v, tw[sk<R>(j * k * tstep)]);
-        x[b][j] = v;
+        for (int j = 0; j < RR; ++j) {
+          const Cx<R> v = src[sk(i + j * m)];
+          // j k tstep <= (RR - 1)(p - 1) n / (p RR) < n: the twiddle index needs no reduction
+          x[b][j] = j ? twiddle<DIR>(v, tw[sk(j * k * tstep)]) : v;
+        }
       }
-      dft<R, RR>(x[b], tw, m);
     }
   }
-  __syncthreads();
 #pragma unroll
   for (int b = 0; b < MAXB; ++b) {
     const int bf = threadIdx.x + b * kFftThreads;
     if (bf < total) {
-      int l, i, k;
-      split(bf, l, i, k);
+      dft<R, RR, DIR>(x[b]);
+      if (EDGE >= 2) {
+        int l, i;
+        split(bf, l, i);
+        if (EDGE == 2) {
+          io.template store<RR>(l, i, m, x[b]);
+        } else {
+          io.template factor<RR>(l, i, m, x[b]);
+          dft<R, RR, -DIR>(x[b]);
+        }
+      }
+    }
+  }
+  if (EDGE == 2) return;
+  if (EDGE != 1) __syncthreads();
+#pragma unroll
+  for (int b = 0; b < MAXB; ++b) {
+    const int bf = threadIdx.x + b * kFftThreads;
+    if (bf < total) {
+      int l, i;
+      split(bf, l, i);
+      const int k = EDGE == 3 ? 0 : rem(i), q = EDGE == 3 ? 1 : p;
       Cx<R>* dst = buf + l * LS;
       const int o = (i - k) * RR + k;
 #pragma unroll
-      for (int j = 0; j < RR; ++j) dst[sk<R>(o + j * p)] = x[b][j];
+      for (int j = 0; j < RR; ++j) dst[sk(o + j * q)] = x[b][j];
     }
   }
   __syncthreads();
 }
 
 // Any radix, out of place between two LDS planes (used when a length has a prime factor > 7).
-// Indices as in stage_inplace (quotients by multiply-high, twiddle index below n); the DFT table
+// Indices as in stage (quotients by multiply-high, twiddle index below n); the DFT table
 // index (j q mod RR) m is carried from one q to the next.
-template <typename R>
+template <typename R, int DIR>
 __device__ __forceinline__ void stage_generic(const Cx<R>* in, Cx<R>* out, const Cx<R>* __restrict__ tw, int n,
-                                              int B, int RR, int p, FastDiv mdiv, FastDiv pdiv) {
+                                              int B, int LS, int RR, int p, FastDiv mdiv, FastDiv pdiv) {
   const int m = n / RR;
   const int tstep = n / (p * RR);
-  const int LS = line_slots<R>(n);
   for (int bf = threadIdx.x; bf < B * m; bf += kFftThreads) {
     const int l = fdiv(bf, mdiv), i = bf - l * m, k = i - fdiv(i, pdiv) * p;
     const Cx<R>* src = in + l * LS;
@@ -250,55 +337,50 @@ __device__ __forceinline__ void stage_generic(const Cx<R>* in, Cx<R>* out, const
       Cx<R> acc{0, 0};
       int jq = 0;   // j q mod RR
       for (int q = 0; q < RR; ++q) {
-        Cx<R> v = src[sk<R>(i + q * m)];
-        if (k) v = cmul(v, tw[sk<R>(q * k * tstep)]);
-        const Cx<R> t = cmul(v, tw[sk<R>(jq * m)]);
+        Cx<R> v = src[sk(i + q * m)];
+        if (k) v = twiddle<DIR>(v, tw[sk(q * k * tstep)]);
+        const Cx<R> t = twiddle<DIR>(v, tw[sk(jq * m)]);
         acc.x += t.x;
         acc.y += t.y;
         jq += j;
         if (jq >= RR) jq -= RR;
       }
-      dst[sk<R>(o + j * p)] = acc;
+      dst[sk(o + j * p)] = acc;
     }
   }
   __syncthreads();
 }
 
-// The stages of one transform of a workgroup's B lines, from buf0 (buf1: the second plane of the
-// generic stages); returns the plane that holds the result.
-template <typename R, bool POW2>
-__device__ __forceinline__ Cx<R>* run_stages(const AxisPlan& plan, Cx<R>* buf0, Cx<R>* buf1, const Cx<R>* tw, int n,
-                                             int B, int inplace) {
-  if (POW2) {
-    for (int s = 0; s < plan.nstage; ++s) {
-      const int p = plan.span[s];
-      switch (plan.radix[s]) {
-        case 2: stage_inplace<R, 2, true>(buf0, tw, n, B, p); break;
-        case 4: stage_inplace<R, 4, true>(buf0, tw, n, B, p); break;
-        default: stage_inplace<R, 8, true>(buf0, tw, n, B, p); break;
-      }
+template <typename R, int DIR, int EDGE, bool P2, typename IO>
+__device__ __forceinline__ void run_stage(const IO& io, const AxisPlan& plan, int s, Cx<R>* buf, const Cx<R>* tw,
+                                          int B, int LS) {
+  const int n = plan.n, p = plan.span[s];
+  const FastDiv md = plan.mdiv[s], pd = plan.pdiv[s];
+  if (P2) {
+    switch (plan.radix[s]) {
+      case 2: stage<R, 2, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
+      case 4: stage<R, 4, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
+      default: stage<R, 8, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
     }
-    return buf0;
-  }
-  if (inplace) {
-    for (int s = 0; s < plan.nstage; ++s) {
-      const int p = plan.span[s];
-      const FastDiv md = plan.mdiv[s], pd = plan.pdiv[s];
-      switch (plan.radix[s]) {
-        case 2: stage_inplace<R, 2>(buf0, tw, n, B, p, md, pd); break;
-        case 3: stage_inplace<R, 3>(buf0, tw, n, B, p, md, pd); break;
-        case 4: stage_inplace<R, 4>(buf0, tw, n, B, p, md, pd); break;
-        case 5: stage_inplace<R, 5>(buf0, tw, n, B, p, md, pd); break;
-        case 7: stage_inplace<R, 7>(buf0, tw, n, B, p, md, pd); break;
-        default: stage_inplace<R, 8>(buf0, tw, n, B, p, md, pd); break;
-      }
+  } else {
+    switch (plan.radix[s]) {
+      case 2: stage<R, 2, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
+      case 3: stage<R, 3, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
+      case 4: stage<R, 4, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
+      case 5: stage<R, 5, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
+      case 6: stage<R, 6, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
+      case 7: stage<R, 7, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
+      case 8: stage<R, 8, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
+      default: stage<R, 10, DIR, EDGE, P2>(io, buf, tw, n, B, LS, p, md, pd); break;
     }
-    return buf0;
   }
-  Cx<R>* in = buf0;
-  Cx<R>* out = buf1;
+}
+
+template <typename R, int DIR>
+__device__ __forceinline__ Cx<R>* run_generic(const AxisPlan& plan, Cx<R>* in, Cx<R>* out, const Cx<R>* tw, int B,
+                                              int LS) {
   for (int s = 0; s < plan.nstage; ++s) {
-    stage_generic<R>(in, out, tw, n, B, plan.radix[s], plan.span[s], plan.mdiv[s], plan.pdiv[s]);
+    stage_generic<R, DIR>(in, out, tw, plan.n, B, LS, plan.radix[s], plan.span[s], plan.mdiv[s], plan.pdiv[s]);
     Cx<R>* t = in;
     in = out;
     out = t;
@@ -306,100 +388,241 @@ __device__ __forceinline__ Cx<R>* run_stages(const AxisPlan& plan, Cx<R>* buf0, 
   return in;
 }
 
-// One FFT pass along one axis.  INV: inverse (conjugated) transform, unnormalised.
-// inplace: all radices <= 8 (LDS = table + B lines); otherwise two planes of B lines.
-// POW2: the length is a power of two (radices 8, 4, 2 only), which keeps the
-// register footprint of the butterflies, and so the kernel's, small.
-// MUL (axis 0 of the free-space solve only): forward transform, product with the Green's
-// function transform, inverse transform, all on the lines held in LDS.
-template <typename R, bool INV, bool POW2, bool MUL = false>
-__global__ __launch_bounds__(kFftThreads) void k_fft_axis(Cx<R>* __restrict__ data, const Cx<R>* __restrict__ twg,
-                                                       AxisPlan plan, AxisLines ln, int inplace, GreenView<R> gv) {
-  extern __shared__ unsigned char smem[];
-  const int n = plan.n;
-  const int B = ln.B;
-  const int LS = line_slots<R>(n);
-  Cx<R>* tw = (Cx<R>*)smem;
-  Cx<R>* buf0 = tw + table_slots<R>(n);
-  Cx<R>* buf1 = buf0 + (int64_t)B * LS;
-  const int lines_per_row = (ln.nl1 + B - 1) / B;
-  const int64_t wg = blockIdx.x;
-  const int64_t l0 = wg / lines_per_row;
-  const int l1b = (int)(wg % lines_per_row) * B;
-  for (int q = threadIdx.x; q < n; q += kFftThreads) {
-    Cx<R> w = twg[q];
-    if (INV) w.y = -w.y;
-    tw[sk<R>(q)] = w;
+__device__ __forceinline__ double periodic_freq(int i, int n, double step) {
+  return (i > n / 2 - 1 ? (double)(i - n) : (double)i) / (n * step);
+}
+
+// Memory side of a pass: element j of butterfly i of workgroup line l is position i + j m.
+template <typename R, typename TO, int KIND>
+struct LineIO {
+  Cx<R>* data;          // the workgroup's first line (complex side)
+  const R* rin;         // FROM_REAL: the workgroup's first pair
+  TO* rout;             // TO_REAL
+  const AxisLines& ln;
+  const FactorView<R>& fv;
+  int n, l0, l1b, nb;
+
+  __device__ __forceinline__ bool rows() const {
+    return KIND == FROM_REAL || KIND == TO_REAL || ln.stride == 1;
   }
-  const int64_t base0 = l0 * ln.s0 + (int64_t)l1b * ln.s1;
-  const int nb = min(B, ln.nl1 - l1b);
-  // element e of the workgroup's B lines: line l, position a (line-major on the contiguous axis,
-  // line-minor otherwise, so a load instruction reads B adjacent lines); POW2 plans have B a
-  // power of two as well, and the split is shifts and masks
-  const int lgn = POW2 ? __builtin_ctz(n) : 0, lgb = POW2 ? __builtin_ctz(B) : 0;
-  auto split = [&](int e) __attribute__((always_inline)) {   // (line, position); e < B n <= 8192
-    if (ln.stride == 1) {
-      const int l = POW2 ? e >> lgn : fdiv(e, plan.ndiv);
-      return make_int2(l, e - l * n);
-    }
-    const int a = POW2 ? e >> lgb : fdiv(e, ln.bdiv);
-    return make_int2(POW2 ? e & (B - 1) : e - a * B, a);
-  };
-  // all of a thread's loads are issued before any is used (B n <= kMax: 8 or 16 per thread)
-  constexpr int kPer = FftPts<R, POW2>::kMax / kFftThreads;
-  Cx<R> ld[kPer];
+  __device__ __forceinline__ FastDiv bdiv() const { return ln.bdiv; }
+  // the second line of the last pair may not exist
+  __device__ __forceinline__ bool second(int l) const { return 2 * (l1b + l) + 1 < ln.nr1; }
+
+  template <int RR>
+  __device__ __forceinline__ void load(int l, int i, int m, Cx<R>* x) const {
+    if (KIND == FROM_REAL) {
+      const R* a = rin + (int64_t)(2 * l) * ln.nr2;
+      const bool two = second(l);
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const int e = threadIdx.x + q * kFftThreads;
-    ld[q] = Cx<R>{0, 0};
-    if (e < B * n) {
-      const int2 la = split(e);
-      if (la.x < nb && la.y < ln.nin) ld[q] = data[base0 + (int64_t)la.x * ln.s1 + (int64_t)la.y * ln.stride];
-    }
-  }
+      for (int j = 0; j < RR; ++j) {
+        const int e = i + j * m;
+        x[j] = Cx<R>{0, 0};
+        if (l < nb && e < ln.nin) {
+          x[j].x = a[e];
+          if (two) x[j].y = a[e + ln.nr2];
+        }
+      }
+    } else if (KIND == TO_REAL) {
+      // X = A + i B of the Hermitian halves A and B; their first and middle values are real
+      const Cx<R>* a = data + (int64_t)(2 * l) * ln.s1;
+      const bool two = second(l);
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const int e = threadIdx.x + q * kFftThreads;
-    if (e < B * n) {
-      const int2 la = split(e);
-      buf0[la.x * LS + sk<R>(la.y)] = ld[q];
-    }
-  }
-  __syncthreads();
-  Cx<R>* res = run_stages<R, POW2>(plan, buf0, buf1, tw, n, B, inplace);
-  if (MUL) {
-    // line (j, k) = (l0, l1b + l), position i; the octant index folds each of them
-    const int j = (int)l0, jj = min(j, gv.m1 - j);
-    for (int e = threadIdx.x; e < B * n; e += kFftThreads) {
-      const int2 la = split(e);
-      if (la.x < nb) {
-        const int k = l1b + la.x, i = la.y;
-        const R f = gv.g[((int64_t)min(i, gv.m0 - i) * gv.o1 + jj) * gv.o2 + min(k, gv.m2 - k)] * gv.scale;
-        Cx<R>& v = res[la.x * LS + sk<R>(la.y)];
-        v.x *= f;
-        v.y *= f;
+      for (int j = 0; j < RR; ++j) {
+        const int e = i + j * m, k = min(e, n - e);
+        x[j] = Cx<R>{0, 0};
+        if (l < nb) {
+          Cx<R> u = a[k], v{0, 0};
+          if (two) v = a[k + ln.s1];
+          const R sg = 2 * k == n || k == 0 ? (R)0 : e == k ? (R)1 : (R)-1;
+          x[j] = Cx<R>{u.x - sg * v.y, sg * u.y + v.x};
+        }
+      }
+    } else {
+      const Cx<R>* a = data + (int64_t)l * ln.s1 + (int64_t)i * ln.stride;
+#pragma unroll
+      for (int j = 0; j < RR; ++j) {
+        x[j] = Cx<R>{0, 0};
+        if (l < nb && i + j * m < ln.nin) x[j] = a[(int64_t)(j * m) * ln.stride];
       }
     }
-    for (int q = threadIdx.x; q < n; q += kFftThreads) tw[sk<R>(q)].y = -tw[sk<R>(q)].y;
-    __syncthreads();
-    res = run_stages<R, POW2>(plan, res, res == buf0 ? buf1 : buf0, tw, n, B, inplace);
   }
-  for (int e = threadIdx.x; e < B * n; e += kFftThreads) {
-    const int2 la = split(e);
-    if (la.x < nb && la.y < ln.nout)
-      data[base0 + (int64_t)la.x * ln.s1 + (int64_t)la.y * ln.stride] = res[la.x * LS + sk<R>(la.y)];
+
+  template <int RR>
+  __device__ __forceinline__ void store(int l, int i, int m, const Cx<R>* x) const {
+    if (l >= nb) return;
+    if (KIND == TO_REAL) {
+      TO* a = rout + (int64_t)(2 * l) * ln.nr2;
+      const bool two = second(l);
+#pragma unroll
+      for (int j = 0; j < RR; ++j) {
+        const int e = i + j * m;
+        if (e < ln.nout) {
+          a[e] = (TO)x[j].x;
+          if (two) a[e + ln.nr2] = (TO)x[j].y;
+        }
+      }
+    } else {
+      Cx<R>* a = data + (int64_t)l * ln.s1 + (int64_t)i * ln.stride;
+#pragma unroll
+      for (int j = 0; j < RR; ++j)
+        if (i + j * m < ln.nout) a[(int64_t)(j * m) * ln.stride] = x[j];
+    }
+  }
+
+  // TURN_*: line (j, k) = (l0, l1b + l) with k <= m2 / 2, position along axis 0
+  template <int RR>
+  __device__ __forceinline__ void factor(int l, int i, int m, Cx<R>* x) const {
+    if (l >= nb) return;
+    const int k = l1b + l;
+    if (KIND == TURN_FREE) {
+      const R* g = fv.g + (int64_t)min(l0, fv.m1 - l0) * fv.o2 + k;
+      const int64_t gs = (int64_t)fv.o1 * fv.o2;
+#pragma unroll
+      for (int j = 0; j < RR; ++j) {
+        const int e = i + j * m;
+        const R f = g[min(e, n - e) * gs] * fv.scale;
+        x[j].x *= f;
+        x[j].y *= f;
+      }
+    } else {
+      // -1 / (4 pi^2 |k|^2), 0 at k = 0 (kernel_fft.cu:82-106).  The frequency of an odd axis is not
+      // antisymmetric there (index n / 2 counts as -(n + 1) / 2); the real part of the full inverse
+      // transform, which is the result, has the mean of the factors at k and -k.
+      const double ky = periodic_freq(l0, fv.m1, fv.step), kz = periodic_freq(k, fv.m2, fv.step);
+      const double kyz = ky * ky, kz2 = kz * kz;
+      const bool odd = (fv.m0 | fv.m1 | fv.m2) & 1;
+      double my = ky, mz = kz;
+      if (odd) {
+        my = periodic_freq(l0 ? fv.m1 - l0 : 0, fv.m1, fv.step);
+        mz = periodic_freq(k ? fv.m2 - k : 0, fv.m2, fv.step);
+      }
+#pragma unroll
+      for (int j = 0; j < RR; ++j) {
+        const int e = i + j * m;
+        if ((e | l0 | k) == 0) {
+          x[j] = Cx<R>{0, 0};
+          continue;
+        }
+        const double kx = periodic_freq(e, n, fv.step);
+        double f = -1.0 / (4.0 * M_PI * M_PI * (kx * kx + kyz + kz2)) * fv.norm;
+        if (odd) {
+          const double mx = periodic_freq(e ? n - e : 0, n, fv.step);
+          f = 0.5 * (f + -1.0 / (4.0 * M_PI * M_PI * (mx * mx + my * my + mz * mz)) * fv.norm);
+        }
+        x[j].x = (R)(x[j].x * f);
+        x[j].y = (R)(x[j].y * f);
+      }
+    }
+  }
+};
+
+// One pass along one axis (unnormalised transforms).  PATH GENERIC (a prime factor above 7, or a
+// single stage): the lines are loaded into LDS, the stages run between two planes and the result
+// is stored from there.  FP64, 240 x 256 x 200 in free space (480 x 512 x 400), complex passes on all of
+// the padded axis 2 with an LDS exchange at both ends -> these: x 1840 -> 590 us (0.8 GB moved), y 300 -> 125 and
+// 121, z 260 -> 106 and 100.  What is left in x: LDS busy for 55 % of the time, arithmetic for 39 %.
+template <typename R, typename TO, int KIND, int PATH>
+__global__ __launch_bounds__(kFftThreads) void k_fft_axis(Cx<R>* __restrict__ data, const R* __restrict__ rin,
+                                                       TO* __restrict__ rout, const Cx<R>* __restrict__ twg,
+                                                       AxisPlan plan, AxisPlan back, AxisLines ln,
+                                                       FactorView<R> fv) {
+  extern __shared__ unsigned char smem[];
+  constexpr bool TURN = KIND == TURN_FREE || KIND == TURN_PERIODIC;
+  constexpr int DIR = KIND == INVERSE || KIND == TO_REAL ? 1 : -1;
+  constexpr bool P2 = PATH == POW2;
+  const int n = plan.n;
+  const int B = ln.B;
+  const int LS = line_slots(n);
+  Cx<R>* tw = (Cx<R>*)smem;
+  Cx<R>* buf0 = tw + table_slots(n);
+  Cx<R>* buf1 = buf0 + (int64_t)B * LS;
+  const int lines_per_row = (ln.nl1 + B - 1) / B;
+  const int l0 = blockIdx.x / lines_per_row;
+  const int l1b = (blockIdx.x % lines_per_row) * B;
+  constexpr bool REAL = KIND == FROM_REAL || KIND == TO_REAL;
+  const int64_t first = (int64_t)l0 * ln.s0 + (int64_t)(REAL ? 2 * l1b : l1b) * ln.s1;
+  const int64_t rfirst = REAL ? ((int64_t)l0 * ln.nr1 + 2 * l1b) * ln.nr2 : 0;
+  const LineIO<R, TO, KIND> io{data + first, rin + rfirst, rout + rfirst, ln, fv, n, l0, l1b,
+                               min(B, ln.nl1 - l1b)};
+  for (int q = threadIdx.x; q < n; q += kFftThreads) tw[sk(q)] = twg[q];
+  Cx<R>* res = buf0;
+  if (PATH == GENERIC) {
+    const bool rows = io.rows();
+    auto split = [&](int e) __attribute__((always_inline)) {   // (line, position)
+      if (rows) {
+        const int l = fdiv(e, plan.ndiv);
+        return make_int2(l, e - l * n);
+      }
+      const int a = fdiv(e, ln.bdiv);
+      return make_int2(e - a * B, a);
+    };
+    for (int e = threadIdx.x; e < B * n; e += kFftThreads) {
+      const int2 la = split(e);
+      io.template load<1>(la.x, la.y, 0, buf0 + la.x * LS + sk(la.y));
+    }
+    __syncthreads();
+    res = run_generic<R, DIR>(plan, buf0, buf1, tw, B, LS);
+    if (TURN) {
+      for (int e = threadIdx.x; e < B * n; e += kFftThreads) {
+        const int2 la = split(e);
+        io.template factor<1>(la.x, la.y, 0, res + la.x * LS + sk(la.y));
+      }
+      __syncthreads();
+      res = run_generic<R, 1>(plan, res, res == buf0 ? buf1 : buf0, tw, B, LS);
+    }
+    if (KIND != FROM_REAL) {
+      for (int e = threadIdx.x; e < B * n; e += kFftThreads) {
+        const int2 la = split(e);
+        io.template store<1>(la.x, la.y, 0, res + la.x * LS + sk(la.y));
+      }
+    }
+  } else {
+    const int last = plan.nstage - 1;   // >= 1
+    run_stage<R, DIR, 1, P2>(io, plan, 0, buf0, tw, B, LS);
+    for (int s = 1; s < last; ++s) run_stage<R, DIR, 0, P2>(io, plan, s, buf0, tw, B, LS);
+    if (TURN) {
+      run_stage<R, DIR, 3, P2>(io, plan, last, buf0, tw, B, LS);
+      for (int s = 1; s < last; ++s) run_stage<R, 1, 0, P2>(io, back, s, buf0, tw, B, LS);
+      run_stage<R, 1, 2, P2>(io, back, last, buf0, tw, B, LS);
+    } else if (KIND == FROM_REAL) {
+      run_stage<R, DIR, 0, P2>(io, plan, last, buf0, tw, B, LS);
+    } else {
+      run_stage<R, DIR, 2, P2>(io, plan, last, buf0, tw, B, LS);
+    }
+  }
+  if (KIND == FROM_REAL) {
+    // Z = A + i B: A_k = (Z_k + conj Z_-k) / 2, B_k = (Z_k - conj Z_-k) / 2i
+    const int h = n / 2 + 1;
+    for (int e = threadIdx.x; e < B * h; e += kFftThreads) {
+      const int l = fdiv(e, ln.hdiv), k = e - l * h;
+      if (l < io.nb) {
+        const Cx<R>* z = res + l * LS;
+        const Cx<R> u = z[sk(k)], v = z[sk(k ? n - k : 0)];
+        Cx<R>* a = io.data + (int64_t)(2 * l) * ln.s1 + k;
+        a[0] = Cx<R>{(R)0.5 * (u.x + v.x), (R)0.5 * (u.y - v.y)};
+        if (io.second(l)) a[ln.s1] = Cx<R>{(R)0.5 * (u.y + v.y), (R)0.5 * (v.x - u.x)};
+      }
+    }
   }
 }
 
-// rhs, C order, into a [m0][m1][m2] complex buffer (m >= n: zero padding already in place).
-// Tile: 32 i x 32 k at fixed j; Q is read along i (x-fastest) and written along k.
+// rhs, C order [n0][n1][n2].  Tile: 32 i x 32 k at fixed j; Q is read along i (x-fastest) and written
+// along k.  The nuclei whose cutoff sphere reaches the tile's box are listed first (in order, 256 at a
+// time): 50 atoms at 240 x 256 x 200, 253 us testing every atom at every voxel, 79 us so.
 template <typename R, typename TI>
 __global__ __launch_bounds__(kThreads) void k_rhs(const TI* __restrict__ q, const double4* __restrict__ atoms,
-                                                  int natoms, GeomView g, double sigma, double cut2, int m1, int m2,
-                                                  Cx<R>* __restrict__ out) {
+                                                  int natoms, GeomView g, double sigma, double cut2,
+                                                  R* __restrict__ out) {
   __shared__ double tile[32][33];
+  __shared__ double4 near[kThreads];
+  __shared__ int cnt[kThreads / 64];
   const int i0 = blockIdx.x * 32, k0 = blockIdx.z * 32, j = blockIdx.y;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 32 x 8
+  const double step = g.h / kAng2Bor;
+  const double norm = 1.0 / (sigma * sigma * sigma * 2.0 * M_PI * sqrt(2.0 * M_PI));
+  const double inv2s2 = 1.0 / (2.0 * sigma * sigma);
+#pragma unroll
   for (int r = ty; r < 32; r += 8) {
     const int i = i0 + tx, k = k0 + r;
     double v = 0.0;
@@ -407,45 +630,59 @@ __global__ __launch_bounds__(kThreads) void k_rhs(const TI* __restrict__ q, cons
     tile[r][tx] = v;
   }
   __syncthreads();
-  const double step = g.h / kAng2Bor;
-  const double norm = 1.0 / (sigma * sigma * sigma * 2.0 * M_PI * sqrt(2.0 * M_PI));
-  const double inv2s2 = 1.0 / (2.0 * sigma * sigma);
-  for (int r = ty; r < 32; r += 8) {
-    const int i = i0 + r, k = k0 + tx;
-    if (i >= g.nx || k >= g.nz) continue;
-    double rho = tile[tx][r] / (-(step * step * step));
-    const double x = g.ox / kAng2Bor + (i + 0.5) * step;
-    const double y = g.oy / kAng2Bor + (j + 0.5) * step;
-    const double z = g.oz / kAng2Bor + (k + 0.5) * step;
-    for (int a = 0; a < natoms; ++a) {
-      const double4 A = atoms[a];
-      const double dx = x - A.x * kRBohr, dy = y - A.y * kRBohr, dz = z - A.z * kRBohr;
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      if (r2 <= cut2) rho += A.w * norm * exp(-r2 * inv2s2);
+  const double y = g.oy / kAng2Bor + (j + 0.5) * step;
+  const double z = g.oz / kAng2Bor + (k0 + tx + 0.5) * step;
+  double rho[4], x[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int r = ty + 8 * c;
+    rho[c] = tile[tx][r] / (-(step * step * step));
+    x[c] = g.ox / kAng2Bor + (i0 + r + 0.5) * step;
+  }
+  const double xm = g.ox / kAng2Bor + (i0 + 16) * step, zm = g.oz / kAng2Bor + (k0 + 16) * step, hw = 16.0 * step;
+  for (int a0 = 0; a0 < natoms; a0 += kThreads) {
+    // the box around the voxel centres, half a step wider: rounding cannot lose an atom
+    double4 A{0, 0, 0, 0};
+    bool in = false;
+    if (a0 + (int)threadIdx.x < natoms) {
+      A = atoms[a0 + threadIdx.x];
+      A.x *= kRBohr;
+      A.y *= kRBohr;
+      A.z *= kRBohr;
+      const double bx = fmax(fabs(A.x - xm) - hw, 0.0), by = fmax(fabs(A.y - y) - 0.5 * step, 0.0),
+                   bz = fmax(fabs(A.z - zm) - hw, 0.0);
+      in = bx * bx + by * by + bz * bz <= cut2;
     }
-    out[((int64_t)i * m1 + j) * m2 + k] = Cx<R>{(R)(-rho / kEps0), (R)0};
+    const uint64_t ball = __ballot(in);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) cnt[wave] = __popcll(ball);
+    __syncthreads();
+    int at = __popcll(ball & (((uint64_t)1 << lane) - 1)), n = 0;
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; ++w) {
+      at += w < wave ? cnt[w] : 0;
+      n += cnt[w];
+    }
+    if (in) near[at] = A;
+    __syncthreads();
+    for (int t = 0; t < n; ++t) {
+      const double4 C = near[t];
+      const double dy = y - C.y, dz = z - C.z;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const double dx = x[c] - C.x;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        if (r2 <= cut2) rho[c] += C.w * norm * exp(-r2 * inv2s2);
+      }
+    }
+    __syncthreads();
   }
-}
-
-// periodic Poisson in k space, normalisation of the inverse transform folded in (kernel_fft.cu:82-106)
-template <typename R>
-__global__ void k_poisson_periodic(Cx<R>* __restrict__ a, int n0, int n1, int n2, double step, double scale) {
-  const int64_t N = (int64_t)n0 * n1 * n2;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= N) return;
-  const int k = (int)(idx % n2), j = (int)((idx / n2) % n1), i = (int)(idx / ((int64_t)n1 * n2));
-  if (idx == 0) {
-    a[0] = Cx<R>{0, 0};
-    return;
+  const int k = k0 + tx;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int i = i0 + ty + 8 * c;
+    if (i < g.nx && k < g.nz) out[((int64_t)i * g.ny + j) * g.nz + k] = (R)(-rho[c] / kEps0);
   }
-  const double kx = (i > n0 / 2 - 1 ? (double)(i - n0) : (double)i) / (n0 * step);
-  const double ky = (j > n1 / 2 - 1 ? (double)(j - n1) : (double)j) / (n1 * step);
-  const double kz = (k > n2 / 2 - 1 ? (double)(k - n2) : (double)k) / (n2 * step);
-  const double f = -1.0 / (4.0 * M_PI * M_PI * (kx * kx + ky * ky + kz * kz)) * scale;
-  Cx<R> v = a[idx];
-  v.x = (R)(v.x * f);
-  v.y = (R)(v.y * f);
-  a[idx] = v;
 }
 
 // g(d) at unit grid step on the m0 x m1 x m2 cyclic grid (m >= 2n), C order: |d_i| = min(i, m - i),
@@ -476,18 +713,33 @@ __global__ void k_green_store(const Cx<R>* __restrict__ a, R* __restrict__ gh, i
   gh[idx] = (R)((double)a[((int64_t)i * m1 + j) * m2 + k].x * scale);
 }
 
-template <typename R, typename TO>
-__global__ void k_extract(const Cx<R>* __restrict__ a, int m1, int m2, int n0, int n1, int n2, TO* __restrict__ out) {
-  const int64_t N = (int64_t)n0 * n1 * n2;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= N) return;
-  const int k = (int)(idx % n2), j = (int)((idx / n2) % n1), i = (int)(idx / ((int64_t)n1 * n2));
-  out[idx] = (TO)a[((int64_t)i * m1 + j) * m2 + k].x;
+// ------------------------------------------------------------------ host: plans
+// Stage radices of a length, largest first.  Powers of two and lengths without a prime factor above 7:
+// as few stages as radices up to 8 (10) allow, of those the smallest sum (480 = 10 8 6, 400 = 10 8 5,
+// 1024 = 8 8 4 4); otherwise 8, 4, 2, 3, 5, 7 and the larger primes.
+void best_radices(int n, bool pow2, std::vector<int>& cur, std::vector<int>& best) {
+  if (n == 1) {
+    auto sum = [](const std::vector<int>& v) {
+      int t = 0;
+      for (int r : v) t += r;
+      return t;
+    };
+    if (best.empty() || cur.size() < best.size() || (cur.size() == best.size() && sum(cur) < sum(best))) best = cur;
+    return;
+  }
+  if (!best.empty() && cur.size() + 1 > best.size()) return;
+  for (int r : {10, 8, 7, 6, 5, 4, 3, 2}) {
+    if (n % r || (!cur.empty() && r > cur.back()) || (pow2 && (r & (r - 1)))) continue;
+    cur.push_back(r);
+    best_radices(n / r, pow2, cur, best);
+    cur.pop_back();
+  }
 }
 
-// ------------------------------------------------------------------ host: plans
 std::vector<int> factorize(int n) {
-  std::vector<int> f;
+  std::vector<int> f, cur;
+  best_radices(n, (n & (n - 1)) == 0, cur, f);
+  if (!f.empty()) return f;
   for (int r : {8, 4, 2, 3, 5, 7}) {
     while (n % r == 0) {
       f.push_back(r);
@@ -572,24 +824,12 @@ int freespace_len(int n) {
   }
 }
 
-// one pass along `axis` of a C-order [m0][m1][m2] buffer, on the lines whose
-// other two indices are below (lim_a, lim_b) (in increasing axis order); positions >= nin
-// are read as zero and positions >= nout are not written.  gv: forward transform, product
-// with the Green's function transform and inverse transform in one pass (axis 0 only).
-template <typename R, bool INV>
-int fft_pass(qm_ctx* ctx, hipStream_t s, Cx<R>* data, const int m[3], int axis, int lim_a, int lim_b, int nin,
-             int nout, const GreenView<R>* gv = nullptr) {
-  const int n = m[axis];
-  const Cx<R>* tw = nullptr;
-  int rc = twiddle_table<R>(ctx, n, &tw);
-  if (rc) return rc;
+AxisPlan make_plan(int n, const std::vector<int>& f) {
   AxisPlan plan{};
   plan.n = n;
-  std::vector<int> f = factorize(n);
-  QM_REQUIRE(ctx, (int)f.size() <= kMaxStages, QM_ELIMIT, "fft: too many stages for length %d", n);
-  int span = 1;
   plan.nstage = (int)f.size();
   plan.ndiv = FastDiv::of(n);
+  int span = 1;
   for (size_t q = 0; q < f.size(); ++q) {
     plan.radix[q] = f[q];
     plan.span[q] = span;
@@ -597,28 +837,49 @@ int fft_pass(qm_ctx* ctx, hipStream_t s, Cx<R>* data, const int m[3], int axis, 
     plan.pdiv[q] = FastDiv::of(span);
     span *= f[q];
   }
-  const int64_t st[3] = {(int64_t)m[1] * m[2], (int64_t)m[2], 1};
+  return plan;
+}
+
+// One pass along `axis` (length n) of a C-order [..][m1][row] complex buffer, on the lines whose other
+// two indices are below (lim_a, lim_b) (in increasing axis order); positions >= nin are read as zero and
+// positions >= nout are not written.  FROM_REAL / TO_REAL (axis 2): rin / rout is a real
+// [lim_a][lim_b][nin / nout] array, the complex lines hold n / 2 + 1 values.
+template <typename R, typename TO, int KIND>
+int fft_pass(qm_ctx* ctx, hipStream_t s, Cx<R>* data, const R* rin, TO* rout, int n, int m1, int row, int axis,
+             int lim_a, int lim_b, int nin, int nout, const FactorView<R>& fv = FactorView<R>{}) {
+  constexpr bool REAL = KIND == FROM_REAL || KIND == TO_REAL;
+  const Cx<R>* tw = nullptr;
+  int rc = twiddle_table<R>(ctx, n, &tw);
+  if (rc) return rc;
+  const std::vector<int> f = factorize(n);
+  QM_REQUIRE(ctx, (int)f.size() <= kMaxStages, QM_ELIMIT, "fft: too many stages for length %d", n);
+  const AxisPlan plan = make_plan(n, f);
+  const AxisPlan back = make_plan(n, std::vector<int>(f.rbegin(), f.rend()));
+  const int64_t st[3] = {(int64_t)m1 * row, (int64_t)row, 1};
   AxisLines ln{};
   ln.stride = st[axis];
-  int oa = axis == 0 ? 1 : 0;            // other axes, oa < ob
-  int ob = axis == 2 ? 1 : 2;
+  const int oa = axis == 0 ? 1 : 0, ob = axis == 2 ? 1 : 2;   // other axes, oa < ob
   ln.nl0 = lim_a;
-  ln.nl1 = lim_b;
+  ln.nl1 = REAL ? (lim_b + 1) / 2 : lim_b;
   ln.s0 = st[oa];
   ln.s1 = st[ob];
   ln.nin = nin;
   ln.nout = nout;
-  QM_REQUIRE(ctx, nin >= 1 && nin <= n && nout >= 1 && nout <= n && (!gv || axis == 0), QM_EINVAL,
-             "fft: bad pass");
-  bool inplace = true;
-  for (int r : f) inplace = inplace && r <= 8;
-  const int planes = inplace ? 1 : 2;
-  // B lines of n points per workgroup: B * n <= kMax (the register staging bound of stage_inplace)
-  const bool pow2 = (n & (n - 1)) == 0;
+  ln.nr1 = lim_b;
+  ln.nr2 = KIND == TO_REAL ? nout : nin;
+  ln.hdiv = FastDiv::of(n / 2 + 1);
+  QM_REQUIRE(ctx, nin >= 1 && nin <= n && nout >= 1 && nout <= n && (axis == 2 || !REAL), QM_EINVAL, "fft: bad pass");
+  bool radix = f.size() >= 2;
+  for (int r : f) radix = radix && r <= 10;
+  const int planes = radix ? 1 : 2;
+  const bool pow2 = radix && (n & (n - 1)) == 0;
+  // B lines of n points per workgroup: B * n <= kMax (the register bound of a stage), whole cache lines
+  // of adjacent lines where that allows it
   const int kMaxPts = pow2 ? FftPts<R, true>::kMax : FftPts<R, false>::kMax;
   QM_REQUIRE(ctx, n <= 4096, QM_ELIMIT, "fft: length %d exceeds 4096", n);
   int B = std::max(1, std::min(16, kMaxPts / n));
-  if (!inplace) B = std::max(1, std::min(B, 2048 / n));
+  if (!radix) B = std::max(1, std::min(B, 2048 / n));
+  if (axis != 2 && B > 8) B = B / 8 * 8;
   B = std::max(1, std::min(B, ln.nl1));
   if (pow2)
     while (B & (B - 1)) B &= B - 1;   // the power-of-two kernel splits indices by shifts
@@ -626,39 +887,34 @@ int fft_pass(qm_ctx* ctx, hipStream_t s, Cx<R>* data, const int m[3], int axis, 
   ln.bdiv = FastDiv::of(B);
   const int lines_per_row = (ln.nl1 + B - 1) / B;
   const int64_t nwg = (int64_t)ln.nl0 * lines_per_row;
-  const size_t shmem = sizeof(Cx<R>) * ((size_t)table_slots<R>(n) + (size_t)planes * B * line_slots<R>(n));
+  const size_t shmem = sizeof(Cx<R>) * ((size_t)table_slots(n) + (size_t)planes * B * line_slots(n));
   QM_REQUIRE(ctx, shmem <= (size_t)128 * 1024, QM_ELIMIT, "fft: length %d needs %zu bytes of LDS per workgroup", n,
              shmem);
   QM_REQUIRE(ctx, nwg <= 0x7fffffff, QM_ELIMIT, "fft: too many lines");
   if (nwg == 0) return QM_OK;
   static bool attr_set = false;
   if (!attr_set) {
-    const void* fns[4] = {(const void*)k_fft_axis<R, INV, false>, (const void*)k_fft_axis<R, INV, true>,
-                          (const void*)k_fft_axis<R, false, false, true>, (const void*)k_fft_axis<R, false, true, true>};
+    const void* fns[3] = {(const void*)k_fft_axis<R, TO, KIND, POW2>, (const void*)k_fft_axis<R, TO, KIND, RADIX>,
+                          (const void*)k_fft_axis<R, TO, KIND, GENERIC>};
     for (const void* f : fns)
       QM_CHECK_HIP(ctx, hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024));
     attr_set = true;
   }
   ProfScope ps(ctx, s, QM_K_FFT_AXIS);
-  const GreenView<R> g0 = gv ? *gv : GreenView<R>{};
   const dim3 grid((unsigned)nwg), thr(kFftThreads);
-  const int ip = inplace ? 1 : 0;
-  if (gv) {
-    if (pow2)
-      hipLaunchKernelGGL((k_fft_axis<R, false, true, true>), grid, thr, shmem, s, data, tw, plan, ln, 1, g0);
-    else
-      hipLaunchKernelGGL((k_fft_axis<R, false, false, true>), grid, thr, shmem, s, data, tw, plan, ln, ip, g0);
-  } else if (pow2) {
-    hipLaunchKernelGGL((k_fft_axis<R, INV, true>), grid, thr, shmem, s, data, tw, plan, ln, 1, g0);
-  } else {
-    hipLaunchKernelGGL((k_fft_axis<R, INV, false>), grid, thr, shmem, s, data, tw, plan, ln, ip, g0);
-  }
+  if (pow2)
+    hipLaunchKernelGGL((k_fft_axis<R, TO, KIND, POW2>), grid, thr, shmem, s, data, rin, rout, tw, plan, back, ln, fv);
+  else if (radix)
+    hipLaunchKernelGGL((k_fft_axis<R, TO, KIND, RADIX>), grid, thr, shmem, s, data, rin, rout, tw, plan, back, ln, fv);
+  else
+    hipLaunchKernelGGL((k_fft_axis<R, TO, KIND, GENERIC>), grid, thr, shmem, s, data, rin, rout, tw, plan, back, ln,
+                       fv);
   QM_CHECK_LAUNCH(ctx);
   return QM_OK;
 }
 
 template <typename R>
-int green_hat(qm_ctx* ctx, hipStream_t s, const int m[3], Cx<R>* work, const R** out) {
+int green_hat(qm_ctx* ctx, hipStream_t s, const int m[3], const R** out) {
   if (!ctx->fft) ctx->fft = new FftPlanCache();
   FftPlanCache& fc = *ctx->fft;
   for (auto& gr : fc.greens)
@@ -668,12 +924,15 @@ int green_hat(qm_ctx* ctx, hipStream_t s, const int m[3], Cx<R>* work, const R**
       return QM_OK;
     }
   const int64_t M = (int64_t)m[0] * m[1] * m[2];
+  Cx<R>* work = nullptr;
+  int rc = qm_ws(ctx, s, WS_FFT_A, sizeof(Cx<R>) * (size_t)M, (void**)&work);
+  if (rc) return rc;
   hipLaunchKernelGGL(k_green<R>, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, s, work, m[0], m[1], m[2]);
   QM_CHECK_LAUNCH(ctx);
-  int rc;
-  if ((rc = fft_pass<R, false>(ctx, s, work, m, 2, m[0], m[1], m[2], m[2]))) return rc;
-  if ((rc = fft_pass<R, false>(ctx, s, work, m, 1, m[0], m[2], m[1], m[1]))) return rc;
-  if ((rc = fft_pass<R, false>(ctx, s, work, m, 0, m[1], m[2], m[0], m[0]))) return rc;
+  R* const none = nullptr;
+  if ((rc = fft_pass<R, R, FORWARD>(ctx, s, work, none, none, m[2], m[1], m[2], 2, m[0], m[1], m[2], m[2]))) return rc;
+  if ((rc = fft_pass<R, R, FORWARD>(ctx, s, work, none, none, m[1], m[1], m[2], 1, m[0], m[2], m[1], m[1]))) return rc;
+  if ((rc = fft_pass<R, R, FORWARD>(ctx, s, work, none, none, m[0], m[1], m[2], 0, m[1], m[2], m[0], m[0]))) return rc;
   const int o[3] = {m[0] / 2 + 1, m[1] / 2 + 1, m[2] / 2 + 1};
   const int64_t O = (int64_t)o[0] * o[1] * o[2];
   // make room: release the least recently used transforms (work queued earlier on s still reads them)
@@ -706,50 +965,42 @@ int hartree_fft(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, const
   const int n[3] = {g->nx, g->ny, g->nz};
   const int m[3] = {fs ? freespace_len(n[0]) : n[0], fs ? freespace_len(n[1]) : n[1],
                     fs ? freespace_len(n[2]) : n[2]};
-  const int64_t M = (int64_t)m[0] * m[1] * m[2];
-  Cx<R>* work = nullptr;
-  int rc = qm_ws(ctx, s, WS_FFT_A, sizeof(Cx<R>) * (size_t)M, (void**)&work);
-  if (rc) return rc;
-  GreenView<R> gv{};
+  int rc;
+  FactorView<R> fv{};
+  fv.m0 = m[0];
+  fv.m1 = m[1];
+  fv.m2 = m[2];
+  fv.step = g->step / kAng2Bor;
   if (fs) {
-    if ((rc = green_hat<R>(ctx, s, m, work, &gv.g))) return rc;
-    const double h_ang = g->step / kAng2Bor;
-    gv.m0 = m[0];
-    gv.m1 = m[1];
-    gv.m2 = m[2];
-    gv.o1 = m[1] / 2 + 1;
-    gv.o2 = m[2] / 2 + 1;
-    gv.scale = (R)(h_ang * h_ang);
+    if ((rc = green_hat<R>(ctx, s, m, &fv.g))) return rc;
+    fv.o1 = m[1] / 2 + 1;
+    fv.o2 = m[2] / 2 + 1;
+    fv.scale = (R)(fv.step * fv.step);
+  } else {
+    fv.norm = 1.0 / (double)((int64_t)m[0] * m[1] * m[2]);
   }
+  // half spectrum [n0][m1][hs] and the real right-hand side [n0][n1][n2]
+  const int h2 = m[2] / 2 + 1, al = (int)(128 / sizeof(Cx<R>));
+  const int hs = h2 >= 4 * al ? (h2 + al - 1) / al * al : h2;
+  const size_t W = (size_t)n[0] * m[1] * hs, N = (size_t)n[0] * n[1] * n[2];
+  Cx<R>* work = nullptr;
+  if ((rc = qm_ws(ctx, s, WS_FFT_A, sizeof(Cx<R>) * W + sizeof(R) * N, (void**)&work))) return rc;
+  R* rhs = (R*)(work + W);
+  R* const none = nullptr;
   const GeomView gview = geom_view(g);
   const double cut2 = (cutoff * sigma) * (cutoff * sigma);
-  // rhs on [i < n0][j < n1][k < n2]; every pass reads only positions already written (the
-  // padding is never cleared: it is read as zero) and writes only positions read later
   hipLaunchKernelGGL((k_rhs<R, TIO>), dim3((n[0] + 31) / 32, n[1], (n[2] + 31) / 32), dim3(kThreads), 0, s, q,
-                     (const double4*)mol->atoms, mol->natoms, gview, sigma, cut2, m[1], m[2], work);
+                     (const double4*)mol->atoms, mol->natoms, gview, sigma, cut2, rhs);
   QM_CHECK_LAUNCH(ctx);
-  // forward: z on lines (i < n0, j < n1), y on (i < n0, all k), x on all (j, k); inverse in reverse
-  if ((rc = fft_pass<R, false>(ctx, s, work, m, 2, n[0], n[1], n[2], m[2]))) return rc;
-  if ((rc = fft_pass<R, false>(ctx, s, work, m, 1, n[0], m[2], n[1], m[1]))) return rc;
-  if (fs) {
-    // x: forward, times G^, inverse, keeping i < n0
-    if ((rc = fft_pass<R, false>(ctx, s, work, m, 0, m[1], m[2], n[0], n[0], &gv))) return rc;
-  } else {
-    if ((rc = fft_pass<R, false>(ctx, s, work, m, 0, m[1], m[2], m[0], m[0]))) return rc;
-    const unsigned blocks = (unsigned)((M + 255) / 256);
-    const double step_ang = g->step / kAng2Bor;
-    hipLaunchKernelGGL(k_poisson_periodic<R>, dim3(blocks), dim3(256), 0, s, work, m[0], m[1], m[2], step_ang,
-                       1.0 / (double)M);
-    QM_CHECK_LAUNCH(ctx);
-    if ((rc = fft_pass<R, true>(ctx, s, work, m, 0, m[1], m[2], m[0], m[0]))) return rc;
-  }
-  if ((rc = fft_pass<R, true>(ctx, s, work, m, 1, n[0], m[2], m[1], n[1]))) return rc;
-  if ((rc = fft_pass<R, true>(ctx, s, work, m, 2, n[0], n[1], m[2], n[2]))) return rc;
-  const int64_t N = (int64_t)n[0] * n[1] * n[2];
-  hipLaunchKernelGGL((k_extract<R, TIO>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, (const Cx<R>*)work,
-                     m[1], m[2], n[0], n[1], n[2], out);
-  QM_CHECK_LAUNCH(ctx);
-  return QM_OK;
+  if ((rc = fft_pass<R, R, FROM_REAL>(ctx, s, work, rhs, none, m[2], m[1], hs, 2, n[0], n[1], n[2], h2))) return rc;
+  if ((rc = fft_pass<R, R, FORWARD>(ctx, s, work, none, none, m[1], m[1], hs, 1, n[0], h2, n[1], m[1]))) return rc;
+  if (fs)
+    rc = fft_pass<R, R, TURN_FREE>(ctx, s, work, none, none, m[0], m[1], hs, 0, m[1], h2, n[0], n[0], fv);
+  else
+    rc = fft_pass<R, R, TURN_PERIODIC>(ctx, s, work, none, none, m[0], m[1], hs, 0, m[1], h2, n[0], n[0], fv);
+  if (rc) return rc;
+  if ((rc = fft_pass<R, R, INVERSE>(ctx, s, work, none, none, m[1], m[1], hs, 1, n[0], h2, m[1], n[1]))) return rc;
+  return fft_pass<R, TIO, TO_REAL>(ctx, s, work, none, out, m[2], m[1], hs, 2, n[0], n[1], h2, n[2]);
 }
 
 }  // namespace
