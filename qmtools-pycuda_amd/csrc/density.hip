@@ -623,10 +623,21 @@ struct Vec8<__bf16> {
 // L2 copy of the row tile's basis values; the heaviest block goes first.
 constexpr int kTT = 128, kTKS = 16, kTPad = 8, kTWG = 512;
 
+// Workgroup b goes to XCD b mod 8 and there, whatever the load, to one of 4 shader engines in turn: with
+// slot = b / 8, slot mod 4 decides.  An even number of column blocks per tile would send the same blocks,
+// whose lengths differ, to the same engines, so their order is turned with the tile.  60 atoms, 256^3, tiles
+// sorted by length: FP64 35.5 ms with one workgroup per tile, 44.2 with two and 66.6 with four in fixed order,
+// 36.0 and 36.7 turned; split 14.3 and 18.0, turned 13.4 and 13.7.  Odd numbers turn by themselves (turned
+// as well: FP64 with three 36.4 -> 40.1).
 __device__ __forceinline__ bool tile_coords(int b, int nrt, int ncb, int& rt, int& cb) {
   const int xcd = b & 7, slot = b >> 3;
   const int rl = slot / ncb;
-  cb = ncb - 1 - (slot - rl * ncb);
+  int k = slot - rl * ncb;
+  if (!(ncb & 1)) {
+    k += rl + (rl >> 1);
+    k -= k / ncb * ncb;
+  }
+  cb = ncb - 1 - k;
   // row tile 8 rl + xcd, turned by a hash of rl within its group of 8: with tiles per grid row a multiple of
   // 8, a fixed xcd would own fixed x ranges of the grid, and the one through the molecule's middle would
   // finish last (the CUs were busy 64-81% of the launch)
@@ -797,6 +808,7 @@ struct BlockTiles {
   int ng;                 // groups of the whole basis: stride of a tile's list, values and partial sums
   const uint16_t* list;   // [row tile][ng]: active groups in increasing order
   const int* cnt;         // [row tile]: how many
+  const int* order;       // the contraction's order of the row tiles, null: as numbered
 };
 
 __host__ __device__ inline int64_t block_tiles(const GeomView& g) {
@@ -871,6 +883,42 @@ template <int GS>
 __global__ __launch_bounds__(kTT) void k_tile_list(MolView m, GeomView g, BlockTiles b, int all,
                                                    uint16_t* __restrict__ list, int* __restrict__ cnt) {
   tile_list_body<GS>(m, g, b, blockIdx.x, all, list, cnt);
+}
+
+// The row tiles of a chunk by falling length of their lists (counting sort, one workgroup), the order in which
+// the contraction takes them: in grid order the last workgroups of a launch are long ones as often as not, and
+// the shader engines' shares differ.  60 atoms, 256^3: FP64 contraction 31.7 -> 27.7 ms (20 launches, 7 us of
+// sorting each), split 7.74 -> 7.47 ms (10 launches, 11.5 us).  Below kOrderMin tiles all workgroups run at
+// once; above kOrderMax (small bases) the end of the launch no longer counts and the sort would.
+constexpr int kOrderMin = 1024, kOrderMax = 32768;
+__global__ __launch_bounds__(1024) void k_tile_order(const int* __restrict__ cnt, int nrt, int* __restrict__ order) {
+  __shared__ int at[kMaxGroups + 1];
+  __shared__ int sums[1024];
+  constexpr int PT = (kMaxGroups + 1024) / 1024;   // bins per thread, longest lists first
+  const int t = threadIdx.x;
+  for (int i = t; i <= kMaxGroups; i += 1024) at[i] = 0;
+  __syncthreads();
+  for (int i = t; i < nrt; i += 1024) atomicAdd(&at[kMaxGroups - cnt[i]], 1);
+  __syncthreads();
+  int mine[PT], total = 0;
+#pragma unroll
+  for (int q = 0; q < PT; ++q) {
+    mine[q] = total;
+    if (t * PT + q <= kMaxGroups) total += at[t * PT + q];
+  }
+  sums[t] = total;
+  __syncthreads();
+  for (int d = 1; d < 1024; d <<= 1) {
+    const int v = t >= d ? sums[t - d] : 0;
+    __syncthreads();
+    sums[t] += v;
+    __syncthreads();
+  }
+#pragma unroll
+  for (int q = 0; q < PT; ++q)
+    if (t * PT + q <= kMaxGroups) at[t * PT + q] = sums[t] - total + mine[q];
+  __syncthreads();
+  for (int i = t; i < nrt; i += 1024) order[atomicAdd(&at[kMaxGroups - cnt[i]], 1)] = i;
 }
 
 // Walks the listed groups of a row tile as runs of consecutive functions (wave uniform): run(j, fj, f0, f1)
@@ -1075,7 +1123,9 @@ __global__ __launch_bounds__(kTWG, 4) void k_contract_f64_blocks(const double* _
                                                                  const double* __restrict__ M, int np, BlockTiles b,
                                                                  int nrt, int ny, double* __restrict__ part) {
   int rt, y;
-  if (tile_coords(blockIdx.x, nrt, ny, rt, y)) f64_block_tile(rt, ny - 1 - y, ny, phi, M, np, b, part);
+  if (!tile_coords(blockIdx.x, nrt, ny, rt, y)) return;
+  if (b.order) rt = b.order[rt];
+  f64_block_tile(rt, ny - 1 - y, ny, phi, M, np, b, part);
 }
 
 // Density of a voxel: partial sums of its row tiles in list order (FP64: one per group; split: two per block
@@ -1613,8 +1663,9 @@ __global__ __launch_bounds__(512, 4) void k_contract_split_blocks(const T16* __r
                                                                   int np_part, int nrt, int ny,
                                                                   double* __restrict__ part) {
   int rt, y;
-  if (tile_coords(blockIdx.x, nrt, ny, rt, y))
-    split_block_tile<T16>(rt, ny - 1 - y, ny, phi, p_hi, p_lo, np, b, np_part, part);
+  if (!tile_coords(blockIdx.x, nrt, ny, rt, y)) return;
+  if (b.order) rt = b.order[rt];
+  split_block_tile<T16>(rt, ny - 1 - y, ny, phi, p_hi, p_lo, np, b, np_part, part);
 }
 
 // ---------------------------------------------------------------------------
@@ -2550,12 +2601,13 @@ float split_phi_scale(const qm_mol* m);
 // Workgroups per row tile (ncb column blocks at most).  Bases of up to two blocks: one, because a workgroup's
 // start (count, list, first loads: about 7 us) costs more than a second block holds (246 functions, FP64,
 // 6.6 M points: 3.0 ms with one, 4.2 ms with two), unless the tiles alone do not fill the 512 workgroup slots.
-// Larger ones: several, side by side on one XCD, so that the blocks of a tile share its basis values in L2
-// (606 functions, 0.88 M points: FP64 2.05 / 1.90 / 1.71 / 1.66 ms with 1 / 2 / 3 / 5; split, 1.77 M points,
-// 0.94 / 0.88 / 0.82 / 0.81 ms, but a batch of 5-80 atoms 11.1 / 12.5 / 11.5 / 13.0 ms).
+// Larger ones: two, side by side on one XCD, so that the blocks of a tile share its basis values in L2, or one
+// per block where the tiles are few.  606 functions, 1 / 2 / 3 / 5 workgroups: FP64, 512 tiles 335 / 307 / 292 /
+// 261 us, 2048 tiles 1126 / 803 / 779 / 783 us, 6912 tiles 2.33 / 2.22 / 2.25 / 2.27 ms; split, 512 tiles 140 /
+// 142 / 132 / 125 us, 2048 tiles 351 / 343 / 343 / 345 us, 6912 tiles 0.93 / 0.84 / 0.84 / 1.44 ms.
 inline int block_split(int nrt, int ncb, bool f64) {
   if (ncb <= 2) return nrt >= 512 ? 1 : ncb;
-  return f64 ? ncb : 3;
+  return nrt >= (f64 ? 4096 : 1024) ? 2 : ncb;
 }
 // Workgroups per four tiles in the basis-value launch (blk of them): 2048 workgroups of four waves fill the
 // chip; with fewer the list (n8 units of 8 functions at most) is shared out.
@@ -2584,22 +2636,26 @@ int density_blocks(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, in
   int rc = QM_OK;
   if ((rc = qm_ws(ctx, s, WS_PHI, tile_bytes * rows, (void**)&phi))) return rc;
   if ((rc = qm_ws(ctx, s, WS_PART, sizeof(double) * kTT * (size_t)nparts * rows, (void**)&part))) return rc;
-  if ((rc = qm_ws(ctx, s, WS_MASK, (sizeof(int) + sizeof(uint16_t) * (size_t)ng) * rows, (void**)&lists))) return rc;
+  if ((rc = qm_ws(ctx, s, WS_MASK, (2 * sizeof(int) + sizeof(uint16_t) * (size_t)ng) * rows, (void**)&lists))) return rc;
   int* cnt = (int*)lists;
-  uint16_t* list = (uint16_t*)(lists + sizeof(int) * rows);
+  int* order = cnt + rows;
+  uint16_t* list = (uint16_t*)(lists + 2 * sizeof(int) * rows);
   const float S = f64 ? 1.f : split_phi_scale(mol);
   const double h3 = g->step * g->step * g->step;
   const double scale = (f64 ? h3 : h3 / mol->pfac / ((double)S * S)) / nsub3;
   const T* M = (const T*)(f64 ? (const void*)mol->M64 : std::is_same<T, _Float16>::value ? mol->P16 : mol->Pb16);
   for (int64_t T0 = 0; T0 < ntiles; T0 += nT) {
-    const BlockTiles b{(int)T0, (int)std::min(nT, ntiles - T0), nsub, ng, list, cnt};
-    const int nrt = b.nT * nsub3, pblk = f64 ? (nrt + 1) / 2 : (nrt + kPhiTiles - 1) / kPhiTiles;
+    const int nTc = (int)std::min(nT, ntiles - T0), nrt = nTc * nsub3;
+    const bool sorted = nrt >= kOrderMin && nrt <= kOrderMax;
+    const BlockTiles b{(int)T0, nTc, nsub, ng, list, cnt, sorted ? order : nullptr};
+    const int pblk = f64 ? (nrt + 1) / 2 : (nrt + kPhiTiles - 1) / kPhiTiles;
     const dim3 pgrid(pblk, phi_split(pblk, ng << (GS - 3)));
     const int ny = block_split(nrt, ncb, f64);
     const dim3 cgrid(tile_grid(nrt, ny));
     {
       ProfScope ps(ctx, s, f64 ? QM_K_PHI : QM_K_PHI_SPLIT);
       hipLaunchKernelGGL(k_tile_list<GS>, dim3(nrt), dim3(kTT), 0, s, mv, gv, b, f64 && !ctx->tile_skip, list, cnt);
+      if (sorted) hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, (const int*)cnt, nrt, order);
       if constexpr (f64)
         hipLaunchKernelGGL(k_phi_f64_blocks, pgrid, dim3(kPhiThreads), 0, s, mv, (const int2*)mol->kgroups, gv, b, nrt,
                            phi);

@@ -73,3 +73,26 @@ def test_basis_points_in_the_callers_order():
     nat.call("qm_basis_points", device_molecule(mol).handle, nat.stream(), nat.dptr(d), 70, nat.dptr(phi))
     got = phi.cpu().numpy().reshape(mol.nbf, 70)
     assert numpy.abs(got - want).max() <= 1e-13 * numpy.abs(want).max()
+
+
+@pytest.mark.parametrize("shape", [(88, 372, 4), (128, 32, 32), (121, 65, 37), (256, 128, 128), (256, 129, 128)])
+def test_block_tiles_sorted_launches(shape):
+    """1023 tiles (as numbered), 1024, 2720 and 32768 (by list length), 33792 (as numbered); the gates of the full
+    grids on z slabs of 4 planes."""
+    import qmtools
+    from oracle import density as od
+    from qmtools import _native as nat, synth
+    mol = synth.synthetic_molecule(3, 12, qmtools.BasisSet(BASIS))
+    h = 0.2
+    o = mol.coords.mean(0) - 0.5 * h * numpy.array(shape) + 0.05
+    nx, ny, nz = shape
+    system = _system(mol)
+    slabs = {k: od.density_grid_raw(system, nx, ny, 4, h, o + numpy.array([0, 0, k * h]), 1).reshape(4, ny, nx)
+             for k in {0, (nz // 2) // 4 * 4, nz - 4}}
+    top = max(numpy.abs(w).max() for w in slabs.values())
+    print("[case] sorted tiles", shape, flush=True)
+    for prec, tol in ((nat.QM_PREC_FP64, 1e-10), (nat.QM_PREC_F16X3, 1e-6)):
+        got = _raw(mol, (*shape, h, tuple(o)), 1, prec).reshape(nz, ny, nx)
+        assert numpy.isfinite(got).all()
+        for k, want in slabs.items():
+            assert numpy.abs(got[k:k + 4] - want).max() <= tol * top
