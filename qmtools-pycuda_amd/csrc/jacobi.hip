@@ -784,8 +784,8 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   return QM_OK;
 }
 
-// 256^3, 2000 sweeps: 128.5 -> 1.47 ms with the charge and the boundary; 72 x 64 x 56 to a delta of 1e-4:
-// 45 -> 0.62 ms.
+// 256^3, 2000 sweeps: 128.5 -> 1.12 ms with the charge and the boundary; 72 x 64 x 56 to a delta of 1e-4:
+// 45 -> 0.58 ms.
 int jacobi_fp64(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const double* rho, double* v, double* tmp,
                 int64_t max_sweeps, double tol, int check_every, int64_t* done_out, double* delta_out) {
   if (max_sweeps >= qm_sine_sweeps(g) && qm_sine_fits(g)) {

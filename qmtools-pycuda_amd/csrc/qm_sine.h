@@ -7,8 +7,9 @@
 
 struct SinePlan {
   int nx, ny;               // grid row and plane sizes
-  int m[3], ld[3];          // interior points per axis, row length of S
-  const double* S[3];       // S_kn = sqrt(2 / (m + 1)) sin(pi k n / (m + 1)), zero padded
+  int m[3], ld[3];          // interior points per axis, row length of the tables
+  const double* S[3];       // S_kn = sqrt(2 / (m + 1)) sin(pi k n / (m + 1)), n <= (m + 1) / 2: odd k,
+  const double* So[3];      // even k (1-based), zero padded
   const double* s2[3];      // sin^2(pi k / (2 (m + 1))), k = 1 .. m
   double* part;             // partial sums of an x pass
   double* sum;              // their sum
@@ -47,8 +48,8 @@ int qm_sine_x_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a
 // bisection in the logarithm of delta.
 int qm_sine_first_below(int64_t n, double dn, double tol, const std::function<int(int64_t, double*)>& delta_at,
                         int64_t* at, double* delta);
-// Sweep counts from which a closed form is taken: it costs what 21 sweeps do at 256^3 (1.32 ms against 64 us a
-// sweep; its 12 n flops a point grow with the axis, a sweep's 24 bytes do not) and about 20 on small grids
+// Sweep counts from which a closed form is taken: it costs what 15 sweeps do at 256^3 (0.92 ms against 64 us a
+// sweep; its 6 n flops a point grow with the axis, a sweep's 24 bytes do not) and about 20 on small grids
 // (eight launches against one replayed node a sweep).
 inline int64_t qm_sine_sweeps(const qm_geom* g) {
   const int n = g->nx > g->ny ? g->nx : g->ny;

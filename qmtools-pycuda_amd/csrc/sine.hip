@@ -9,15 +9,20 @@
 // change of the n-th sweep (the convergence test) is 3 transforms of a^(n-1) times the stored spectrum.
 //
 // One axis is a product with the symmetric m x m matrix S_kn = sqrt(2 / (m + 1)) sin(pi k n / (m + 1)), which
-// is its own inverse.  A matrix product takes 2 m flops per point where an FFT would take about
-// 2.5 log2 m per real point, but it runs on the FP64 matrix cores for any m (an FFT of the odd extension has
-// length 2 (m + 1) = 510 for 256 points, with factors 17 and 51), and one pass reads and writes each
-// value once like an FFT pass: 256^3, 6 transforms: 50 GFLOP, 1.6 GB.
+// is its own inverse.  Its rows are even or odd under n -> m + 1 - n in turn, so the product is two of half the
+// size: the rows of odd k take the sums u_j = x_j + x_m+1-j, those of even k the differences, m flops per point.
+// An FFT would take about 2.5 log2 m per real point, but this runs on the FP64 matrix cores for any m (an FFT of
+// the odd extension has length 2 (m + 1) = 510 for 256 points, with factors 17 and 51), and one pass reads and
+// writes each value once like an FFT pass: 256^3, 6 transforms: 25 GFLOP, 1.6 GB.
 //
-// Kernel: a workgroup of 8 waves owns 16 LT lines and keeps their values in LDS ([line tile][n][16 lines]:
-// an MFMA operand row is 128 contiguous bytes, and 4 consecutive rows cover all 64 banks); wave w owns the row tiles w,
-// w + 8, .. of the result and reads S from L2 (64 points: 32 KB, 254: 516 KB) straight into operands.  Lines are
-// read whole before anything is stored, so a pass works in place.
+// Kernel: a workgroup of 8 waves owns 16 LT lines and keeps their sums and differences in LDS ([line tile][j]
+// [16 lines]: an MFMA operand row is 128 contiguous bytes, and 4 consecutive rows cover all 64 banks; the lines of
+// row j are permuted by j mod 16, so that 16 values of one line spread over the banks too, as lines along x are
+// loaded and stored); waves 0-3 own the rows of odd k, waves 4-7 those of even k, and read S from L2 (64 points:
+// 16 KB, 254: 258 KB) straight into operands.  Lines are read whole before anything is stored, so a pass works
+// in place.  254^3, with all of S and rows shared out among 8 waves -> these: x from the residual 242 -> 188 us, y 192 ->
+// 128, z forward, factor and back 448 -> 314, x added to V 228 -> 160 (262 MB a pass: 53 us of copying; the products
+// 58 us at the rate of a large one); load, product and store of a workgroup follow each other, two share a CU.
 #include <algorithm>
 #include <cmath>
 
@@ -76,7 +81,8 @@ __device__ __forceinline__ double factor(const SinePlan& p, const SineFactor& f,
 
 template <int LT, int RT, int AX, int LOAD, bool MID, int STORE>
 __global__ __launch_bounds__(kThreads) void k_sine(Args a) {
-  __shared__ __align__(16) double x[LT][128 * RT][16];
+  constexpr int HP = 64 * RT;         // rows 0 ..: sums, rows HP ..: differences
+  __shared__ __align__(16) double x[LT][2 * HP][16];
   __shared__ int64_t base[16 * LT];   // first interior point of each line
   __shared__ int2 mode[16 * LT];      // its indices along the two other axes
   const SinePlan& p = a.p;
@@ -84,6 +90,7 @@ __global__ __launch_bounds__(kThreads) void k_sine(Args a) {
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int li = lane & 15, lk = lane >> 4;
   const int m = p.m[AX], ld = p.ld[AX];
+  const int half = (m + 1) / 2;       // sums; m / 2 differences
   const int m0 = AX == 0 ? p.m[1] : p.m[0];   // fast one of the other axes
   const int m1 = AX == 2 ? p.m[1] : p.m[2];
   const int64_t nx = p.nx, nxy = (int64_t)p.nx * p.ny;
@@ -97,73 +104,97 @@ __global__ __launch_bounds__(kThreads) void k_sine(Args a) {
     mode[t] = make_int2(u, w);
   }
   __syncthreads();
+  auto at = [&](int line, int row) __attribute__((always_inline)) -> double& {
+    return x[line >> 4][row][(line ^ row) & 15];
+  };
   // mode (kx, ky, kz) of element n of line t
   auto fac = [&](int line, int n) __attribute__((always_inline)) -> double {
     const int2 u = mode[line];
     return AX == 0 ? factor(p, a.f, n, u.x, u.y) : AX == 1 ? factor(p, a.f, u.x, n, u.y) : factor(p, a.f, u.x, u.y, n);
   };
-  const int rows = (m + 15) / 16 * 16;
   bool bad = false;
-  // lines along x: 16 threads per 128 bytes of a line; else consecutive threads take neighbouring lines
+  auto load = [&](int line, int n) __attribute__((always_inline)) -> double {
+    const int64_t idx = base[line] + n * stride;
+    if (LOAD == LOAD_RESIDUAL) {
+      const double* __restrict__ V = a.in;
+      double s = V[idx - 1] + V[idx + 1];
+      s += V[idx + nx];
+      s += V[idx - nx];
+      s += V[idx + nxy];
+      s += V[idx - nxy];
+      const double v = fma(-a.rho[idx], a.hinv, s) * (1.0 / 6.0) - V[idx];
+      bad = bad || !(fabs(v) < INFINITY);
+      return v;
+    }
+    const double v = a.in[idx];
+    if (LOAD != LOAD_SCALED) return v;
+    {
+#pragma clang fp contract(off)   // the product is rounded before the sums, as where it is kept in between (MID)
+      const double scaled = v * fac(line, n);
+      return scaled;
+    }
+  };
+  // element e of the workgroup's count * 16 LT: lines along x: 16 threads per 128 bytes of a line; else
+  // consecutive threads take neighbouring lines
+  auto split = [&](int e, int& line, int& n) __attribute__((always_inline)) {
+    line = AX == 0 ? (e >> 4) % (16 * LT) : e % (16 * LT);
+    n = AX == 0 ? (e & 15) + 16 * ((e >> 4) / (16 * LT)) : e / (16 * LT);
+  };
+  const int rows = (half + 15) / 16 * 16;
   for (int e = t; e < rows * 16 * LT; e += kThreads) {
-    const int line = AX == 0 ? (e >> 4) % (16 * LT) : e % (16 * LT);
-    const int n = AX == 0 ? (e & 15) + 16 * ((e >> 4) / (16 * LT)) : e / (16 * LT);
-    double v = 0.0;
-    if (n < m) {
-      const int64_t idx = base[line] + n * stride;
-      if (LOAD == LOAD_RESIDUAL) {
-        const double* __restrict__ V = a.in;
-        double s = V[idx - 1] + V[idx + 1];
-        s += V[idx + nx];
-        s += V[idx - nx];
-        s += V[idx + nxy];
-        s += V[idx - nxy];
-        v = fma(-a.rho[idx], a.hinv, s) * (1.0 / 6.0) - V[idx];
-        bad = bad || !(fabs(v) < INFINITY);
-      } else {
-        v = a.in[idx];
-        if (LOAD == LOAD_SCALED) v *= fac(line, n);
+    int line, j;
+    split(e, line, j);
+    double u = 0.0, v = 0.0;
+    if (j < half) {
+      u = load(line, j);
+      const int n = m - 1 - j;
+      if (n != j) {
+        const double w = load(line, n);
+        v = u - w;
+        u += w;
       }
     }
-    x[line >> 4][n][line & 15] = v;
+    at(line, j) = u;
+    at(line, HP + j) = v;
   }
   if (LOAD == LOAD_RESIDUAL && bad) atomicOr(p.flag, 1);
   __syncthreads();
 
-  const double* __restrict__ S = p.S[AX];
+  const int odd = wave >> 2, w4 = wave & 3;   // odd: differences, rows k = 2 r + 1 (0-based)
+  const int kk = odd ? m / 2 : half;
+  const double* __restrict__ S = odd ? p.So[AX] : p.S[AX];
   d4 acc[RT][LT];
   auto product = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int l = 0; l < LT; ++l) acc[r][l] = d4{0, 0, 0, 0};
-    const double* __restrict__ Sw = S + (int64_t)lk * ld + 16 * wave + li;
+    const double* __restrict__ Sw = S + (int64_t)lk * ld + 16 * w4 + li;
+    const int lx = li ^ lk;
     auto run = [&](auto nrc) __attribute__((always_inline)) {
       constexpr int NR = decltype(nrc)::value;
 #pragma unroll 4
-      for (int n0 = 0; n0 < m; n0 += 4) {   // rows m .. of S and of x are zero
+      for (int n0 = 0; n0 < kk; n0 += 4) {   // rows beyond the half of S and of x are zero
         double b[LT], s[NR > 0 ? NR : 1];
 #pragma unroll
-        for (int r = 0; r < NR; ++r) s[r] = Sw[(int64_t)n0 * ld + 128 * r];
+        for (int r = 0; r < NR; ++r) s[r] = Sw[(int64_t)n0 * ld + 64 * r];
 #pragma unroll
-        for (int l = 0; l < LT; ++l) b[l] = x[l][n0 + lk][li];
+        for (int l = 0; l < LT; ++l) b[l] = x[l][HP * odd + n0 + lk][lx ^ (n0 & 12)];
 #pragma unroll
         for (int r = 0; r < NR; ++r)
 #pragma unroll
-          for (int l = 0; l < LT; ++l)   // along x the lines go first, so that 16 lanes store 16 points of a line
-            acc[r][l] = AX == 0 ? __builtin_amdgcn_mfma_f64_16x16x4f64(b[l], s[r], acc[r][l], 0, 0, 0)
-                                : __builtin_amdgcn_mfma_f64_16x16x4f64(s[r], b[l], acc[r][l], 0, 0, 0);
+          for (int l = 0; l < LT; ++l) acc[r][l] = __builtin_amdgcn_mfma_f64_16x16x4f64(s[r], b[l], acc[r][l], 0, 0, 0);
       }
     };
-    // row tiles of this wave: wave + 8 r < rows / 16 (uniform)
-    const int nr = max(0, (rows / 16 - wave + 7) / 8);
+    // row tiles of this wave: w4 + 4 r < (kk + 15) / 16 (uniform)
+    const int nr = max(0, ((kk + 15) / 16 - w4 + 3) / 4);
     if (nr == RT) run(std::integral_constant<int, RT>());
     else if (RT > 1 && nr == RT - 1) run(std::integral_constant<int, RT - 1>());
     else if (RT > 2 && nr == RT - 2) run(std::integral_constant<int, (RT > 2 ? RT - 2 : 0)>());
     else if (RT > 3 && nr == RT - 3) run(std::integral_constant<int, (RT > 3 ? RT - 3 : 0)>());
     else if (RT > 4 && nr == RT - 4) run(std::integral_constant<int, (RT > 4 ? RT - 4 : 0)>());
   };
-  // element of acc[r][l][q]: along x (line 16 l + 4 q + lk, n = 16 (wave + 8 r) + li), else the reverse
+  // element of acc[r][l][q]: line 16 l + li, n = 2 (16 (w4 + 4 r) + 4 q + lk) + odd
   auto each = [&](auto&& f) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < RT; ++r)
@@ -171,27 +202,52 @@ __global__ __launch_bounds__(kThreads) void k_sine(Args a) {
       for (int l = 0; l < LT; ++l)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int line = 16 * l + (AX == 0 ? 4 * q + lk : li);
-          const int n = 16 * (wave + 8 * r) + (AX == 0 ? li : 4 * q + lk);
-          if (n < m) f(line, n, acc[r][l][q]);
+          const int n = 2 * (16 * (w4 + 4 * r) + 4 * q + lk) + odd;
+          if (n < m) f(16 * l + li, n, acc[r][l][q]);
         }
   };
   product();
   if (MID) {
+    // scaled values at the rows of their sums and differences, then folded in place
     __syncthreads();
-    each([&](int line, int n, double v) { x[line >> 4][n][line & 15] = v * fac(line, n); });
+    each([&](int line, int n, double v) { at(line, n < half ? n : HP + m - 1 - n) = v * fac(line, n); });
+    __syncthreads();
+    for (int e = t; e < half * 16 * LT; e += kThreads) {
+      const int line = e % (16 * LT), j = e / (16 * LT);
+      double u = at(line, j), v = 0.0;
+      if (m - 1 - j != j) {
+        const double w = at(line, HP + j);
+        v = u - w;
+        u += w;
+      }
+      at(line, j) = u;
+      at(line, HP + j) = v;
+    }
     __syncthreads();
     product();
   }
   double sum = 0.0;
-  each([&](int line, int n, double v) {
+  auto store = [&](int line, int n, double v) __attribute__((always_inline)) {
     if (l0 + line >= nl) return;
     const int64_t idx = base[line] + n * stride;
     if (STORE == STORE_PLAIN) a.out[idx] = v;
     else if (STORE == STORE_ADD) a.out[idx] += v;
     else if (STORE == STORE_SUM) sum += fabs(v);
     else sum += fabs(a.out[idx] + v);
-  });
+  };
+  if (AX == 0 && STORE != STORE_SUM) {
+    // along x a wave's values are every other point: through LDS, so that whole cache lines are stored
+    __syncthreads();
+    each([&](int line, int n, double v) { at(line, n) = v; });
+    __syncthreads();
+    for (int e = t; e < (m + 15) / 16 * 16 * 16 * LT; e += kThreads) {
+      int line, n;
+      split(e, line, n);
+      if (n < m) store(line, n, at(line, n));
+    }
+  } else {
+    each(store);
+  }
   if (STORE == STORE_SUM || STORE == STORE_SUMV) {
     __shared__ double red[8];
 #pragma unroll
@@ -206,22 +262,24 @@ __global__ __launch_bounds__(kThreads) void k_sine(Args a) {
   }
 }
 
-// S_kn with zero columns up to ld and zero rows up to a multiple of 4, and sin^2(pi k / (2 (m + 1)))
+// The halves of S (row j: input, column r: output 2 r or 2 r + 1, 0-based) with zero columns up to ld and zero rows
+// up to a multiple of 4, and sin^2(pi k / (2 (m + 1)))
 __global__ __launch_bounds__(256) void k_sine_tables(SinePlan p) {
   const int ax = blockIdx.y, m = p.m[ax], ld = p.ld[ax];
-  const int rows = (m + 3) / 4 * 4;
-  double* __restrict__ S = const_cast<double*>(p.S[ax]);
+  const int half = (m + 1) / 2, rows = (half + 3) / 4 * 4;
   double* __restrict__ s2 = const_cast<double*>(p.s2[ax]);
   if (ax == 0 && blockIdx.x == 0 && threadIdx.x == 0) *p.flag = 0;
   const double scale = sqrt(2.0 / (m + 1));
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < rows * ld; i += gridDim.x * 256) {
-    const int n = i / ld, k = i - n * ld;
-    const int64_t r = (int64_t)(n + 1) * (k + 1) % (2 * (m + 1));
-    S[i] = n < m && k < m ? scale * sinpi((double)r / (m + 1)) : 0.0;
-    if (i < m) {
-      const double h = sinpi((double)(i + 1) / (2 * (m + 1)));
-      s2[i] = h * h;
-    }
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < 2 * rows * ld; i += gridDim.x * 256) {
+    const int odd = i >= rows * ld, q = i - odd * rows * ld;
+    const int j = q / ld, r = q - j * ld, k = 2 * r + odd;
+    const int64_t a = (int64_t)(j + 1) * (k + 1) % (2 * (m + 1));
+    const bool in = k < m && j < (odd ? m / 2 : half);
+    const_cast<double*>(odd ? p.So[ax] : p.S[ax])[q] = in ? scale * sinpi((double)a / (m + 1)) : 0.0;
+  }
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < m; i += gridDim.x * 256) {
+    const double h = sinpi((double)(i + 1) / (2 * (m + 1)));
+    s2[i] = h * h;
   }
 }
 
@@ -293,13 +351,15 @@ int qm_sine_plan(qm_ctx* ctx, hipStream_t s, const qm_geom* g, SinePlan* p) {
   const int n[3] = {g->nx, g->ny, g->nz};
   p->nx = g->nx;
   p->ny = g->ny;
-  size_t doubles = 0, off[3], most = 0;
+  size_t doubles = 0, off[3], table[3], most = 0;
   for (int d = 0; d < 3; ++d) {
     p->m[d] = n[d] - 2;
-    p->ld[d] = (p->m[d] + 15) / 16 * 16;
+    const int half = (p->m[d] + 1) / 2;
+    p->ld[d] = (half + 15) / 16 * 16;
+    table[d] = (size_t)((half + 3) / 4 * 4) * p->ld[d];
     off[d] = doubles;
-    most = std::max(most, (size_t)((p->m[d] + 3) / 4 * 4) * p->ld[d]);
-    doubles += (size_t)((p->m[d] + 3) / 4 * 4) * p->ld[d] + p->ld[d];
+    most = std::max(most, 2 * table[d]);
+    doubles += 2 * table[d] + p->m[d];
   }
   // partial sums of an x pass, then the flag
   const size_t nparts = ((size_t)p->m[1] * p->m[2] + 15) / 16;
@@ -308,7 +368,8 @@ int qm_sine_plan(qm_ctx* ctx, hipStream_t s, const qm_geom* g, SinePlan* p) {
   if (rc) return rc;
   for (int d = 0; d < 3; ++d) {
     p->S[d] = w + off[d];
-    p->s2[d] = p->S[d] + (size_t)((p->m[d] + 3) / 4 * 4) * p->ld[d];
+    p->So[d] = p->S[d] + table[d];
+    p->s2[d] = p->So[d] + table[d];
   }
   p->part = w + doubles;
   p->sum = p->part + nparts;
