@@ -305,156 +305,90 @@ inline int pick_zs2(int nx, int ny, int nz, int fixed) {
   return std::max(4, (nz + tz - 1) / tz);
 }
 
-// FP32 two-sweep pass with two adjacent columns per lane (8-byte loads and stores, half the
-// lane shuffles per point).  A strip spans 128 columns, lane L holding columns i and i + 1 with
-// i = 124 bx - 2 + 2L; the first sweep is formed on all 128 columns and the second on columns
-// 2 ... 125, the strip's 124 outputs.  The first sweep at the two outer columns sees a clamped
-// or the lane's own value as its missing neighbour; it feeds only the second sweep at columns 1
-// and 126, which is not stored, so no halo column is loaded.  nx must be even: pairs start at
-// even columns and lie wholly inside or outside the grid.  Each point's arithmetic and summation
-// order are those of the one-column kernels, so the results are bitwise the same.
-constexpr int kWP = 2 * kSW - 4;   // output columns per strip
-constexpr int kR2P = 4;            // rows per strip
-template <int R>
-struct Strip2P {
-  static constexpr int W = kWP;
-  static constexpr int TY = R * kSWaves;
+// FP32, T sweeps per pass on tiles that a workgroup keeps on chip: 32 columns x 16 rows x RZ planes, of which
+// the inner part, T points from the sides, is stored.  A thread owns one column of RZ points, V and rho in
+// registers; x neighbours come from the adjacent lanes (a wave holds two rows of 32), y neighbours through
+// LDS, z neighbours from the thread's registers.  Every point of the tile is relaxed in every sweep; values
+// near its sides lack a neighbour and are not those of the sweep, but they move inwards by one point a
+// sweep and so never reach what is stored.  Each stored point's arithmetic and summation order are those of T
+// single sweeps, so the result is bitwise the same.
+//
+// All loads of a tile are in flight at once, where strips that march through the planes (4 rows of 2 columns per
+// lane, loads two planes ahead) waited for one plane after the other: us per sweep on n^3, strips of two sweeps
+// -> tiles of two (RZ 10), of three (RZ 12): 32: 4.1 -> 2.0, 1.5; 64: 4.3 -> 2.0, 1.6; 96: 5.1 -> 2.5, 2.5; 128:
+// 6.7 -> 3.9, 3.7; 160: 11.6 -> 6.0, 6.3; 192: 13.1 -> 9.0, 10.1; 256: 26.2 -> 22.4, 22.0 (201 MB a pass: 41 us
+// of copying).  32 rows, 64 columns or other heights are slower on most of these.
+constexpr int kTileX = 32, kTileRows = 16;
+template <int T>
+struct Tile {
+  static constexpr int RZ = T == 3 ? 12 : 10;
+  static constexpr int X = kTileX - 2 * T, Y = kTileRows - 2 * T, Z = RZ - 2 * T;   // what is stored
 };
+// grids on which three sweeps per pass are the faster ones (see above): 144^3
+constexpr int64_t kTile3Points = 144 * 144 * 144;
 
-template <int R>
-__device__ __forceinline__ void strip2p_body(int bx, int by, int bz, int zs, const float* __restrict__ rho,
-                                             const float* __restrict__ v, float* __restrict__ vout, int nx, int ny,
-                                             int nz, float h) {
-  constexpr int R0 = R + 4, R1 = R + 2;
-  const int lane = threadIdx.x;
-  const int wy = __builtin_amdgcn_readfirstlane(threadIdx.y);
-  const int i = bx * kWP - 2 + 2 * lane;   // first column of the lane's pair (even)
-  const int j0 = by * Strip2P<R>::TY + wy * R;
-  if (j0 >= ny) return;                    // whole wave idle; the kernel has no barrier
-  const int z0 = bz * zs, z1 = min(nz, z0 + zs);
-  const size_t sy = (size_t)nx, sz = (size_t)nx * ny;
-  // clamped pair: values read at it only feed outer-layer points (copied) or points outside the grid
-  const unsigned ic = (unsigned)min(max(i, 0), nx - 2);
-  auto row = [&](int j) -> size_t { return sy * (size_t)min(max(j, 0), ny - 1); };
-  auto pln = [&](int k) -> size_t { return sz * (size_t)min(max(k, 0), nz - 1); };
-  auto ld = [](const float* __restrict__ p, size_t off) -> float2 { return *(const float2*)(p + off); };
+template <int T>
+__device__ __forceinline__ void tile_body(int bx, int by, int bz, const float* __restrict__ rho,
+                                          const float* __restrict__ v, float* __restrict__ vout, int nx, int ny,
+                                          int nz, float h) {
+  constexpr int RZ = Tile<T>::RZ;
+  __shared__ float ex[RZ][kTileRows][kTileX];
+  const int lx = threadIdx.x & (kTileX - 1), ly = threadIdx.x / kTileX;
+  const int i = bx * Tile<T>::X - T + lx, j = by * Tile<T>::Y - T + ly, k0 = bz * Tile<T>::Z - T;
+  const bool hold = i <= 0 || i >= nx - 1 || j <= 0 || j >= ny - 1;
+  const size_t sz = (size_t)nx * ny;
+  // clamped: values read there only feed points of the outer layer, which are held, or outside the grid
+  const size_t col = (size_t)min(max(j, 0), ny - 1) * nx + min(max(i, 0), nx - 1);
+  float e[RZ], q[RZ];
+#pragma unroll
+  for (int z = 0; z < RZ; ++z) {
+    const size_t at = sz * (size_t)min(max(k0 + z, 0), nz - 1) + col;
+    e[z] = v[at];
+    q[z] = rho[at];
+  }
   const float hinv = 1.0f / h;
-  const bool xb0 = i <= 0 || i >= nx - 1, xb1 = i + 1 <= 0 || i + 1 >= nx - 1;
-  const bool store = lane >= 1 && lane <= kSW - 2 && i < nx;
-  float2 am[R0], ac[R0], ap[R0];   // V on planes m-1, m, m+1, rows j0-2+q
-  float2 bmm[R1], bm[R1];          // first sweep on planes m-2, m-1, rows j0-1+p
-  float2 rc[R1], rm[R1];           // rho of planes m and m-1 (rows j0-1+p)
-  // loads two planes ahead into ping-pong buffers, as in the one-column kernel
-  float2 an[2][R0], rn[2][R1];
-  const int m0 = z0 - 1;
-  auto request = [&](int m, auto buf) __attribute__((always_inline)) {
-    constexpr int b = decltype(buf)::value;
-    const size_t pv = pln(m + 3), pr = pln(m + 2);
+  const int yp = min(ly + 1, kTileRows - 1), ym = max(ly - 1, 0);
 #pragma unroll
-    for (int q = 0; q < R0; ++q) an[b][q] = ld(v, pv + row(j0 - 2 + q) + ic);
+  for (int t = 0; t < T; ++t) {
+    if (t) __syncthreads();
 #pragma unroll
-    for (int p = 0; p < R1; ++p) rn[b][p] = ld(rho, pr + row(j0 - 1 + p) + ic);
-  };
+    for (int z = 0; z < RZ; ++z) ex[z][ly][lx] = e[z];
+    __syncthreads();
+    float below = e[0];
 #pragma unroll
-  for (int q = 0; q < R0; ++q) {
-    am[q] = ld(v, pln(m0 - 1) + row(j0 - 2 + q) + ic);
-    ac[q] = ld(v, pln(m0) + row(j0 - 2 + q) + ic);
-    ap[q] = ld(v, pln(m0 + 1) + row(j0 - 2 + q) + ic);
-    an[1][q] = ld(v, pln(m0 + 2) + row(j0 - 2 + q) + ic);
+    for (int z = 0; z < RZ; ++z) {
+      const float c = e[z];
+      // the lanes next to this one (wave_shr:1, wave_shl:1)
+      const int ci = __builtin_bit_cast(int, c);
+      const float l = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, ci, 0x138, 0xf, 0xf, true));
+      const float r = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, ci, 0x130, 0xf, 0xf, true));
+      float s = l + r;
+      s += ex[z][yp][lx];
+      s += ex[z][ym][lx];
+      s += e[z + 1 < RZ ? z + 1 : z];
+      s += below;
+      s = fmaf(-q[z], hinv, s);
+      const int k = k0 + z;
+      below = c;
+      e[z] = hold || k <= 0 || k >= nz - 1 ? c : s * (float)(1.0 / 6.0);
+    }
   }
+  if (lx < T || lx >= kTileX - T || ly < T || ly >= kTileRows - T || i >= nx || j >= ny) return;
 #pragma unroll
-  for (int p = 0; p < R1; ++p) {
-    rc[p] = ld(rho, pln(m0) + row(j0 - 1 + p) + ic);
-    rn[1][p] = ld(rho, pln(m0 + 1) + row(j0 - 1 + p) + ic);
-    rm[p] = make_float2(0.f, 0.f);
-    bmm[p] = make_float2(0.f, 0.f);
-    bm[p] = make_float2(0.f, 0.f);
-  }
-  // V' at the pair from its x neighbours (l, c.x) and (c.y, r) and the four others
-  auto relax = [&](float2 c, float l, float r, float2 yp, float2 ym, float2 zp, float2 zm, float2 q, bool o0,
-                   bool o1) __attribute__((always_inline)) -> float2 {
-    float s0 = l + c.y;
-    s0 += yp.x;
-    s0 += ym.x;
-    s0 += zp.x;
-    s0 += zm.x;
-    s0 = fmaf(-q.x, hinv, s0);
-    float s1 = c.x + r;
-    s1 += yp.y;
-    s1 += ym.y;
-    s1 += zp.y;
-    s1 += zm.y;
-    s1 = fmaf(-q.y, hinv, s1);
-    return make_float2(o0 ? c.x : s0 * (float)(1.0 / 6.0), o1 ? c.y : s1 * (float)(1.0 / 6.0));
-  };
-  auto step = [&](int m, auto buf) __attribute__((always_inline)) {
-    constexpr int b = decltype(buf)::value;
-    request(m, buf);
-    // first sweep on plane m
-    const bool zb1 = m <= 0 || m >= nz - 1;
-    float2 bc[R1];
-#pragma unroll
-    for (int p = 0; p < R1; ++p) {
-      const int j = j0 - 1 + p;
-      const float2 c = ac[p + 1];
-      const float l = __shfl_up(c.y, 1, kSW);
-      const float r = __shfl_down(c.x, 1, kSW);
-      const bool o = zb1 || j <= 0 || j >= ny - 1;
-      bc[p] = relax(c, l, r, ac[p + 2], ac[p], ap[p + 1], am[p + 1], rc[p], o || xb0, o || xb1);
-    }
-    // second sweep on plane m-1
-    const int k = m - 1;
-    if (k >= z0) {
-      const bool zb2 = k == 0 || k == nz - 1;
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int j = j0 + r;
-        const float2 c = bm[r + 1];
-        const float l = __shfl_up(c.y, 1, kSW);
-        const float rr = __shfl_down(c.x, 1, kSW);
-        const bool o = zb2 || j == 0 || j == ny - 1;
-        const float2 val = relax(c, l, rr, bm[r + 2], bm[r], bc[r + 1], bmm[r + 1], rm[r + 1], o || xb0, o || xb1);
-        if (store && j < ny) *(float2*)(vout + sz * (size_t)k + sy * (size_t)j + (unsigned)i) = val;
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < R0; ++q) {
-      am[q] = ac[q];
-      ac[q] = ap[q];
-      ap[q] = an[1 - b][q];
-    }
-#pragma unroll
-    for (int p = 0; p < R1; ++p) {
-      bmm[p] = bm[p];
-      bm[p] = bc[p];
-      rm[p] = rc[p];
-      rc[p] = rn[1 - b][p];
-    }
-  };
-  int m = m0;
-  for (; m + 1 <= z1; m += 2) {
-    step(m, std::integral_constant<int, 0>());
-    step(m + 1, std::integral_constant<int, 1>());
-  }
-  if (m <= z1) step(m, std::integral_constant<int, 0>());
+  for (int z = T; z < RZ - T; ++z)
+    if (k0 + z < nz) vout[sz * (size_t)(k0 + z) + col] = e[z];
 }
 
-template <int R>
-__global__ __launch_bounds__(kSW* kSWaves) void k_sweep_strip2p(const float* __restrict__ rho,
-                                                                const float* __restrict__ v, float* __restrict__ vout,
-                                                                int nx, int ny, int nz, int zs, float h) {
-  strip2p_body<R>(blockIdx.x, blockIdx.y, blockIdx.z, zs, rho, v, vout, nx, ny, nz, h);
-}
-
-// planes per workgroup of the paired two-sweep kernel (as pick_zs2)
-// the paired kernel's grids: even nx
-inline bool pairs_fit(int nx, int ny) { return nx % 2 == 0 && ny > 0; }
-
-inline int pick_zs2p(int nx, int ny, int nz, int fixed) {
-  if (fixed > 0) return std::min(fixed, nz);
-  const int tiles = ((nx + kWP - 1) / kWP) * ((ny + Strip2P<kR2P>::TY - 1) / Strip2P<kR2P>::TY);
-  const int tz = std::max(1, 1024 / tiles);
-  return std::max(4, (nz + tz - 1) / tz);
+// tx x ty x .. tiles; consecutive ones on one XCD (workgroup b runs on XCD b mod 8), whose L2 then serves the
+// points that they share
+template <int T>
+__global__ __launch_bounds__(kTileX* kTileRows) void k_sweep_tile(const float* __restrict__ rho,
+                                                                  const float* __restrict__ v,
+                                                                  float* __restrict__ vout, int nx, int ny, int nz,
+                                                                  int tx, int ty, float h) {
+  const int xcd = blockIdx.x & 7, per = gridDim.x >> 3, more = gridDim.x & 7;
+  const int b = xcd * per + min(xcd, more) + (int)(blockIdx.x >> 3);
+  tile_body<T>(b % tx, b / tx % ty, b / (tx * ty), rho, v, vout, nx, ny, nz, h);
 }
 
 // planes per workgroup: about 1024 workgroups (4096 waves) for the chip, at least 4 planes each;
@@ -613,19 +547,22 @@ int sweep(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const T* rho, const T* a
   return QM_OK;
 }
 
+template <int T>
+int sweep_tile(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const float* rho, const float* a, float* b) {
+  const int tx = (g->nx + Tile<T>::X - 1) / Tile<T>::X, ty = (g->ny + Tile<T>::Y - 1) / Tile<T>::Y;
+  const int64_t tiles = (int64_t)tx * ty * ((g->nz + Tile<T>::Z - 1) / Tile<T>::Z);
+  QM_REQUIRE(ctx, tiles <= 0x7fffffff, QM_ELIMIT, "jacobi: too many tiles");
+  hipLaunchKernelGGL(k_sweep_tile<T>, dim3((unsigned)tiles), dim3(kTileX * kTileRows), 0, s, rho, a, b, g->nx, g->ny,
+                     g->nz, tx, ty, (float)g->step);
+  QM_CHECK_LAUNCH(ctx);
+  return QM_OK;
+}
+
 // two sweeps a -> b in one pass (bitwise the same as sweep(a -> t), sweep(t -> b))
 template <typename T>
 int sweep2(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const T* rho, const T* a, T* b, bool prof = true) {
   ProfScope ps(ctx, s, QM_K_JACOBI, 2, prof);
-  if (sizeof(T) == 4 && ctx->jacobi_pairs && pairs_fit(g->nx, g->ny)) {
-    const int zs = pick_zs2p(g->nx, g->ny, g->nz, ctx->jacobi_zs);
-    const dim3 grid((g->nx + kWP - 1) / kWP, (g->ny + Strip2P<kR2P>::TY - 1) / Strip2P<kR2P>::TY,
-                    (g->nz + zs - 1) / zs);
-    hipLaunchKernelGGL(k_sweep_strip2p<kR2P>, grid, dim3(kSW, kSWaves), 0, s, (const float*)rho, (const float*)a,
-                       (float*)b, g->nx, g->ny, g->nz, zs, (float)g->step);
-    QM_CHECK_LAUNCH(ctx);
-    return QM_OK;
-  }
+  if (sizeof(T) == 4 && ctx->jacobi_pairs) return sweep_tile<2>(ctx, s, g, (const float*)rho, (const float*)a, (float*)b);
   constexpr int R = r2<T>();
   const int zs = pick_zs2<T>(g->nx, g->ny, g->nz, ctx->jacobi_zs);
   const dim3 grid((g->nx + Strip2<R>::W - 1) / Strip2<R>::W, (g->ny + Strip2<R>::TY - 1) / Strip2<R>::TY,
@@ -883,11 +820,12 @@ int jacobi_fp32(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const double* rho,
   // one residual block of m sweeps: residual, m FP32 sweeps, correction (kernels only).
   // With convergence checks the correction starts from cleared buffers and the block ends in
   // two single sweeps (e last, t the one before); without, the residual kernel also forms the
-  // first sweep (into t) and the other m - 1 run as two-sweep passes (a single one if odd).
+  // first sweep (into t) and the other m - 1 run as passes of three and two sweeps (a single one where
+  // these do not add up): three at a time on small grids, else for an odd number's sake only.
   auto enqueue = [&](hipStream_t q, int64_t m, bool prof) -> int {
     float* a = e;
     float* b = t;
-    int64_t P, S;
+    int64_t P, S, Q = 0;
     if (checks) {
       hipLaunchKernelGGL(k_residual, sweep_grid(g), dim3(kBX, kBY), 0, q, rho, (const double*)v, r, nullptr, g->nx,
                          g->ny, g->nz, g->step);
@@ -897,8 +835,18 @@ int jacobi_fp32(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const double* rho,
       hipLaunchKernelGGL(k_residual, sweep_grid(g), dim3(kBX, kBY), 0, q, rho, (const double*)v, r, t, g->nx,
                          g->ny, g->nz, g->step);
       std::swap(a, b);
-      P = (m - 1) / 2;
-      S = (m - 1) % 2;
+      if (ctx->jacobi_pairs && m > 3) {
+        Q = n <= kTile3Points ? (m - 1) / 3 : (m - 1) % 2;
+        if ((m - 1 - 3 * Q) % 2) --Q;   // a remainder of 1: one pass of three less, two of two more
+      }
+      P = (m - 1 - 3 * Q) / 2;
+      S = (m - 1 - 3 * Q) % 2;
+    }
+    for (int64_t j = 0; j < Q; ++j) {
+      ProfScope ps(ctx, q, QM_K_JACOBI, 3, prof);
+      int r1 = sweep_tile<3>(ctx, q, g, r, a, b);
+      if (r1) return r1;
+      std::swap(a, b);
     }
     for (int64_t j = 0; j < P; ++j) {
       int r1 = sweep2<float>(ctx, q, g, r, a, b, prof);
@@ -1045,7 +993,7 @@ struct JItem {
   float* r32;
   int blk0, bx, by;          // pointwise kernels: 64 x 4 tiles, one z plane per block
   int blk0s, tbx, tby, zs;   // sweep: 64 x 32 tiles (four 64 x 8 strips), zs planes per block
-  int blk0t, tbx2, tby2, zs2;  // two-sweep pass: 62-column strips (124 with paired columns)
+  int blk0t, tbx2, tby2, zs2;  // two-sweep pass: 62-column strips or tiles
 };
 
 __device__ __forceinline__ int find_item(const JItem* __restrict__ it, int n, int b) {
@@ -1100,16 +1048,13 @@ __global__ __launch_bounds__(kSW* kSWaves) void kb_sweep2(const JItem* __restric
                           q.nx, q.ny, q.nz, (T)q.h);
 }
 
-template <int R>
-__global__ __launch_bounds__(kSW* kSWaves) void kb_sweep2p(const JItem* __restrict__ items, int n, int dir) {
+__global__ __launch_bounds__(kTileX* kTileRows) void kb_sweep_tile(const JItem* __restrict__ items, int n, int dir) {
   const JItem& q = items[find_item_t(items, n, blockIdx.x)];
   const int local = blockIdx.x - q.blk0t;
   const int bx = local % q.tbx2;
   const int rest = local / q.tbx2;
-  const int by = rest % q.tby2;
-  const int bz = rest / q.tby2;
-  strip2p_body<R>(bx, by, bz, q.zs2, (const float*)q.rho, (const float*)(dir ? q.b : q.a), (float*)(dir ? q.a : q.b),
-                  q.nx, q.ny, q.nz, (float)q.h);
+  tile_body<2>(bx, rest % q.tby2, rest / q.tby2, (const float*)q.rho, (const float*)(dir ? q.b : q.a),
+               (float*)(dir ? q.a : q.b), q.nx, q.ny, q.nz, (float)q.h);
 }
 
 template <typename T>
@@ -1224,11 +1169,9 @@ extern "C" int qm_jacobi_batch(qm_ctx* ctx, void* stream, int n, const qm_geom* 
   int blocks = 0, sblocks = 0, tblocks = 0;
   size_t f32_elems = 0;
   constexpr int RD = kR2D, RF = kR2F;
-  // FP32 two-sweep passes take the paired-column kernel when every grid has an even nx
-  bool pairs = !f64 && ctx->jacobi_pairs;
-  for (int i = 0; i < n && pairs; ++i) pairs = pairs_fit(geoms[i].nx, geoms[i].ny);
-  const int W = pairs ? kWP : Strip2<RD>::W;
-  const int TY = f64 ? Strip2<RD>::TY : pairs ? Strip2P<kR2P>::TY : Strip2<RF>::TY;
+  const bool tile = !f64 && ctx->jacobi_pairs;   // FP32 two-sweep passes by tiles
+  const int W = tile ? Tile<2>::X : Strip2<RD>::W;
+  const int TY = f64 ? Strip2<RD>::TY : tile ? Tile<2>::Y : Strip2<RF>::TY;
   // two-sweep passes: one slab length for the whole batch, for about 1024 workgroups in all
   // (per-grid slabs of small grids would be a few planes, each re-reading 4 halo planes)
   int64_t tile_planes = 0;
@@ -1253,7 +1196,7 @@ extern "C" int qm_jacobi_batch(qm_ctx* ctx, void* stream, int n, const qm_geom* 
     q.blk0s = sblocks;
     sblocks += q.tbx * q.tby * ((q.nz + q.zs - 1) / q.zs);
     {
-      q.zs2 = std::min(zs2_batch, q.nz);
+      q.zs2 = tile ? Tile<2>::Z : std::min(zs2_batch, q.nz);
       q.tbx2 = (q.nx + W - 1) / W;
       q.tby2 = (q.ny + TY - 1) / TY;
       q.blk0t = tblocks;
@@ -1310,7 +1253,7 @@ extern "C" int qm_jacobi_batch(qm_ctx* ctx, void* stream, int n, const qm_geom* 
       hipLaunchKernelGGL(kb_residual, grid, thr, 0, t, dt, n);
       dir = 1;
       for (int64_t q = 0; q < (kf - 1) / 2; ++q, dir ^= 1) {
-        if (pairs) hipLaunchKernelGGL(kb_sweep2p<kR2P>, tgrid, sthr, 0, t, dt, n, dir);
+        if (tile) hipLaunchKernelGGL(kb_sweep_tile, tgrid, dim3(kTileX * kTileRows), 0, t, dt, n, dir);
         else hipLaunchKernelGGL(kb_sweep2<float>, tgrid, sthr, 0, t, dt, n, dir);
       }
       if ((kf - 1) & 1) {
@@ -1334,7 +1277,7 @@ extern "C" int qm_jacobi_batch(qm_ctx* ctx, void* stream, int n, const qm_geom* 
     // block length and the precision
     std::vector<char> key(sizeof(int) * 4 + sizeof(void*) + tbytes);
     {
-      const int hdr[4] = {n, block, f64 ? 1 : 0, pairs ? 1 : 0};
+      const int hdr[4] = {n, block, f64 ? 1 : 0, tile ? 1 : 0};
       std::memcpy(key.data(), hdr, sizeof(hdr));
       std::memcpy(key.data() + sizeof(hdr), &dtab, sizeof(void*));
       std::memcpy(key.data() + sizeof(hdr) + sizeof(void*), items.data(), tbytes);

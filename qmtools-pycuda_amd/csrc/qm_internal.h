@@ -117,7 +117,7 @@ struct qm_ctx {
   int split_tm = 3;                     // split contraction variant (0..3 tiled, 4 fused, 64 / 128 all-columns)
   int f64_variant = 4;                  // FP64 contraction: 0 wave-cyclic, 1 dense per-wave, 2 tiled, 3 rows, 4 block tiles + DMA
   int jacobi_zs = 0;                    // z planes per Jacobi sweep workgroup (0 = chosen per grid)
-  int jacobi_pairs = 1;                 // FP32 two-sweep passes with two columns per lane (even nx)
+  int jacobi_pairs = 1;                 // FP32 passes of several sweeps by tiles (else one-column strips)
   int tile_skip = 1;                    // contractions skip basis-function groups that are zero on a row tile
   int ncu = 256;                        // compute units of the device
   std::vector<ProfRec> recs;
