@@ -3032,23 +3032,20 @@ int qm_density(qm_ctx* ctx, qm_mol* mol, void* stream, const qm_geom* g, int sub
       return qm_fail(ctx, QM_EINVAL, "density: bad precision %d", precision);
   }
   if (rc) return rc;
-  if (normalize || raw_total) {
+  if (normalize) {
+    if ((rc = qm_normalize_dev(ctx, s, out_dtype, out, npoints(g), mol->qtot, raw_total ? ctx->host_scalars : nullptr)))
+      return rc;
+  } else if (raw_total) {
     double* dtot = nullptr;
     rc = qm_ws(ctx, s, WS_SCALAR, 256, (void**)&dtot);
     if (rc) return rc;
     rc = qm_reduce_dev(ctx, s, QM_RED_SUM, out_dtype, out, nullptr, npoints(g), dtot);
     if (rc) return rc;
-    if (raw_total) {
-      QM_CHECK_HIP(ctx, hipMemcpyAsync(ctx->host_scalars, dtot, sizeof(double), hipMemcpyDeviceToHost, s));
-    }
-    if (normalize) {
-      rc = qm_scale_dev(ctx, s, out_dtype, out, npoints(g), nullptr, mol->qtot, dtot);
-      if (rc) return rc;
-    }
-    if (raw_total) {
-      QM_CHECK_HIP(ctx, hipStreamSynchronize(s));
-      *raw_total = ctx->host_scalars[0];
-    }
+    QM_CHECK_HIP(ctx, hipMemcpyAsync(ctx->host_scalars, dtot, sizeof(double), hipMemcpyDeviceToHost, s));
+  }
+  if (raw_total) {
+    QM_CHECK_HIP(ctx, hipStreamSynchronize(s));
+    *raw_total = ctx->host_scalars[0];
   }
   return QM_OK;
 }
@@ -3447,13 +3444,9 @@ struct Round {
 int batch_normalize(qm_ctx* ctx, hipStream_t s, int nmol, qm_mol* const* mols, const qm_geom* geoms,
                     void* const* outs, int out_dtype, int normalize) {
   if (!normalize) return QM_OK;
-  double* tot = nullptr;
-  int rc = QM_OK;
-  if ((rc = qm_ws(ctx, s, WS_BATCH2, sizeof(double) * (size_t)nmol, (void**)&tot))) return rc;
   for (int i = 0; i < nmol; ++i) {
-    if ((rc = qm_reduce_dev(ctx, s, QM_RED_SUM, out_dtype, outs[i], nullptr, npoints(&geoms[i]), tot + i))) return rc;
-    if ((rc = qm_scale_dev(ctx, s, out_dtype, outs[i], npoints(&geoms[i]), nullptr, mols[i]->qtot, tot + i)))
-      return rc;
+    const int rc = qm_normalize_dev(ctx, s, out_dtype, outs[i], npoints(&geoms[i]), mols[i]->qtot, nullptr);
+    if (rc) return rc;
   }
   return QM_OK;
 }

@@ -70,7 +70,6 @@ enum WsSlot {
   WS_GTO,          // Hermite distributions
   WS_MISC,
   WS_BATCH,        // batched-launch tables
-  WS_BATCH2,
   WS_VNE,          // diffusion V_ne partials and loop state
   WS_PART,         // per-column-block partial densities of the tiled contraction
   WS_MASK,         // per-tile lists of the active basis-function groups
@@ -186,6 +185,8 @@ int qm_check_geom(qm_ctx* ctx, const qm_geom* g);
 // deterministic FP64 reductions (reduce.hip)
 int qm_reduce_dev(qm_ctx* ctx, hipStream_t s, int op, int dtype, const void* a, const void* b,
                   int64_t n, double* dev_result);
+// a times `total` over the sum of a; the sum to host_sum (pinned memory, readable once s has run) unless null
+int qm_normalize_dev(qm_ctx* ctx, hipStream_t s, int dtype, void* a, int64_t n, double total, double* host_sum);
 int qm_scale_dev(qm_ctx* ctx, hipStream_t s, int dtype, void* a, int64_t n, const double* dev_num,
                  double num_const, const double* dev_den);
 // density-matrix device forms (density.hip)

@@ -114,12 +114,12 @@ def _as_device(grid, dtype):
     return t if t.dtype == want else t.to(want)
 
 
-def _result_grid(template, dtype):
+def _result_grid(template, dtype, clear=True):
     """A new single-field grid with the geometry of `template` for a computed result: its device
-    buffer is allocated and cleared on the device, and the host `qube` keeps the zeros of a fresh
-    grid (nothing is copied between host and device)."""
+    buffer is allocated and cleared (unless the call writes every value) on the device, and the host
+    `qube` keeps the zeros of a fresh grid (nothing is copied between host and device)."""
     g = Grid.emptyAs(template, nfields=1, dtype=dtype)
-    g.d_qube = _device.zeros(g.qube.size, dtype)
+    g.d_qube = (_device.zeros if clear else _device.empty)(g.qube.size, dtype)
     return g
 
 
@@ -138,7 +138,7 @@ class QMTools:
         """
         p = _prec(precision)
         dt = numpy.float64 if p == "fp64" else numpy.float32
-        cgrid = _result_grid(grid, dt)
+        cgrid = _result_grid(grid, dt, clear=False)
         dm = device_molecule(molecule)
         raw = ctypes.c_double(0.0)
         nat.call("qm_density", dm.handle, nat.stream(), ctypes.byref(nat.geom(cgrid)), int(subgrid), _PREC[p],
