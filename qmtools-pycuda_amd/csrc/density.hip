@@ -5,8 +5,9 @@
 // per chunk of points:
 //
 //   1. k_phi_*:      Phi[t][f] for all points t of the chunk and basis
-//                    functions f (one thread per point, shells are wave
-//                    uniform, writes coalesced along t);
+//                    functions f (shells are wave uniform, writes coalesced
+//                    along t); the default kernels work on compact tiles of
+//                    voxels and evaluate the functions that reach them;
 //   2. k_contract_*: rho_t = sum_n Phi[t][n] (Phi P)[t][n], the diagonal of
 //                    Phi P Phi^T, as an MFMA GEMM with the row-dot fused
 //                    into the epilogue (no X = Phi P round trip to HBM).
