@@ -36,13 +36,13 @@ import numpy  # noqa: E402
 HBM_PEAK_GBS = 8000.0
 # HBM bytes per contraction launch measured with rocprofv3 FETCH_SIZE (x2 calibration) and
 # WRITE_SIZE (x1) for this workload; source: profiles/mol60_grid256_pmc_traffic.md
-# (precision, nbf_pad, variant): (points per launch, HBM bytes per launch)
-MEASURED_TRAFFIC = {("fp64", 640, "tiles_dma"): (838784, 3499848 * 1024 * 2 + 32765 * 1024),
+# (precision, nbf_pad, variant): (points, HBM bytes) of a launch or a step's launches
+MEASURED_TRAFFIC = {("fp64", 640, "tiles_dma"): (16777216, 25779000 * 1024 * 2 + 2091000 * 1024),   # 20 launches
                     ("fp64", 640, "tiles"): (838784, 6138183 * 1024 * 2 + 32765 * 1024),
                     ("fp64", 640, "rows"): (838784, 3870778 * 1024 * 2 + 65536 * 1024),
                     ("fp64", 640, "lds"): (838784, 4444220 * 1024 * 2 + 190037 * 1024),
                     ("fp64", 640, "direct"): (838784, 7883104 * 1024 * 2 + 6553 * 1024),
-                    ("mixed", 640, 3): (1677696, 1995799 * 1024 * 2 + 65535 * 1024),
+                    ("mixed", 640, 3): (16777216, 12941000 * 1024 * 2 + 709000 * 1024),   # 10 launches
                     ("mixed", 640, 1): (1677696, 2246457 * 1024 * 2 + 65535 * 1024),
                     ("mixed", 640, 0): (1677696, 2397406 * 1024 * 2 + 65535 * 1024),
                     ("mixed", 640, 2): (1677696, 2526254 * 1024 * 2 + 65535 * 1024),
@@ -130,6 +130,19 @@ class Workload:
         self.nat.check(self.nat.library().qm_profile_read(self.nat.context(), kid, ctypes.byref(tot),
                                                           ctypes.byref(n)), self.nat.context())
         return tot.value, n.value
+
+
+def active_flops(mol, grid, dense=False, samples=20000):
+    """Flops per voxel that the contraction cannot do without: nbf (nbf + 1) + 2 nbf (dense: 2 nbf^2 + 2 nbf) of the
+    functions with a primitive above e^-50 there (beyond, the basis values are zero), mean of seeded voxels."""
+    nx, ny, nz, h, o = grid.geometry()
+    rng = numpy.random.default_rng(1)
+    pts = numpy.array(o) + (rng.integers((nx, ny, nz), size=(samples, 3)) + 0.5) * h
+    amin = numpy.array([mol.prim_alpha[q:q + k].min() for q, k in zip(mol.shell_poff, mol.shell_nprim)])
+    n = numpy.zeros(samples)
+    for c, a, L in zip(mol.coords[mol.shell_atom], amin, mol.shell_L):
+        n += (2 * L + 1) * (((pts - c) ** 2).sum(1) * a <= 50.0)
+    return float(((2.0 if dense else 1.0) * n * n + (2.0 if dense else 3.0) * n).mean())
 
 
 def pct(vals, q):
@@ -284,14 +297,16 @@ def cold_request(basis):
 
 
 def jacobi_section(w, sweeps=200):
-    """Jacobi sweeps on the 256^3 grid of the 60-atom workload: ms per sweep and HBM roofline fraction."""
+    """`sweeps` Jacobi sweeps on the 256^3 grid of the 60-atom workload: ms, and the bytes that cannot be avoided
+    against the HBM peak.  FP64 runs in closed form, six one-axis transforms that read and write each value once
+    (96 B/point whatever the count); FP32 sweeps read V and rho and write V' (12 B/point per sweep)."""
     import torch
     import qmtools
     from qmtools import _native as nat
     out = {}
     qg = qmtools.Grid.emptyAs(w.grid)
     qg.d_qube = w.q64.clone()
-    for prec, bps in (("fp64", 24.0), ("mixed", 12.0)):
+    for prec, bytes_per_point in (("fp64", 96.0), ("mixed", 12.0 * sweeps)):
         qmtools.QMTools.Compute_hartree_iter(qg, w.mol, tolerance=None, max_sweeps=50, boundary="multipole",
                                              precision=prec, copyBack=False)
         torch.cuda.synchronize()
@@ -303,10 +318,10 @@ def jacobi_section(w, sweeps=200):
         wall = time.perf_counter() - t0
         nat.library().qm_profile(nat.context(), 0)
         ms, n = w.kernel_ms(nat.QM_K_JACOBI)
-        per = ms / max(n, 1)
-        gbs = bps * w.N / (per * 1e-3) / 1e9
-        out[prec] = {"ms_per_sweep": per, "sweeps": n, "wall_ms_per_sweep": wall * 1000 / sweeps,
-                     "algorithmic_bytes_per_point": bps, "achieved_GBs": gbs, "hbm_frac": gbs / HBM_PEAK_GBS}
+        gbs = bytes_per_point * w.N / (ms * 1e-3) / 1e9
+        out[prec] = {"sweeps": n, "ms": ms, "ms_per_sweep": ms / max(n, 1), "wall_ms": wall * 1000,
+                     "closed_form": prec == "fp64", "algorithmic_bytes_per_point": bytes_per_point,
+                     "achieved_GBs": gbs, "hbm_frac": gbs / HBM_PEAK_GBS}
     return out
 
 
@@ -505,23 +520,22 @@ def main():
             other_out["contraction_avg_ms"] = km / max(kn, 1)
             other_out["contraction_launches_per_step"] = kn / 2
             # the split contraction on the FP16 MFMAs: 3 products of the triangular form per point
-            nbf_m = w.mol.nbf
             pts_m = w.N / max(kn / 2, 1)
-            ach_m = 3.0 * (nbf_m * (nbf_m + 1.0) + 2.0 * nbf_m) * pts_m / (km / max(kn, 1) * 1e-3) / 1e12
+            ach_m = 3.0 * active_flops(w.mol, w.grid) * pts_m / (km / max(kn, 1) * 1e-3) / 1e12
             other_out["contraction_roofline"] = {"bound": "mfma", "achieved": ach_m, "peak": F16_MFMA_PEAK_TFLOPS,
                                                  "unit": "TFLOP/s", "frac": ach_m / F16_MFMA_PEAK_TFLOPS,
-                                                 "algorithmic": "3 x (nbf (nbf + 1) + 2 nbf) FP16 MFMA flops/point"}
+                                                 "algorithmic": "3 x (n (n + 1) + 2 n) FP16 MFMA flops/point, n = functions "
+                                                                "within their cutoff of the point"}
             log(f"mixed breakdown: {other_out['breakdown_ms_per_step']}")
         w.q64.copy_(q64)
 
-    # roofline of the dominant kernel (the density contraction).  The LDS-staged
-    # kernels contract with the upper-triangular M = D + 2U of the symmetric P,
-    # nbf (nbf + 1) + 2 nbf flops per point (half the dense 2 nbf^2 + 2 nbf);
-    # the barrier-free FP64 variant is dense.
+    # roofline of the dominant kernel (the density contraction): the products of the functions that are not
+    # zero at a point, n (n + 1) + 2 n flops with the upper-triangular M = D + 2U of the symmetric P (half the
+    # dense 2 n^2 + 2 n, which the barrier-free FP64 variant forms, over all functions)
     nbf = w.mol.nbf
     launch_pts = w.N / max(k_n / args.steps, 1)
     dense = args.precision == "fp64" and tune["fp64"].get("f64_variant", 0) == 1
-    per_point = (2.0 * nbf * nbf if dense else nbf * (nbf + 1.0)) + 2.0 * nbf
+    per_point = 2.0 * nbf * nbf + 2.0 * nbf if dense else active_flops(w.mol, w.grid)
     flops_per_launch = per_point * launch_pts
     mult = 1.0 if args.precision == "fp64" else 3.0     # hi/lo split executes 3 products
     avg_ms = k_ms / max(k_n, 1)
@@ -611,12 +625,10 @@ def main():
                      "achieved": achieved, "peak": peak, "unit": "TFLOP/s", "frac": achieved / peak,
                      "traffic": traffic,
                      "traffic_source": "profiles/mol60_grid256_pmc_traffic.md",
-                     "algorithmic": (f"({'2 nbf^2' if dense else 'nbf (nbf + 1)'} + 2 nbf) flops/point x "
-                                     f"{launch_pts:.0f} points/launch"
+                     "algorithmic": (f"{per_point:.4g} flops/point x {launch_pts:.0f} points/launch"
                                      + (" x 3 split products" if mult > 1 else "")
-                                     + ("" if dense else " (triangular M = D + 2U of symmetric P)")
-                                     + ("" if mult > 1 else "; counts the whole triangle, of which the kernel "
-                                        "skips the groups of 16 functions that are zero on a row tile")),
+                                     + (" (2 nbf^2 + 2 nbf)" if dense else " (n (n + 1) + 2 n, n = functions within "
+                                        "their cutoff of the point, triangular M = D + 2U of symmetric P)")),
                      "dense_equivalent_tflops": dense_equiv,
                      "avg_ms": avg_ms, "launches": k_n},
         "breakdown_ms_per_step": {"contraction": k_ms / args.steps, "phi": phi_ms / args.steps,

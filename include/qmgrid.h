@@ -183,7 +183,12 @@ int qm_multipole_boundary(qm_ctx* ctx, void* stream, const qm_geom* g, int dtype
  * precision QM_PREC_FP64: FP64 sweeps in pairs v->tmp->v; every `check_every`
  *   sweeps (even, > 0) computes delta = sum|v - tmp| like the reference loop
  *   (which checks every 100 iterations = 200 sweeps) and stops when
- *   delta <= tolerance.
+ *   delta <= tolerance.  From about 32 + n / 16 sweeps on (n the longest
+ *   axis, at most 1026 points) the result and the checks are computed in
+ *   closed form by sine transforms: to rounding those of the sweeps, in a time
+ *   that does not follow their number; the call then waits for `stream`.
+ *   While `stream` is being captured, with a residual that is not finite or a
+ *   tolerance below 1e-12 sum|V|, the sweeps are run.
  * precision QM_PREC_FP32: rho and v are FP64 buffers, tmp is unused; every
  *   `check_every` sweeps (> 0, e.g. 50) the FP64 residual charge is formed
  *   and the block's sweeps run in FP32 on the correction (defect correction:
@@ -239,7 +244,9 @@ int qm_vne_classic(qm_ctx* ctx, qm_mol* mol, void* stream, const qm_geom* g, int
  * Runs pairs of sweeps v -> tmp -> v until sum|v - tmp| / npts <= tolerance
  * (checked after each pair) or until the pair count exceeds maxiters (finite;
  * the reference's default is 10 npts^(1/3)), then *converged = 0.  A
- * tolerance >= 1 runs no sweep, as in the reference.  Synchronises `stream`. */
+ * tolerance >= 1 runs no sweep, as in the reference.  FP64 pairs are computed
+ * in closed form where qm_jacobi's sweeps are (weights that are not negative
+ * and sum to at most 1).  Synchronises `stream`. */
 int qm_vne_diffusion(qm_ctx* ctx, qm_mol* mol, void* stream, const qm_geom* g, int dtype, double adsorb,
                      double diff, double tolerance, double maxiters, void* v, void* tmp, int64_t* pairs,
                      double* delta, int* converged);
@@ -276,23 +283,23 @@ int qm_jacobi_batch(qm_ctx* ctx, void* stream, int n, const qm_geom* geoms, cons
 enum {
   QM_TUNE_SPLIT_VARIANT = 0, /* 16-bit split contraction, 128 x 128 tiles with per-block partial sums:
                                0 / 2 = FP32 basis values split while staged (8 / 4 waves), 1 = basis values
-                               written pre-split, staged through registers, 3 = pre-split, fetched by LDS DMA
-                               (default); 4 = basis values evaluated inside the contraction kernel, 128 points
+                               written pre-split, staged through registers, 3 = pre-split block tiles of 8 x 4 x 4
+                               voxels with lists of active functions (default); 4 = basis values evaluated inside the contraction kernel, 128 points
                                x 320 columns per workgroup (no basis-value buffer; slower on the 60-atom
                                workload); 5 = pre-split, DMA, 256 points x 320 columns per workgroup and
                                128 x 80 per wave (slower); 64 or 128 = points per workgroup of the
                                all-columns kernel */
   QM_TUNE_F64_VARIANT = 1,  /* FP64 contraction: 0 = all columns per workgroup (wave-cyclic tiles), 1 = per-wave
                                loads of the dense P, no barriers, 2 = 128 x 128 tiles with per-block partial sums,
-                               3 = 128 x 64 tiles with diagonal skipping, 4 = 128 x 128 tiles fed by LDS DMA with
-                               diagonal skipping (default) */
+                               3 = 128 x 64 tiles with diagonal skipping, 4 = block tiles of 8 x 4 x 4 voxels with
+                               lists of active functions, fed by LDS DMA (default; above 32768 functions 2) */
   QM_TUNE_JACOBI_ZS = 2,    /* z planes per Jacobi sweep workgroup, 0 = chosen per grid (the two-sweep passes
                                of qm_jacobi_batch: one length for the whole batch), else 1..4096 */
   QM_TUNE_JACOBI_PAIRS = 3, /* FP32 Jacobi passes of two and three sweeps: 1 = tiles kept on chip (default), 0 = strips
                                of one column per lane (two sweeps); the results are bitwise the same */
-  QM_TUNE_TILE_SKIP = 4,    /* FP64 contraction with LDS DMA: 1 = skip the products of basis-function groups
-                               that are zero on a whole row tile (default), 0 = form every product; they add
-                               exact zeros, so the results are the same */
+  QM_TUNE_TILE_SKIP = 4,    /* FP64 block tiles: 1 = list the basis-function groups that reach a tile (default),
+                               0 = list every group; what is left out are exact zeros, so the results are the
+                               same */
   QM_TUNE_COUNT = 5
 };
 int qm_tune_set(qm_ctx* ctx, int knob, int value);
@@ -315,7 +322,7 @@ enum {
   QM_K_PHI_SPLIT = 3,          /* basis values, FP32 + 16-bit split */
   QM_K_FFT_AXIS = 4,           /* one FFT pass along one axis */
   QM_K_GTO = 5,                /* Hermite/Boys potential */
-  QM_K_JACOBI = 6,             /* one Jacobi sweep (FP64 or FP32) */
+  QM_K_JACOBI = 6,             /* Jacobi sweeps (FP64 or FP32; a closed form counts as its sweeps) */
   QM_K_VNE = 7,                /* one pair of diffusion V_ne sweeps with its convergence test */
   QM_K_COUNT = 8
 };
