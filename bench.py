@@ -326,8 +326,8 @@ def jacobi_section(w, sweeps=200):
 
 
 def vne_section(w, pairs=25):
-    """Diffusion pseudo-V_ne on the 256^3 grid: fixed pair count, per-sweep time and HBM fraction
-    (16 B/point/sweep FP64: read V, write V')."""
+    """Diffusion pseudo-V_ne on the 256^3 grid, a fixed pair count in FP64: one sweep and sine transforms (closed
+    form), so the time does not follow the count and has no bytes per sweep."""
     import warnings
     import qmtools
     from qmtools import _native as nat
@@ -338,11 +338,8 @@ def vne_section(w, pairs=25):
         v = qmtools.QMTools.Compute_VNe(w.grid, w.mol, tolerance=-1.0, maxiters=pairs - 1, copyBack=False)
         wall = time.perf_counter() - t0
     nat.library().qm_profile(nat.context(), 0)
-    ms, n = w.kernel_ms(nat.QM_K_VNE)
-    per_sweep = ms / max(n, 1) / 2
-    gbs = 16.0 * w.N / (per_sweep * 1e-3) / 1e9
-    return {"pairs": int(v.pairs), "ms_per_sweep": per_sweep, "wall_ms_per_pair": wall * 1e3 / max(v.pairs, 1),
-            "algorithmic_bytes_per_point": 16.0, "achieved_GBs": gbs, "hbm_frac": gbs / HBM_PEAK_GBS}
+    ms, _ = w.kernel_ms(nat.QM_K_VNE)
+    return {"pairs": int(v.pairs), "closed_form": True, "ms": ms, "wall_ms": wall * 1e3}
 
 
 def batched_section(basis, count, sweeps, seed=41):
