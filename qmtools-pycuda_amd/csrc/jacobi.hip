@@ -714,6 +714,8 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   const double floor = 1e-12 * total;
   if (!(floor < INFINITY) || (tol < floor && delta < floor)) return QM_OK;
   if ((rc = qm_sine_x_add(ctx, s, p, w, v))) return rc;
+  // with a tolerance the call returns once v is final, as the loop does
+  QM_CHECK_HIP(ctx, hipStreamSynchronize(s));
   *done_out = at;
   *delta_out = delta;
   *converged_out = converged;

@@ -365,6 +365,7 @@ int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, d
   const double floor = 1e-12 * total / n;
   if (!(floor < INFINITY) || !(d < INFINITY) || (tol < floor && d < floor)) return QM_OK;
   if ((rc = qm_sine_x(ctx, s, p, v))) return rc;
+  QM_CHECK_HIP(ctx, hipStreamSynchronize(s));   // the call returns once v is final, as the loop does
   *pairs = at;
   *delta = d;
   *conv = ok ? 1 : 0;

@@ -1,0 +1,64 @@
+"""Closed forms of the relaxations against the stream order that the C interface promises."""
+import ctypes
+
+import numpy
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _charge(shape, seed):
+    import torch
+    g = torch.Generator(device="cpu").manual_seed(seed)
+    return torch.randn(shape[0] * shape[1] * shape[2], dtype=torch.float64, generator=g).cuda()
+
+
+def _jacobi(stream, shape, rho, v, tmp, sweeps, tol=-1.0, every=0):
+    from qmtools import _native as nat
+    done, delta = ctypes.c_int64(0), ctypes.c_double(0)
+    rc = nat.library().qm_jacobi(nat.context(), ctypes.c_void_p(stream.cuda_stream),
+                                 ctypes.byref(nat.geom((*shape, 0.3, (0.0, 0.0, 0.0)))), nat.QM_PREC_FP64,
+                                 nat.dptr(rho), nat.dptr(v), nat.dptr(tmp), sweeps, tol, every, ctypes.byref(done),
+                                 ctypes.byref(delta))
+    assert rc in (nat.QM_OK, nat.QM_ENOCONV)   # a cap reached first is an outcome too
+    return done.value
+
+
+def test_jacobi_with_a_tolerance_returns_finished():
+    """With a tolerance the outcome goes to host scalars, so nothing is left on the stream at the return."""
+    import torch
+    shape = (256, 256, 256)
+    rho = _charge(shape, 1)
+    v, tmp = torch.zeros_like(rho), torch.empty_like(rho)
+    s = torch.cuda.Stream()
+    print("[case] tolerance, stream idle at return", flush=True)
+    with torch.cuda.stream(s):
+        for _ in range(2):
+            v.zero_()
+            torch.cuda.synchronize()
+            _jacobi(s, shape, rho, v, tmp, 4000, 1e3, 40)
+            assert s.query()
+
+
+def test_vne_returns_finished():
+    """qm_vne_diffusion synchronises its stream."""
+    import torch
+    import qmtools
+    from conftest import BASIS
+    from qmtools import _native as nat, synth
+    from qmtools.qmtools import device_molecule
+    mol = synth.synthetic_molecule(6, 3, qmtools.BasisSet(BASIS))
+    shape, h = (256, 256, 256), 0.1
+    o = mol.coords.mean(0) - 0.5 * h * numpy.array(shape)
+    v = torch.empty(shape[0] * shape[1] * shape[2], dtype=torch.float64, device="cuda")
+    t = torch.empty_like(v)
+    handle = device_molecule(mol).handle
+    s = torch.cuda.Stream()
+    pairs, delta, conv = ctypes.c_int64(0), ctypes.c_double(0), ctypes.c_int(0)
+    print("[case] V_ne, stream idle at return", flush=True)
+    for _ in range(2):
+        torch.cuda.synchronize()
+        nat.call("qm_vne_diffusion", handle, ctypes.c_void_p(s.cuda_stream), ctypes.byref(nat.geom((*shape, h, tuple(o)))),
+                 nat.QM_F64, 0.05, 0.02, 1e-6, 100.0, nat.dptr(v), nat.dptr(t), ctypes.byref(pairs),
+                 ctypes.byref(delta), ctypes.byref(conv))
+        assert s.query()
