@@ -157,6 +157,7 @@ int qm_ctx_destroy(qm_ctx* ctx) {
     if (w.ptr) (void)hipFreeAsync(w.ptr, nullptr);
   (void)hipStreamSynchronize(nullptr);
   if (ctx->host_scalars) (void)hipHostFree(ctx->host_scalars);
+  if (ctx->sine_done) (void)hipEventDestroy(ctx->sine_done);
   qm_reclaim_graphs(ctx, true);
   if (ctx->jgraph_exec) (void)hipGraphExecDestroy(ctx->jgraph_exec);
   if (ctx->jgraph) (void)hipGraphDestroy(ctx->jgraph);

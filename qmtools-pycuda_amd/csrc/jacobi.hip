@@ -660,8 +660,10 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   }
   const int64_t checks = tol >= 0 && check_every > 0 ? max_sweeps / check_every : 0;
   double* w = nullptr;
-  int rc = QM_OK;
-  if (checks > 0 && qm_ws(ctx, s, WS_JAC_A, sizeof(double) * (size_t)npoints(g), (void**)&w)) {
+  SineUse use(ctx, s);
+  int rc = use.begin();
+  if (rc) return rc;
+  if (checks > 0 && qm_ws(ctx, s, WS_SINE_W, sizeof(double) * (size_t)npoints(g), (void**)&w)) {
     ctx->err.clear();
     return QM_OK;
   }
@@ -715,6 +717,7 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   if (!(floor < INFINITY) || (tol < floor && delta < floor)) return QM_OK;
   if ((rc = qm_sine_x_add(ctx, s, p, w, v))) return rc;
   // with a tolerance the call returns once v is final, as the loop does
+  use.end();
   QM_CHECK_HIP(ctx, hipStreamSynchronize(s));
   *done_out = at;
   *delta_out = delta;

@@ -74,6 +74,7 @@ enum WsSlot {
   WS_PART,         // per-column-block partial densities of the tiled contraction
   WS_MASK,         // per-tile lists of the active basis-function groups
   WS_SINE,         // sine-transform matrices and partial sums
+  WS_SINE_W,       // work grid of the closed forms' convergence checks
   WS_COUNT
 };
 
@@ -99,6 +100,7 @@ struct qm_ctx {
   Workspace ws[WS_COUNT];
   double* host_scalars = nullptr;   // pinned host buffer for results
   FftPlanCache* fft = nullptr;
+  hipEvent_t sine_done = nullptr;   // after the last closed form's use of WS_SINE and WS_SINE_W (SineUse)
   bool prof = false;
   hipStream_t graph_stream = nullptr;   // non-blocking stream for graph capture (default priority)
   std::vector<LiveGraph> graphs;        // graphs whose replays may still run
@@ -185,6 +187,10 @@ int qm_check_geom(qm_ctx* ctx, const qm_geom* g);
 // deterministic FP64 reductions (reduce.hip)
 int qm_reduce_dev(qm_ctx* ctx, hipStream_t s, int op, int dtype, const void* a, const void* b,
                   int64_t n, double* dev_result);
+constexpr int kRedMaxBlocks = 2048;   // block partials of a reduction at most
+// the same with the block partials in `part` (kRedMaxBlocks doubles) instead of the context's workspace
+int qm_reduce_part_dev(qm_ctx* ctx, hipStream_t s, int op, int dtype, const void* a, const void* b, int64_t n,
+                       double* part, double* dev_result);
 // a times `total` over the sum of a; the sum to host_sum (pinned memory, readable once s has run) unless null
 int qm_normalize_dev(qm_ctx* ctx, hipStream_t s, int dtype, void* a, int64_t n, double total, double* host_sum);
 int qm_scale_dev(qm_ctx* ctx, hipStream_t s, int dtype, void* a, int64_t n, const double* dev_num,

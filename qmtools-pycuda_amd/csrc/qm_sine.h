@@ -12,6 +12,7 @@ struct SinePlan {
   const double* So[3];      // even k (1-based), zero padded
   const double* s2[3];      // sin^2(pi k / (2 (m + 1))), k = 1 .. m
   double* part;             // partial sums of an x pass
+  double* red;              // block partials of their reduction
   double* sum;              // their sum
   int* flag;                // set when a residual is not finite
 };
@@ -24,6 +25,23 @@ struct SineFactor {
   double n;                 // whole number below 2^53
   int odd;                  // n is odd
   double w0, w1, w2, w3;    // SINE_VNE: 1 - a = w0 + w1 sum (1 - c) + w2 sum (1 - c c') + w3 (1 - c c' c''), c = cos theta
+};
+
+// Held by a closed form from before its plan to its last launch.  The sweeps work in the caller's buffers
+// alone, so calls on several streams of one context may be in flight together; the closed forms share the
+// context's tables and work grid, and are ordered one after the other by an event.  (Nothing else uses these
+// workspaces: the reductions have their own partials, red, instead of WS_RED.)
+struct SineUse {
+  qm_ctx* ctx;
+  hipStream_t s;
+  bool held = false;
+  SineUse(qm_ctx* c, hipStream_t st) : ctx(c), s(st) {}
+  int begin();
+  void end() {
+    if (held) (void)hipEventRecord(ctx->sine_done, s);
+    held = false;
+  }
+  ~SineUse() { end(); }
 };
 
 bool qm_sine_fits(const qm_geom* g);   // every axis has 1 .. 1024 interior points

@@ -12,7 +12,6 @@
 namespace {
 
 constexpr int kRedThreads = 256;
-constexpr int kRedMaxBlocks = 2048;
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -225,6 +224,11 @@ int qm_reduce_dev(qm_ctx* ctx, hipStream_t s, int op, int dtype, const void* a, 
   int rc = qm_ws(ctx, s, WS_RED, sizeof(double) * kRedMaxBlocks, &part);
   if (rc) return rc;
   return reduce_into(ctx, s, op, dtype, a, b, n, (double*)part, dev_result);
+}
+
+int qm_reduce_part_dev(qm_ctx* ctx, hipStream_t s, int op, int dtype, const void* a, const void* b, int64_t n,
+                       double* part, double* dev_result) {
+  return reduce_into(ctx, s, op, dtype, a, b, n, part, dev_result);
 }
 
 int qm_normalize_dev(qm_ctx* ctx, hipStream_t s, int dtype, void* a, int64_t n, double total, double* host_sum) {

@@ -340,6 +340,13 @@ int qm_sine_first_below(int64_t n, double dn, double tol, const std::function<in
   return QM_OK;
 }
 
+int SineUse::begin() {
+  if (!ctx->sine_done) QM_CHECK_HIP(ctx, hipEventCreateWithFlags(&ctx->sine_done, hipEventDisableTiming));
+  QM_CHECK_HIP(ctx, hipStreamWaitEvent(s, ctx->sine_done, 0));
+  held = true;
+  return QM_OK;
+}
+
 bool qm_sine_fits(const qm_geom* g) {
   const int n[3] = {g->nx, g->ny, g->nz};
   for (int d = 0; d < 3; ++d)
@@ -361,10 +368,10 @@ int qm_sine_plan(qm_ctx* ctx, hipStream_t s, const qm_geom* g, SinePlan* p) {
     most = std::max(most, 2 * table[d]);
     doubles += 2 * table[d] + p->m[d];
   }
-  // partial sums of an x pass, then the flag
+  // partial sums of an x pass, their reduction's, its result, then the flag
   const size_t nparts = ((size_t)p->m[1] * p->m[2] + 15) / 16;
   double* w = nullptr;
-  int rc = qm_ws(ctx, s, WS_SINE, sizeof(double) * (doubles + nparts + 4), (void**)&w);
+  int rc = qm_ws(ctx, s, WS_SINE, sizeof(double) * (doubles + nparts + kRedMaxBlocks + 4), (void**)&w);
   if (rc) return rc;
   for (int d = 0; d < 3; ++d) {
     p->S[d] = w + off[d];
@@ -372,7 +379,8 @@ int qm_sine_plan(qm_ctx* ctx, hipStream_t s, const qm_geom* g, SinePlan* p) {
     p->s2[d] = p->So[d] + table[d];
   }
   p->part = w + doubles;
-  p->sum = p->part + nparts;
+  p->red = p->part + nparts;
+  p->sum = p->red + kRedMaxBlocks;
   p->flag = (int*)(p->sum + 1);
   hipLaunchKernelGGL(k_sine_tables, dim3((unsigned)std::min<size_t>(512, (most + 255) / 256), 3), dim3(256), 0, s, *p);
   QM_CHECK_LAUNCH(ctx);
@@ -430,7 +438,8 @@ int qm_sine_x_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a
   int rc = v ? pass<0, LOAD_PLAIN, false, STORE_SUMV>(ctx, s, r) : pass<0, LOAD_PLAIN, false, STORE_SUM>(ctx, s, r);
   if (rc) return rc;
   const int64_t nl = (int64_t)p.m[1] * p.m[2], lines = p.m[0] <= 256 ? 32 : 16;
-  if ((rc = qm_reduce_dev(ctx, s, QM_RED_SUM, QM_F64, p.part, nullptr, (nl + lines - 1) / lines, p.sum))) return rc;
+  if ((rc = qm_reduce_part_dev(ctx, s, QM_RED_SUM, QM_F64, p.part, nullptr, (nl + lines - 1) / lines, p.red,
+                               p.sum))) return rc;
   QM_CHECK_HIP(ctx, hipMemcpyAsync(ctx->host_scalars + 2, p.sum, sizeof(double), hipMemcpyDeviceToHost, s));
   QM_CHECK_HIP(ctx, hipStreamSynchronize(s));
   *host_sum = ctx->host_scalars[2];

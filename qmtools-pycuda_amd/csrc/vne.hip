@@ -322,8 +322,10 @@ int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, d
   const double gap = (double)((long double)ads - D * (6.0L + 12.0L / r2 + 8.0L / r3 - (long double)kVneSelf));   // 1 - row sum
   if (!(dif >= 0.0) || !(1.0 - dif * kVneSelf - ads >= 0.0) || !(gap >= 0.0)) return QM_OK;
   const double n = (double)npoints(g);
+  SineUse use(ctx, s);
   SinePlan p;
   int rc;
+  if ((rc = use.begin())) return rc;
   if ((rc = qm_sine_plan(ctx, s, g, &p))) return rc;
   ProfScope ps(ctx, s, QM_K_VNE, (int)std::min<int64_t>(cap, 1 << 30));
   // the first sweep of a zero field is the source
@@ -365,6 +367,7 @@ int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, d
   const double floor = 1e-12 * total / n;
   if (!(floor < INFINITY) || !(d < INFINITY) || (tol < floor && d < floor)) return QM_OK;
   if ((rc = qm_sine_x(ctx, s, p, v))) return rc;
+  use.end();
   QM_CHECK_HIP(ctx, hipStreamSynchronize(s));   // the call returns once v is final, as the loop does
   *pairs = at;
   *delta = d;

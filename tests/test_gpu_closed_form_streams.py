@@ -62,3 +62,59 @@ def test_vne_returns_finished():
                  nat.QM_F64, 0.05, 0.02, 1e-6, 100.0, nat.dptr(v), nat.dptr(t), ctypes.byref(pairs),
                  ctypes.byref(delta), ctypes.byref(conv))
         assert s.query()
+
+
+@pytest.mark.parametrize("other", ["fixed", "tolerance", "fp32", "vne"])
+def test_calls_on_two_streams_of_one_context(other):
+    """A fixed-count relaxation in flight on one stream and another call on a second one: the bits of either alone."""
+    import torch
+    import qmtools
+    from conftest import BASIS
+    from qmtools import _native as nat, synth
+    from qmtools.qmtools import device_molecule
+    mol = synth.synthetic_molecule(4, 3, qmtools.BasisSet(BASIS))
+    handle = device_molecule(mol).handle
+    big, small = (200, 190, 180), (40, 66, 34)
+    rb, rs = _charge(big, 2), _charge(small, 3)
+
+    def first(s):
+        v = torch.zeros_like(rb)
+        t = torch.empty_like(rb)
+        torch.cuda.synchronize()
+        return v, t, lambda: _jacobi(s, big, rb, v, t, 500)
+
+    def second(s):
+        v = torch.zeros_like(rs)
+        t = torch.empty_like(rs)
+        torch.cuda.synchronize()
+        if other == "vne":
+            g = nat.geom((*small, 0.5, tuple(mol.coords.mean(0) - 0.25 * numpy.array(small))))
+            p, d, c = ctypes.c_int64(0), ctypes.c_double(0), ctypes.c_int(0)
+            return v, t, lambda: nat.call("qm_vne_diffusion", handle, ctypes.c_void_p(s.cuda_stream), ctypes.byref(g),
+                                          nat.QM_F64, 0.05, 0.02, 1e-7, 400.0, nat.dptr(v), nat.dptr(t),
+                                          ctypes.byref(p), ctypes.byref(d), ctypes.byref(c))
+        if other == "fp32":
+            d, n = ctypes.c_double(0), ctypes.c_int64(0)
+            return v, t, lambda: nat.call("qm_jacobi", ctypes.c_void_p(s.cuda_stream),
+                                          ctypes.byref(nat.geom((*small, 0.3, (0.0, 0.0, 0.0)))), nat.QM_PREC_FP32,
+                                          nat.dptr(rs), nat.dptr(v), None, 500, -1.0, 50, ctypes.byref(n),
+                                          ctypes.byref(d))
+        tol = (1e-3, 40) if other == "tolerance" else (-1.0, 0)
+        return v, t, lambda: _jacobi(s, small, rs, v, t, 700, *tol)
+
+    sa, sb = torch.cuda.Stream(), torch.cuda.Stream()
+    want = []
+    for make, s in ((first, sa), (second, sb)):
+        v, _, run = make(s)
+        run()
+        torch.cuda.synchronize()
+        want.append(v.cpu().numpy())
+    print("[case] two streams, one context:", other, flush=True)
+    for order in (0, 1, 0, 1):
+        va, _ta, ra = first(sa)
+        vb, _tb, rb2 = second(sb)
+        for run in ((ra, rb2) if order == 0 else (rb2, ra)):
+            run()
+        torch.cuda.synchronize()
+        assert numpy.array_equal(va.cpu().numpy(), want[0])
+        assert numpy.array_equal(vb.cpu().numpy(), want[1])
