@@ -188,8 +188,8 @@ int qm_multipole_boundary(qm_ctx* ctx, void* stream, const qm_geom* g, int dtype
  *   closed form by sine transforms: to rounding those of the sweeps, in a time
  *   that does not follow their number; the call then waits for `stream` (with
  *   a tolerance until v is final, else for the residual of v as given).
- *   While `stream` is being captured, with a residual that is not finite or a
- *   tolerance below 1e-12 sum|V|, the sweeps are run.
+ *   While `stream` is being captured, with a residual that is not finite or
+ *   above 1e290, or a tolerance below 1e-12 sum|V|, the sweeps are run.
  *   tmp is work space; what it holds on return is not specified.
  * precision QM_PREC_FP32: rho and v are FP64 buffers, tmp is unused; every
  *   `check_every` sweeps (> 0, e.g. 50) the FP64 residual charge is formed

@@ -642,8 +642,8 @@ struct GraphBlock {
 
 // FP64 sweeps in closed form by sine transforms (sine.hip): V_n = V + sum_{j<n} A^j (V_1 - V).  *done stays
 // false where the sweeps have to be run instead: under stream capture (the call waits for a flag), a residual
-// that is not finite somewhere (it would spread over the whole grid at once), no room for the check's
-// buffer, or a tolerance that the sweeps' rounding decides.
+// that is not finite somewhere (it would spread over the whole grid at once) or so large that a transform
+// might overflow, no room for the check's buffer, or a tolerance that the sweeps' rounding decides.
 //
 // Convergence checks: delta after n sweeps is |A^(n-1) (V_1 - V)|_1, and A (neighbour sums / 6) does not
 // increase that norm, so the first check with delta <= tol is found by bisection over the checks, in the

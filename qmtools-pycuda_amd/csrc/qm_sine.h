@@ -14,7 +14,7 @@ struct SinePlan {
   double* part;             // partial sums of an x pass
   double* red;              // block partials of their reduction
   double* sum;              // their sum
-  int* flag;                // set when a residual is not finite
+  int* flag;                // set when a residual is not finite or near the end of the range
 };
 
 enum { SINE_JACOBI = 0, SINE_VNE = 1 };     // which sweep's eigenvalue a
@@ -48,7 +48,7 @@ bool qm_sine_fits(const qm_geom* g);   // every axis has 1 .. 1024 interior poin
 // tables in the context's workspace, valid on s until the next plan; clears the flag
 int qm_sine_plan(qm_ctx* ctx, hipStream_t s, const qm_geom* g, SinePlan* p);
 // The passes read and write interior points only and work in place where one buffer is given.
-// x and y transforms of (one Jacobi sweep of v) - v; sets the plan's flag if that is not finite somewhere
+// x and y transforms of (one Jacobi sweep of v) - v; sets the plan's flag if that is not finite, or 1e290 and more, somewhere
 int qm_sine_residual_xy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* rho, const double* v, double h,
                         double* out);
 int qm_sine_xy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* a);

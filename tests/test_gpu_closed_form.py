@@ -77,6 +77,20 @@ def test_values_that_are_not_finite_stay_local():
     assert numpy.isfinite(row[:60 - 46]).all() and numpy.isfinite(row[60 + 46:]).all()
 
 
+def test_charges_near_the_end_of_the_range():
+    """Charges whose transform overflows while the relaxed field does not (here by a factor of 50)."""
+    from oracle import jacobi as oj
+    shape = (64, 64, 64)
+    rho = numpy.full(64 ** 3, -1.8e305)
+    v0 = numpy.zeros_like(rho)
+    want = oj.jacobi(rho, *shape, 0.3, 131, bvals=v0, v0=v0)
+    assert numpy.isfinite(want).all()
+    print("[case] closed form, huge charges", flush=True)
+    rc, got, done, _ = _jacobi(shape, rho, v0, 131)
+    assert rc == 0 and done == 131
+    assert numpy.abs(got - want).max() <= 1e-12 * numpy.abs(want).max()
+
+
 @pytest.mark.parametrize("adsorb,diff,tol,maxiters", [(0.1, 0.01, 1e-9, None), (0.05, 0.02, 1e-9, None),
                                                       (0.05, 0.02, 1e-6, 400.5), (0.02, 0.02, 1e-6, 40),
                                                       (0.4, 0.05, 1e-9, None), (0.05, 0.02, -1.0, 24)])
