@@ -2679,10 +2679,19 @@ int density_blocks(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, in
   return QM_OK;
 }
 
-// a tile's groups fit a workgroup's list: 32768 basis functions in FP64, where larger bases take variant 2
-// (a split basis beyond 65536 functions would need 34 GB for M and is refused by its allocation)
+// a tile's groups fit a workgroup's list: 32768 basis functions in FP64, where larger bases take variant 2, and 65536 in
+// the split path, where larger ones are refused (split_blocks_limit; the matrix upload refuses them too: k_split_P's
+// launch would exceed 2^32 threads)
 inline bool f64_blocks(const qm_ctx* ctx, const qm_mol* mol) {
   return ctx->f64_variant == 4 && (mol->nbf + 15) / 16 <= kMaxGroups;
+}
+
+int split_blocks_limit(qm_ctx* ctx, const qm_mol* mol, int precision) {
+  const bool split = precision == QM_PREC_F16X3 || precision == QM_PREC_BF16X3;
+  const bool blocks = ctx->split_tm == 3 || (ctx->split_tm == 4 && !fused_fits(mol));
+  QM_REQUIRE(ctx, !split || !blocks || (mol->nbf + 31) / 32 <= kMaxGroups, QM_ELIMIT,
+             "density: %d basis functions, the split path takes at most %d", mol->nbf, 32 * kMaxGroups);
+  return QM_OK;
 }
 
 template <typename TO>
@@ -3011,6 +3020,7 @@ int qm_density(qm_ctx* ctx, qm_mol* mol, void* stream, const qm_geom* g, int sub
   rc = qm_check_geom(ctx, g);
   if (rc) return rc;
   QM_REQUIRE(ctx, mol && out, QM_EINVAL, "density: null argument");
+  if ((rc = split_blocks_limit(ctx, mol, precision))) return rc;
   QM_REQUIRE(ctx, mol->has_dm, QM_EINVAL, "density: molecule has no density matrix");
   QM_REQUIRE(ctx, subgrid >= 1 && subgrid <= 16, QM_EINVAL, "density: subgrid must be 1..16");
   QM_REQUIRE(ctx, out_dtype == QM_F64 || out_dtype == QM_F32, QM_EINVAL, "density: bad output dtype");
@@ -3548,6 +3558,7 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
   QM_REQUIRE(ctx, out_dtype == QM_F64 || out_dtype == QM_F32, QM_EINVAL, "density_batch: bad output dtype");
   if (nmol == 0) return QM_OK;
   for (int i = 0; i < nmol; ++i) {
+    if (mols[i] && (rc = split_blocks_limit(ctx, mols[i], precision))) return rc;
     QM_REQUIRE(ctx, mols[i] && mols[i]->has_dm && outs[i], QM_EINVAL, "density_batch: item %d incomplete", i);
     if ((rc = qm_check_geom(ctx, &geoms[i]))) return rc;
   }

@@ -96,3 +96,30 @@ def test_block_tiles_sorted_launches(shape):
         assert numpy.isfinite(got).all()
         for k, want in slabs.items():
             assert numpy.abs(got[k:k + 4] - want).max() <= tol * top
+
+
+@pytest.mark.parametrize("nbf,limit", [(65536, False), (65537, True)])
+@pytest.mark.parametrize("prec", ["QM_PREC_F16X3", "QM_PREC_BF16X3", "QM_PREC_FP64"])
+def test_basis_beyond_the_lists_of_the_split_path(nbf, limit, prec):
+    """A tile's list holds 2048 groups of 32 functions: the split path refuses a larger basis before it looks for a
+    density matrix, single and batched (FP64 takes larger ones; here the matrix is missing)."""
+    import torch
+    from qmtools import _native as nat
+    zero, one = numpy.zeros(nbf, dtype=numpy.int32), numpy.ones(nbf, dtype=numpy.int32)
+    z, xyz, alpha = numpy.array([6], dtype=numpy.int32), numpy.zeros(3), numpy.ones(1)
+    mol = ctypes.c_void_p()
+    nat.call("qm_mol_create", 1, nat.i32p(z), nat.f64p(xyz), nbf, nat.i32p(zero), nat.i32p(zero), nat.i32p(one),
+             nat.i32p(zero), 1, nat.f64p(alpha), nat.f64p(alpha), ctypes.byref(mol))
+    lib, ctx = nat.library(), nat.context()
+    print("[case] list limit", nbf, prec, flush=True)
+    try:
+        out = torch.zeros(512, dtype=torch.float64, device="cuda")
+        g = nat.geom((8, 8, 8, 0.3, (0.0, 0.0, 0.0)))
+        want = nat.QM_ELIMIT if limit and prec != "QM_PREC_FP64" else nat.QM_EINVAL
+        p = getattr(nat, prec)
+        assert lib.qm_density(ctx, mol, nat.stream(), ctypes.byref(g), 1, p, nat.QM_F64, nat.dptr(out), 0, None) == want
+        outs = (ctypes.c_void_p * 1)(out.data_ptr())
+        assert lib.qm_density_batch(ctx, nat.stream(), 1, (ctypes.c_void_p * 1)(mol.value), (nat.Geom * 1)(g), outs, p,
+                                    nat.QM_F64, 0) == want
+    finally:
+        lib.qm_mol_destroy(ctx, mol)
