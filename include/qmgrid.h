@@ -302,7 +302,9 @@ enum {
   QM_TUNE_TILE_SKIP = 4,    /* FP64 block tiles: 1 = list the basis-function groups that reach a tile (default),
                                0 = list every group; what is left out are exact zeros, so the results are the
                                same */
-  QM_TUNE_COUNT = 5
+  QM_TUNE_PHI_MIB = 5,      /* MiB of basis values that a density call (a round of qm_density_batch) holds at a time,
+                               1..4096 (default); the results do not depend on it */
+  QM_TUNE_COUNT = 6
 };
 int qm_tune_set(qm_ctx* ctx, int knob, int value);
 int qm_tune_get(qm_ctx* ctx, int knob, int* value);

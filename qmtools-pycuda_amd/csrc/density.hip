@@ -805,11 +805,12 @@ constexpr int kMaxGroups = 2048;   // groups per tile that a workgroup can list 
 
 struct BlockTiles {
   int T0, nT;             // tiles T0 .. T0 + nT - 1 of the grid (x fastest)
-  int nsub;               // row tile rt = s nT + (T - T0) holds sub-point s of tile T's voxels
+  int nsub;               // row tile rt = (s - s0) nT + (T - T0) holds sub-point s of tile T's voxels
   int ng;                 // groups of the whole basis: stride of a tile's list, values and partial sums
   const uint16_t* list;   // [row tile][ng]: active groups in increasing order
   const int* cnt;         // [row tile]: how many
   const int* order;       // the contraction's order of the row tiles, null: as numbered
+  int s0, ns;             // sub-points s0 .. s0 + ns - 1 of nsub^3
 };
 
 __host__ __device__ inline int64_t block_tiles(const GeomView& g) {
@@ -828,9 +829,9 @@ __device__ __forceinline__ void block_origin(const GeomView& g, int T, int& i0, 
 // grid repeat its last plane, row or column and are not stored.
 __device__ __forceinline__ void block_point(const GeomView& g, const BlockTiles& b, int rt, int p, double& x, double& y,
                                             double& z) {
-  const int s = rt / b.nT;
+  const int part = rt / b.nT, s = b.s0 + part;
   int i0, j0, k0;
-  block_origin(g, b.T0 + (rt - s * b.nT), i0, j0, k0);
+  block_origin(g, b.T0 + (rt - part * b.nT), i0, j0, k0);
   const int i = min(i0 + (p & 7), g.nx - 1), j = min(j0 + ((p >> 3) & 3), g.ny - 1), k = min(k0 + (p >> 5), g.nz - 1);
   const int sx = s % b.nsub, sy = (s / b.nsub) % b.nsub, sz = s / (b.nsub * b.nsub);
   const double inv = 1.0 / b.nsub;
@@ -1130,14 +1131,15 @@ __global__ __launch_bounds__(kTWG, 4) void k_contract_f64_blocks(const double* _
 }
 
 // Density of a voxel: partial sums of its row tiles in list order (FP64: one per group; split: two per block
-// of 4 groups), times scale, summed over its sub-points.  One thread per tile point.
+// of 4 groups), times scale, summed over its sub-points in order; sums of launches that hold only some of
+// them are carried in acc.  One thread per tile point.
 template <bool SPLIT>
 __device__ __forceinline__ int block_parts(int cnt) { return SPLIT ? (cnt + 3) / 4 * 2 : cnt; }
 
 template <bool SPLIT, typename TO>
 __device__ __forceinline__ void blocks_finish_body(int64_t idx, const GeomView& g, const BlockTiles& b,
                                                    const double* __restrict__ part, double scale,
-                                                   TO* __restrict__ out) {
+                                                   double* __restrict__ acc, TO* __restrict__ out) {
   const int tl = (int)(idx / kTT), p = (int)(idx % kTT);
   if (tl >= b.nT) return;
   int i, j, k;
@@ -1147,8 +1149,8 @@ __device__ __forceinline__ void blocks_finish_body(int64_t idx, const GeomView& 
   k += p >> 5;
   if (i >= g.nx || j >= g.ny || k >= g.nz) return;
   const int stride = block_parts<SPLIT>(b.ng);
-  double v = 0.0;
-  for (int s = 0; s < b.nsub * b.nsub * b.nsub; ++s) {
+  double v = b.s0 ? acc[idx] : 0.0;
+  for (int s = 0; s < b.ns; ++s) {
     const int rt = s * b.nT + tl;
     const int n = block_parts<SPLIT>(b.cnt[rt]);
     const double* __restrict__ mine = part + (int64_t)rt * stride * kTT + p;
@@ -1156,13 +1158,14 @@ __device__ __forceinline__ void blocks_finish_body(int64_t idx, const GeomView& 
     for (int q = 0; q < n; ++q) r += mine[(int64_t)q * kTT];
     v += r * scale;
   }
-  store_rho<TO>(out, i + (int64_t)g.nx * (j + (int64_t)g.ny * k), v);
+  if (b.s0 + b.ns < b.nsub * b.nsub * b.nsub) acc[idx] = v;
+  else store_rho<TO>(out, i + (int64_t)g.nx * (j + (int64_t)g.ny * k), v);
 }
 
 template <bool SPLIT, typename TO>
 __global__ __launch_bounds__(256) void k_blocks_finish(GeomView g, BlockTiles b, const double* __restrict__ part,
-                                                       double scale, TO* __restrict__ out) {
-  blocks_finish_body<SPLIT, TO>((int64_t)blockIdx.x * 256 + threadIdx.x, g, b, part, scale, out);
+                                                       double scale, double* __restrict__ acc, TO* __restrict__ out) {
+  blocks_finish_body<SPLIT, TO>((int64_t)blockIdx.x * 256 + threadIdx.x, g, b, part, scale, acc, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -2505,8 +2508,6 @@ __global__ void k_split_P(const double* __restrict__ P64, int npad, float pfac, 
 
 int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 
-constexpr size_t kPhiBudget = (size_t)4 << 30;   // bytes of basis values per chunk
-
 }  // namespace
 
 int qm_density_upload_P(qm_ctx* ctx, qm_mol* mol, hipStream_t s) {
@@ -2614,8 +2615,10 @@ inline int block_split(int nrt, int ncb, bool f64) {
 // chip; with fewer the list (n8 units of 8 functions at most) is shared out.
 inline int phi_split(int blk, int n8) { return std::max(1, std::min({n8, 64, 2048 / std::max(blk, 1)})); }
 
-// Block tiles (the default contractions): chunks of tiles whose basis values fit kPhiBudget with every
-// group listed (a tile leaves the part of its space that it does not need untouched).
+// Block tiles (the default contractions): chunks of tiles whose basis values fit the context's budget with every
+// group listed (a tile leaves the part of its space that it does not need untouched).  Where one tile with all of its
+// sub-points does not fit (subgrid 16: 4096 row tiles, 5.9 GiB with 1500 FP64 functions), it is taken in chunks of
+// sub-points.
 // FP64 (T = double, groups of 16) or split (T = _Float16 / __bf16, groups of 32; M in hi and lo planes).
 template <typename T, typename TO>
 int density_blocks(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, int nsub, TO* out) {
@@ -2628,16 +2631,19 @@ int density_blocks(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, in
   const MolView mv = mol->view();
   const int64_t ntiles = block_tiles(gv);
   const size_t tile_bytes = (f64 ? sizeof(double) : 4) * (size_t)kTT * (ng << GS);
-  int64_t nT = std::max<int64_t>((int64_t)(kPhiBudget / tile_bytes) / nsub3, 1);
+  const int64_t fit = std::max<int64_t>((int64_t)(ctx->phi_budget / tile_bytes), 1);   // row tiles
+  const int ns = (int)std::min<int64_t>(fit, nsub3);
+  int64_t nT = std::max<int64_t>(fit / nsub3, 1);
   nT = std::min(nT, std::min(ntiles, std::max<int64_t>((1 << 22) / nsub3, 1)));
-  const int64_t rows = nT * nsub3;
+  const int64_t rows = nT * ns;
   T* phi = nullptr;
-  double* part = nullptr;
+  double *part = nullptr, *acc = nullptr;
   char* lists = nullptr;
   int rc = QM_OK;
   if ((rc = qm_ws(ctx, s, WS_PHI, tile_bytes * rows, (void**)&phi))) return rc;
   if ((rc = qm_ws(ctx, s, WS_PART, sizeof(double) * kTT * (size_t)nparts * rows, (void**)&part))) return rc;
   if ((rc = qm_ws(ctx, s, WS_MASK, (2 * sizeof(int) + sizeof(uint16_t) * (size_t)ng) * rows, (void**)&lists))) return rc;
+  if (ns < nsub3 && (rc = qm_ws(ctx, s, WS_RHO, sizeof(double) * kTT * (size_t)nT, (void**)&acc))) return rc;
   int* cnt = (int*)lists;
   int* order = cnt + rows;
   uint16_t* list = (uint16_t*)(lists + 2 * sizeof(int) * rows);
@@ -2646,35 +2652,38 @@ int density_blocks(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, in
   const double scale = (f64 ? h3 : h3 / mol->pfac / ((double)S * S)) / nsub3;
   const T* M = (const T*)(f64 ? (const void*)mol->M64 : std::is_same<T, _Float16>::value ? mol->P16 : mol->Pb16);
   for (int64_t T0 = 0; T0 < ntiles; T0 += nT) {
-    const int nTc = (int)std::min(nT, ntiles - T0), nrt = nTc * nsub3;
-    const bool sorted = nrt >= kOrderMin && nrt <= kOrderMax;
-    const BlockTiles b{(int)T0, nTc, nsub, ng, list, cnt, sorted ? order : nullptr};
-    const int pblk = f64 ? (nrt + 1) / 2 : (nrt + kPhiTiles - 1) / kPhiTiles;
-    const dim3 pgrid(pblk, phi_split(pblk, ng << (GS - 3)));
-    const int ny = block_split(nrt, ncb, f64);
-    const dim3 cgrid(tile_grid(nrt, ny));
-    {
-      ProfScope ps(ctx, s, f64 ? QM_K_PHI : QM_K_PHI_SPLIT);
-      hipLaunchKernelGGL(k_tile_list<GS>, dim3(nrt), dim3(kTT), 0, s, mv, gv, b, f64 && !ctx->tile_skip, list, cnt);
-      if (sorted) hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, (const int*)cnt, nrt, order);
+    const int nTc = (int)std::min(nT, ntiles - T0);
+    for (int s0 = 0; s0 < nsub3; s0 += ns) {
+      const int nsc = std::min(ns, nsub3 - s0), nrt = nTc * nsc;
+      const bool sorted = nrt >= kOrderMin && nrt <= kOrderMax;
+      const BlockTiles b{(int)T0, nTc, nsub, ng, list, cnt, sorted ? order : nullptr, s0, nsc};
+      const int pblk = f64 ? (nrt + 1) / 2 : (nrt + kPhiTiles - 1) / kPhiTiles;
+      const dim3 pgrid(pblk, phi_split(pblk, ng << (GS - 3)));
+      const int ny = block_split(nrt, ncb, f64);
+      const dim3 cgrid(tile_grid(nrt, ny));
+      {
+        ProfScope ps(ctx, s, f64 ? QM_K_PHI : QM_K_PHI_SPLIT);
+        hipLaunchKernelGGL(k_tile_list<GS>, dim3(nrt), dim3(kTT), 0, s, mv, gv, b, f64 && !ctx->tile_skip, list, cnt);
+        if (sorted) hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, (const int*)cnt, nrt, order);
+        if constexpr (f64)
+          hipLaunchKernelGGL(k_phi_f64_blocks, pgrid, dim3(kPhiThreads), 0, s, mv, (const int2*)mol->kgroups, gv, b, nrt,
+                             phi);
+        else
+          hipLaunchKernelGGL(k_phi_split_blocks<T>, pgrid, dim3(kPhiThreads), 0, s, mv, (const float2*)mol->prims_l2e,
+                             (const int2*)mol->kgroups, gv, b, nrt, S, phi);
+      }
+      QM_CHECK_LAUNCH(ctx);
+      ProfScope pc(ctx, s, f64 ? QM_K_DENSITY_CONTRACT : QM_K_DENSITY_SPLIT);
       if constexpr (f64)
-        hipLaunchKernelGGL(k_phi_f64_blocks, pgrid, dim3(kPhiThreads), 0, s, mv, (const int2*)mol->kgroups, gv, b, nrt,
-                           phi);
+        hipLaunchKernelGGL(k_contract_f64_blocks, cgrid, dim3(kTWG), 0, s, (const double*)phi, M, np, b, nrt, ny, part);
       else
-        hipLaunchKernelGGL(k_phi_split_blocks<T>, pgrid, dim3(kPhiThreads), 0, s, mv, (const float2*)mol->prims_l2e,
-                           (const int2*)mol->kgroups, gv, b, nrt, S, phi);
+        hipLaunchKernelGGL(k_contract_split_blocks<T>, cgrid, dim3(512), 0, s, (const T*)phi, M, M + (int64_t)np * np, np,
+                           b, nparts, nrt, ny, part);
+      QM_CHECK_LAUNCH(ctx);
+      hipLaunchKernelGGL((k_blocks_finish<!f64, TO>), dim3((unsigned)(((int64_t)b.nT * kTT + 255) / 256)), dim3(256), 0, s,
+                         gv, b, (const double*)part, scale, acc, out);
+      QM_CHECK_LAUNCH(ctx);
     }
-    QM_CHECK_LAUNCH(ctx);
-    ProfScope pc(ctx, s, f64 ? QM_K_DENSITY_CONTRACT : QM_K_DENSITY_SPLIT);
-    if constexpr (f64)
-      hipLaunchKernelGGL(k_contract_f64_blocks, cgrid, dim3(kTWG), 0, s, (const double*)phi, M, np, b, nrt, ny, part);
-    else
-      hipLaunchKernelGGL(k_contract_split_blocks<T>, cgrid, dim3(512), 0, s, (const T*)phi, M, M + (int64_t)np * np, np,
-                         b, nparts, nrt, ny, part);
-    QM_CHECK_LAUNCH(ctx);
-    hipLaunchKernelGGL((k_blocks_finish<!f64, TO>), dim3((unsigned)(((int64_t)b.nT * kTT + 255) / 256)), dim3(256), 0, s,
-                       gv, b, (const double*)part, scale, out);
-    QM_CHECK_LAUNCH(ctx);
   }
   return QM_OK;
 }
@@ -2700,7 +2709,7 @@ int density_fp64(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, int 
   const int np = mol->nbf_pad;
   const int nsub3 = nsub * nsub * nsub;
   const int64_t nvox_tot = npoints(g);
-  int64_t maxpts = (int64_t)(kPhiBudget / ((size_t)np * sizeof(double)));
+  int64_t maxpts = (int64_t)(ctx->phi_budget / ((size_t)np * sizeof(double)));
   maxpts = std::max<int64_t>(maxpts / kTileM * kTileM, kTileM);
   int64_t nvox = std::max<int64_t>(maxpts / nsub3, 1);
   nvox = std::min<int64_t>(nvox, nvox_tot);
@@ -2819,7 +2828,7 @@ int density_wide(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, int 
   const int np = mol->nbf_pad;
   const int nsub3 = nsub * nsub * nsub;
   const int64_t nvox_tot = npoints(g);
-  int64_t maxpts = (int64_t)(kPhiBudget / ((size_t)np * sizeof(float)));
+  int64_t maxpts = (int64_t)(ctx->phi_budget / ((size_t)np * sizeof(float)));
   maxpts = std::max<int64_t>(maxpts / kWP * kWP, kWP);
   int64_t nvox = std::max<int64_t>(maxpts / nsub3, 1);
   nvox = std::min<int64_t>(nvox, nvox_tot);
@@ -2932,7 +2941,7 @@ int density_split(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, int
   const int np = mol->nbf_pad;
   const int nsub3 = nsub * nsub * nsub;
   const int64_t nvox_tot = npoints(g);
-  int64_t maxpts = (int64_t)(kPhiBudget / ((size_t)np * sizeof(float)));
+  int64_t maxpts = (int64_t)(ctx->phi_budget / ((size_t)np * sizeof(float)));
   maxpts = std::max<int64_t>(maxpts / kTileM * kTileM, kTileM);
   int64_t nvox = std::max<int64_t>(maxpts / nsub3, 1);
   nvox = std::min<int64_t>(nvox, nvox_tot);
@@ -3107,6 +3116,12 @@ int qm_tune_set(qm_ctx* ctx, int knob, int value) {
     ctx->tile_skip = value;
     return QM_OK;
   }
+  if (knob == QM_TUNE_PHI_MIB) {
+    QM_REQUIRE(ctx, value >= 1 && value <= (int)(kPhiBudget >> 20), QM_EINVAL, "tune: basis values of 1..%d MiB",
+               (int)(kPhiBudget >> 20));
+    ctx->phi_budget = (size_t)value << 20;
+    return QM_OK;
+  }
   return qm_fail(ctx, QM_EINVAL, "tune: unknown knob %d", knob);
 }
 
@@ -3132,6 +3147,10 @@ int qm_tune_get(qm_ctx* ctx, int knob, int* value) {
   }
   if (knob == QM_TUNE_TILE_SKIP) {
     *value = ctx->tile_skip;
+    return QM_OK;
+  }
+  if (knob == QM_TUNE_PHI_MIB) {
+    *value = (int)(ctx->phi_budget >> 20);
     return QM_OK;
   }
   return qm_fail(ctx, QM_EINVAL, "tune: unknown knob %d", knob);
@@ -3374,7 +3393,7 @@ template <bool SPLIT, typename TO>
 __global__ __launch_bounds__(kPhiThreads) void kb_blocks_finish(const BChunk* __restrict__ c, int n) {
   const BChunk& q = c[find_chunk(c, n, blockIdx.x, true)];
   blocks_finish_body<SPLIT, TO>((int64_t)(blockIdx.x - q.blk0_phi) * kPhiThreads + threadIdx.x, q.g, q.b, q.part,
-                                q.scale, (TO*)q.out);
+                                q.scale, nullptr, (TO*)q.out);
 }
 
 // the basis-value launches of a round of block tiles
@@ -3585,7 +3604,7 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
   bool blocks = f64 || sv == 3;   // block tiles
   for (int i = 0; f64 && i < nmol; ++i) blocks = blocks && f64_blocks(ctx, mols[i]);
   const int gs = f64 ? 4 : 5;     // log2 of the functions per group
-  // chunks per molecule, packed into rounds of at most kPhiBudget bytes of basis values
+  // chunks per molecule, packed into rounds of at most phi_budget bytes of basis values
   std::vector<BChunk> table;
   std::vector<Round> rounds;
   std::vector<BChunk> cur;
@@ -3633,7 +3652,7 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
     const int nphi = blocks ? ng << gs : np;   // functions stored per point
     const int64_t N = blocks ? block_tiles(geom_view(&geoms[i])) * kTT : npoints(&geoms[i]);
     const int64_t cap = std::max<int64_t>(kTileM, std::min<int64_t>(kBatchChunk,
-                                          (int64_t)(kPhiBudget / ((size_t)nphi * elt)) / kTileM * kTileM));
+                                          (int64_t)(ctx->phi_budget / ((size_t)nphi * elt)) / kTileM * kTileM));
     for (int64_t v0 = 0; v0 < N; v0 += cap) {
       BChunk c{};
       c.mol = m->view();
@@ -3650,12 +3669,12 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
         c.ncb = f64 ? (ng + 7) / 8 : (ng + 3) / 4;
         c.ny = block_split(c.ld / kTT, c.ncb, f64);
         c.b = BlockTiles{(int)(v0 / kTT), c.ld / kTT, 1, ng, (const uint16_t*)(uintptr_t)list_bytes,
-                         (const int*)(uintptr_t)cnt_bytes};   // offsets for now, rebased below
+                         (const int*)(uintptr_t)cnt_bytes, nullptr, 0, 1};   // offsets for now, rebased below
         list_bytes += sizeof(uint16_t) * (size_t)ng * c.b.nT;
         cnt_bytes += sizeof(int) * (size_t)c.b.nT;
       }
       const size_t bytes = (size_t)nphi * c.ld * elt;
-      if (cur_bytes + bytes > kPhiBudget) flush();
+      if (cur_bytes + bytes > ctx->phi_budget) flush();
       c.phi = (void*)(uintptr_t)cur_bytes;            // offsets for now, rebased below
       c.pscale = (float*)(uintptr_t)cur_ps;
       c.part = (double*)(uintptr_t)cur_part;

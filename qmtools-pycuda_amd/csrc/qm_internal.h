@@ -94,6 +94,8 @@ struct LiveGraph {
   hipEvent_t done;
 };
 
+constexpr size_t kPhiBudget = (size_t)4 << 30;   // bytes of basis values per chunk
+
 struct qm_ctx {
   int device = 0;
   std::string err;
@@ -120,6 +122,7 @@ struct qm_ctx {
   int jacobi_zs = 0;                    // z planes per Jacobi sweep workgroup (0 = chosen per grid)
   int jacobi_pairs = 1;                 // FP32 passes of several sweeps by tiles (else one-column strips)
   int tile_skip = 1;                    // contractions skip basis-function groups that are zero on a row tile
+  size_t phi_budget = kPhiBudget;       // bytes of basis values per chunk
   int ncu = 256;                        // compute units of the device
   std::vector<ProfRec> recs;
 };

@@ -123,3 +123,32 @@ def test_basis_beyond_the_lists_of_the_split_path(nbf, limit, prec):
                                     nat.QM_F64, 0) == want
     finally:
         lib.qm_mol_destroy(ctx, mol)
+
+
+@pytest.mark.parametrize("shape,subgrid", [((9, 6, 5), 3), ((8, 4, 4), 5), ((3, 2, 1), 16)])
+@pytest.mark.parametrize("prec", ["QM_PREC_FP64", "QM_PREC_F16X3"])
+def test_sub_points_beyond_the_workspace_budget(shape, subgrid, prec):
+    """A budget of 1 MiB holds 4 (FP64) or 9 (split) row tiles of 199 functions, fewer than one tile's sub-points:
+    the workspaces stay within it and the bits are those of the whole tile at once."""
+    import torch
+    import qmtools
+    from qmtools import _native as nat, synth
+    from qmtools.qmtools import device_molecule
+    mol = synth.synthetic_molecule(20, 6, qmtools.BasisSet(BASIS))
+    h = 0.7
+    o = mol.coords.mean(0) - 0.5 * h * numpy.array(shape) + 0.1
+    want = _raw(mol, (*shape, h, tuple(o)), subgrid, getattr(nat, prec))
+    handle = device_molecule(mol).handle
+    print("[case] sub-point chunks", shape, subgrid, prec, mol.nbf, flush=True)
+    ctx = nat.new_context()
+    try:
+        nat.call_ctx(ctx, "qm_tune_set", nat.QM_TUNE_PHI_MIB, 1)
+        got = torch.full((want.size,), float("nan"), dtype=torch.float64, device="cuda")
+        nat.call_ctx(ctx, "qm_density", handle, nat.stream(), ctypes.byref(nat.geom((*shape, h, tuple(o)))), subgrid,
+                     getattr(nat, prec), nat.QM_F64, nat.dptr(got), 0, None)
+        assert numpy.array_equal(got.cpu().numpy(), want)
+        held = ctypes.c_int64(0)
+        nat.library().qm_ctx_memory(ctx, ctypes.byref(held))
+        assert held.value <= (1 << 20) * 5 // 4   # partial sums: an eighth of the basis values at most
+    finally:
+        nat.destroy_context(ctx)
