@@ -154,13 +154,30 @@ def _green_points(reqs):
     return loose + sum((a // 2 + 1) * (b // 2 + 1) * (c // 2 + 1) for a, b, c in shapes)
 
 
+def _list_groups(req, precision):
+    """Groups of functions (16 in FP64, 32 in the split path) that a tile of 128 points can list."""
+    return -(-int(req.mol.nbf) // (16 if precision == "fp64" else 32))
+
+
+def _partial_share(req, precision):
+    """Partial densities and scales of a round as a share of its basis values: per point one FP64 sum for every
+    group (FP64) or two for every four groups (split), and one FP32 scale."""
+    ng = _list_groups(req, precision)
+    if precision == "fp64":
+        return (8 * ng + 4) / (128 * ng)
+    return (16 * -(-ng // 4) + 4) / (128 * ng)
+
+
 def workspace_estimate(reqs, precision="mixed", poisson="jacobi"):
     """Device bytes a lane's native context grows to while it runs this batch: basis values of one
-    round, the FP32 Jacobi correction buffers or the FFT work buffer and Green's-function cache."""
+    round with their partial densities and scales, the tiles' function lists, the FP32 Jacobi correction
+    buffers or the FFT work buffer and Green's-function cache."""
     elt = 8 if precision == "fp64" else 4
     npts = sum(r.npts for r in reqs)
     nbf_pad = max(((int(r.mol.nbf) + 63) // 64 * 64 for r in reqs), default=0)
     phi = min(_PHI_BUDGET, npts * nbf_pad * elt)
+    phi += int(phi * max((_partial_share(r, precision) for r in reqs), default=0.0))
+    phi += sum((r.npts + 127) // 128 * (4 + 2 * _list_groups(r, precision)) for r in reqs)
     if poisson == "fft":
         cplx = 16 if precision == "fp64" else 8
         padded = [_padded_points(r) for r in reqs]
