@@ -698,7 +698,8 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   if ((rc = qm_sine_z(ctx, s, p, tmp))) return rc;
   auto delta_at = [&](int64_t c, double* d) -> int {   // check c: after c check_every sweeps
     int r = qm_sine_scale_zy(ctx, s, p, sweeps_factor(SINE_POWER, c * check_every - 1), tmp, w);
-    return r ? r : qm_sine_x_sum(ctx, s, p, w, nullptr, d);
+    if (!r) r = qm_sine_x_sum(ctx, s, p, w, nullptr);
+    return r ? r : qm_sine_sum(ctx, s, p, d);
   };
   double dhi = 0.0;   // delta at the last check; the wait makes the flag readable
   if ((rc = delta_at(checks, &dhi))) return rc;
@@ -712,13 +713,13 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   }
   if ((rc = qm_sine_scale_zy(ctx, s, p, sweeps_factor(SINE_SUM, at), tmp, w))) return rc;
   double total = 0.0;
-  if ((rc = qm_sine_x_sum(ctx, s, p, w, v, &total))) return rc;
+  if ((rc = qm_sine_x_sum(ctx, s, p, w, v)) || (rc = qm_sine_sum(ctx, s, p, &total))) return rc;
   const double floor = 1e-12 * total;
   if (!(floor < INFINITY) || (tol < floor && delta < floor)) return QM_OK;
   if ((rc = qm_sine_x_add(ctx, s, p, w, v))) return rc;
   // with a tolerance the call returns once v is final, as the loop does
-  use.end();
   QM_CHECK_HIP(ctx, hipStreamSynchronize(s));
+  use.waited();
   *done_out = at;
   *delta_out = delta;
   *converged_out = converged;

@@ -102,7 +102,8 @@ struct qm_ctx {
   Workspace ws[WS_COUNT];
   double* host_scalars = nullptr;   // pinned host buffer for results
   FftPlanCache* fft = nullptr;
-  hipEvent_t sine_done = nullptr;   // after the last closed form's use of WS_SINE and WS_SINE_W (SineUse)
+  hipEvent_t sine_done = nullptr;   // after the last closed form's use of WS_SINE and WS_SINE_W (SineUse),
+  bool sine_pending = false;        // which may be in flight still
   bool prof = false;
   hipStream_t graph_stream = nullptr;   // non-blocking stream for graph capture (default priority)
   std::vector<LiveGraph> graphs;        // graphs whose replays may still run

@@ -346,7 +346,7 @@ int qm_sine_first_below(int64_t n, double dn, double tol, const std::function<in
 
 int SineUse::begin() {
   if (!ctx->sine_done) QM_CHECK_HIP(ctx, hipEventCreateWithFlags(&ctx->sine_done, hipEventDisableTiming));
-  QM_CHECK_HIP(ctx, hipStreamWaitEvent(s, ctx->sine_done, 0));
+  if (ctx->sine_pending) QM_CHECK_HIP(ctx, hipStreamWaitEvent(s, ctx->sine_done, 0));
   held = true;
   return QM_OK;
 }
@@ -436,14 +436,16 @@ int qm_sine_x_add(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a
   return pass<0, LOAD_PLAIN, false, STORE_ADD>(ctx, s, plain_args(p, a, v));
 }
 
-int qm_sine_x_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, const double* v, double* host_sum) {
+int qm_sine_x_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, const double* v) {
   Args r = plain_args(p, a, const_cast<double*>(v));
   r.part = p.part;
   int rc = v ? pass<0, LOAD_PLAIN, false, STORE_SUMV>(ctx, s, r) : pass<0, LOAD_PLAIN, false, STORE_SUM>(ctx, s, r);
   if (rc) return rc;
   const int64_t nl = (int64_t)p.m[1] * p.m[2], lines = p.m[0] <= 256 ? 32 : 16;
-  if ((rc = qm_reduce_part_dev(ctx, s, QM_RED_SUM, QM_F64, p.part, nullptr, (nl + lines - 1) / lines, p.red,
-                               p.sum))) return rc;
+  return qm_reduce_part_dev(ctx, s, QM_RED_SUM, QM_F64, p.part, nullptr, (nl + lines - 1) / lines, p.red, p.sum);
+}
+
+int qm_sine_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* host_sum) {
   QM_CHECK_HIP(ctx, hipMemcpyAsync(ctx->host_scalars + 2, p.sum, sizeof(double), hipMemcpyDeviceToHost, s));
   QM_CHECK_HIP(ctx, hipStreamSynchronize(s));
   *host_sum = ctx->host_scalars[2];

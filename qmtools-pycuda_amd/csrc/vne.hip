@@ -347,7 +347,8 @@ int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, d
   };
   auto delta_at = [&](int64_t pr, double* d) -> int {
     int r = qm_sine_scale_zy(ctx, s, p, factor(SINE_POWER, 2 * pr - 1), tmp, v);
-    if (!r) r = qm_sine_x_sum(ctx, s, p, v, nullptr, d);
+    if (!r) r = qm_sine_x_sum(ctx, s, p, v, nullptr);
+    if (!r) r = qm_sine_sum(ctx, s, p, d);
     *d /= n;
     return r;
   };
@@ -363,12 +364,13 @@ int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, d
   if (!ok && (rc = delta_at(cap, &d))) return rc;
   double total = 0.0;
   if ((rc = qm_sine_scale_zy(ctx, s, p, factor(SINE_SUM, 2 * at), tmp, v))) return rc;
-  if ((rc = qm_sine_x_sum(ctx, s, p, v, nullptr, &total))) return rc;
+  if ((rc = qm_sine_x_sum(ctx, s, p, v, nullptr))) return rc;
+  if ((rc = qm_sine_x(ctx, s, p, v))) return rc;
+  // one wait for the sum and the last pass (the loop would clear v): the call returns once v is final, as the loop does
+  if ((rc = qm_sine_sum(ctx, s, p, &total))) return rc;
+  use.waited();
   const double floor = 1e-12 * total / n;
   if (!(floor < INFINITY) || !(d < INFINITY) || (tol < floor && d < floor)) return QM_OK;
-  if ((rc = qm_sine_x(ctx, s, p, v))) return rc;
-  use.end();
-  QM_CHECK_HIP(ctx, hipStreamSynchronize(s));   // the call returns once v is final, as the loop does
   *pairs = at;
   *delta = d;
   *conv = ok ? 1 : 0;
