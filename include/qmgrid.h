@@ -304,7 +304,9 @@ enum {
                                same */
   QM_TUNE_PHI_MIB = 5,      /* MiB of basis values that a density call (a round of qm_density_batch) holds at a time,
                                1..4096 (default); the results do not depend on it */
-  QM_TUNE_COUNT = 6
+  QM_TUNE_WS_MIB = 6,       /* MiB that each workspace of the context may grow to, 0 = no limit (default); a call that
+                               needs more takes a path that does not, or returns QM_ENOMEM */
+  QM_TUNE_COUNT = 7
 };
 int qm_tune_set(qm_ctx* ctx, int knob, int value);
 int qm_tune_get(qm_ctx* ctx, int knob, int* value);

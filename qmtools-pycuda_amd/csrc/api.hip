@@ -40,7 +40,7 @@ int qm_ws(qm_ctx* ctx, hipStream_t s, int slot, size_t bytes, void** out) {
     }
     size_t want = std::max(bytes, (size_t)4096);
     want = (want + 4095) & ~(size_t)4095;
-    if (hipMallocAsync(&w.ptr, want, s) != hipSuccess) {
+    if ((ctx->ws_limit && want > ctx->ws_limit) || hipMallocAsync(&w.ptr, want, s) != hipSuccess) {
       (void)hipGetLastError();
       w.ptr = nullptr;
       return qm_fail(ctx, QM_ENOMEM, "workspace %d: cannot allocate %zu bytes", slot, want);

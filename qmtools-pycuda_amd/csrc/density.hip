@@ -3122,6 +3122,11 @@ int qm_tune_set(qm_ctx* ctx, int knob, int value) {
     ctx->phi_budget = (size_t)value << 20;
     return QM_OK;
   }
+  if (knob == QM_TUNE_WS_MIB) {
+    QM_REQUIRE(ctx, value >= 0, QM_EINVAL, "tune: negative workspace limit");
+    ctx->ws_limit = (size_t)value << 20;
+    return QM_OK;
+  }
   return qm_fail(ctx, QM_EINVAL, "tune: unknown knob %d", knob);
 }
 
@@ -3151,6 +3156,10 @@ int qm_tune_get(qm_ctx* ctx, int knob, int* value) {
   }
   if (knob == QM_TUNE_PHI_MIB) {
     *value = (int)(ctx->phi_budget >> 20);
+    return QM_OK;
+  }
+  if (knob == QM_TUNE_WS_MIB) {
+    *value = (int)(ctx->ws_limit >> 20);
     return QM_OK;
   }
   return qm_fail(ctx, QM_EINVAL, "tune: unknown knob %d", knob);

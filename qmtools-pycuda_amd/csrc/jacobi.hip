@@ -643,7 +643,7 @@ struct GraphBlock {
 // FP64 sweeps in closed form by sine transforms (sine.hip): V_n = V + sum_{j<n} A^j (V_1 - V).  *done stays
 // false where the sweeps have to be run instead: under stream capture (the call waits for a flag), a residual
 // that is not finite somewhere (it would spread over the whole grid at once) or so large that a transform
-// might overflow, no room for the check's buffer, or a tolerance that the sweeps' rounding decides.
+// might overflow, no room for the tables or the check's buffer, or a tolerance that the sweeps' rounding decides.
 //
 // Convergence checks: delta after n sweeps is |A^(n-1) (V_1 - V)|_1, and A (neighbour sums / 6) does not
 // increase that norm, so the first check with delta <= tol is found by bisection over the checks, in the
@@ -669,7 +669,9 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   }
   SinePlan p;
   ProfScope ps(ctx, s, QM_K_JACOBI, (int)std::min<int64_t>(max_sweeps, 1 << 30));
-  if ((rc = qm_sine_plan(ctx, s, g, &p))) return rc;
+  rc = qm_sine_plan(ctx, s, g, &p);
+  if (rc == QM_ENOMEM) ctx->err.clear();   // the sweeps need no tables
+  if (rc) return rc == QM_ENOMEM ? QM_OK : rc;
   if ((rc = qm_sine_residual_xy(ctx, s, p, rho, v, g->step, tmp))) return rc;
   int* bad = (int*)(ctx->host_scalars + 3);
   auto sweeps_factor = [](int kind, int64_t n) {

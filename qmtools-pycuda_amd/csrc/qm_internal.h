@@ -124,6 +124,7 @@ struct qm_ctx {
   int jacobi_pairs = 1;                 // FP32 passes of several sweeps by tiles (else one-column strips)
   int tile_skip = 1;                    // contractions skip basis-function groups that are zero on a row tile
   size_t phi_budget = kPhiBudget;       // bytes of basis values per chunk
+  size_t ws_limit = 0;                  // bytes per workspace, 0 = no limit
   int ncu = 256;                        // compute units of the device
   std::vector<ProfRec> recs;
 };

@@ -311,7 +311,7 @@ __global__ __launch_bounds__(256) void k_vne_finish(const double* __restrict__ p
 // sum_{j<n} A^j s, and the n-th changes the field by A^(n-1) s.  Taken where A has no negative weight and no
 // row sum above 1 (the usual parameters: a voxel keeps 1 - 16.79 DIF - ADS >= 0, and ADS >= 2.31 DIF), because then
 // sum |A^(n-1) s| never grows and the first pair at the tolerance is found by bisection.  *finished stays
-// false where that does not hold, or where the sweeps' rounding (about 1e-16 of the field) decides the test.
+// false where that does not hold, where the tables cannot be had, or where the sweeps' rounding (about 1e-16 of the field) decides the test.
 // v is the work buffer (its outer layer stays 0), tmp holds the spectrum.
 // 120 x 120 x 64, 974 pairs: 27.1 -> 0.36 ms.
 int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, double ads, double dif, double tol,
@@ -326,7 +326,9 @@ int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, d
   SinePlan p;
   int rc;
   if ((rc = use.begin())) return rc;
-  if ((rc = qm_sine_plan(ctx, s, g, &p))) return rc;
+  rc = qm_sine_plan(ctx, s, g, &p);
+  if (rc == QM_ENOMEM) ctx->err.clear();   // the sweeps need no tables
+  if (rc) return rc == QM_ENOMEM ? QM_OK : rc;
   ProfScope ps(ctx, s, QM_K_VNE, (int)std::min<int64_t>(cap, 1 << 30));
   // the first sweep of a zero field is the source
   hipLaunchKernelGGL(k_vne_sweep<double>, grid, block, 0, s, (const double*)v, tmp, (const double4*)mol->atoms,

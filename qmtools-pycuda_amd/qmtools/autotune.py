@@ -17,7 +17,7 @@ from . import _native as nat
 
 _KNOBS = {"split_variant": nat.QM_TUNE_SPLIT_VARIANT, "f64_variant": nat.QM_TUNE_F64_VARIANT,
           "jacobi_zs": nat.QM_TUNE_JACOBI_ZS, "jacobi_pairs": nat.QM_TUNE_JACOBI_PAIRS,
-          "tile_skip": nat.QM_TUNE_TILE_SKIP, "phi_mib": nat.QM_TUNE_PHI_MIB}
+          "tile_skip": nat.QM_TUNE_TILE_SKIP, "phi_mib": nat.QM_TUNE_PHI_MIB, "ws_mib": nat.QM_TUNE_WS_MIB}
 _PREC = {"fp64": nat.QM_PREC_FP64, "mixed": nat.QM_PREC_F16X3, "f16": nat.QM_PREC_F16X3,
          "bf16": nat.QM_PREC_BF16X3}
 

@@ -106,3 +106,51 @@ def test_under_stream_capture():
             assert numpy.array_equal(v.cpu().numpy(), want.cpu().numpy())
     finally:
         nat.destroy_context(ctx)
+
+
+@pytest.mark.parametrize("tol", [-1.0, 1e-6])
+def test_no_room_for_the_tables(tol):
+    """The sweeps need no workspace of the grid's size: where the sine tables cannot be had they run instead."""
+    from qmtools import _native as nat
+    shape = (530, 20, 24)
+    rho, v0 = _state(shape, 7)
+    want, got = v0.clone(), v0.clone()
+    for _ in range(9):
+        _jacobi(shape, rho, want, 20)
+    print("[case] closed form, no room", tol, flush=True)
+    ctx = nat.new_context()
+    try:
+        nat.call_ctx(ctx, "qm_tune_set", nat.QM_TUNE_WS_MIB, 1)
+        rc, done, _ = _jacobi(shape, rho, got, 180, tol, 60, ctx)
+        assert rc == (nat.QM_OK if tol < 0 else nat.QM_ENOCONV) and done == 180
+        assert numpy.array_equal(got.cpu().numpy(), want.cpu().numpy())
+    finally:
+        nat.destroy_context(ctx)
+
+
+def test_no_room_for_the_tables_of_vne():
+    import torch
+    import qmtools
+    from conftest import BASIS
+    from oracle import vne as ov
+    from qmtools import _native as nat, synth
+    from qmtools.qmtools import device_molecule
+    mol = synth.synthetic_molecule(6, 3, qmtools.BasisSet(BASIS))
+    shape, h = (530, 12, 10), 0.5
+    o = mol.coords.mean(0) - 0.5 * h * numpy.array(shape)
+    v = torch.empty(shape[0] * shape[1] * shape[2], dtype=torch.float64, device="cuda")
+    t = torch.empty_like(v)
+    p, d, c = ctypes.c_int64(0), ctypes.c_double(0), ctypes.c_int(0)
+    handle = device_molecule(mol).handle
+    print("[case] V_ne closed form, no room", flush=True)
+    ctx = nat.new_context()
+    try:
+        nat.call_ctx(ctx, "qm_tune_set", nat.QM_TUNE_WS_MIB, 1)
+        nat.call_ctx(ctx, "qm_vne_diffusion", handle, nat.stream(), ctypes.byref(nat.geom((*shape, h, tuple(o)))),
+                     nat.QM_F64, 0.05, 0.02, 1e-7, 200.0, nat.dptr(v), nat.dptr(t), ctypes.byref(p), ctypes.byref(d),
+                     ctypes.byref(c))
+    finally:
+        nat.destroy_context(ctx)
+    want, wp, wd, wc = ov.vne_diffusion(mol.types, mol.coords, *shape, h, o, 0.05, 0.02, 1e-7, 200.0)
+    assert p.value == wp and bool(c.value) == wc
+    assert numpy.abs(v.cpu().numpy().reshape(want.shape) - want).max() <= 1e-12 * numpy.abs(want).max()
