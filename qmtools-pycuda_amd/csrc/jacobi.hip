@@ -668,7 +668,7 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
     return QM_OK;
   }
   SinePlan p;
-  ProfScope ps(ctx, s, QM_K_JACOBI, (int)std::min<int64_t>(max_sweeps, 1 << 30));
+  ProfScope ps(ctx, s, QM_K_JACOBI, 0);   // counts as the sweeps that it stands for
   rc = qm_sine_plan(ctx, s, g, &p);
   if (rc == QM_ENOMEM) ctx->err.clear();   // the sweeps need no tables
   if (rc) return rc == QM_ENOMEM ? QM_OK : rc;
@@ -693,6 +693,7 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
     (void)hipEventDestroy(ev);
     if (rc || *bad) return rc;
     if ((rc = qm_sine_x_add(ctx, s, p, tmp, v))) return rc;
+    ps.weight = (int)std::min<int64_t>(max_sweeps, 1 << 30);
     *done_out = max_sweeps;
     *finished = true;
     return QM_OK;
@@ -722,6 +723,7 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   // with a tolerance the call returns once v is final, as the loop does
   QM_CHECK_HIP(ctx, hipStreamSynchronize(s));
   use.waited();
+  ps.weight = (int)std::min<int64_t>(at, 1 << 30);
   *done_out = at;
   *delta_out = delta;
   *converged_out = converged;

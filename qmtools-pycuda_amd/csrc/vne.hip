@@ -329,7 +329,7 @@ int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, d
   rc = qm_sine_plan(ctx, s, g, &p);
   if (rc == QM_ENOMEM) ctx->err.clear();   // the sweeps need no tables
   if (rc) return rc == QM_ENOMEM ? QM_OK : rc;
-  ProfScope ps(ctx, s, QM_K_VNE, (int)std::min<int64_t>(cap, 1 << 30));
+  ProfScope ps(ctx, s, QM_K_VNE, 0);   // counts as the pairs that it stands for
   // the first sweep of a zero field is the source
   hipLaunchKernelGGL(k_vne_sweep<double>, grid, block, 0, s, (const double*)v, tmp, (const double4*)mol->atoms,
                      mol->natoms, geom_view(g), zs, ads, dif, (double*)nullptr, st);
@@ -373,6 +373,7 @@ int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, d
   use.waited();
   const double floor = 1e-12 * total / n;
   if (!(floor < INFINITY) || !(d < INFINITY) || (tol < floor && d < floor)) return QM_OK;
+  ps.weight = (int)std::min<int64_t>(at, 1 << 30);
   *pairs = at;
   *delta = d;
   *conv = ok ? 1 : 0;

@@ -154,3 +154,22 @@ def test_no_room_for_the_tables_of_vne():
     want, wp, wd, wc = ov.vne_diffusion(mol.types, mol.coords, *shape, h, o, 0.05, 0.02, 1e-7, 200.0)
     assert p.value == wp and bool(c.value) == wc
     assert numpy.abs(v.cpu().numpy().reshape(want.shape) - want).max() <= 1e-12 * numpy.abs(want).max()
+
+
+@pytest.mark.parametrize("tol,decided", [(1e2, True), (0.0, False)])
+def test_profile_counts_the_sweeps_that_were_done(tol, decided):
+    """A closed form that stops at a check counts as the sweeps up to it, one that is left to the sweeps as nothing."""
+    from qmtools import _native as nat
+    shape = (12, 10, 9)
+    rho, v = _state(shape, 4)
+    ctx = nat.new_context()
+    print("[case] closed form, profile", tol, flush=True)
+    try:
+        nat.call_ctx(ctx, "qm_profile", 1)
+        rc, done, _ = _jacobi(shape, rho, v, 3000, tol, 30, ctx)
+        assert rc == nat.QM_OK and (done < 3000 or not decided)
+        ms, n = ctypes.c_double(0), ctypes.c_int64(0)
+        nat.call_ctx(ctx, "qm_profile_read", nat.QM_K_JACOBI, ctypes.byref(ms), ctypes.byref(n))
+        assert n.value == done
+    finally:
+        nat.destroy_context(ctx)
