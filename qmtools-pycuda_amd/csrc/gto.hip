@@ -162,7 +162,11 @@ __device__ __forceinline__ double dist_sum(const double* __restrict__ ds, int lo
 struct DistLists {
   const double* d[kLmax + 1];
   int n[kLmax + 1];
+  int cost;                 // of all lists (dist_cost)
 };
+
+// cost of a distribution, about proportional to its FP64 operations
+__host__ __device__ constexpr int dist_cost(int L) { return L == 0 ? 5 : L == 1 ? 6 : L == 2 ? 8 : L == 3 ? 12 : 20; }
 
 // Point of thread t of workgroup b: a list or a grid's nodes in order, or (blocks) a grid in blocks of 8^3 per workgroup
 // and 4^3 per wave, so that the points of a wave mostly take the same branch of the Boys function.  idx < 0: none.
@@ -198,6 +202,9 @@ __device__ __forceinline__ int64_t gto_point(const double* __restrict__ pts, con
 // points: 3.1 -> 1.7 ms with shared primitive pairs and one multiply-add per Taylor term; 16 atoms,
 // 48 x 40 x 56 nodes: 2.9 -> 1.3 ms, with the nodes taken in 4^3 blocks.
 constexpr int kGtoThreads = 512;
+// SHARES: a chunk takes an equal share of lists.cost, else a slice of every list (as a branch in one kernel this cost the
+// long chunks 1 %)
+template <bool SHARES>
 __global__ __launch_bounds__(kGtoThreads) void k_gto(DistLists lists, const double* __restrict__ boys_tab,
                                                      const double* __restrict__ pts, GeomView g, int64_t npts,
                                                      int blocks, int nchunk, double* __restrict__ partial) {
@@ -206,11 +213,18 @@ __global__ __launch_bounds__(kGtoThreads) void k_gto(DistLists lists, const doub
   double cx, cy, cz;
   const int64_t idx = gto_point(pts, g, npts, blockIdx.x, threadIdx.x, blocks, cx, cy, cz);
   double acc = 0.0;
+  int c0 = (int)((int64_t)lists.cost * chunk / nchunk), c1 = (int)((int64_t)lists.cost * (chunk + 1) / nchunk);
 #define QM_GTO_L(LL)                                                                                                 \
   {                                                                                                                  \
     const int n = lists.n[LL];                                                                                       \
     const int per = (n + nchunk - 1) / nchunk;                                                                       \
-    const int lo = min(n, chunk * per), hi = min(n, lo + per);                                                       \
+    int lo = min(n, chunk * per), hi = min(n, lo + per);                                                             \
+    if (SHARES) {                                                                                                    \
+      lo = min(n, max(0, (c0 + dist_cost(LL) - 1) / dist_cost(LL)));                                                 \
+      hi = min(n, max(0, (c1 + dist_cost(LL) - 1) / dist_cost(LL)));                                                 \
+      c0 -= n * dist_cost(LL);                                                                                       \
+      c1 -= n * dist_cost(LL);                                                                                       \
+    }                                                                                                                \
     if (hi > lo) { /* the same for the whole workgroup */                                                            \
       __syncthreads();                                                                                               \
       for (int i = threadIdx.x; i < kBoysPts * kBoysN; i += kGtoThreads) tab[i] = boys_tab[LL * kBoysPts * kBoysN + i]; \
@@ -580,16 +594,24 @@ int gto_eval(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const double* pts, const G
   const int64_t blocked = pts ? 0 : (int64_t)((gv.nx + 7) / 8) * ((gv.ny + 7) / 8) * ((gv.nz + 7) / 8);
   const bool blocks = !pts && 20 * blocked <= 21 * linear;
   const int64_t pblocks = blocks ? blocked : linear;
-  // enough workgroups for 256 CUs: split the distributions over chunks when points are few
-  int nchunk = (int)std::max<int64_t>(1, std::min<int64_t>(256, 2048 / std::max<int64_t>(pblocks, 1)));
-  nchunk = std::max(1, std::min(nchunk, std::max(1, total / 64)));
+  // Enough workgroups for 256 CUs: the distributions are split over chunks when points are few, at least 64 of them to a
+  // chunk, or 32 of up to 2048 (the last kernel adds the chunks up one after the other).  Short chunks take a share of the
+  // total cost, so that they run one or two of the lists, since each refills the table in LDS; long ones a slice of every
+  // list.  2, 5, 9, 12 atoms (185, 1148, 3292, 5347 distributions), 700 points, us: slices of 64 36, 40, 53, 62; shares
+  // of 64 34, 33, 46, 56; of 32 20, 28, 49, 66.
+  const int few = total / (total <= 2048 ? 32 : 64);
+  const int64_t fill = std::min<int64_t>(256, 2048 / std::max<int64_t>(pblocks, 1));
+  const int nchunk = (int)std::max<int64_t>(1, std::min<int64_t>(fill, few));
+  const bool shares = total < 256 * nchunk;
+  dl.cost = 0;
+  for (int L = 0; shares && L <= kLmax; ++L) dl.cost += dl.n[L] * dist_cost(L);
   double* partial = nullptr;
   if ((rc = qm_ws(ctx, s, WS_GTO, sizeof(double) * (size_t)nchunk * npts, (void**)&partial))) return rc;
   QM_REQUIRE(ctx, pblocks <= 0x7fffffff, QM_ELIMIT, "gto: too many points");
   {
     ProfScope ps(ctx, s, QM_K_GTO);
-    hipLaunchKernelGGL(k_gto, dim3((unsigned)pblocks, nchunk), dim3(kGtoThreads), 0, s, dl, (const double*)c->boys,
-                     pts, gv, npts, blocks ? 1 : 0, nchunk, partial);
+    hipLaunchKernelGGL(shares ? k_gto<true> : k_gto<false>, dim3((unsigned)pblocks, nchunk), dim3(kGtoThreads), 0, s, dl,
+                       (const double*)c->boys, pts, gv, npts, blocks ? 1 : 0, nchunk, partial);
   }
   QM_CHECK_LAUNCH(ctx);
   hipLaunchKernelGGL(k_gto_finish<TO>, dim3((unsigned)((npts + 255) / 256)), dim3(256), 0, s,

@@ -74,3 +74,26 @@ def test_thin_grids_cost_what_their_nodes_cost(shape):
             best = min(best, e0.elapsed_time(e1))
         return best
     assert time(grid) <= 2.0 * time(points)
+
+
+@pytest.mark.parametrize("natoms", [1, 2, 5, 7, 9])
+@pytest.mark.parametrize("npts", [1, 700, 5000])
+def test_shares_of_the_distributions(natoms, npts):
+    """Few distributions and few points: chunks of equal cost over all lists (1 to 64 of them); the gate, 1e-10."""
+    import torch
+    from oracle import gto as og
+    from oracle.basisfile import read_basis
+    from oracle.system import make_system
+    from qmtools import _native as nat
+    from qmtools.qmtools import device_molecule
+    mol = _molecule(natoms)
+    pts = mol.coords.mean(0) + numpy.random.default_rng(natoms).uniform(-6, 6, size=(npts, 3))
+    some = numpy.unique(numpy.r_[0:min(npts, 40), max(npts - 8, 0):npts])
+    want = og.potential(make_system(mol.types, mol.coords, mol.dm, read_basis(BASIS)), pts[some])
+    d = torch.tensor(pts.ravel(), device="cuda")
+    out = torch.full((npts,), float("nan"), dtype=torch.float64, device="cuda")
+    print("[case] gto shares", natoms, npts, flush=True)
+    nat.call("qm_hartree_gto_points", device_molecule(mol).handle, nat.stream(), nat.dptr(d), npts, nat.dptr(out))
+    got = out.cpu().numpy()
+    assert numpy.isfinite(got).all()
+    assert numpy.abs(got[some] - want).max() <= 1e-10 * numpy.abs(want).max()
