@@ -152,3 +152,38 @@ def test_sub_points_beyond_the_workspace_budget(shape, subgrid, prec):
         assert held.value <= (1 << 20) * 5 // 4   # partial sums: an eighth of the basis values at most
     finally:
         nat.destroy_context(ctx)
+
+
+def _best_ms(run, reps=6):
+    import torch
+    best = 1e9
+    for _ in range(reps):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        run()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
+def _density_call(mol, geom, subgrid, prec):
+    import torch
+    from qmtools import _native as nat
+    from qmtools.qmtools import device_molecule
+    handle, g = device_molecule(mol).handle, nat.geom(geom)
+    out = torch.empty(geom[0] * geom[1] * geom[2], dtype=torch.float64, device="cuda")
+    return lambda: nat.call("qm_density", handle, nat.stream(), ctypes.byref(g), subgrid, prec, nat.QM_F64, nat.dptr(out),
+                            0, None)
+
+
+def test_sub_points_cost_what_their_grid_costs():
+    """16^3 voxels of 4^3 sub-points are the points of 64^3 voxels: no more than 1.8 times their time."""
+    import qmtools
+    from qmtools import _native as nat, synth
+    mol = synth.synthetic_molecule(12, 3, qmtools.BasisSet(BASIS))
+    o = tuple(mol.coords.mean(0) - 9.0)
+    print("[case] sub-points, time", flush=True)
+    sub = _best_ms(_density_call(mol, (16, 16, 16, 18.0 / 16, o), 4, nat.QM_PREC_FP64))
+    fine = _best_ms(_density_call(mol, (64, 64, 64, 18.0 / 64, o), 1, nat.QM_PREC_FP64))
+    assert sub <= 1.8 * fine
