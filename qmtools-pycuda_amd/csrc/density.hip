@@ -799,8 +799,6 @@ __device__ __forceinline__ void tiled_f64_body(int rt, int cb, const double* __r
 // cutoff), so the sums are the same bit for bit with every group listed (QM_TUNE_TILE_SKIP = 0).
 // On 60 atoms in a 28 bohr box 45% of the FP64 groups (52% of the split ones) are active and 26% (33%) of the
 // triangle is left.  60 atoms at 256^3, density call: FP64 110 -> 43 ms, split 25.3 -> 16.7 ms.
-constexpr int kBTX = 8, kBTY = 4, kBTZ = 4;
-static_assert(kBTX * kBTY * kBTZ == kTT, "a block tile is one row tile");
 constexpr int kMaxGroups = 2048;   // groups per tile that a workgroup can list in LDS
 
 struct BlockTiles {
@@ -811,18 +809,46 @@ struct BlockTiles {
   const int* cnt;         // [row tile]: how many
   const int* order;       // the contraction's order of the row tiles, null: as numbered
   int s0, ns;             // sub-points s0 .. s0 + ns - 1 of nsub^3
+  int lx, ly;             // log2 of a tile's voxels along x and y (block_shape)
 };
 
-__host__ __device__ inline int64_t block_tiles(const GeomView& g) {
-  return (int64_t)((g.nx + kBTX - 1) / kBTX) * ((g.ny + kBTY - 1) / kBTY) * ((g.nz + kBTZ - 1) / kBTZ);
+// A tile's shape: 8 x 4 x 4 voxels, but on an axis that holds no more than half of an edge the edge is halved and the
+// shortest one that its axis still exceeds is doubled, so that planes and lines fill their tiles (8 x 4 x 4 holds
+// a quarter of its points on a plane, a 16th or 32nd on a line).  30 atoms, two sub-points per axis, FP64 and split, us:
+// 100 x 100 x 1 605 -> 217 and 237 -> 85, 1 x 1 x 3000 1463 -> 109 and 558 -> 51.
+inline void block_shape(const GeomView& g, int l[3]) {
+  const int n[3] = {g.nx, g.ny, g.nz};
+  int spare = 0;
+  l[0] = 3;
+  l[1] = l[2] = 2;
+  for (int d = 0; d < 3; ++d)
+    for (; l[d] > 0 && 1 << (l[d] - 1) >= n[d]; --l[d]) ++spare;
+  for (; spare > 0; --spare) {
+    int to = -1;
+    for (int d = 0; d < 3; ++d)
+      if (1 << l[d] < n[d] && (to < 0 || l[d] < l[to])) to = d;
+    ++l[to < 0 ? 0 : to];
+  }
 }
 
-__device__ __forceinline__ void block_origin(const GeomView& g, int T, int& i0, int& j0, int& k0) {
-  const int ntx = (g.nx + kBTX - 1) / kBTX, nty = (g.ny + kBTY - 1) / kBTY;
+inline int64_t block_tiles(const GeomView& g, const int l[3]) {
+  auto tiles = [](int n, int lg) { return ((int64_t)n + (1 << lg) - 1) >> lg; };
+  return tiles(g.nx, l[0]) * tiles(g.ny, l[1]) * tiles(g.nz, l[2]);
+}
+
+__device__ __forceinline__ void block_origin(const GeomView& g, const BlockTiles& b, int T, int& i0, int& j0, int& k0) {
+  const int ntx = (g.nx + (1 << b.lx) - 1) >> b.lx, nty = (g.ny + (1 << b.ly) - 1) >> b.ly;
   const int q = T / ntx;
-  i0 = (T - q * ntx) * kBTX;
-  k0 = q / nty * kBTZ;
-  j0 = (q - q / nty * nty) * kBTY;
+  i0 = (T - q * ntx) << b.lx;
+  k0 = q / nty << (7 - b.lx - b.ly);
+  j0 = (q - q / nty * nty) << b.ly;
+}
+
+// voxel of point p of a tile, from the tile's first
+__device__ __forceinline__ void block_voxel(const BlockTiles& b, int p, int& i, int& j, int& k) {
+  i += p & ((1 << b.lx) - 1);
+  j += (p >> b.lx) & ((1 << b.ly) - 1);
+  k += p >> (b.lx + b.ly);
 }
 
 // Position of point p of row tile rt (same arithmetic as chunk_point); points of an edge tile beyond the
@@ -830,9 +856,12 @@ __device__ __forceinline__ void block_origin(const GeomView& g, int T, int& i0, 
 __device__ __forceinline__ void block_point(const GeomView& g, const BlockTiles& b, int rt, int p, double& x, double& y,
                                             double& z) {
   const int part = rt / b.nT, s = b.s0 + part;
-  int i0, j0, k0;
-  block_origin(g, b.T0 + (rt - part * b.nT), i0, j0, k0);
-  const int i = min(i0 + (p & 7), g.nx - 1), j = min(j0 + ((p >> 3) & 3), g.ny - 1), k = min(k0 + (p >> 5), g.nz - 1);
+  int i, j, k;
+  block_origin(g, b, b.T0 + (rt - part * b.nT), i, j, k);
+  block_voxel(b, p, i, j, k);
+  i = min(i, g.nx - 1);
+  j = min(j, g.ny - 1);
+  k = min(k, g.nz - 1);
   const int sx = s % b.nsub, sy = (s / b.nsub) % b.nsub, sz = s / (b.nsub * b.nsub);
   const double inv = 1.0 / b.nsub;
   x = g.ox + ((double)i + (sx + 0.5) * inv) * g.h;
@@ -1170,10 +1199,8 @@ __device__ __forceinline__ void blocks_finish_body(int64_t idx, const GeomView& 
   const int tl = (int)(idx / kTT), p = (int)(idx % kTT);
   if (tl >= b.nT) return;
   int i, j, k;
-  block_origin(g, b.T0 + tl, i, j, k);
-  i += p & 7;
-  j += (p >> 3) & 3;
-  k += p >> 5;
+  block_origin(g, b, b.T0 + tl, i, j, k);
+  block_voxel(b, p, i, j, k);
   if (i >= g.nx || j >= g.ny || k >= g.nz) return;
   const int64_t stride = (int64_t)block_parts<SPLIT>(b.ng) * kTT;
   double v = b.s0 ? acc[idx] : 0.0;
@@ -2663,7 +2690,9 @@ int density_blocks(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, in
   const int nsub3 = nsub * nsub * nsub;
   const GeomView gv = geom_view(g);
   const MolView mv = mol->view();
-  const int64_t ntiles = block_tiles(gv);
+  int shape[3];
+  block_shape(gv, shape);
+  const int64_t ntiles = block_tiles(gv, shape);
   const size_t tile_bytes = (f64 ? sizeof(double) : 4) * (size_t)kTT * (ng << GS);
   const int64_t fit = std::max<int64_t>((int64_t)(ctx->phi_budget / tile_bytes), 1);   // row tiles
   const int ns = (int)std::min<int64_t>(fit, nsub3);
@@ -2690,7 +2719,7 @@ int density_blocks(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, in
     for (int s0 = 0; s0 < nsub3; s0 += ns) {
       const int nsc = std::min(ns, nsub3 - s0), nrt = nTc * nsc;
       const bool sorted = nrt >= kOrderMin && nrt <= kOrderMax;
-      const BlockTiles b{(int)T0, nTc, nsub, ng, list, cnt, sorted ? order : nullptr, s0, nsc};
+      const BlockTiles b{(int)T0, nTc, nsub, ng, list, cnt, sorted ? order : nullptr, s0, nsc, shape[0], shape[1]};
       const int pblk = f64 ? (nrt + 1) / 2 : (nrt + kPhiTiles - 1) / kPhiTiles;
       const dim3 pgrid(pblk, phi_split(pblk, ng << (GS - 3)));
       const int ny = block_split(nrt, ncb, f64);
@@ -3696,7 +3725,9 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
     // block tiles: points of whole tiles, in tile order
     const int ng = (m->nbf + (1 << gs) - 1) >> gs;
     const int nphi = blocks ? ng << gs : np;   // functions stored per point
-    const int64_t N = blocks ? block_tiles(geom_view(&geoms[i])) * kTT : npoints(&geoms[i]);
+    int shape[3];
+    block_shape(geom_view(&geoms[i]), shape);
+    const int64_t N = blocks ? block_tiles(geom_view(&geoms[i]), shape) * kTT : npoints(&geoms[i]);
     const int64_t cap = std::max<int64_t>(kTileM, std::min<int64_t>(kBatchChunk,
                                           (int64_t)(ctx->phi_budget / ((size_t)nphi * elt)) / kTileM * kTileM));
     for (int64_t v0 = 0; v0 < N; v0 += cap) {
@@ -3715,7 +3746,7 @@ extern "C" int qm_density_batch(qm_ctx* ctx, void* stream, int nmol, qm_mol* con
         c.ncb = f64 ? (ng + 7) / 8 : (ng + 3) / 4;
         c.ny = block_split(c.ld / kTT, c.ncb, f64);
         c.b = BlockTiles{(int)(v0 / kTT), c.ld / kTT, 1, ng, (const uint16_t*)(uintptr_t)list_bytes,
-                         (const int*)(uintptr_t)cnt_bytes, nullptr, 0, 1};   // offsets for now, rebased below
+                         (const int*)(uintptr_t)cnt_bytes, nullptr, 0, 1, shape[0], shape[1]};   // offsets for now, rebased below
         list_bytes += sizeof(uint16_t) * (size_t)ng * c.b.nT;
         cnt_bytes += sizeof(int) * (size_t)c.b.nT;
       }

@@ -187,3 +187,49 @@ def test_sub_points_cost_what_their_grid_costs():
     sub = _best_ms(_density_call(mol, (16, 16, 16, 18.0 / 16, o), 4, nat.QM_PREC_FP64))
     fine = _best_ms(_density_call(mol, (64, 64, 64, 18.0 / 64, o), 1, nat.QM_PREC_FP64))
     assert sub <= 1.8 * fine
+
+
+THIN = [(1, 1, 300), (1, 300, 1), (300, 1, 1), (40, 37, 1), (1, 40, 37), (37, 1, 40), (2, 70, 9), (70, 3, 9), (9, 70, 2),
+        (5, 1, 1), (3, 3, 3)]
+
+
+@pytest.mark.parametrize("shape", THIN)
+@pytest.mark.parametrize("subgrid", [1, 2])
+def test_tiles_of_thin_grids(shape, subgrid):
+    """Tiles that follow a thin grid's shape; the gates of the full grids, single and (one sub-point) batched."""
+    import torch
+    import qmtools
+    from oracle import density as od
+    from qmtools import _native as nat, synth
+    from qmtools.qmtools import device_molecule
+    mol = synth.synthetic_molecule(7, 6, qmtools.BasisSet(BASIS))
+    h = 0.4
+    o = mol.coords.mean(0) - 0.5 * h * numpy.array(shape) + 0.1
+    print("[case] thin tiles", shape, subgrid, flush=True)
+    want = od.density_grid_raw(_system(mol), *shape, h, o, subgrid)
+    top = numpy.abs(want).max()
+    for prec, tol in ((nat.QM_PREC_FP64, 1e-10), (nat.QM_PREC_F16X3, 1e-6)):
+        got = _raw(mol, (*shape, h, tuple(o)), subgrid, prec)
+        assert numpy.abs(got - want).max() <= tol * top
+        if subgrid > 1:
+            continue
+        out = torch.full((want.size,), float("nan"), dtype=torch.float64, device="cuda")
+        g = (nat.Geom * 1)(nat.geom((*shape, h, tuple(o))))
+        nat.call("qm_density_batch", nat.stream(), 1, (ctypes.c_void_p * 1)(device_molecule(mol).handle), g,
+                 (ctypes.c_void_p * 1)(out.data_ptr()), prec, nat.QM_F64, 0)
+        assert numpy.abs(out.cpu().numpy() - want).max() <= tol * top
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 3072), (3072, 1, 1), (64, 48, 1)])
+def test_thin_grids_cost_what_a_box_costs(shape):
+    """3072 voxels of 2^3 sub-points on a line or plane across the molecule: at most three times a box of as many."""
+    import qmtools
+    from qmtools import _native as nat, synth
+    mol = synth.synthetic_molecule(12, 3, qmtools.BasisSet(BASIS))
+    print("[case] thin tiles, time", shape, flush=True)
+
+    def best(sh):
+        h = 18.0 / max(sh)
+        o = tuple(mol.coords.mean(0) - 0.5 * h * numpy.array(sh))
+        return _best_ms(_density_call(mol, (*sh, h, o), 2, nat.QM_PREC_FP64))
+    assert best(shape) <= 3.0 * best((16, 16, 12))
