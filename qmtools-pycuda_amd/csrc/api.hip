@@ -233,7 +233,7 @@ static void free_mol_device(qm_mol* m) {
   if (m->Pb16) (void)hipFree(m->Pb16);
   qm_gto_cache_free(m->gto);
   m->gto = nullptr;
-  m->atoms = nullptr; m->shells = nullptr; m->prims = nullptr;
+  m->atoms = nullptr; m->shells = nullptr; m->shells_user = nullptr; m->prims = nullptr;
   m->P64 = nullptr; m->M64 = nullptr; m->P16 = nullptr; m->Pb16 = nullptr;
 }
 
@@ -274,7 +274,7 @@ int qm_mol_create(qm_ctx* ctx, int natoms, const int* Z, const double* xyz_bohr,
     d.L = shell_L[s];
     d.nprim = shell_nprim[s];
     d.poff = shell_poff[s];
-    d.bf_user = bf;
+    d.bf = d.bf_user = bf;
     if (d.atom < 0 || d.atom >= natoms || d.L < 0 || d.L > 2 || d.nprim <= 0 || d.poff < 0 ||
         d.poff + d.nprim > nprim) {
       delete m;
@@ -287,6 +287,7 @@ int qm_mol_create(qm_ctx* ctx, int natoms, const int* Z, const double* xyz_bohr,
     bf += 2 * d.L + 1;
     m->h_shells[s] = d;
   }
+  std::vector<DevShell> both = m->h_shells;   // the caller's order, later after the internal one
   {
     const std::vector<int> order = shell_order(m->xyz, natoms, m->h_shells);
     std::vector<DevShell> sorted(nshell);
@@ -305,6 +306,7 @@ int qm_mol_create(qm_ctx* ctx, int natoms, const int* Z, const double* xyz_bohr,
     }
     m->h_shells.swap(sorted);
   }
+  both.insert(both.begin(), m->h_shells.begin(), m->h_shells.end());
   m->nbf = bf;
   m->nbf_pad = (bf + 63) / 64 * 64;
   m->h_alpha.assign(alpha, alpha + nprim);
@@ -328,7 +330,7 @@ int qm_mol_create(qm_ctx* ctx, int natoms, const int* Z, const double* xyz_bohr,
   }
 
   if (hipMalloc(&m->atoms, sizeof(double4) * natoms) != hipSuccess ||
-      hipMalloc(&m->shells, sizeof(DevShell) * nshell) != hipSuccess ||
+      hipMalloc(&m->shells, sizeof(DevShell) * both.size()) != hipSuccess ||
       hipMalloc(&m->prims, sizeof(double2) * nprim) != hipSuccess ||
       hipMalloc(&m->prims_l2e, sizeof(float2) * nprim) != hipSuccess ||
       hipMalloc(&m->kgroups, sizeof(int2) * kg.size()) != hipSuccess) {
@@ -338,7 +340,7 @@ int qm_mol_create(qm_ctx* ctx, int natoms, const int* Z, const double* xyz_bohr,
     return qm_fail(ctx, QM_ENOMEM, "molecule tables: device allocation failed");
   }
   if (hipMemcpy(m->atoms, at.data(), sizeof(double4) * natoms, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(m->shells, m->h_shells.data(), sizeof(DevShell) * nshell, hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(m->shells, both.data(), sizeof(DevShell) * both.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(m->prims, pr.data(), sizeof(double2) * nprim, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(m->prims_l2e, pr32.data(), sizeof(float2) * nprim, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(m->kgroups, kg.data(), sizeof(int2) * kg.size(), hipMemcpyHostToDevice) != hipSuccess) {
@@ -347,6 +349,7 @@ int qm_mol_create(qm_ctx* ctx, int natoms, const int* Z, const double* xyz_bohr,
     delete m;
     return qm_fail(ctx, QM_EHIP, "molecule tables: upload failed: %s", hipGetErrorString(e));
   }
+  m->shells_user = m->shells + nshell;
   *out = m;
   return QM_OK;
 }

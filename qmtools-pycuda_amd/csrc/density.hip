@@ -143,7 +143,8 @@ __device__ __forceinline__ void phi_f64_body(int blk, const MolView& m, const Ge
   } else {
     chunk_point(g, v0, nvox, nsub, t, x, y, z);
   }
-  // shells come grouped by atom: the offset to the nucleus is formed once per atom (uniform test)
+  // the offset to the nucleus is formed where the atom changes (uniform test): once per atom in the caller's order of
+  // the shells (point lists), for most shells in the internal order
   int atom = -1;
   double dx = 0, dy = 0, dz = 0, r2 = 0;
   for (int s = 0; s < m.nshell; ++s) {
@@ -164,7 +165,7 @@ __device__ __forceinline__ void phi_f64_body(int blk, const MolView& m, const Ge
         if (e < kExpCut) radial += pc.y * exp(-e);   // beyond: below 2e-22 of the coefficient
       }
     }
-    double* __restrict__ col = phi + (int64_t)(pts ? sh.bf_user : sh.bf) * ld + t;   // point lists: caller's order
+    double* __restrict__ col = phi + (int64_t)sh.bf * ld + t;
     shell_emit<double>(sh.L, dx, dy, dz, radial, [&](int c, double val) { col[(int64_t)c * ld] = val; });
   }
   for (int f = m.nbf; f < nbf_pad; ++f) phi[(int64_t)f * ld + t] = 0.0;
@@ -3143,7 +3144,8 @@ int qm_basis_points(qm_ctx* ctx, qm_mol* mol, void* stream, const double* pts, i
   QM_REQUIRE(ctx, npts > 0 && npts < ((int64_t)1 << 30), QM_ELIMIT, "basis_points: bad point count");
   // writes phi[f * npts + t] for f < nbf (ld = npts); rows beyond nbf are not stored
   const int n = (int)npts;
-  const MolView mv = mol->view();
+  MolView mv = mol->view();
+  mv.shells = mol->shells_user;
   GeomView gv{};
   gv.nx = 1; gv.ny = 1; gv.nz = 1; gv.h = 1.0;
   hipLaunchKernelGGL(k_phi_f64, dim3((n + kPhiThreads - 1) / kPhiThreads), dim3(kPhiThreads), 0,

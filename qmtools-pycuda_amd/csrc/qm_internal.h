@@ -133,6 +133,7 @@ struct qm_mol {
   int natoms = 0, nshell = 0, nprim = 0, nbf = 0, nbf_pad = 0;
   double4* atoms = nullptr;
   DevShell* shells = nullptr;
+  DevShell* shells_user = nullptr;  // the same in the caller's order, bf too (qm_basis_points); behind shells
   double2* prims = nullptr;
   float2* prims_l2e = nullptr;      // (alpha log2 e, coeff) in FP32 for the FP32 basis kernel
   int2* kgroups = nullptr;          // per 8 functions (nbf_pad / 8): shell of the first function, its m index
