@@ -921,8 +921,12 @@ __global__ __launch_bounds__(kTT) void k_tile_list(MolView m, GeomView g, BlockT
 // the contraction takes them: in grid order the last workgroups of a launch are long ones as often as not, and
 // the shader engines' shares differ.  60 atoms, 256^3: FP64 contraction 31.7 -> 27.7 ms (20 launches, 7 us of
 // sorting each), split 7.74 -> 7.47 ms (10 launches, 11.5 us).  Below kOrderMin tiles all workgroups run at
-// once; above kOrderMax (small bases) the end of the launch no longer counts and the sort would.
+// once; above kOrderMax the end of the launch no longer counts and the sort would.  Nor is it worth its time for
+// short lists: whole calls with and without sorting, 96^3 and 128^3, us: FP64, 14 functions 96 and 78, 209 and 173; 85: 276
+// and 271, 615 and 605; 123: 412 and 416, 931 and 951; split, 52 functions 120 and 104, 297 and 263; 199: 401 and 376,
+// 850 and 821; 303: 531 and 524, 1170 and 1153.
 constexpr int kOrderMin = 1024, kOrderMax = 32768;
+constexpr int kOrderGroups64 = 8, kOrderGroupsSplit = 16;
 __global__ __launch_bounds__(1024) void k_tile_order(const int* __restrict__ cnt, int nrt, int* __restrict__ order) {
   __shared__ int at[kMaxGroups + 1];
   __shared__ int sums[1024];
@@ -2719,7 +2723,7 @@ int density_blocks(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, in
     const int nTc = (int)std::min(nT, ntiles - T0);
     for (int s0 = 0; s0 < nsub3; s0 += ns) {
       const int nsc = std::min(ns, nsub3 - s0), nrt = nTc * nsc;
-      const bool sorted = nrt >= kOrderMin && nrt <= kOrderMax;
+      const bool sorted = ng >= (f64 ? kOrderGroups64 : kOrderGroupsSplit) && nrt >= kOrderMin && nrt <= kOrderMax;
       const BlockTiles b{(int)T0, nTc, nsub, ng, list, cnt, sorted ? order : nullptr, s0, nsc, shape[0], shape[1]};
       const int pblk = f64 ? (nrt + 1) / 2 : (nrt + kPhiTiles - 1) / kPhiTiles;
       const dim3 pgrid(pblk, phi_split(pblk, ng << (GS - 3)));

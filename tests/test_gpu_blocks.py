@@ -233,3 +233,25 @@ def test_thin_grids_cost_what_a_box_costs(shape):
         o = tuple(mol.coords.mean(0) - 0.5 * h * numpy.array(sh))
         return _best_ms(_density_call(mol, (*sh, h, o), 2, nat.QM_PREC_FP64))
     assert best(shape) <= 3.0 * best((16, 16, 12))
+
+
+@pytest.mark.parametrize("shape", [(128, 32, 32), (121, 65, 37)])
+@pytest.mark.parametrize("natoms,prec", [(13, "QM_PREC_FP64"), (50, "QM_PREC_FP64"), (50, "QM_PREC_F16X3")])
+def test_sorted_launches_of_larger_bases(natoms, prec, shape):
+    """1024 and 2720 tiles of 8 and more groups (FP64) or 16 and more (split), taken by list length: the bits of
+    launches of fewer than 1024 tiles, which are taken as numbered."""
+    import qmtools
+    from qmtools import _native as nat, autotune, synth
+    mol = synth.synthetic_molecule(natoms, 12, qmtools.BasisSet(BASIS))
+    assert mol.nbf > (112 if prec == "QM_PREC_FP64" else 480)
+    h = 0.25
+    o = mol.coords.mean(0) - 0.5 * h * numpy.array(shape) + 0.05
+    print("[case] sorted tiles, larger basis", natoms, mol.nbf, shape, prec, flush=True)
+    got = _raw(mol, (*shape, h, tuple(o)), 1, getattr(nat, prec))
+    old = autotune.get("phi_mib")
+    autotune.set("phi_mib", 64)   # at least 131 072 bytes a tile: at most 512 tiles
+    try:
+        want = _raw(mol, (*shape, h, tuple(o)), 1, getattr(nat, prec))
+    finally:
+        autotune.set("phi_mib", old)
+    assert numpy.isfinite(got).all() and numpy.array_equal(got, want)
