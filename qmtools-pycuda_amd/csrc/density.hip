@@ -1176,15 +1176,15 @@ __device__ __forceinline__ int block_parts(int cnt) { return SPLIT ? (cnt + 3) /
 // n values kTT apart, added in order, eight loads in flight
 __device__ __forceinline__ double add_parts(const double* __restrict__ a, int n) {
   double r = 0.0;
-  int q = 0;
-  for (; q + 8 <= n; q += 8) {
+  for (int q = 0; q < n; q += 8) {
     double v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = a[(int64_t)(q + u) * kTT];
+    for (int u = 0; u < 8; ++u)
+      if (q + u < n) v[u] = a[(int64_t)(q + u) * kTT];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) r += v[u];
+    for (int u = 0; u < 8; ++u)
+      if (q + u < n) r += v[u];
   }
-  for (; q < n; ++q) r += a[(int64_t)q * kTT];
   return r;
 }
 
