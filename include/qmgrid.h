@@ -186,8 +186,8 @@ int qm_multipole_boundary(qm_ctx* ctx, void* stream, const qm_geom* g, int dtype
  *   delta <= tolerance.  From about 32 + n / 16 sweeps on (n the longest
  *   axis, at most 1026 points) the result and the checks are computed in
  *   closed form by sine transforms: to rounding those of the sweeps, in a time
- *   that does not follow their number; the call then waits for `stream` (with
- *   a tolerance until v is final, else for the residual of v as given).
+ *   that does not follow their number; with a tolerance the call returns
+ *   once v is final.
  *   While `stream` is being captured, with a residual that is not finite or
  *   above 1e290, or a tolerance below 1e-12 sum|V|, the sweeps are run.
  *   tmp is work space; what it holds on return is not specified.

@@ -641,9 +641,10 @@ struct GraphBlock {
 };
 
 // FP64 sweeps in closed form by sine transforms (sine.hip): V_n = V + sum_{j<n} A^j (V_1 - V).  *done stays
-// false where the sweeps have to be run instead: under stream capture (the call waits for a flag), a residual
-// that is not finite somewhere (it would spread over the whole grid at once) or so large that a transform
-// might overflow, no room for the tables or the check's buffer, or a tolerance that the sweeps' rounding decides.
+// false where the sweeps have to be run instead: under stream capture, no room for the tables or the check's
+// buffer, and, with a tolerance, a residual that is not finite somewhere (it would spread over the whole grid at
+// once) or so large that a transform might overflow, or a tolerance that the sweeps' rounding decides.  Without a
+// tolerance the call only queues work, so such a residual is found on the device and its sweeps run there.
 //
 // Convergence checks: delta after n sweeps is |A^(n-1) (V_1 - V)|_1, and A (neighbour sums / 6) does not
 // increase that norm, so the first check with delta <= tol is found by bisection over the checks, in the
@@ -673,7 +674,6 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
   if (rc == QM_ENOMEM) ctx->err.clear();   // the sweeps need no tables
   if (rc) return rc == QM_ENOMEM ? QM_OK : rc;
   if ((rc = qm_sine_residual_xy(ctx, s, p, rho, v, g->step, tmp))) return rc;
-  int* bad = (int*)(ctx->host_scalars + 3);
   auto sweeps_factor = [](int kind, int64_t n) {
     SineFactor f{};
     f.sweep = SINE_JACOBI;
@@ -682,22 +682,18 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
     f.odd = (int)(n & 1);
     return f;
   };
-  QM_CHECK_HIP(ctx, hipMemcpyAsync(bad, p.flag, sizeof(int), hipMemcpyDeviceToHost, s));
   if (checks == 0) {
-    // the transforms go on in tmp while the host waits for the flag; V is only touched after that
-    hipEvent_t ev;
-    QM_CHECK_HIP(ctx, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    rc = hipEventRecord(ev, s) == hipSuccess ? qm_sine_z_scale_zy(ctx, s, p, sweeps_factor(SINE_SUM, max_sweeps), tmp)
-                                             : qm_fail(ctx, QM_EHIP, "jacobi: event record failed");
-    if (!rc && hipEventSynchronize(ev) != hipSuccess) rc = qm_fail(ctx, QM_EHIP, "jacobi: event wait failed");
-    (void)hipEventDestroy(ev);
-    if (rc || *bad) return rc;
+    // queued as a whole: V is only touched where the flag is not set, and relaxed by sweeps where it is
+    if ((rc = qm_sine_z_scale_zy(ctx, s, p, sweeps_factor(SINE_SUM, max_sweeps), tmp))) return rc;
     if ((rc = qm_sine_x_add(ctx, s, p, tmp, v))) return rc;
+    if ((rc = qm_sine_sweeps_if(ctx, s, p, g, rho, v, tmp, max_sweeps))) return rc;
     ps.weight = (int)std::min<int64_t>(max_sweeps, 1 << 30);
     *done_out = max_sweeps;
     *finished = true;
     return QM_OK;
   }
+  int* bad = (int*)(ctx->host_scalars + 3);
+  QM_CHECK_HIP(ctx, hipMemcpyAsync(bad, p.flag, sizeof(int), hipMemcpyDeviceToHost, s));
   if ((rc = qm_sine_z(ctx, s, p, tmp))) return rc;
   auto delta_at = [&](int64_t c, double* d) -> int {   // check c: after c check_every sweeps
     int r = qm_sine_scale_zy(ctx, s, p, sweeps_factor(SINE_POWER, c * check_every - 1), tmp, w);

@@ -15,6 +15,7 @@ struct SinePlan {
   double* red;              // block partials of their reduction
   double* sum;              // their sum
   int* flag;                // set when a residual is not finite or near the end of the range
+  unsigned long long* ctl;  // of qm_sine_sweeps_if: workgroups so far, arrivals at its barriers, workgroups that take part
 };
 
 enum { SINE_JACOBI = 0, SINE_VNE = 1 };     // which sweep's eigenvalue a
@@ -51,7 +52,7 @@ struct SineUse {
 };
 
 bool qm_sine_fits(const qm_geom* g);   // every axis has 1 .. 1024 interior points
-// tables in the context's workspace, valid on s until the next plan; clears the flag
+// tables in the context's workspace, valid on s until the next plan; clears the flag and ctl
 int qm_sine_plan(qm_ctx* ctx, hipStream_t s, const qm_geom* g, SinePlan* p);
 // The passes read and write interior points only and work in place where one buffer is given.
 // x and y transforms of (one Jacobi sweep of v) - v; sets the plan's flag if that is not finite, or 1e290 and more, somewhere
@@ -65,7 +66,10 @@ int qm_sine_z_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const Sine
 int qm_sine_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const SineFactor& f, const double* spectrum,
                      double* out);
 int qm_sine_x(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* a);
-int qm_sine_x_add(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, double* v);   // v += x transform of a
+int qm_sine_x_add(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, double* v);   // v += x transform of a, unless the flag is set
+// `sweeps` Jacobi sweeps of v (tmp: work space) if the flag is set, else nothing
+int qm_sine_sweeps_if(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const qm_geom* g, const double* rho, double* v,
+                      double* tmp, int64_t sweeps);
 // sum over the interior of |x transform of a| (v null) or |v + x transform of a|, on the device; qm_sine_sum waits for s
 // and returns it
 int qm_sine_x_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, const double* v);

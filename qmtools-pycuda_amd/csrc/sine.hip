@@ -90,6 +90,7 @@ __global__ __launch_bounds__(kThreads) void k_sine(Args a) {
   __shared__ int64_t base[16 * LT];   // first interior point of each line
   __shared__ int2 mode[16 * LT];      // its indices along the two other axes
   const SinePlan& p = a.p;
+  if (STORE == STORE_ADD && *p.flag) return;   // left to qm_sine_sweeps_if
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int li = lane & 15, lk = lane >> 4;
@@ -272,7 +273,10 @@ __global__ __launch_bounds__(256) void k_sine_tables(SinePlan p) {
   const int ax = blockIdx.y, m = p.m[ax], ld = p.ld[ax];
   const int half = (m + 1) / 2, rows = (half + 3) / 4 * 4;
   double* __restrict__ s2 = const_cast<double*>(p.s2[ax]);
-  if (ax == 0 && blockIdx.x == 0 && threadIdx.x == 0) *p.flag = 0;
+  if (ax == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
+    *p.flag = 0;
+    p.ctl[0] = p.ctl[1] = p.ctl[2] = 0;
+  }
   const double scale = sqrt(2.0 / (m + 1));
   for (int i = blockIdx.x * 256 + threadIdx.x; i < 2 * rows * ld; i += gridDim.x * 256) {
     const int odd = i >= rows * ld, q = i - odd * rows * ld;
@@ -285,6 +289,80 @@ __global__ __launch_bounds__(256) void k_sine_tables(SinePlan p) {
     const double h = sinpi((double)(i + 1) / (2 * (m + 1)));
     s2[i] = h * h;
   }
+}
+
+// The sweeps of a relaxation whose residual is left to them, in one launch behind the closed form, so that the host
+// need not wait for the flag: without it the workgroups return at once (3 us; a wait for the flag held the caller
+// for all earlier work of the stream).  A sweep is followed by a barrier of the workgroups that take part.  These are
+// the ones that run when the first of them closes the count; a workgroup that starts later returns, so a barrier only
+// waits for workgroups that are running and every wait ends, whatever else the GPU runs.  The arithmetic of a
+// point is that of the sweep kernels.
+constexpr unsigned long long kClosed = 1ull << 32;
+__global__ __launch_bounds__(kThreads) void k_sweeps_if(const int* flag, unsigned long long* ctl, const double* rho,
+                                                        double* v, double* tmp, int nx, int ny, int nz, double hinv,
+                                                        int64_t sweeps) {
+  if (*flag == 0) return;
+  __shared__ unsigned long long in;   // this workgroup's number and, once closed, the count
+  if (threadIdx.x == 0) {
+    unsigned long long at = __hip_atomic_fetch_add(&ctl[0], 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (at == 0) {   // the first one gives the others some time
+      for (int i = 0; i < 4096; ++i) {
+        if (__hip_atomic_load(&ctl[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x) break;
+        __builtin_amdgcn_s_sleep(8);
+      }
+      const unsigned long long n = __hip_atomic_fetch_or(&ctl[0], kClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // the count at closing, for the others (ctl[0] may grow by late ones)
+      __hip_atomic_store(&ctl[2], n, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    in = at;
+  }
+  __syncthreads();
+  const unsigned long long me = in;
+  if (me & kClosed) return;   // late
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long n;
+    while ((n = __hip_atomic_load(&ctl[2], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT)) == 0) __builtin_amdgcn_s_sleep(8);
+    in = n;
+  }
+  __syncthreads();
+  const int64_t count = (int64_t)in;
+  const int64_t sz = (int64_t)nx * ny, n = sz * nz;
+  const int64_t lo = n * (int64_t)me / count, hi = n * ((int64_t)me + 1) / count;
+  unsigned long long target = 0;
+  auto barrier = [&]() {
+    target += count;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");   // every wave's own stores, before thread 0 arrives
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      __hip_atomic_fetch_add(&ctl[1], 1ull, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+      while (__hip_atomic_load(&ctl[1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < target) __builtin_amdgcn_s_sleep(1);
+    }
+    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  };
+  double *src = v, *dst = tmp;
+  for (int64_t q = 0; q < sweeps; ++q) {
+    for (int64_t e = lo + threadIdx.x; e < hi; e += kThreads) {
+      const int i = (int)(e % nx), j = (int)(e / nx % ny), k = (int)(e / sz);
+      double r = src[e];
+      if (i > 0 && i < nx - 1 && j > 0 && j < ny - 1 && k > 0 && k < nz - 1) {
+        double s = src[e - 1] + src[e + 1];
+        s += src[e + nx];
+        s += src[e - nx];
+        s += src[e + sz];
+        s += src[e - sz];
+        r = fma(-rho[e], hinv, s) * (1.0 / 6.0);
+      }
+      dst[e] = r;
+    }
+    barrier();
+    double* t = src;
+    src = dst;
+    dst = t;
+  }
+  if (src != v)
+    for (int64_t e = lo + threadIdx.x; e < hi; e += kThreads) v[e] = src[e];
 }
 
 template <int LT, int RT, int AX, int LOAD, bool MID, int STORE>
@@ -345,7 +423,10 @@ int qm_sine_first_below(int64_t n, double dn, double tol, const std::function<in
 }
 
 int SineUse::begin() {
-  if (!ctx->sine_done) QM_CHECK_HIP(ctx, hipEventCreateWithFlags(&ctx->sine_done, hipEventDisableTiming));
+  // orders streams of this device only: without fences to the host and other devices 200 sweeps of 64^3 take 51.5
+  // instead of 57 us
+  if (!ctx->sine_done)
+    QM_CHECK_HIP(ctx, hipEventCreateWithFlags(&ctx->sine_done, hipEventDisableTiming | hipEventDisableSystemFence));
   if (ctx->sine_pending) QM_CHECK_HIP(ctx, hipStreamWaitEvent(s, ctx->sine_done, 0));
   held = true;
   return QM_OK;
@@ -375,7 +456,7 @@ int qm_sine_plan(qm_ctx* ctx, hipStream_t s, const qm_geom* g, SinePlan* p) {
   // partial sums of an x pass, their reduction's, its result, then the flag
   const size_t nparts = ((size_t)p->m[1] * p->m[2] + 15) / 16;
   double* w = nullptr;
-  int rc = qm_ws(ctx, s, WS_SINE, sizeof(double) * (doubles + nparts + kRedMaxBlocks + 4), (void**)&w);
+  int rc = qm_ws(ctx, s, WS_SINE, sizeof(double) * (doubles + nparts + kRedMaxBlocks + 8), (void**)&w);
   if (rc) return rc;
   for (int d = 0; d < 3; ++d) {
     p->S[d] = w + off[d];
@@ -386,6 +467,7 @@ int qm_sine_plan(qm_ctx* ctx, hipStream_t s, const qm_geom* g, SinePlan* p) {
   p->red = p->part + nparts;
   p->sum = p->red + kRedMaxBlocks;
   p->flag = (int*)(p->sum + 1);
+  p->ctl = (unsigned long long*)(p->sum + 2);
   hipLaunchKernelGGL(k_sine_tables, dim3((unsigned)std::min<size_t>(512, (most + 255) / 256), 3), dim3(256), 0, s, *p);
   QM_CHECK_LAUNCH(ctx);
   return QM_OK;
@@ -434,6 +516,14 @@ int qm_sine_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const SineFa
 
 int qm_sine_x_add(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, double* v) {
   return pass<0, LOAD_PLAIN, false, STORE_ADD>(ctx, s, plain_args(p, a, v));
+}
+
+int qm_sine_sweeps_if(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const qm_geom* g, const double* rho, double* v,
+                      double* tmp, int64_t sweeps) {
+  hipLaunchKernelGGL(k_sweeps_if, dim3((unsigned)ctx->ncu), dim3(kThreads), 0, s, (const int*)p.flag, p.ctl, rho, v, tmp,
+                     g->nx, g->ny, g->nz, 1.0 / g->step, sweeps);
+  QM_CHECK_LAUNCH(ctx);
+  return QM_OK;
 }
 
 int qm_sine_x_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, const double* v) {

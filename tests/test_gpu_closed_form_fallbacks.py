@@ -173,3 +173,32 @@ def test_profile_counts_the_sweeps_that_were_done(tol, decided):
         assert n.value == done
     finally:
         nat.destroy_context(ctx)
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 3), (12, 10, 9), (70, 33, 20)])
+@pytest.mark.parametrize("where", ["rho nan", "rho inf", "v inside", "v outside", "huge"])
+@pytest.mark.parametrize("sweeps", [45, 80])
+def test_residuals_left_to_the_sweeps(shape, where, sweeps):
+    """Charges or values that are not finite, or too large for the transforms: the sweeps' bits, odd and even counts."""
+    from qmtools import _native as nat
+    rho, v0 = _state(shape, 8)
+    nx, ny, nz = shape
+    at = nx // 2 + nx * (ny // 2 + ny * (nz // 2))
+    if where == "rho nan":
+        rho[at] = float("nan")
+    elif where == "rho inf":
+        rho[at] = float("inf")
+        rho[1 + nx * (1 + ny)] = float("-inf")
+    elif where == "v inside":
+        v0[at] = float("nan")
+    elif where == "v outside":
+        v0[nx // 2 + nx * (ny // 2)] = float("inf")
+    else:
+        rho[at] = 1e300
+    want, got = v0.clone(), v0.clone()
+    for q in range(0, sweeps, 20):
+        _jacobi(shape, rho, want, min(20, sweeps - q))
+    print("[case] left to the sweeps", shape, where, sweeps, flush=True)
+    rc, done, _ = _jacobi(shape, rho, got, sweeps)
+    assert rc == nat.QM_OK and done == sweeps
+    numpy.testing.assert_array_equal(got.cpu().numpy(), want.cpu().numpy())

@@ -118,3 +118,32 @@ def test_calls_on_two_streams_of_one_context(other):
         torch.cuda.synchronize()
         assert numpy.array_equal(va.cpu().numpy(), want[0])
         assert numpy.array_equal(vb.cpu().numpy(), want[1])
+
+
+def test_a_fixed_count_does_not_wait_for_the_stream():
+    """Without a tolerance the call returns with its work queued: what ran on the stream before is still running."""
+    import torch
+    shape = (96, 80, 72)
+    rho = _charge(shape, 5)
+    v, tmp = torch.zeros_like(rho), torch.empty_like(rho)
+    s = torch.cuda.Stream()
+    a = torch.randn(8192, 8192, device="cuda")
+    b = torch.empty_like(a)
+    print("[case] fixed count, stream busy at return", flush=True)
+    with torch.cuda.stream(s):
+        torch.mm(a, a, out=b)
+        _jacobi(s, shape, rho, v, tmp, 500)   # workspaces and tables exist from here on
+        torch.cuda.synchronize()
+        v.zero_()
+        for _ in range(40):
+            torch.mm(a, a, out=b)
+        busy = torch.cuda.Event()
+        busy.record(s)
+        _jacobi(s, shape, rho, v, tmp, 500)
+        waited = busy.query()
+    torch.cuda.synchronize()
+    assert not waited
+    want = torch.zeros_like(rho)
+    _jacobi(torch.cuda.current_stream(), shape, rho, want, tmp, 500)
+    torch.cuda.synchronize()
+    assert numpy.array_equal(v.cpu().numpy(), want.cpu().numpy())
