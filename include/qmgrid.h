@@ -212,7 +212,9 @@ int qm_jacobi(qm_ctx* ctx, void* stream, const qm_geom* g, int precision, const 
  * mode QM_FFT_PERIODIC: V^ = rhs^ * (-1/(4 pi^2 |k|^2)), V^(0) = 0 (reference semantics);
  * mode QM_FFT_FREESPACE: convolution with 1/(4 pi eps0 r) on a 2x zero-padded grid.
  * q: electrons per voxel, x-fastest (dtype); out: V in volts, C order [i][j][k] (dtype).
- * precision QM_PREC_FP64 (complex128) or QM_PREC_FP32 (complex64).
+ * precision QM_PREC_FP64 (complex128) or QM_PREC_FP32 (complex64).  Transform lengths (the axes, in free space
+ * padded to at least twice as long) of up to 4096 points in complex64, and in complex128 of 3855, or 2560 with a
+ * prime factor above 7; longer ones return QM_ELIMIT.
  * Replaces gpu_add_nuclear_charge + gpu_poisson_frequency_solve (kernel_fft.cu:23-106),
  * the cuFFT plans and QMTools.Compute_hartree_fft (qmtools.py:2578-2639). */
 int qm_hartree_fft(qm_ctx* ctx, qm_mol* mol, void* stream, const qm_geom* g, int precision,

@@ -879,7 +879,10 @@ int fft_pass(qm_ctx* ctx, hipStream_t s, Cx<R>* data, const R* rin, TO* rout, in
   // B lines of n points per workgroup: B * n <= kMax (the register bound of a stage), whole cache lines
   // of adjacent lines where that allows it
   const int kMaxPts = pow2 ? FftPts<R, true>::kMax : FftPts<R, false>::kMax;
-  QM_REQUIRE(ctx, n <= 4096, QM_ELIMIT, "fft: length %d exceeds 4096", n);
+  // complex128: LDS would hold slightly longer lines than these, which callers have been refused
+  const bool smooth = std::all_of(f.begin(), f.end(), [](int r) { return r <= 10; });
+  const int limit = sizeof(R) == 4 ? 4096 : smooth ? 3855 : 2560;
+  QM_REQUIRE(ctx, n <= limit, QM_ELIMIT, "fft: length %d exceeds %d", n, limit);
   int B = std::max(1, std::min(16, kMaxPts / n));
   if (!radix) B = std::max(1, std::min(B, 2048 / n));
   if (axis != 2 && B > 8) B = B / 8 * 8;

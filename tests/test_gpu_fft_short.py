@@ -67,3 +67,23 @@ def test_eight_points_cost_no_more_than_sixteen():
         return t
     print("[case] fft short axes, time", flush=True)
     assert best(8) <= 1.5 * best(16)
+
+
+@pytest.mark.parametrize("n,prec,ok", [(2560, "FP64", True), (2558, "FP64", True), (2561, "FP64", False),
+                                       (2564, "FP64", False), (2638, "FP64", False), (3840, "FP64", True),
+                                       (3888, "FP64", False), (3969, "FP64", False), (4096, "FP64", False),
+                                       (2564, "FP32", True), (3969, "FP32", True), (4096, "FP32", True)])
+def test_length_limits(n, prec, ok):
+    """Lengths beyond the documented limits are refused, whatever the axis."""
+    from qmtools import _native as nat
+    for axis in range(3):
+        shape = [2, 2, 2]
+        shape[axis] = n
+        print("[case] fft length", shape, prec, flush=True)
+        run = _call(tuple(shape), numpy.full(4 * n, 0.01), getattr(nat, "QM_PREC_" + prec), nat.QM_FFT_PERIODIC)[4]
+        if ok:
+            run()
+        else:
+            with pytest.raises(nat.QMError) as e:
+                run()
+            assert e.value.code == nat.QM_ELIMIT
