@@ -205,7 +205,7 @@ __device__ __forceinline__ void phi_f32_body(int blk, const MolView& m, const fl
   // offsets to the nucleus are formed in FP64 and rounded once: rounding x and R
   // separately to FP32 costs ~1e-6 bohr, i.e. ~1e-4 relative error in tight primitives
   float vmax = 0.f;
-  int atom = -1;   // shells come grouped by atom: offsets once per atom
+  int atom = -1;   // offsets where the atom changes: for most shells, which are sorted by cutoff
   float dx = 0.f, dy = 0.f, dz = 0.f, r2 = 0.f;
   for (int s = 0; s < m.nshell; ++s) {
     const DevShell sh = m.shells[s];
@@ -298,7 +298,7 @@ __device__ __forceinline__ void phi_split_body(int blk, const MolView& m, const 
     }
     ++f;
   };
-  int atom = -1;   // shells come grouped by atom: offsets once per atom
+  int atom = -1;   // offsets where the atom changes: for most shells, which are sorted by cutoff
   float dx = 0.f, dy = 0.f, dz = 0.f, r2 = 0.f;
   for (int s = 0; s < m.nshell; ++s) {
     const DevShell sh = m.shells[s];
@@ -628,9 +628,9 @@ constexpr int kTT = 128, kTKS = 16, kTPad = 8, kTWG = 512;
 // Workgroup b goes to XCD b mod 8 and there, whatever the load, to one of 4 shader engines in turn: with
 // slot = b / 8, slot mod 4 decides.  An even number of column blocks per tile would send the same blocks,
 // whose lengths differ, to the same engines, so their order is turned with the tile.  60 atoms, 256^3, tiles
-// sorted by length: FP64 35.5 ms with one workgroup per tile, 44.2 with two and 66.6 with four in fixed order,
-// 36.0 and 36.7 turned; split 14.3 and 18.0, turned 13.4 and 13.7.  Odd numbers turn by themselves (turned
-// as well: FP64 with three 36.4 -> 40.1).
+// sorted by length, two and four workgroups per tile: FP64 44.2 and 66.6 ms in fixed order, 36.0 and 36.7 turned;
+// split 14.3 and 18.0, turned 13.4 and 13.7.  Odd numbers turn by themselves (turned as well: FP64 with three 36.4 ->
+// 40.1).
 __device__ __forceinline__ bool tile_coords(int b, int nrt, int ncb, int& rt, int& cb) {
   const int xcd = b & 7, slot = b >> 3;
   const int rl = slot / ncb;
@@ -799,7 +799,8 @@ __device__ __forceinline__ void tiled_f64_body(int rt, int cb, const double* __r
 // whole basis.  What is left out are exact zeros (the basis-value kernels write 0 beyond a shell's
 // cutoff), so the sums are the same bit for bit with every group listed (QM_TUNE_TILE_SKIP = 0).
 // On 60 atoms in a 28 bohr box 45% of the FP64 groups (52% of the split ones) are active and 26% (33%) of the
-// triangle is left.  60 atoms at 256^3, density call: FP64 110 -> 43 ms, split 25.3 -> 16.7 ms.
+// triangle is left.  60 atoms at 256^3, density call, x-line tiles -> these with what follows (sorted tiles, two points per
+// lane): FP64 110 -> 36 ms, split 25.3 -> 13.5 ms.
 constexpr int kMaxGroups = 2048;   // groups per tile that a workgroup can list in LDS
 
 struct BlockTiles {
@@ -1775,12 +1776,12 @@ __global__ __launch_bounds__(512, 4) void k_contract_split_blocks(const T16* __r
 // table read during the stages is an LDS read.
 // LDS: 32 KB basis values + 80 KB M + 4 KB row-dot + up to 40 KB of tables.
 //
-// Measured on the 60-atom, 256^3 workload: 68 ms per grid against 27 ms for
-// basis values written to memory plus the DMA tiles (variant 3).  The single
+// Measured on the 60-atom, 256^3 workload: 54 ms per grid (68 before the shells
+// were sorted by cutoff) against 13.5 ms for variant 3.  The single
 // producer wave per SIMD is the bound: its evaluation (LDS table reads in a
 // dependent chain per shell, FP64 offsets, per-slot selection of the harmonic)
 // takes about 3 us per stage, against well under 1 us of MFMAs; with the
-// evaluation switched off the kernel takes 24 ms.  Kept as a variant (no
+// evaluation switched off the kernel took 24 ms.  Kept as a variant (no
 // basis-value buffer at all) and timed by the autotuner.
 constexpr int kFP = 128;          // points per workgroup
 constexpr int kFCT = 20;          // 16-column tiles per column group
@@ -2672,7 +2673,9 @@ float split_phi_scale(const qm_mol* m);
 // Larger ones: two, side by side on one XCD, so that the blocks of a tile share its basis values in L2, or one
 // per block where the tiles are few.  606 functions, 1 / 2 / 3 / 5 workgroups: FP64, 512 tiles 335 / 307 / 292 /
 // 261 us, 2048 tiles 1126 / 803 / 779 / 783 us, 6912 tiles 2.33 / 2.22 / 2.25 / 2.27 ms; split, 512 tiles 140 /
-// 142 / 132 / 125 us, 2048 tiles 351 / 343 / 343 / 345 us, 6912 tiles 0.93 / 0.84 / 0.84 / 1.44 ms.
+// 142 / 132 / 125 us, 2048 tiles 351 / 343 / 343 / 345 us, 6912 tiles 0.93 / 0.84 / 0.84 / 1.44 ms.  Whole calls of 10
+// (split) and 20 launches of about 6550 tiles, 1 / 2 / 3 / 4 / 5: FP64 36.1 / 36.8 / 37.1 / 37.5 / 37.8 ms, split 13.8 / 13.5 /
+// 13.6 / 13.7 / 13.8 ms: between one and two, FP64 goes either way by 2 to 5 %, so both precisions take two.
 inline int block_split(int nrt, int ncb, bool f64) {
   if (ncb <= 2) return nrt >= 512 ? 1 : ncb;
   return nrt >= (f64 ? 4096 : 1024) ? 2 : ncb;

@@ -317,7 +317,7 @@ inline int pick_zs2(int nx, int ny, int nz, int fixed) {
 // lane, loads two planes ahead) waited for one plane after the other: us per sweep on n^3, strips of two sweeps
 // -> tiles of two (RZ 10), of three (RZ 12): 32: 4.1 -> 2.0, 1.5; 64: 4.3 -> 2.0, 1.6; 96: 5.1 -> 2.5, 2.5; 128:
 // 6.7 -> 3.9, 3.7; 160: 11.6 -> 6.0, 6.3; 192: 13.1 -> 9.0, 10.1; 256: 26.2 -> 22.4, 22.0 (201 MB a pass: 41 us
-// of copying).  32 rows, 64 columns or other heights are slower on most of these.
+// of copying; whole relaxations there gain less, 29 -> 27.5 us a sweep with their residual and correction).  32 rows, 64 columns or other heights are slower on most of these.
 constexpr int kTileX = 32, kTileRows = 16;
 template <int T>
 struct Tile {

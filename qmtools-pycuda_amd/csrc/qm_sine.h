@@ -78,9 +78,10 @@ int qm_sine_sum(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* host_sum)
 // bisection in the logarithm of delta.
 int qm_sine_first_below(int64_t n, double dn, double tol, const std::function<int(int64_t, double*)>& delta_at,
                         int64_t* at, double* delta);
-// Sweep counts from which a closed form is taken: it costs what 15 sweeps do at 256^3 (0.92 ms against 64 us a
-// sweep; its 6 n flops a point grow with the axis, a sweep's 24 bytes do not) and about 20 on small grids
-// (eight launches against one replayed node a sweep).
+// Sweep counts from which a closed form is taken.  It costs what 5 to 11 sweeps do (us, closed form and one sweep: 16^3 31
+// and 7.0, 64^3 52 and 9.0, 128^3 114 and 12.3, 256^3 850 and 83; its 6 n flops a point grow with the axis, a sweep's
+// 24 bytes do not).  The line lies well above that crossing: short counts keep the bits of the sweeps, so that calls
+// of up to 32 sweeps, one after the other, add up to the bits of the loop.
 inline int64_t qm_sine_sweeps(const qm_geom* g) {
   const int n = g->nx > g->ny ? g->nx : g->ny;
   return 32 + (n > g->nz ? n : g->nz) / 16;

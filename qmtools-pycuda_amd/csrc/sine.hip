@@ -35,7 +35,7 @@ namespace {
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 512;
-constexpr int kMaxM = 1024;       // interior points per axis (139 KB of LDS)
+constexpr int kMaxM = 1024;       // interior points per axis (131 KB of LDS)
 // Residuals from here on, and those that are not finite, are left to the sweeps.  A transform grows values by at most
 // m sqrt(2 / (m + 1)) < 46 an axis and the factor is below 1 / (1 - a) < 2.2e5, so six transforms stay below 2.1e15
 // times the residual, 2.1e305; sweeps reach the end of the range only where the field itself does.
@@ -372,7 +372,7 @@ void launch(hipStream_t s, const Args& a) {
                      dim3(kThreads), 0, s, a);
 }
 
-// 32 lines per workgroup (34 or 68 KB of LDS, two workgroups per CU) up to 256 points, 16 beyond
+// 32 lines per workgroup (33 or 66 KB of LDS, two workgroups per CU) up to 256 points, 16 beyond
 template <int AX, int LOAD, bool MID, int STORE>
 int pass(qm_ctx* ctx, hipStream_t s, const Args& a) {
   const int m = a.p.m[AX];
