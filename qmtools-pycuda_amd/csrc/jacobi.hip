@@ -711,14 +711,14 @@ int jacobi_closed_form(qm_ctx* ctx, hipStream_t s, const qm_geom* g, const doubl
     at *= check_every;
   }
   if ((rc = qm_sine_scale_zy(ctx, s, p, sweeps_factor(SINE_SUM, at), tmp, w))) return rc;
+  // one wait for the sum and the last pass, which leaves v alone where the sum leaves the tolerance undecided: with a
+  // tolerance the call returns once v is final, as the loop does
   double total = 0.0;
-  if ((rc = qm_sine_x_sum(ctx, s, p, w, v)) || (rc = qm_sine_sum(ctx, s, p, &total))) return rc;
-  const double floor = 1e-12 * total;
-  if (!(floor < INFINITY) || (tol < floor && delta < floor)) return QM_OK;
-  if ((rc = qm_sine_x_add(ctx, s, p, w, v))) return rc;
-  // with a tolerance the call returns once v is final, as the loop does
-  QM_CHECK_HIP(ctx, hipStreamSynchronize(s));
+  if ((rc = qm_sine_x_sum(ctx, s, p, w, v)) || (rc = qm_sine_x_add_decided(ctx, s, p, w, v, tol, delta)) ||
+      (rc = qm_sine_sum(ctx, s, p, &total)))
+    return rc;
   use.waited();
+  if (sine_undecided(total, tol, delta)) return QM_OK;
   ps.weight = (int)std::min<int64_t>(at, 1 << 30);
   *done_out = at;
   *delta_out = delta;

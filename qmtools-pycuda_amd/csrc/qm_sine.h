@@ -28,6 +28,13 @@ struct SineFactor {
   double w0, w1, w2, w3;    // SINE_VNE: 1 - a = w0 + w1 sum (1 - c) + w2 sum (1 - c c') + w3 (1 - c c' c''), c = cos theta
 };
 
+// A tolerance below 1e-12 of the field's size is decided by the rounding of the sweeps, about 1e-16 of it: total is
+// sum |V| (per point where delta is), delta the change that the closed form found.
+__host__ __device__ inline bool sine_undecided(double total, double tol, double delta) {
+  const double floor = 1e-12 * total;
+  return !(floor < INFINITY) || (tol < floor && delta < floor);
+}
+
 // Held by a closed form from before its plan to its last launch.  The sweeps work in the caller's buffers
 // alone, so calls on several streams of one context may be in flight together; the closed forms share the
 // context's tables and work grid, and are ordered one after the other by an event.  (Nothing else uses these
@@ -67,6 +74,9 @@ int qm_sine_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const SineFa
                      double* out);
 int qm_sine_x(qm_ctx* ctx, hipStream_t s, const SinePlan& p, double* a);
 int qm_sine_x_add(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, double* v);   // v += x transform of a, unless the flag is set
+// the same, unless sine_undecided(sum, tol, delta) with the sum of the last qm_sine_x_sum
+int qm_sine_x_add_decided(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, double* v, double tol,
+                          double delta);
 // `sweeps` Jacobi sweeps of v (tmp: work space) if the flag is set, else nothing
 int qm_sine_sweeps_if(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const qm_geom* g, const double* rho, double* v,
                       double* tmp, int64_t sweeps);

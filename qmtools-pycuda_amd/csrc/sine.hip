@@ -52,6 +52,8 @@ struct Args {
   double hinv;
   SineFactor f;
   double* part;             // STORE_SUM: sum |x|, STORE_SUMV: sum |out + x|, one per workgroup
+  const double* gate;       // STORE_ADD: nothing is added if sine_undecided(*gate, tol, delta)
+  double tol, delta;
 };
 
 // q = 1 - a and c = 1 + a of the sweep's eigenvalue a at mode (kx, ky, kz) (0-based), from sin^2 of the half
@@ -90,7 +92,8 @@ __global__ __launch_bounds__(kThreads) void k_sine(Args a) {
   __shared__ int64_t base[16 * LT];   // first interior point of each line
   __shared__ int2 mode[16 * LT];      // its indices along the two other axes
   const SinePlan& p = a.p;
-  if (STORE == STORE_ADD && *p.flag) return;   // left to qm_sine_sweeps_if
+  // left to qm_sine_sweeps_if or to the caller
+  if (STORE == STORE_ADD && (*p.flag || (a.gate && sine_undecided(*a.gate, a.tol, a.delta)))) return;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int li = lane & 15, lk = lane >> 4;
@@ -516,6 +519,15 @@ int qm_sine_scale_zy(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const SineFa
 
 int qm_sine_x_add(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, double* v) {
   return pass<0, LOAD_PLAIN, false, STORE_ADD>(ctx, s, plain_args(p, a, v));
+}
+
+int qm_sine_x_add_decided(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const double* a, double* v, double tol,
+                          double delta) {
+  Args r = plain_args(p, a, v);
+  r.gate = p.sum;
+  r.tol = tol;
+  r.delta = delta;
+  return pass<0, LOAD_PLAIN, false, STORE_ADD>(ctx, s, r);
 }
 
 int qm_sine_sweeps_if(qm_ctx* ctx, hipStream_t s, const SinePlan& p, const qm_geom* g, const double* rho, double* v,

@@ -371,8 +371,7 @@ int vne_closed_form(qm_ctx* ctx, qm_mol* mol, hipStream_t s, const qm_geom* g, d
   // one wait for the sum and the last pass (the loop would clear v): the call returns once v is final, as the loop does
   if ((rc = qm_sine_sum(ctx, s, p, &total))) return rc;
   use.waited();
-  const double floor = 1e-12 * total / n;
-  if (!(floor < INFINITY) || !(d < INFINITY) || (tol < floor && d < floor)) return QM_OK;
+  if (!(d < INFINITY) || sine_undecided(total / n, tol, d)) return QM_OK;
   ps.weight = (int)std::min<int64_t>(at, 1 << 30);
   *pairs = at;
   *delta = d;
